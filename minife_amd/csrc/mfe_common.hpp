@@ -141,6 +141,10 @@ struct mfe_csr {
   // per (block, plane, slot) the base and the power of two of the offsets,
   // side by side (boxpack_kq[2 * group], boxpack_kq[2 * group + 1]).
   bool boxpack_valid = false, boxpack32_valid = false;
+  // Per field width (mfe_pack.hpp's kPackWidths), the upper slots (and the FP64
+  // boundary stream's lower slots) whose every group fits it, found while the
+  // layout is built.
+  unsigned boxpack_fits[6] = {}, boxpack32_fits[6] = {}, boxwpack_fits[6] = {};
   int boxpack_form = 0, boxpack32_form = 0;
   int boxpack_cap = 0, boxpack32_cap = 0;
   unsigned *boxpack_pw = nullptr, *boxpack32_pw = nullptr;

@@ -810,84 +810,6 @@ __host__ __device__ inline unsigned box_mask(int ix, int iy, int iz, int gx, int
 }
 __device__ inline int slot_rank(unsigned mask, int s) { return __popc(mask & ((1u << s) - 1u)); }
 
-// One workgroup per (block, plane), thread t's node: its 14 upper slots into
-// U and its lower slots whose neighbour lies outside the block into W (entry
-// inv[t * 13 + s]); 0 where the slot is out of range or the node past the
-// box's edge, so every entry is written.  The block-plane's CSR rows are
-// staged in LDS first (each of its 16 grid lines' rows is one contiguous run
-// of values: coalesced loads instead of one 216-byte-strided row per
-// thread).  With CHECK, also the symmetry check of the pairs the layout takes from LDS: every lower slot
-// whose neighbour lies in the same 16 x 16 block -- against the neighbour's
-// entry in LDS (same plane) or in A's values (the plane below).  Pairs that
-// cross the block's edge are read from W, the row's own values, and need no
-// check.  A mismatch stores 1 into bad[0].
-constexpr int kSymStage = 27 * kBlock;  // values of a block-plane's rows
-template <typename Tout, bool CHECK>
-__global__ __launch_bounds__(kBlock) void boxsym_fill_staged_kernel(
-    BoxGeom g, const int* __restrict__ ro, const double* __restrict__ vals,
-    const int* __restrict__ inv, Tout* __restrict__ U, Tout* __restrict__ W, unsigned* bad) {
-  __shared__ double sv[kSymStage];
-  __shared__ int lbase[kBoxBY + 1];  // LDS position of each line's first value
-  __shared__ int lfirst[kBoxBY];     // ro[] of each line's first row
-  const int blk = (int)(blockIdx.x / (unsigned)g.gz), z = (int)(blockIdx.x % (unsigned)g.gz);
-  const int bx = blk % g.nbx, by = blk / g.nbx;
-  const int t = (int)threadIdx.x, tx = t % kBoxBX, ty = t / kBoxBX;
-  const int nxl = min(kBoxBX, g.gx - bx * kBoxBX);  // live nodes per line
-  if (t < kBoxBY) {
-    const int iy = by * kBoxBY + t;
-    int cnt = 0, first = 0;
-    if (iy < g.gy) {
-      const int64_t r0 = ((int64_t)z * g.gy + iy) * g.gx + bx * kBoxBX;
-      first = ro[r0];
-      cnt = ro[r0 + nxl] - first;
-    }
-    lfirst[t] = first;
-    lbase[t + 1] = cnt;
-  }
-  __syncthreads();
-  if (t == 0) {
-    lbase[0] = 0;
-    for (int l = 0; l < kBoxBY; ++l) lbase[l + 1] += lbase[l];
-  }
-  __syncthreads();
-  for (int l = 0; l < kBoxBY; ++l) {
-    const int cnt = lbase[l + 1] - lbase[l];
-    for (int i = t; i < cnt; i += kBlock) sv[lbase[l] + i] = vals[(int64_t)lfirst[l] + i];
-  }
-  __syncthreads();
-  const int ix = bx * kBoxBX + tx, iy = by * kBoxBY + ty;
-  const bool live = ix < g.gx && iy < g.gy;
-  const int64_t row = ((int64_t)z * g.gy + iy) * g.gx + ix;
-  const unsigned m = live ? box_mask(ix, iy, z, g.gx, g.gy, g.gz) : 0u;
-  const double* rv = sv + (live ? lbase[ty] + (ro[row] - lfirst[ty]) : 0);
-#pragma unroll
-  for (int u = 0; u < kSymU; ++u) {
-    const int s = 13 + u;
-    U[sym_at(g, blk, z, u, t)] = ((m >> s) & 1u) ? (Tout)rv[slot_rank(m, s)] : Tout(0);
-  }
-  const int64_t wbase = ((int64_t)blk * g.gz + z) * kSymNB;
-  bool ok = true;
-  for (int s = 0; s < 13; ++s) {
-    const int e = inv[t * 13 + s];
-    const bool in = (m >> s) & 1u;
-    if (e >= 0) {
-      W[wbase + e] = in ? (Tout)rv[slot_rank(m, s)] : Tout(0);
-      continue;
-    }
-    if (!CHECK || !in) continue;
-    // in-block neighbour: its mirrored entry must hold the same bits
-    const int sz = s / 9 - 1, sy = (s / 3) % 3 - 1, sx = s % 3 - 1;
-    const int cx = ix + sx, cy = iy + sy, cz = z + sz;
-    const unsigned mc = box_mask(cx, cy, cz, g.gx, g.gy, g.gz);
-    const int64_t c = cx + (int64_t)g.gx * (cy + (int64_t)g.gy * cz);
-    double vc;
-    if (sz == 0) vc = sv[lbase[ty + sy] + (ro[c] - lfirst[ty + sy]) + slot_rank(mc, 26 - s)];
-    else vc = vals[ro[c] + slot_rank(mc, 26 - s)];
-    ok = ok && __double_as_longlong(vc) == __double_as_longlong(rv[slot_rank(m, s)]);
-  }
-  if (CHECK && !ok) bad[0] = 1u;
-}
-
 // The tables of the symmetric layout: entry e = pair (t, s) of a block row t
 // and a lower slot s whose neighbour is outside the 16 x 16 block, in (t, s)
 // order; tab[e] = where the kernel writes its value (reading row t and the
@@ -1040,70 +962,13 @@ static int build_box(mfe_ctx* ctx, mfe_csr* A) {
   return MFE_OK;
 }
 
-// The symmetric box layout of A's values as T; MFE_OK with the layout absent
-// when it does not fit in memory.  The first build for A's current values
-// also checks the symmetry the layout relies on (A->boxsym_state 1 or 2;
-// synchronises the stream) and frees the layout again when it fails.
-template <typename T>
-static int build_boxsym(mfe_ctx* ctx, mfe_csr* A) {
-  const BoxGeom g = A->box_geom;
-  if (!A->boxsym_tab) {
-    std::vector<int> tab;
-    boxsym_tables(tab);
-    if (tab.empty()) return fail(ctx, MFE_UNSUPPORTED, "symmetric layout tables");
-    if (!try_alloc(&A->boxsym_tab, sizeof(int) * tab.size())) return MFE_OK;
-    if (int st = upload_bytes(ctx, A->boxsym_tab, tab.data(), sizeof(int) * tab.size())) return st;
-  }
-  T** du;
-  T** dw;
-  if constexpr (std::is_same<T, double>::value) {
-    du = &A->boxsym_u;
-    dw = &A->boxsym_w;
-  } else {
-    du = &A->boxsym_u32;
-    dw = &A->boxsym_w32;
-  }
-  if (!*du && !try_alloc(du, sizeof(T) * (size_t)sym_entries(g))) return MFE_OK;
-  if (!*dw && !try_alloc(dw, sizeof(T) * (size_t)sym_bnd_entries(g))) return MFE_OK;
-  const unsigned grid = (unsigned)((int64_t)g.nbx * g.nby * g.gz);
-  const bool check = A->boxsym_state == 0;
-  unsigned* bad = reinterpret_cast<unsigned*>(ctx->d_scalars + 16);
-  if (check) {
-    MFE_CHECK(ctx, hipMemsetAsync(bad, 0, sizeof(unsigned), ctx->stream));
-    boxsym_fill_staged_kernel<T, true><<<grid, kBlock, 0, ctx->stream>>>(
-        g, A->row_offsets, A->vals, A->boxsym_tab + kSymNB, *du, *dw, bad);
-  } else {
-    boxsym_fill_staged_kernel<T, false><<<grid, kBlock, 0, ctx->stream>>>(
-        g, A->row_offsets, A->vals, A->boxsym_tab + kSymNB, *du, *dw, nullptr);
-  }
-  MFE_LAUNCHED(ctx, "boxsym_fill_staged_kernel");
-  if (check) {
-    unsigned hbad = 0;
-    if (int st = download_bytes(ctx, &hbad, bad, sizeof(unsigned))) return st;
-    A->boxsym_state = hbad ? 2 : 1;
-    if (hbad) {  // not symmetric: the box layout with all 27 slots instead
-      hipFree(*du);
-      hipFree(*dw);
-      *du = nullptr;
-      *dw = nullptr;
-      return MFE_OK;
-    }
-  }
-  if constexpr (std::is_same<T, double>::value) A->boxsym_valid = true;
-  else A->boxsym32_valid = true;
-  return MFE_OK;
-}
-
 // The packed form of a box layout's values (mfe_pack.hpp; SymPack: the
-// symmetric layout's upper slots).  First pass, one workgroup per (block,
-// plane): for each of the NS slots, the least
-// exponent qe of any value's lowest set bit (values other than +0.0 and 1.0;
-// -0.0, infinities and NaNs make the slot unpackable in that group), then the
-// least and greatest k = v / 2^qe.  The slot fits W bits in the group when
-// every |k| < 2^53 (FP32: 2^24) and they span at most 2^W - 3 (W of
-// kPackWidths; 32 for FP64 only).  Writes kmax to kq[2 * group]
-// and 2^qe to kq[2 * group + 1]; fits[i] keeps the slots that fit
-// kPackWidths[i] bits in every group.
+// symmetric layout's upper slots).  The layout's build finds per (block,
+// plane, slot) group the least exponent qe of any value's lowest set bit
+// (values other than +0.0 and 1.0; -0.0, infinities and NaNs make the slot
+// unpackable in that group) and the least and greatest k = v / 2^qe.  The
+// slot fits W bits in the group when every |k| < 2^53 (FP32: 2^24) and they
+// span at most 2^W - 3 (W of kPackWidths; 32 for FP64 only).
 template <typename T>
 struct PackBits;
 template <>
@@ -1138,67 +1003,253 @@ struct PackBits<float> {
   __device__ static bool same(float a, float b) { return __float_as_int(a) == __float_as_int(b); }
 };
 
-template <typename V, typename Op>
-__device__ __forceinline__ V block_reduce(V v, V* sh, Op op) {
-  const int lane = (int)threadIdx.x % kWave, wave = (int)threadIdx.x / kWave;
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v = op(v, (V)__shfl_xor(v, off, kWave));
-  if (lane == 0) sh[wave] = v;
-  __syncthreads();
-  V r = sh[0];
-#pragma unroll
-  for (int w = 1; w < kBlock / kWave; ++w) r = op(r, sh[w]);
-  __syncthreads();  // sh is reused by the next reduction
-  return r;
-}
-
-template <typename T, int NS>
-__global__ __launch_bounds__(kBlock) void boxpack_scan_kernel(const T* __restrict__ U,
-                                                              T* __restrict__ kq,
-                                                              unsigned* fits) {
+// Least lowest-set-bit exponent and range of a group's values (+0.0 and 1.0
+// apart; -0.0, infinities and NaNs set bad), 16 lanes per group.
+template <typename T>
+struct PackRange {
   using B = PackBits<T>;
-  __shared__ int si[kBlock / kWave];
-  __shared__ T st[kBlock / kWave];
-  const int64_t grp0 = (int64_t)blockIdx.x * NS;  // blockIdx.x = block * gz + plane
-  const int t = (int)threadIdx.x;
-  auto imin = [](int a, int b) { return min(a, b); };
-  auto tmin = [](T a, T b) { return a < b ? a : b; };
-  auto tmax = [](T a, T b) { return a > b ? a : b; };
-  unsigned m[kPackNumWidths] = {};
-  for (int u = 0; u < NS; ++u) {
-    const int64_t grp = grp0 + u;
-    const T v = U[grp * kBlock + t];
-    const int lb = B::lowbit(v);
-    const bool special = lb == INT_MAX;
-    const int bad = block_reduce(lb == INT_MIN ? 1 : 0, si, [](int a, int b) { return max(a, b); });
-    const int qe = block_reduce(lb, si, imin);  // INT_MAX: no value to pack
-    bool ok = !bad;
-    T kmin = T(0), kmax = T(0), qv = T(1);
-    if (ok && qe != INT_MAX) {
-      qv = B::pow2(qe);
-      const T k = special ? T(0) : v / qv;  // exact: v is a whole multiple of 2^qe
-      const bool kok = special || fabs(k) < B::kLimit;
-      ok = block_reduce(kok ? 1 : 0, si, imin) != 0;
-      kmin = block_reduce(special ? (T)B::kLimit : k, st, tmin);
-      kmax = block_reduce(special ? -(T)B::kLimit : k, st, tmax);
+  int lb = INT_MAX, bad = 0;
+  T lo = T(0), hi = T(0);  // of the values seen so far (lb != INT_MAX)
+  __device__ void add(T v) {
+    const int l = B::lowbit(v);
+    if (l == INT_MAX) return;
+    if (l == INT_MIN) {
+      bad = 1;
+      return;
     }
-    if (t == 0) {
-      kq[2 * grp] = kmax;
-      kq[2 * grp + 1] = qv;
+    lo = lb == INT_MAX || v < lo ? v : lo;
+    hi = lb == INT_MAX || v > hi ? v : hi;
+    lb = min(lb, l);
+  }
+  __device__ void join16() {
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) {
+      const int l = __shfl_xor(lb, off, kWave);
+      const T ol = __shfl_xor(lo, off, kWave), oh = __shfl_xor(hi, off, kWave);
+      bad |= __shfl_xor(bad, off, kWave);
+      if (l == INT_MAX) continue;
+      lo = lb == INT_MAX || ol < lo ? ol : lo;
+      hi = lb == INT_MAX || oh > hi ? oh : hi;
+      lb = min(lb, l);
+    }
+  }
+  // The group's power of two and greatest multiple, and the widths of
+  // kPackWidths (bit i) that hold it.  A multiple v / q is exact, and the
+  // least and greatest one are those of the least and greatest value.
+  __device__ unsigned widths(T& kmax, T& qv) const {
+    bool ok = !bad;
+    T kmin = T(0);
+    kmax = T(0);
+    qv = T(1);
+    if (ok && lb != INT_MAX) {
+      qv = B::pow2(lb);
+      kmin = lo / qv;
+      kmax = hi / qv;
+      ok = fabs(kmin) < B::kLimit && fabs(kmax) < B::kLimit;
     }
     const T span = kmax - kmin;  // exact: both are integers below the limit
+    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < kPackNumWidths; ++i) {
       const int w = kPackWidths[i];
       const bool allowed = sizeof(T) == 8 || w <= 24;
-      if (ok && allowed && span <= T((double)((1ull << w) - 3ull))) m[i] |= 1u << u;
+      if (ok && allowed && span <= T((double)((1ull << w) - 3ull))) m |= 1u << i;
     }
+    return m;
   }
-  if (t == 0)
-    for (int i = 0; i < kPackNumWidths; ++i) atomicAnd(fits + i, m[i]);
+};
+
+// Device words of a plan build (PlanWords at d_scalars + kPlanWordsAt).
+struct PlanWords {
+  unsigned asym;                     // 1: a mirrored pair differs
+  unsigned pack_bad, wpack_bad;      // 1: a packed value does not decode to itself
+  unsigned pad;
+  unsigned fits[kPackNumWidths];     // per width of kPackWidths: the slots every group fits
+  unsigned wfits[kPackNumWidths];    // the boundary stream's lower slots
+};
+constexpr int kPlanWordsAt = 16;
+static_assert(sizeof(PlanWords) <= 32 * sizeof(double), "d_scalars holds 64 doubles");
+
+__global__ void plan_words_kernel(PlanWords* w) {
+  const int i = (int)threadIdx.x;
+  if (i == 0) w->asym = w->pack_bad = w->wpack_bad = w->pad = 0u;
+  if (i < kPackNumWidths) w->fits[i] = w->wfits[i] = ~0u;
 }
 
-// Second pass: the fields of PF's slots (each fits its width W in every
+// The symmetric layout of A's values and, in the same pass, what its packed
+// form and its symmetry check need.  A workgroup owns one 16 x 16 block and a
+// range of planes (g.zc); per plane thread t's node writes its 14 upper slots
+// to U and its lower slots whose neighbour lies outside the block to W (entry
+// inv[t * 13 + s]), 0 where the slot is out of range or the node past the
+// box's edge, so every entry is written.
+//   The block-plane's CSR rows are staged in LDS (16 lanes per grid line, whose
+// rows' values are one contiguous run: coalesced loads instead of one
+// 216-byte-strided row per thread), the next plane's loads in flight while
+// this one is worked on; positions follow from the box's closed-form row
+// offsets.
+//   CHECK: every lower slot whose neighbour lies in the block must hold the
+// bits of that neighbour's mirrored upper slot (from LDS: this plane's, or
+// the plane before's kept in `up`); pairs across the block's edge are read
+// from W, the row's own values, and need none.
+//   With kq (and wkq: the boundary stream's groups), per (block, plane, slot)
+// group the least exponent of any value's lowest set bit and the range of
+// the values (16 threads per slot), giving kmax and q (kq[2 group], [+ 1];
+// wkq[rec + 2 s], [+ 1]) and the widths every group fits.
+//   What bounds it: HBM, 27 values read and 14 + 282/256 written per row (9.2
+// GB at 300^3).  Filling one plane per workgroup and scanning U and W in two
+// kernels of their own took 7.5 + 7.9 + 2.1 ms there (serial loads of one
+// line after another, mirrored entries gathered from memory, 70 workgroup
+// reductions per plane).
+constexpr int kSymStage = 27 * kBlock;  // values of a block-plane's rows
+template <typename T, bool CHECK>
+__global__ __launch_bounds__(kBlock, 2) void boxsym_build_kernel(
+    BoxGeom g, const double* __restrict__ vals, const int* __restrict__ tab, T* __restrict__ U,
+    T* __restrict__ W, T* __restrict__ kq, T* __restrict__ wkq, PlanWords* words) {
+  __shared__ double sv[kSymStage];  // the staged rows, then this plane's upper slots [u][t]
+  __shared__ double up[CHECK ? 9 : 1][kBlock];  // the plane before's upper slots 18 + j
+  __shared__ T sw[kSymNB];
+  double(*const su)[kBlock] = reinterpret_cast<double(*)[kBlock]>(sv);
+  const int wg = (int)blockIdx.x;
+  const int chunk = wg % g.nzc, blk = wg / g.nzc;
+  const int bx = blk % g.nbx, by = blk / g.nbx;
+  const int t = (int)threadIdx.x, tx = t % kBoxBX, ty = t / kBoxBX;
+  const int x0 = bx * kBoxBX, ix = x0 + tx, iy = by * kBoxBY + ty;
+  const int nxl = min(kBoxBX, g.gx - x0);  // live nodes per line
+  const bool lline = iy < g.gy, live = ix < g.gx && lline;
+  const int z0 = chunk * g.zc, z1 = min(z0 + g.zc, g.gz);
+  // entries before node i of an axis of g nodes, each with its in-range neighbours
+  auto pre = [](int i, int gn) { return i == 0 ? 0 : 3 * i - 1 - (i == gn ? 1 : 0); };
+  auto cnt = [](int i, int gn) { return 1 + (i > 0) + (i < gn - 1); };
+  const int64_t Sx = pre(g.gx, g.gx), Sy = pre(g.gy, g.gy);
+  const int cy = cnt(iy, g.gy);
+  const int px = pre(ix < g.gx ? ix : x0, g.gx) - pre(x0, g.gx);
+  const int lx = pre(x0 + nxl, g.gx) - pre(x0, g.gx);
+  double v[27];
+  auto load = [&](int z) {  // the 16 lanes of a line take its values in turn
+    const int cz = cnt(z, g.gz);
+    const int64_t first =
+        lline ? pre(z, g.gz) * Sy * Sx + cz * (pre(iy, g.gy) * Sx + cy * (int64_t)pre(x0, g.gx)) : 0;
+    const int len = lline ? cz * cy * lx : 0;
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+      const int i = tx + kBoxBX * k;
+      v[k] = i < len ? vals[first + i] : 0.0;
+    }
+  };
+  int e[13];
+#pragma unroll
+  for (int s = 0; s < 13; ++s) e[s] = tab[kSymNB + t * 13 + s];
+  const int gs = t / 16, gp = t % 16;  // the slot and part this thread scans
+  int we[2] = {-1, -1};
+  if (gs < kSymWGroups) {
+    we[0] = tab[kSymWListAt + gs * kSymWListLen + gp];
+    we[1] = tab[kSymWListAt + gs * kSymWListLen + gp + 16];
+  }
+  unsigned fit = ~0u, wfit = ~0u;
+  bool same = true;
+  if (CHECK) {
+#pragma unroll
+    for (int j = 0; j < 9; ++j) up[CHECK ? j : 0][t] = 0.0;
+  }
+  const int zb = CHECK && z0 > 0 ? z0 - 1 : z0;  // one plane early for the checks across planes
+  load(zb);
+  for (int z = zb; z < z1; ++z) {
+    const bool own = z >= z0;
+#pragma unroll
+    for (int k = 0; k < 27; ++k) sv[ty * (27 * kBoxBX) + tx + kBoxBX * k] = v[k];
+    __syncthreads();
+    const unsigned m = live ? box_mask(ix, iy, z, g.gx, g.gy, g.gz) : 0u;
+    double r[27];
+    {
+      int at = ty * (27 * kBoxBX) + cnt(z, g.gz) * cy * px;
+#pragma unroll
+      for (int s = 0; s < 27; ++s) {
+        const bool in = (m >> s) & 1u;
+        r[s] = in ? sv[at] : 0.0;
+        at += in ? 1 : 0;
+      }
+    }
+    if (z + 1 < z1) load(z + 1);
+    if (own) {
+#pragma unroll
+      for (int u = 0; u < kSymU; ++u) U[sym_at(g, blk, z, u, t)] = (T)r[13 + u];
+      const int64_t wbase = ((int64_t)blk * g.gz + z) * kSymNB;
+#pragma unroll
+      for (int s = 0; s < 13; ++s) {
+        if (e[s] >= 0) {
+          W[wbase + e[s]] = (T)r[s];
+          sw[e[s]] = (T)r[s];
+        } else if (CHECK && s < 9 && ((m >> s) & 1u)) {
+          const int sy = s / 3 - 1, sx = s % 3 - 1;
+          const double c = up[CHECK ? 8 - s : 0][t + sy * kBoxBX + sx];
+          same = same && __double_as_longlong(c) == __double_as_longlong(r[s]);
+        }
+      }
+    }
+    __syncthreads();  // the staged rows and the plane before's slots are read
+#pragma unroll
+    for (int u = 0; u < kSymU; ++u) su[u][t] = r[13 + u];
+    if (CHECK) {
+#pragma unroll
+      for (int j = 0; j < 9; ++j) up[CHECK ? j : 0][t] = r[18 + j];
+    }
+    __syncthreads();
+    if (own) {
+      if (CHECK) {
+#pragma unroll
+        for (int s = 9; s < 13; ++s)
+          if (e[s] < 0 && ((m >> s) & 1u)) {
+            const int sy = (s - 9) / 3 - 1, sx = (s - 9) % 3 - 1;
+            const double c = su[13 - s][t + sy * kBoxBX + sx];
+            same = same && __double_as_longlong(c) == __double_as_longlong(r[s]);
+          }
+      }
+      const int64_t gi = (int64_t)blk * g.gz + z;
+      if (kq) {
+        PackRange<T> pr;
+        const int u = gs < kSymU ? gs : 0;
+#pragma unroll 4
+        for (int k = 0; k < 16; ++k) pr.add((T)su[u][gp + 16 * ((k + gs) & 15)]);
+        pr.join16();
+        T kmax, qv;
+        const unsigned w = pr.widths(kmax, qv);
+        if (gs < kSymU) {
+          fit &= w;
+          if (gp == 0) {
+            kq[2 * (gi * kSymU + gs)] = kmax;
+            kq[2 * (gi * kSymU + gs) + 1] = qv;
+          }
+        }
+      }
+      if (wkq) {
+        PackRange<T> pr;
+        if (we[0] >= 0) pr.add(sw[we[0]]);
+        if (we[1] >= 0) pr.add(sw[we[1]]);
+        pr.join16();
+        T kmax, qv;
+        const unsigned w = pr.widths(kmax, qv);
+        if (gs < kSymWGroups) {
+          wfit &= w;
+          if (gp == 0) {
+            wkq[gi * kSymWRec + 2 * gs] = kmax;
+            wkq[gi * kSymWRec + 2 * gs + 1] = qv;
+          }
+        }
+      }
+    }
+    __syncthreads();  // sv and sw are written by the next plane
+  }
+  if (CHECK && !same) words->asym = 1u;
+  if (gp == 0) {
+#pragma unroll
+    for (int i = 0; i < kPackNumWidths; ++i) {
+      if (kq && gs < kSymU && !((fit >> i) & 1u)) atomicAnd(&words->fits[i], ~(1u << gs));
+      if (wkq && gs < kSymWGroups && !((wfit >> i) & 1u)) atomicAnd(&words->wfits[i], ~(1u << gs));
+    }
+  }
+}
+
+// The fields of PF's slots (each fits its width W in every
 // group) from kb = kmax - (2^W - 1), so kb is an integer of at most kmax's
 // size and every field lies between 2 (the codes' successor) and 2^W - 1;
 // packed into words, kb replaces kmax.  Every value is decoded as the SpMV decodes it and compared
@@ -1246,14 +1297,75 @@ __global__ __launch_bounds__(kBlock) void boxpack_pack_kernel(const T* __restric
   if (t == 0) kq[2 * NS * (int64_t)gridDim.x + gi] = any ? T(1) : T(0);
 }
 
-// The packed form of the layout U (map P, precision T, `groups` (block,
-// plane) groups), built after the layout: of the forms whose every field fits
-// its width in every group, the one with the fewest bytes per row (fields
-// and full-width values), or none (kPackNone: the SpMV reads the full
-// values).  *kq, *pw and *cap are the
-// layout's arrays (allocated here); *form is set, and left kPackNone when
-// they do not fit in memory.  Synchronises the stream (for the slot sets and
-// the check).
+// The symmetric box layout of A's values as T, with the groups' bases and
+// powers of two and the widths they fit (what build_boxpack needs); MFE_OK
+// with the layout absent when it does not fit in memory.  The first build for
+// A's current values also checks the symmetry the layout relies on
+// (A->boxsym_state 1 or 2) and frees the layout again when it fails.
+// Synchronises the stream.
+template <typename T>
+static int build_boxsym(mfe_ctx* ctx, mfe_csr* A) {
+  constexpr bool f64 = std::is_same<T, double>::value;
+  BoxGeom g = A->box_geom;
+  if (!A->boxsym_tab) {
+    std::vector<int> tab;
+    boxsym_tables(tab);
+    if (tab.empty()) return fail(ctx, MFE_UNSUPPORTED, "symmetric layout tables");
+    if (!try_alloc(&A->boxsym_tab, sizeof(int) * tab.size())) return MFE_OK;
+    if (int st = upload_bytes(ctx, A->boxsym_tab, tab.data(), sizeof(int) * tab.size())) return st;
+  }
+  T **du, **dw, **dk;
+  if constexpr (f64) {
+    du = &A->boxsym_u;
+    dw = &A->boxsym_w;
+    dk = &A->boxpack_kq;
+  } else {
+    du = &A->boxsym_u32;
+    dw = &A->boxsym_w32;
+    dk = &A->boxpack32_kq;
+  }
+  const int64_t groups = (int64_t)g.nbx * g.nby * g.gz;
+  if (!*du && !try_alloc(du, sizeof(T) * (size_t)sym_entries(g))) return MFE_OK;
+  if (!*dw && !try_alloc(dw, sizeof(T) * (size_t)sym_bnd_entries(g))) return MFE_OK;
+  // without room for these the values stay at full width
+  if (!*dk) (void)try_alloc(dk, sizeof(T) * (size_t)(2 * groups * kSymU + groups));
+  T* wkq = nullptr;
+  if constexpr (f64) {
+    if (!A->boxwpack_kq) (void)try_alloc(&A->boxwpack_kq, sizeof(T) * (size_t)(groups * kSymWRec));
+    wkq = A->boxwpack_kq;
+  }
+  const bool check = A->boxsym_state == 0;
+  PlanWords* words = reinterpret_cast<PlanWords*>(ctx->d_scalars + kPlanWordsAt);
+  plan_words_kernel<<<1, kWave, 0, ctx->stream>>>(words);
+  auto run = [&](auto kern) {
+    box_chunks(g, resident_groups((const void*)kern, ctx->cu_count), groups);
+    kern<<<(unsigned)((int64_t)g.nbx * g.nby * g.nzc), kBlock, 0, ctx->stream>>>(
+        g, A->vals, A->boxsym_tab, *du, *dw, *dk, wkq, words);
+  };
+  if (check) run(boxsym_build_kernel<T, true>);
+  else run(boxsym_build_kernel<T, false>);
+  MFE_LAUNCHED(ctx, "boxsym_build_kernel");
+  PlanWords hw;
+  if (int st = download_bytes(ctx, &hw, words, sizeof(hw))) return st;
+  if (check) {
+    A->boxsym_state = hw.asym ? 2 : 1;
+    if (hw.asym) {  // not symmetric: the box layout with all 27 slots instead
+      hipFree(*du);
+      hipFree(*dw);
+      *du = nullptr;
+      *dw = nullptr;
+      return MFE_OK;
+    }
+  }
+  for (int i = 0; i < kPackNumWidths; ++i) {
+    (f64 ? A->boxpack_fits : A->boxpack32_fits)[i] = *dk ? hw.fits[i] : 0u;
+    if (f64) A->boxwpack_fits[i] = wkq ? hw.wfits[i] : 0u;
+  }
+  if constexpr (f64) A->boxsym_valid = true;
+  else A->boxsym32_valid = true;
+  return MFE_OK;
+}
+
 // f(std::integral_constant<int, form>) for a packed form that precision T
 // has (FP32: no 32-bit fields); else hipErrorInvalidValue.
 template <typename T, typename F>
@@ -1275,25 +1387,19 @@ static int with_pack_form(int form, F&& f) {
   return (int)hipErrorInvalidValue;
 }
 
-template <typename T, typename P, int PF>
-static void boxpack_launch(mfe_ctx* ctx, const T* U, T* kq, unsigned* pw, unsigned* bad,
-                           int64_t groups) {
-  boxpack_pack_kernel<T, P, PF><<<(unsigned)groups, kBlock, 0, ctx->stream>>>(U, kq, pw, bad);
-}
-
-template <typename T, typename P>
-static int build_pack(mfe_ctx* ctx, const T* U, int64_t groups, T** kq, unsigned** pw, int* cap,
-                      int* form_out) {
+// The packed form of the symmetric layout U (precision T, `groups` (block,
+// plane) groups), built after the layout: of the forms whose every field fits
+// its width in every group (fits), the one with the fewest bytes per row
+// (fields and full-width values), or none (kPackNone: the SpMV reads the full
+// values).  *pw and *cap are the layout's words (allocated here); the form is
+// left kPackNone when they do not fit in memory.  Enqueues the packing; the
+// caller checks words->pack_bad.
+template <typename T>
+static int enqueue_pack(mfe_ctx* ctx, const T* U, int64_t groups, const unsigned* fits, T* kq,
+                        unsigned** pw, int* cap, PlanWords* words, int* form_out) {
+  using P = SymPack;
   constexpr bool f64 = std::is_same<T, double>::value;
   *form_out = kPackNone;
-  if (!*kq && !try_alloc(kq, sizeof(T) * (size_t)(2 * groups * P::kSlots + groups))) return MFE_OK;
-  unsigned* fits = reinterpret_cast<unsigned*>(ctx->d_scalars + 24);  // per kPackWidths
-  unsigned* bad = reinterpret_cast<unsigned*>(ctx->d_scalars + 28);
-  MFE_CHECK(ctx, hipMemsetAsync(fits, 0xFF, kPackNumWidths * sizeof(unsigned), ctx->stream));
-  boxpack_scan_kernel<T, P::kSlots><<<(unsigned)groups, kBlock, 0, ctx->stream>>>(U, *kq, fits);
-  MFE_LAUNCHED(ctx, "boxpack_scan_kernel");
-  unsigned hf[kPackNumWidths] = {};
-  if (int st = download_bytes(ctx, hf, fits, sizeof(hf))) return st;
   int form = kPackNone;
   int64_t best = 0;
   for (int f = 1; f < kPackForms; ++f) {
@@ -1308,7 +1414,7 @@ static int build_pack(mfe_ctx* ctx, const T* U, int64_t groups, T** kq, unsigned
       }
       int i = 0;
       while (kPackWidths[i] != w) ++i;
-      fits_all = fits_all && ((hf[i] >> s) & 1u);
+      fits_all = fits_all && ((fits[i] >> s) & 1u);
     }
     const int64_t bytes = 4 * (int64_t)P::words(f) + (int64_t)sizeof(T) * fulls;
     if (fits_all && (form == kPackNone || bytes < best)) {
@@ -1316,84 +1422,27 @@ static int build_pack(mfe_ctx* ctx, const T* U, int64_t groups, T** kq, unsigned
       best = bytes;
     }
   }
-  if (form != kPackNone) {
-    const int words = P::words(form);
-    if (*cap < words) {
-      hipFree(*pw);
-      *pw = nullptr;
-      *cap = 0;
-      if (!try_alloc(pw, sizeof(unsigned) * (size_t)(groups * words * kBlock))) return MFE_OK;
-      *cap = words;
-    }
-    MFE_CHECK(ctx, hipMemsetAsync(bad, 0, sizeof(unsigned), ctx->stream));
-    with_pack_form<T>(form, [&](auto pf) {
-      boxpack_launch<T, P, decltype(pf)::value>(ctx, U, *kq, *pw, bad, groups);
-      return 0;
-    });
-    MFE_LAUNCHED(ctx, "boxpack_pack_kernel");
-    unsigned hb = 0;
-    if (int st = download_bytes(ctx, &hb, bad, sizeof(hb))) return st;
-    if (hb) form = kPackNone;  // a value the form cannot reproduce: full values
+  if (form == kPackNone) return MFE_OK;
+  const int nw = P::words(form);
+  if (*cap < nw) {
+    hipFree(*pw);
+    *pw = nullptr;
+    *cap = 0;
+    if (!try_alloc(pw, sizeof(unsigned) * (size_t)(groups * nw * kBlock))) return MFE_OK;
+    *cap = nw;
   }
+  with_pack_form<T>(form, [&](auto pf) {
+    boxpack_pack_kernel<T, P, decltype(pf)::value>
+        <<<(unsigned)groups, kBlock, 0, ctx->stream>>>(U, kq, *pw, &words->pack_bad);
+    return 0;
+  });
+  MFE_LAUNCHED(ctx, "boxpack_pack_kernel");
   *form_out = form;
   return MFE_OK;
 }
 
-// The packed boundary stream (mfe_boxsym.hpp).  First pass, one workgroup
-// per (block, plane), thread s < kSymWGroups for lower slot s: q and the
-// least and greatest multiple over the slot's entries (the list in tab from
-// kSymWListAt), as for the upper values; kmax and q to wkq, and the slots
-// whose multiples fit each width of kPackWidths and-ed into fits.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void boxwpack_scan_kernel(const T* __restrict__ W,
-                                                               const int* __restrict__ tab,
-                                                               T* __restrict__ wkq,
-                                                               unsigned* fits) {
-  using B = PackBits<T>;
-  __shared__ unsigned sfit[kPackNumWidths];
-  const int64_t gi = blockIdx.x;
-  const int t = (int)threadIdx.x;
-  if (t < kPackNumWidths) sfit[t] = ~0u;
-  __syncthreads();
-  if (t < kSymWGroups) {
-    const int* L = tab + kSymWListAt + t * kSymWListLen;
-    const T* w = W + gi * kSymNB;
-    int qe = INT_MAX;
-    bool ok = true;
-    for (int i = 0; i < kSymWListLen && L[i] >= 0; ++i) {
-      const int lb = B::lowbit(w[L[i]]);
-      ok = ok && lb != INT_MIN;
-      if (lb != INT_MIN) qe = min(qe, lb);
-    }
-    T kmin = T(0), kmax = T(0), qv = T(1);
-    if (ok && qe != INT_MAX) {
-      qv = B::pow2(qe);
-      kmin = (T)B::kLimit;
-      kmax = -(T)B::kLimit;
-      for (int i = 0; i < kSymWListLen && L[i] >= 0; ++i) {
-        const T v = w[L[i]];
-        if (B::lowbit(v) == INT_MAX) continue;  // +0.0 or 1.0: a code
-        const T k = v / qv;                     // exact: v is a whole multiple of 2^qe
-        ok = ok && fabs(k) < B::kLimit;
-        kmin = k < kmin ? k : kmin;
-        kmax = k > kmax ? k : kmax;
-      }
-      if (kmin > kmax) kmin = kmax = T(0);  // only codes
-    }
-    wkq[gi * kSymWRec + 2 * t] = kmax;
-    wkq[gi * kSymWRec + 2 * t + 1] = qv;
-    const T span = kmax - kmin;
-    for (int i = 0; i < kPackNumWidths; ++i) {
-      const int wd = kPackWidths[i];
-      const bool allowed = sizeof(T) == 8 || wd <= 24;
-      if (!(ok && allowed && span <= T((double)((1ull << wd) - 3ull)))) atomicAnd(&sfit[i], ~(1u << t));
-    }
-  }
-  __syncthreads();
-  if (t < kPackNumWidths) atomicAnd(fits + t, sfit[t]);
-}
-
-// Second pass for form F: the fields of the (block, plane)'s entries,
+// The packed boundary stream (mfe_boxsym.hpp) in form F: the fields of the
+// (block, plane)'s entries,
 // assembled in LDS, each decoded as the SpMV decodes it and compared bit for
 // bit (*bad = 1 on a mismatch); kb replaces kmax, and the codes flag is set.
 template <typename T, int F>
@@ -1440,79 +1489,72 @@ __global__ __launch_bounds__(kBlock) void boxwpack_pack_kernel(const T* __restri
   if (t == 0) wkq[gi * kSymWRec + 2 * kSymWGroups] = any ? T(1) : T(0);
 }
 
-// The packed boundary stream of A's symmetric layout in precision T: of the
-// forms that give every entry a field and whose widths every group fits, the
-// one with the fewest words, or none (the SpMV reads the full values).
-// Synchronises the stream.
-template <typename T>
-static int build_boxwpack(mfe_ctx* ctx, mfe_csr* A, const T* W, T** wkq, unsigned** wpw,
-                          int* form_out) {
-  constexpr bool f64 = std::is_same<T, double>::value;
-  const BoxGeom g = A->box_geom;
-  const int64_t groups = (int64_t)g.nbx * g.nby * g.gz;
+// The FP64 boundary stream's packed form: of the forms that give every entry a
+// field and whose widths every group fits, the one with the fewest words, or
+// none (the SpMV reads the full values).  Enqueues the packing; the caller
+// checks words->wpack_bad.
+static int enqueue_wpack(mfe_ctx* ctx, mfe_csr* A, int64_t groups, PlanWords* words,
+                         int* form_out) {
   *form_out = kPackNone;
-  if (!*wkq && !try_alloc(wkq, sizeof(T) * (size_t)(groups * kSymWRec))) return MFE_OK;
-  if (!*wpw && !try_alloc(wpw, sizeof(unsigned) * (size_t)(groups * sym_w_words(kPackCube16Near32))))
+  if (!A->boxwpack_pw &&
+      !try_alloc(&A->boxwpack_pw, sizeof(unsigned) * (size_t)(groups * sym_w_words(kPackCube16Near32))))
     return MFE_OK;
-  unsigned* fits = reinterpret_cast<unsigned*>(ctx->d_scalars + 24);
-  unsigned* bad = reinterpret_cast<unsigned*>(ctx->d_scalars + 28);
-  MFE_CHECK(ctx, hipMemsetAsync(fits, 0xFF, kPackNumWidths * sizeof(unsigned), ctx->stream));
-  boxwpack_scan_kernel<T><<<(unsigned)groups, kBlock, 0, ctx->stream>>>(W, A->boxsym_tab, *wkq, fits);
-  MFE_LAUNCHED(ctx, "boxwpack_scan_kernel");
-  unsigned hf[kPackNumWidths] = {};
-  if (int st = download_bytes(ctx, hf, fits, sizeof(hf))) return st;
   auto fit = [&](int wd, unsigned slots) {
     int i = 0;
     while (kPackWidths[i] != wd) ++i;
-    return (hf[i] & slots) == slots;
+    return (A->boxwpack_fits[i] & slots) == slots;
   };
   const unsigned all = (1u << kSymWGroups) - 1u;
   int form = kPackNone;
   for (int f = 1; f < kPackForms; ++f) {
-    if (f == kPackCube16 || (!f64 && pack_wide(f) == 32)) continue;
+    if (f == kPackCube16) continue;
     const bool ok = pack_all(f) ? fit(pack_narrow(f), all)
                                 : fit(pack_narrow(f), all & ~kSymWNear) && fit(pack_wide(f), kSymWNear);
     if (ok && (form == kPackNone || sym_w_words(f) < sym_w_words(form))) form = f;
   }
-  if (form != kPackNone) {
-    MFE_CHECK(ctx, hipMemsetAsync(bad, 0, sizeof(unsigned), ctx->stream));
-    with_pack_form<T>(form, [&](auto pf) {
-      boxwpack_pack_kernel<T, decltype(pf)::value><<<(unsigned)groups, kBlock, 0, ctx->stream>>>(
-          W, A->boxsym_tab, *wkq, *wpw, bad);
-      return 0;
-    });
-    MFE_LAUNCHED(ctx, "boxwpack_pack_kernel");
-    unsigned hb = 0;
-    if (int st = download_bytes(ctx, &hb, bad, sizeof(hb))) return st;
-    if (hb) form = kPackNone;
-  }
+  if (form == kPackNone) return MFE_OK;
+  with_pack_form<double>(form, [&](auto pf) {
+    boxwpack_pack_kernel<double, decltype(pf)::value><<<(unsigned)groups, kBlock, 0, ctx->stream>>>(
+        A->boxsym_w, A->boxsym_tab, A->boxwpack_kq, A->boxwpack_pw, &words->wpack_bad);
+    return 0;
+  });
+  MFE_LAUNCHED(ctx, "boxwpack_pack_kernel");
   *form_out = form;
   return MFE_OK;
 }
 
 // The packed form of A's symmetric layout in precision T (after the layout):
 // the upper values, and the boundary stream where the upper values are packed.
+// A form whose fields do not give back every value is not used.  Synchronises
+// the stream when something was packed.
 template <typename T>
 static int build_boxpack(mfe_ctx* ctx, mfe_csr* A) {
+  constexpr bool f64 = std::is_same<T, double>::value;
   const BoxGeom g = A->box_geom;
   const int64_t groups = (int64_t)g.nbx * g.nby * g.gz;
-  int form = kPackNone;
-  if constexpr (std::is_same<T, double>::value) {
-    if (int st = build_pack<double, SymPack>(ctx, A->boxsym_u, groups, &A->boxpack_kq,
-                                             &A->boxpack_pw, &A->boxpack_cap, &form))
-      return st;
+  PlanWords* words = reinterpret_cast<PlanWords*>(ctx->d_scalars + kPlanWordsAt);
+  plan_words_kernel<<<1, kWave, 0, ctx->stream>>>(words);
+  int form = kPackNone, wform = kPackNone, st = MFE_OK;
+  if constexpr (f64) {
+    st = enqueue_pack<double>(ctx, A->boxsym_u, groups, A->boxpack_fits, A->boxpack_kq,
+                              &A->boxpack_pw, &A->boxpack_cap, words, &form);
+    if (!st && form != kPackNone) st = enqueue_wpack(ctx, A, groups, words, &wform);
+  } else {
+    st = enqueue_pack<float>(ctx, A->boxsym_u32, groups, A->boxpack32_fits, A->boxpack32_kq,
+                             &A->boxpack32_pw, &A->boxpack32_cap, words, &form);
+  }
+  if (st) return st;
+  if (form != kPackNone) {
+    PlanWords hw;
+    if ((st = download_bytes(ctx, &hw, words, sizeof(hw)))) return st;
+    if (hw.wpack_bad) wform = kPackNone;
+    if (hw.pack_bad) form = wform = kPackNone;
+  }
+  if constexpr (f64) {
     A->boxpack_form = form;
-    int wform = kPackNone;
-    if (form != kPackNone)
-      if (int st = build_boxwpack<double>(ctx, A, A->boxsym_w, &A->boxwpack_kq, &A->boxwpack_pw,
-                                          &wform))
-        return st;
     A->boxwpack_form = wform;
     A->boxpack_valid = true;
   } else {
-    if (int st = build_pack<float, SymPack>(ctx, A->boxsym_u32, groups, &A->boxpack32_kq,
-                                            &A->boxpack32_pw, &A->boxpack32_cap, &form))
-      return st;
     A->boxpack32_form = form;
     A->boxpack32_valid = true;
   }
