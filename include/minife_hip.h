@@ -190,7 +190,8 @@ int mfe_make_local_matrix(mfe_ctx* ctx, mfe_csr* A);
  * (the three at full width), 4 all in 12, 5 eleven in 12 and three in 24, 6
  * all in 10, 7 eleven in 10 and three in 22 -- and, once the FP32 copy
  * exists, of the FP32 values in bits 8-15; the FP64 boundary stream's form
- * in bits 16-23, 0 where it is read at full width); and
+ * in bits 16-23, 0 where it has none -- the CG reads it so from 2^23 rows on,
+ * and at full width below); and
  * for the staged-x plan (else 0): runs; most distinct columns of a 256-row
  * tile; stored entries whose local columns are read; slices read as base +
  * lane instead (every row of the slice as wide as the slice, slot j's local

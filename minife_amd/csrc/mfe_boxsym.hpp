@@ -77,12 +77,53 @@ __host__ __device__ constexpr int sym_w_words(int f) {
           kSymWNearCount * (pack_all(f) ? pack_narrow(f) : pack_wide(f)) + 31) / 32 + 1;
 }
 
-// PF != kPackNone: the upper values are read in the packed form of
-// mfe_pack.hpp (SymPack: slot u is upper slot u, one word group), the kb and
-// q of plane z staged in LDS; with WPK (and PF) the boundary stream too, in
-// form wform, from WPW and WKQ (a template argument: the choice between the
-// two loads of the boundary values costs registers where it is made at run
-// time).
+// The upper values' record of a (block, plane), kSymKRec values of T at KQ[rec *
+// kSymKRec]: the bases kb q of the 14 slots, then as 32-bit words the powers of
+// two q (FP64: the high word, the low one being 0) and the codes flag (1: some
+// packed value is +0.0 or 1.0).
+constexpr int kSymKRec = 2 * kSymU + 2;
+template <typename T>
+struct SymRec {
+  T kb[kSymU];
+  unsigned q[kSymU];
+  unsigned codes;
+  // the record at p, the same for every lane (scalar loads)
+  __device__ static SymRec load(const T* p) {
+    SymRec r;
+    const unsigned* w = reinterpret_cast<const unsigned*>(p + kSymU);
+#pragma unroll
+    for (int u = 0; u < kSymU; ++u) {
+      r.kb[u] = p[u];
+      r.q[u] = w[u];
+    }
+    r.codes = w[kSymU];
+    return r;
+  }
+  __device__ T pow2(int u) const {
+    if constexpr (sizeof(T) == 8) return __hiloint2double((int)q[u], 0);
+    else return __uint_as_float(q[u]);
+  }
+};
+
+// One workgroup per (block, z chunk), one node column per thread.  Lower slot s
+// of row r is upper slot 26 - s of the neighbour n = r + off(s), and both its
+// value and its x entry are n's own: n forms the product v x_n and hands it to
+// r through LDS (up: from the plane before; sm: from the same plane), so a row
+// reads 8 + 4 products and the next plane's 9 x entries from LDS instead of
+// 12 values and 27 x entries; its upper same-plane x entries are the ones it
+// read as next-plane entries the step before, and the product from its own
+// column stays in a register.  A boundary entry (a lower slot whose neighbour
+// is outside the block) is multiplied by the ring's x entry by the thread that
+// loaded it.  Products and their order are those of a row-by-row sum.
+//   PF != kPackNone: the upper values are read in the packed form of
+// mfe_pack.hpp (SymPack: slot u is upper slot u, one word group); a plane's
+// record is the same for every lane and is read with scalar loads, issued when
+// the plane before has been decoded (43 scalar registers).  With WPK
+// (and PF) the boundary stream too, in form wform, from WPW and WKQ (a
+// template argument: the choice between the two loads of the boundary values
+// costs registers where it is made at run time); its records differ from lane
+// to lane and are staged in LDS.
+//   Every load runs one plane step ahead of its use.
 template <typename T, bool ZERO_Y, int MODE, int PF = kPackNone, bool WPK = false>
 __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
     BoxGeom g, const T* __restrict__ U, const T* __restrict__ W, const int* __restrict__ btab,
@@ -95,21 +136,24 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
   constexpr PackLayout<P, PF> L{};
   constexpr unsigned kMask = L.mask;  // slots with a field
   constexpr int kWords = L.words;
-  if (done && *done) return;
-  __shared__ T xw[3][kBoxWin];
-  __shared__ T up[9][kBlock];  // previous plane's upper slots 18 + j, by reading row
-  __shared__ T sm[4][kBlock];  // this plane's upper slots 14 + i, by reading row
-  __shared__ T red[4];
-  // kb and q of every slot of a plane (2 * kSymU values) and its codes flag,
-  // then the boundary stream's record (kSymWRec), double-buffered by plane
-  // parity: plane z+1's record is stored during step z
-  constexpr int kRec = 2 * kSymU + 1, kRecAll = kRec + kSymWRec;
   constexpr bool kHasKQ = PF != kPackNone;
   constexpr bool wpk = kHasKQ && WPK;
-  const int nrec = wpk ? kRecAll : kRec;
-  __shared__ T kqs[2][PF != kPackNone ? kRecAll : 1];
-  const int wg = (int)blockIdx.x;
-  const int chunk = wg % g.nzc, blk = wg / g.nzc;
+  if (done && *done) return;
+  __shared__ T xw[3][kBoxWin];
+  __shared__ T up[8][kBlock];  // products of the plane before's upper slots 18 + j
+                               // (j != 4), by reading row
+  __shared__ T sm[4][kBlock];  // products of this plane's upper slots 14 + i, by reading row
+  __shared__ T red[4];
+  // the boundary stream's record, double-buffered by plane parity: plane z+1's
+  // is stored during step z
+  __shared__ T kqs[2][wpk ? kSymWRec : 1];
+  // each XCD takes a contiguous range of tiles numbered block-fastest within a z
+  // chunk: neighbouring blocks then meet in one L2, which serves their x rings
+  // and merges the lines of y that two blocks write (16 nodes start mid-line).
+  // At 300^3 this reads 1.04 GB instead of 1.24 and takes 0.347 ms instead of 0.362.
+  const int tile = xcd_contiguous((int)blockIdx.x, (int)gridDim.x), nblk = g.nbx * g.nby;
+  const int chunk = tile / nblk, blk = tile % nblk;
+  const int wg = blk * g.nzc + chunk;  // index of this workgroup's partial
   const int bx = blk % g.nbx, by = blk / g.nbx;
   const int t = (int)threadIdx.x;
   const int tx = t % kBoxBX, ty = t / kBoxBX;
@@ -118,19 +162,22 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
   const int z0 = chunk * g.zc;
   const int z1 = min(z0 + g.zc, g.gz);
   const int64_t plane = (int64_t)g.gx * g.gy;
-  int64_t woff[2];
-  bool wok[2];
-  int bcode[2];
-  bool bok[2];
+  const int64_t rec0 = (int64_t)blk * g.gz;  // (block, plane) index of plane 0
+  // window cells this thread loads, and its boundary entries: where the value's
+  // product goes and the ring cell of its x entry
+  int woff[2], bcode[2], bcell[2];
+  bool wok[2], bok[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     const int w = t + k * kBlock;
     const int wx = w % kBoxWX, wy = w / kBoxWX;
     const int nx = bx * kBoxBX + wx - 1, ny = by * kBoxBY + wy - 1;
     wok[k] = w < kBoxWin && nx >= 0 && nx < g.gx && ny >= 0 && ny < g.gy;
-    woff[k] = wok[k] ? nx + (int64_t)g.gx * ny : 0;
+    woff[k] = wok[k] ? nx + g.gx * ny : 0;
     bok[k] = w < kSymNB;
     bcode[k] = bok[k] ? btab[w] : 0;
+    const int rt = bcode[k] & 511, s = (bcode[k] >> 26) & 15;
+    bcell[k] = (rt / kBoxBX + 1 + (s / 3) % 3 - 1) * kBoxWX + (rt % kBoxBX + 1 + s % 3 - 1);
   }
   // boundary entry k's field: bit offset (from its table code, recomputed
   // where used rather than held in registers)
@@ -140,13 +187,16 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
     const int nb = (bcode[k] >> 16) & 511;
     return (t + k * kBlock - nb) * wn + nb * wwd;
   };
-  auto load_plane = [&](int z, int slot) {
+  auto x_plane = [&](int z, T* dst) {
     const bool zin = z >= 0 && z < g.gz;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int w = t + k * kBlock;
-      if (w < kBoxWin) xw[slot][w] = (zin && wok[k]) ? x[(int64_t)z * plane + woff[k]] : T(0);
-    }
+    for (int k = 0; k < 2; ++k)
+      dst[k] = zin && wok[k] ? x[(int64_t)z * plane + woff[k]] : T(0);
+  };
+  auto put_plane = [&](int slot, const T* src) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (t + k * kBlock < kBoxWin) xw[slot][t + k * kBlock] = src[k];
   };
   const int lox = ix > 0 ? -1 : 0, hix = ix < g.gx - 1 ? 1 : 0;
   const int loy = iy > 0 ? -1 : 0, hiy = iy < g.gy - 1 ? 1 : 0;
@@ -158,69 +208,58 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
     unsigned pw[kWords > 0 ? kWords : 1];
     T full[kFull > 0 ? kFull : 1];
   };
-  // entry e of (block, plane) gi's record: kb, q of its slots, then its codes flag
-  const int64_t ngroups = (int64_t)g.nbx * g.nby * g.gz;
-  auto kq_at = [&](int64_t gi, int e) {
-    return e < 2 * kSymU ? KQ[gi * (2 * kSymU) + e]
-         : e == 2 * kSymU ? KQ[ngroups * (2 * kSymU) + gi]
-                          : WKQ[gi * kSymWRec + (e - kRec)];
-  };
   auto load_raw = [&](int z, int lo, int cnt, Raw& r) {
-    const int64_t gz_idx = (int64_t)blk * g.gz + z;
 #pragma unroll
     for (int w = 0; w < kWords; ++w)
-      if (L.needed(w, lo, cnt)) r.pw[w] = PW[(gz_idx * kWords + w) * kBlock + t];
+      if (L.needed(w, lo, cnt)) r.pw[w] = PW[((rec0 + z) * kWords + w) * kBlock + t];
 #pragma unroll
     for (int u = lo; u < lo + cnt; ++u)
       if (!((kMask >> u) & 1u)) r.full[u - pack_rank(kMask, u)] = U[sym_at(g, blk, z, u, t)];
   };
-  // upper slots lo .. lo+cnt-1 of a plane from its loads, its kb, q record
-  // kq (in LDS, or in KQ for the first step's previous plane) and its codes
-  // flag (the same in every lane: a branch of the whole wave)
-  auto decode_as = [&](int lo, int cnt, const Raw& r, const T* kq, T* dst, auto codes) {
+  // upper slots lo .. lo+cnt-1 of a plane from its loads; its codes flag
+  // chooses a branch of the whole workgroup
+  auto decode_as = [&](int lo, int cnt, const Raw& r, const SymRec<T>& rec, T* dst, auto codes) {
 #pragma unroll
     for (int i = 0; i < cnt; ++i) {
       const int u = lo + i;
       if (L.width[u]) {
         const unsigned f = pack_field(r.pw + L.word[u], L.width[u], L.shift[u]);
-        dst[i] = pack_decode<T, decltype(codes)::value>(kq[2 * u], kq[2 * u + 1], f);
+        dst[i] = pack_decode<T, decltype(codes)::value>(rec.kb[u], rec.pow2(u), f);
       } else {
         dst[i] = r.full[u - pack_rank(kMask, u)];
       }
     }
   };
-  auto decode = [&](int lo, int cnt, const Raw& r, const T* kq, T flag, T* dst) {
-    if (!kHasKQ || __builtin_amdgcn_readfirstlane(flag != T(0) ? 1 : 0))
-      decode_as(lo, cnt, r, kq, dst, std::true_type{});
-    else
-      decode_as(lo, cnt, r, kq, dst, std::false_type{});
+  auto decode = [&](int lo, int cnt, const Raw& r, const SymRec<T>& rec, T* dst) {
+    if (kHasKQ && rec.codes) decode_as(lo, cnt, r, rec, dst, std::true_type{});
+    else decode_as(lo, cnt, r, rec, dst, std::false_type{});
   };
-  // this row's upper slot (dy, dx) is read by the block row at (tx+dx, ty+dy)
-  auto put_up = [&](const T* u9) {
-#pragma unroll
-    for (int dy = -1; dy <= 1; ++dy)
-#pragma unroll
-      for (int dx = -1; dx <= 1; ++dx) {
-        const int rx = tx + dx, ry = ty + dy;
-        if (rx >= 0 && rx < kBoxBX && ry >= 0 && ry < kBoxBY)
-          up[(dy + 1) * 3 + (dx + 1)][rx + kBoxBX * ry] = u9[(dy + 1) * 3 + (dx + 1)];
-      }
+  SymRec<T> rec;
+  auto load_rec = [&](int z) {
+    if (kHasKQ) rec = SymRec<T>::load(KQ + (rec0 + z) * kSymKRec);
   };
-  // Loads run one plane step ahead: step z's LDS writes and arithmetic go on
-  // while step z+1's x plane, upper values and boundary values are in flight.
-  T xn[2], kqn = T(0);
+  // this row's upper slot (dy, dx) of the next plane is read by the block row at
+  // (tx+dx, ty+dy); its own column's stays in pc
+  T pc = T(0);
+  auto put_up = [&](const T* u9, T xo) {
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+      const int rx = tx + j % 3 - 1, ry = ty + j / 3 - 1;
+      const T p = u9[j] * xo;
+      if (j == 4) pc = p;
+      else if (rx >= 0 && rx < kBoxBX && ry >= 0 && ry < kBoxBY)
+        up[j < 4 ? j : j - 1][rx + kBoxBX * ry] = p;
+    }
+  };
+  T xn[2], wqn = T(0), y0n = T(0), brn = T(0);
   // boundary entry k: its value's bits, or the two words holding its field
   unsigned long long bn[2] = {0ull, 0ull};
   Raw rn;
-  auto fetch = [&](int z) {  // x plane z+1, the values of plane z, kb and q of plane z+1
-    const bool zin = z + 1 < g.gz;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-      xn[k] = (t + k * kBlock < kBoxWin && zin && wok[k]) ? x[(int64_t)(z + 1) * plane + woff[k]]
-                                                          : T(0);
+  auto fetch = [&](int z) {  // x plane z+1, what step z reads, the boundary record of plane z+1
+    x_plane(z + 1, xn);
     if (live) load_raw(z, 0, kSymU, rn);
     if (wpk) {
-      const unsigned* wp = WPW + ((int64_t)blk * g.gz + z) * wwords;
+      const unsigned* wp = WPW + (rec0 + z) * wwords;
 #pragma unroll
       for (int k = 0; k < 2; ++k)
         if (bok[k]) {
@@ -228,7 +267,7 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
           bn[k] = ((unsigned long long)wp[wi + 1] << 32) | wp[wi];
         }
     } else {
-      const int64_t wbase = ((int64_t)blk * g.gz + z) * kSymNB;
+      const int64_t wbase = (rec0 + z) * kSymNB;
 #pragma unroll
       for (int k = 0; k < 2; ++k)
         if (bok[k]) {
@@ -237,35 +276,45 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
           else bn[k] = __float_as_uint(v);
         }
     }
+    if (live) {
+      const int64_t row = (int64_t)z * plane + ix + (int64_t)g.gx * iy;
+      if (ZERO_Y) y0n = y[row];
+      if (MODE == kResid) brn = bvec[row];
+    }
     // issued last: the compiler's waits for the loads above (before their
     // registers are reset) would otherwise include it
-    if (kHasKQ && t < nrec && z + 1 < z1) kqn = kq_at((int64_t)blk * g.gz + z + 1, t);
+    if (wpk && t < kSymWRec && z + 1 < z1) wqn = WKQ[(rec0 + z + 1) * kSymWRec + t];
   };
   T tsum = T(0);
-  // Every lower-slot entry starts at +0.0: the ones that no row writes (a
-  // neighbour past the box's edge inside the block, the plane below the
-  // box's first) then hold +0.0, and every entry is finite.
+  // Every product starts at +0.0: the ones that no row writes (a neighbour past
+  // the box's edge inside the block, the plane below the box's first) stay +0.0.
 #pragma unroll
-  for (int j = 0; j < 9; ++j) up[j][t] = T(0);
+  for (int j = 0; j < 8; ++j) up[j][t] = T(0);
 #pragma unroll
   for (int j = 0; j < 4; ++j) sm[j][t] = T(0);
-  __syncthreads();
-  load_plane(z0 - 1, (z0 + 2) % 3);
-  load_plane(z0, z0 % 3);
-  if (z0 > 0 && live) {
-    Raw r0;
-    T u9[9];
-    load_raw(z0 - 1, 5, 9, r0);
-    const int64_t gi = (int64_t)blk * g.gz + z0 - 1;
-    decode(5, 9, r0, kHasKQ ? KQ + gi * (2 * kSymU) : nullptr, kHasKQ ? kq_at(gi, 2 * kSymU) : T(1),
-           u9);
-    put_up(u9);
-  }
-  if (kHasKQ && t < nrec) kqs[z0 & 1][t] = kq_at((int64_t)blk * g.gz + z0, t);
+  T xa[2], xb[2];
+  Raw r0;
+  x_plane(z0 - 1, xa);
+  x_plane(z0, xb);
+  if (z0 > 0 && live) load_raw(z0 - 1, 5, 9, r0);
+  if (wpk && t < kSymWRec) kqs[z0 & 1][t] = WKQ[(rec0 + z0) * kSymWRec + t];
   fetch(z0);
-  if (kHasKQ) __syncthreads();  // plane z0's kb, q record
+  put_plane((z0 + 2) % 3, xa);
+  put_plane(z0 % 3, xb);
+  __syncthreads();
+  if (z0 > 0 && live) {
+    T u9[9];
+    load_rec(z0 - 1);
+    decode(5, 9, r0, rec, u9);
+    put_up(u9, xw[(z0 + 2) % 3][c0]);
+  }
+  load_rec(z0);
+  T xs[5];  // x of this row and of its upper same-plane neighbours, slots 13 .. 17
+#pragma unroll
+  for (int i = 0; i < 5; ++i)
+    xs[i] = xw[z0 % 3][c0 + (i < 2 ? i : kBoxWX + i - 3)];
   for (int z = z0; z < z1; ++z) {
-    // the boundary values first (into the LDS entries of the rows that read
+    // the boundary products first (into the LDS entries of the rows that read
     // them), while few registers are live
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -274,76 +323,73 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
         if constexpr (sizeof(T) == 8) v = __longlong_as_double((long long)bn[k]);
         else v = __uint_as_float((unsigned)bn[k]);
         if (wpk) {
-          const T* rec = kqs[z & 1] + kRec;
+          const T* rec = kqs[z & 1];
           const int wd = ((bcode[k] >> 25) & 1) ? wwd : wn, sl = (bcode[k] >> 26) & 15;
           const unsigned mask = wd >= 32 ? ~0u : (1u << wd) - 1u;
           const unsigned f = (unsigned)(bn[k] >> (bfield_off(k) & 31)) & mask;
           v = pack_decode<T, true>(rec[2 * sl], rec[2 * sl + 1], f);
         }
         const int rt = bcode[k] & 511, j = (bcode[k] >> 9) & 15;
-        if ((bcode[k] >> 13) & 1) sm[j][rt] = v;
-        else up[j][rt] = v;
+        const bool same = (bcode[k] >> 13) & 1;
+        const T p = v * xw[same ? z % 3 : (z + 2) % 3][bcell[k]];
+        if (same) sm[j][rt] = p;
+        else up[j < 4 ? j : j - 1][rt] = p;
       }
     T u[kSymU];
-    if (live) decode(0, kSymU, rn, kqs[z & 1], kHasKQ ? kqs[z & 1][2 * kSymU] : T(1), u);
-    // plane z+1's record: its buffer was last read by step z-1's decode,
-    // before step z-1's barriers, and is read after this step's first
-    if (kHasKQ && t < nrec && z + 1 < z1) kqs[(z + 1) & 1][t] = kqn;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-      if (t + k * kBlock < kBoxWin) xw[(z + 1) % 3][t + k * kBlock] = xn[k];
-    const int64_t row = (int64_t)z * plane + ix + (int64_t)g.gx * iy;
-    T y0 = T(0), br = T(0);
     if (live) {
-      if (ZERO_Y) y0 = y[row];
-      if (MODE == kResid) br = bvec[row];
-    }
-    if (live) {
+      decode(0, kSymU, rn, rec, u);
       // same-plane upper slots 14 + i at (dy, dx) = (0, 1), (1, -1), (1, 0),
       // (1, 1): read by the block row at (tx+dx, ty+dy)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int dy = i == 0 ? 0 : 1, dx = i == 0 ? 1 : i - 2;
         const int rx = tx + dx, ry = ty + dy;
-        if (rx < kBoxBX && rx >= 0 && ry < kBoxBY) sm[i][rx + kBoxBX * ry] = u[1 + i];
+        const T p = u[1 + i] * xs[0];
+        if (rx < kBoxBX && rx >= 0 && ry < kBoxBY) sm[i][rx + kBoxBX * ry] = p;
       }
     }
+    load_rec(min(z + 1, z1 - 1));
+    // the boundary record of plane z+1: its buffer was last read by step z-1's products,
+    // before step z-1's barriers, and is read after this step's
+    if (wpk && t < kSymWRec && z + 1 < z1) kqs[(z + 1) & 1][t] = wqn;
+    put_plane((z + 1) % 3, xn);
+    const T y0 = y0n, br = brn;
     if (z + 1 < z1) fetch(z + 1);
     __syncthreads();
+    const T xo = xs[0];
     if (live) {
       const int loz = z > 0 ? -1 : 0, hiz = z < g.gz - 1 ? 1 : 0;
       T sum = ZERO_Y ? T(0) * y0 : T(0);
+      // Out of range: the product is +-0.0, which leaves a sum that started at
+      // +0.0 unchanged (a sum of round-to-nearest additions from +0.0 is
+      // never -0.0); a sum that starts at 0*y (ZERO_Y) may be -0.0 and skips
+      // the term.
+      auto add = [&](int s, T p) {
+        const int sz = s / 9 - 1, sy = (s / 3) % 3 - 1, sx = s % 3 - 1;
+        const bool in = sx >= lox && sx <= hix && sy >= loy && sy <= hiy && sz >= loz && sz <= hiz;
+        const T next = sum + p;
+        sum = (ZERO_Y && !in) ? sum : next;
+      };
 #pragma unroll
-      for (int sz = -1; sz <= 1; ++sz) {
-        const T* wp = xw[(z + 3 + sz) % 3];
+      for (int s = 0; s < 9; ++s) add(s, s == 4 ? pc : up[s < 4 ? 7 - s : 8 - s][t]);
 #pragma unroll
-        for (int sy = -1; sy <= 1; ++sy)
+      for (int s = 9; s < 13; ++s) add(s, sm[12 - s][t]);
 #pragma unroll
-          for (int sx = -1; sx <= 1; ++sx) {
-            const int s = (sz + 1) * 9 + (sy + 1) * 3 + (sx + 1);
-            const int nc = c0 + sy * kBoxWX + sx;
-            const bool in = sx >= lox && sx <= hix && sy >= loy && sy <= hiy && sz >= loz &&
-                            sz <= hiz;
-            T v;
-            if (s >= 13) v = u[s - 13];
-            else if (sz < 0) v = up[26 - s - 18][t];
-            else v = sm[26 - s - 14][t];
-            const T p = v * wp[nc];
-            const T next = sum + p;
-            // Out of range: v is finite and the x entry +0.0, so p is +-0.0,
-            // which leaves a sum that started at +0.0 unchanged (a sum of
-            // round-to-nearest additions from +0.0 is never -0.0); a sum
-            // that starts at 0*y (ZERO_Y) may be -0.0 and skips the term.
-            sum = (ZERO_Y && !in) ? sum : next;
-          }
+      for (int i = 0; i < 5; ++i) add(13 + i, u[i] * xs[i]);
+      const T* wp = xw[(z + 1) % 3];
+#pragma unroll
+      for (int j = 0; j < 9; ++j) {
+        const T xv = wp[c0 + (j / 3 - 1) * kBoxWX + j % 3 - 1];
+        add(18 + j, u[5 + j] * xv);
+        if (j >= 4) xs[j - 4] = xv;
       }
       if (MODE == kResid) sum = T(1) * br + T(-1) * sum;
-      y[row] = sum;
-      if (MODE == kDot) tsum += sum * xw[z % 3][c0];
+      y[(int64_t)z * plane + ix + (int64_t)g.gx * iy] = sum;
+      if (MODE == kDot) tsum += sum * xo;
       if (MODE == kResid) tsum += sum * sum;
     }
     __syncthreads();
-    if (live) put_up(u + 5);
+    if (live) put_up(u + 5, xo);
   }
   if (MODE != kPlain) {
     const T s = block_sum<T>(tsum, red);

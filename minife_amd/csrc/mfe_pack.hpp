@@ -7,16 +7,14 @@
 // divides every one of them: the assembled entries are sums of element
 // terms, so even the analytically zero ones -- a cube's face neighbours,
 // about 1e-9 of the diagonal -- are multiples of the terms' last place).
-// The group stores a base kb and q side by side (KQ[2 group], KQ[2 group +
-// 1]) and each value an unsigned field f of W bits: f = 0 stands for +0.0,
-// f = 1 for 1.0 (the padding, Dirichlet rows and zeroed columns), and
-// otherwise the value is (kb + f) * q, exact (kb + f is an integer below
-// 2^53, or 2^24 in FP32, and scaling by a power of two is exact; the plan
-// checks every value).  kb = kmax - (2^W - 1), so the group's multiples fit
-// W bits when they span at most 2^W - 3.  After the 2 * slots * groups
-// entries of KQ, one per (block, plane) is 1 when any of its packed values
-// is +0.0 or 1.0 (a code can occur), else 0: the SpMV then skips the code
-// tests.
+// The group stores a base kb q and q side by side and each value an unsigned
+// field f of W bits: f = 0 stands for +0.0, f = 1 for 1.0 (the padding,
+// Dirichlet rows and zeroed columns), and otherwise the value is (kb + f) * q,
+// formed as f q + kb q and exact (kb + f is an integer below 2^53, or 2^24
+// in FP32, and scaling by a power of two is exact; the plan checks every value).
+// kb = kmax - (2^W - 1), so the group's multiples fit W bits when they span at
+// most 2^W - 3.  One flag per (block, plane) is 1 when any of its packed values
+// is +0.0 or 1.0 (a code can occur), else 0: the SpMV then skips the code tests.
 //
 // A form gives each slot a width: the cube's slots (every slot but the
 // analytically zero ones, NEAR) a narrow width, the NEAR slots the same
@@ -171,12 +169,15 @@ __host__ __device__ inline unsigned pack_field(const unsigned* w, int nw, int sh
   return ((w[0] >> sh) | (w[1] << (32 - sh))) & mask;
 }
 
-// The value of field f.  CODES: the plane may hold +0.0 or 1.0 (the value is
-// computed for every f and the codes selected afterwards, so no branch
-// separates the arithmetic from the loads of kb and q); else f >= 2.
+// The value (kb + f) q of field f from the base kbq = kb q: f q and kb q are
+// whole multiples of q and exact, and so is their sum, the stored value (two
+// instructions with one scalar operand each; an fma would need a copy of one).
+// CODES: the plane may hold +0.0 or 1.0 (the value is computed for every f and
+// the codes selected afterwards, so no branch separates the arithmetic from the
+// loads of kbq and q); else f >= 2.
 template <typename T, bool CODES>
-__device__ __forceinline__ T pack_decode(T kb, T q, unsigned f) {
-  const T v = (kb + (T)f) * q;
+__device__ __forceinline__ T pack_decode(T kbq, T q, unsigned f) {
+  const T v = (T)f * q + kbq;
   if constexpr (!CODES) {
     return v;
   } else {

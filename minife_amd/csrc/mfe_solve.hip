@@ -895,6 +895,14 @@ void box_chunks(BoxGeom& g, int resident, int64_t cap) {
   }
 }
 
+// Resident workgroups of a packed symmetric SpMV: its plane record sits in
+// scalar registers, and with about 100 of them a SIMD holds six waves, which the
+// occupancy query does not count (FP32 at 200^3: 1,521 workgroups 67.8 us,
+// 1,690 -- within the query's seven per CU -- 83.3 us).
+static int packed_resident(const void* kernel, int cus) {
+  return std::min(resident_groups(kernel, cus), 6 * std::max(cus, 1));
+}
+
 static bool box_applies(const mfe_csr* A) {
   return A->spmv_format == MFE_SPMV_AUTO && A->box_elems[0] > 0 && A->nrows > 0 &&
          (int64_t)(A->box_elems[0] + 1) * (A->box_elems[1] + 1) * (A->box_elems[2] + 1) ==
@@ -974,6 +982,7 @@ struct PackBits;
 template <>
 struct PackBits<double> {
   static constexpr double kLimit = 9007199254740992.0;  // 2^53
+  static constexpr int kLeast = -1022;  // a q below the least normal number is not packed
   // exponent of the lowest set bit; INT_MAX for +0.0 and 1.0; INT_MIN if unpackable
   __device__ static int lowbit(double v) {
     const long long b = __double_as_longlong(v);
@@ -991,6 +1000,7 @@ struct PackBits<double> {
 template <>
 struct PackBits<float> {
   static constexpr float kLimit = 16777216.0f;  // 2^24
+  static constexpr int kLeast = -126;
   __device__ static int lowbit(float v) {
     const int b = __float_as_int(v);
     if (b == 0 || v == 1.0f) return INT_MAX;
@@ -1045,7 +1055,7 @@ struct PackRange {
       qv = B::pow2(lb);
       kmin = lo / qv;
       kmax = hi / qv;
-      ok = fabs(kmin) < B::kLimit && fabs(kmax) < B::kLimit;
+      ok = lb >= B::kLeast && fabs(kmin) < B::kLimit && fabs(kmax) < B::kLimit;
     }
     const T span = kmax - kmin;  // exact: both are integers below the limit
     unsigned m = 0;
@@ -1093,7 +1103,7 @@ __global__ void plan_words_kernel(PlanWords* w) {
 // from W, the row's own values, and need none.
 //   With kq (and wkq: the boundary stream's groups), per (block, plane, slot)
 // group the least exponent of any value's lowest set bit and the range of
-// the values (16 threads per slot), giving kmax and q (kq[2 group], [+ 1];
+// the values (16 threads per slot), giving kmax and q (kq[rec + 2 u], [+ 1];
 // wkq[rec + 2 s], [+ 1]) and the widths every group fits.
 //   What bounds it: HBM, 27 values read and 14 + 282/256 written per row (9.2
 // GB at 300^3).  Filling one plane per workgroup and scanning U and W in two
@@ -1216,8 +1226,8 @@ __global__ __launch_bounds__(kBlock, 2) void boxsym_build_kernel(
         if (gs < kSymU) {
           fit &= w;
           if (gp == 0) {
-            kq[2 * (gi * kSymU + gs)] = kmax;
-            kq[2 * (gi * kSymU + gs) + 1] = qv;
+            kq[gi * kSymKRec + 2 * gs] = kmax;
+            kq[gi * kSymKRec + 2 * gs + 1] = qv;
           }
         }
       }
@@ -1249,15 +1259,14 @@ __global__ __launch_bounds__(kBlock, 2) void boxsym_build_kernel(
   }
 }
 
-// The fields of PF's slots (each fits its width W in every
-// group) from kb = kmax - (2^W - 1), so kb is an integer of at most kmax's
-// size and every field lies between 2 (the codes' successor) and 2^W - 1;
-// packed into words, kb replaces kmax.  Every value is decoded as the SpMV decodes it and compared
-// bit for bit (*bad = 1 on a mismatch).  The (block, plane)'s codes flag
-// (after the records) is 1 when any packed value took a code.
+// The fields of PF's slots (each fits its width W in every group) from kb =
+// kmax - (2^W - 1), so kb is an integer of at most kmax's size and every field
+// lies between 2 (the codes' successor) and 2^W - 1; packed into words, kb q
+// replaces kmax.  Every value is decoded as the SpMV decodes it and compared bit
+// for bit (*bad = 1 on a mismatch).  The (block, plane)'s codes flag is 1 when
+// any packed value took a code.
 template <typename T, typename P, int PF>
-__global__ __launch_bounds__(kBlock) void boxpack_pack_kernel(const T* __restrict__ U,
-                                                              T* __restrict__ kq,
+__global__ __launch_bounds__(kBlock) void boxpack_pack_kernel(const T* __restrict__ U, T* kq,
                                                               unsigned* __restrict__ PW,
                                                               unsigned* bad) {
   using B = PackBits<T>;
@@ -1265,11 +1274,21 @@ __global__ __launch_bounds__(kBlock) void boxpack_pack_kernel(const T* __restric
   constexpr int NS = P::kSlots, kWords = L.words;
   const int64_t gi = blockIdx.x;
   const int t = (int)threadIdx.x;
-  T base[NS];
-#pragma unroll
-  for (int u = 0; u < NS; ++u)
-    base[u] = kq[2 * (gi * NS + u)] - T((double)((1ull << L.width[u]) - 1ull));
-  __syncthreads();  // every thread has read kmax before thread 0 replaces it
+  T* const rec = kq + gi * kSymKRec;
+  // the record's slots go through LDS: threads 0 .. 13 read (kmax, q), and after
+  // the barrier (every read is done: its value is in LDS) write the SymRec
+  __shared__ T base[NS], qs[NS];
+  if (t < NS) {
+    base[t] = rec[2 * t] - T((double)((1ull << P::width(PF, t)) - 1ull));
+    qs[t] = rec[2 * t + 1];
+  }
+  __syncthreads();
+  unsigned* const rw = reinterpret_cast<unsigned*>(rec + NS);
+  if (t < NS) {
+    rec[t] = base[t] * qs[t];
+    if constexpr (sizeof(T) == 8) rw[t] = (unsigned)__double2hiint(qs[t]);
+    else rw[t] = __float_as_uint(qs[t]);
+  }
   unsigned pw[kWords];
 #pragma unroll
   for (int w = 0; w < kWords; ++w) pw[w] = 0;
@@ -1277,24 +1296,22 @@ __global__ __launch_bounds__(kBlock) void boxpack_pack_kernel(const T* __restric
 #pragma unroll
   for (int u = 0; u < NS; ++u) {
     if (!L.width[u]) continue;
-    const int64_t grp = gi * NS + u;
-    const T v = U[grp * kBlock + t];
-    const T qv = kq[2 * grp + 1];
+    const T v = U[(gi * NS + u) * kBlock + t];
+    const T qv = qs[u];
     const bool special = B::lowbit(v) == INT_MAX;
     const bool zero = special && v == T(0);
     coded = coded || special;
     const unsigned f = special ? (zero ? 0u : 1u) : (unsigned)(long long)(v / qv - base[u]);
-    ok = ok && B::same(pack_decode<T, true>(base[u], qv, f), v);
+    ok = ok && B::same(pack_decode<T, true>(base[u] * qv, qv, f), v);
     const int w = L.word[u], sh = L.shift[u];
     pw[w] |= f << sh;
     if (L.straddle[u]) pw[w + 1] |= f >> (32 - sh);
-    if (t == 0) kq[2 * grp] = base[u];
   }
 #pragma unroll
   for (int w = 0; w < kWords; ++w) PW[(gi * kWords + w) * kBlock + t] = pw[w];
   if (!ok) *bad = 1u;
   const int any = __syncthreads_or(coded ? 1 : 0);
-  if (t == 0) kq[2 * NS * (int64_t)gridDim.x + gi] = any ? T(1) : T(0);
+  if (t == 0) rw[NS] = any ? 1u : 0u;
 }
 
 // The symmetric box layout of A's values as T, with the groups' bases and
@@ -1328,7 +1345,7 @@ static int build_boxsym(mfe_ctx* ctx, mfe_csr* A) {
   if (!*du && !try_alloc(du, sizeof(T) * (size_t)sym_entries(g))) return MFE_OK;
   if (!*dw && !try_alloc(dw, sizeof(T) * (size_t)sym_bnd_entries(g))) return MFE_OK;
   // without room for these the values stay at full width
-  if (!*dk) (void)try_alloc(dk, sizeof(T) * (size_t)(2 * groups * kSymU + groups));
+  if (!*dk) (void)try_alloc(dk, sizeof(T) * (size_t)(groups * kSymKRec));
   T* wkq = nullptr;
   if constexpr (f64) {
     if (!A->boxwpack_kq) (void)try_alloc(&A->boxwpack_kq, sizeof(T) * (size_t)(groups * kSymWRec));
@@ -1444,7 +1461,7 @@ static int enqueue_pack(mfe_ctx* ctx, const T* U, int64_t groups, const unsigned
 // The packed boundary stream (mfe_boxsym.hpp) in form F: the fields of the
 // (block, plane)'s entries,
 // assembled in LDS, each decoded as the SpMV decodes it and compared bit for
-// bit (*bad = 1 on a mismatch); kb replaces kmax, and the codes flag is set.
+// bit (*bad = 1 on a mismatch); kb q replaces kmax, and the codes flag is set.
 template <typename T, int F>
 __global__ __launch_bounds__(kBlock) void boxwpack_pack_kernel(const T* __restrict__ W,
                                                                const int* __restrict__ tab,
@@ -1476,7 +1493,7 @@ __global__ __launch_bounds__(kBlock) void boxwpack_pack_kernel(const T* __restri
     const bool zero = special && v == T(0);
     coded = coded || special;
     const unsigned f = special ? (zero ? 0u : 1u) : (unsigned)(long long)(v / qs[sl] - base[sl]);
-    ok = ok && B::same(pack_decode<T, true>(base[sl], qs[sl], f), v);
+    ok = ok && B::same(pack_decode<T, true>(base[sl] * qs[sl], qs[sl], f), v);
     const int sh = off & 31;
     atomicOr(&acc[off >> 5], f << sh);
     if (sh + wd > 32) atomicOr(&acc[(off >> 5) + 1], f >> (32 - sh));
@@ -1485,7 +1502,7 @@ __global__ __launch_bounds__(kBlock) void boxwpack_pack_kernel(const T* __restri
   if (t < kWords) WPW[gi * kWords + t] = acc[t];
   if (!ok) *bad = 1u;
   const int any = __syncthreads_or(coded ? 1 : 0);
-  if (t < kSymWGroups) wkq[gi * kSymWRec + 2 * t] = base[t];
+  if (t < kSymWGroups) wkq[gi * kSymWRec + 2 * t] = base[t] * qs[t];
   if (t == 0) wkq[gi * kSymWRec + 2 * kSymWGroups] = any ? T(1) : T(0);
 }
 
@@ -1825,6 +1842,8 @@ static SpmvOp<T> spmv_op(const mfe_csr* A, bool allow_sell = true, bool allow_st
   return op;
 }
 
+constexpr int kWPackRows = 1 << 23;  // rows from which the packed boundary stream is read
+
 // y = A x on stream; *tiles_out = the number of partials written (one per
 // 256 rows in the CSR and SELL formats, one per workgroup in the box layout,
 // never more than max(kVecBlocks, one per 256 rows)).
@@ -1842,7 +1861,7 @@ static int launch_spmv(const SpmvOp<T>& op, const T* x, T* y, const T* bvec, T* 
     {
       if (op.pack) {
         auto run = [&](auto kern) {
-          box_chunks(g, resident_groups((const void*)kern, op.cus), cap);
+          box_chunks(g, packed_resident((const void*)kern, op.cus), cap);
           const int groups = g.nbx * g.nby * g.nzc;
           kern<<<groups, kBlock, 0, stream>>>(g, op.symu, op.symw, op.symtab, x, y, bvec,
                                                partials, done, op.pw, op.pkq, op.wpw, op.wkq,
@@ -1851,11 +1870,14 @@ static int launch_spmv(const SpmvOp<T>& op, const T* x, T* y, const T* bvec, T* 
           return (int)hipGetLastError();
         };
         return with_pack_form<T>(op.pack, [&](auto pf) {
-          // The packed boundary stream only where it was measured faster:
-          // FP64 without ZERO_Y (the CG's kernel); elsewhere the decode's
-          // registers cost more than the bytes it saves.
+          // The packed boundary stream only where it was measured faster: FP64
+          // without ZERO_Y (the CG's kernel) on matrices that the 256 MB of
+          // last-level cache cannot hold with their vectors; elsewhere its decode
+          // costs more than the bytes it saves (packed against full: 300^3 309
+          // and 324 us, 200^3 100 and 100, 128^3 36.6 and 34.2, 64^3 12.4 and
+          // 11.0; matvec_std at 300^3 385 and 371).
           if constexpr (!ZERO_Y && std::is_same<T, double>::value)
-            if (op.wpack) return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, true>);
+            if (op.wpack && n >= kWPackRows) return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, true>);
           return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, false>);
         });
       }
@@ -2924,11 +2946,12 @@ int mfe_spmv_plan(mfe_ctx* ctx, mfe_csr* A, int format, int64_t info[8]) {
                               : (const void*)spmv_box_kernel<double, false, kDot>;
       if (op.pack)
         with_pack_form<double>(op.pack, [&](auto pf) {
-          k = op.wpack ? (const void*)spmv_boxsym_kernel<double, false, kDot, decltype(pf)::value, true>
-                       : (const void*)spmv_boxsym_kernel<double, false, kDot, decltype(pf)::value, false>;
+          k = op.wpack && A->nrows >= kWPackRows
+                  ? (const void*)spmv_boxsym_kernel<double, false, kDot, decltype(pf)::value, true>
+                  : (const void*)spmv_boxsym_kernel<double, false, kDot, decltype(pf)::value, false>;
           return 0;
         });
-      box_chunks(g, resident_groups(k, op.cus),
+      box_chunks(g, op.pack ? packed_resident(k, op.cus) : resident_groups(k, op.cus),
                  std::max<int64_t>(kVecBlocks, cdiv(A->nrows, kSpmvRows)));
       info[0] = op.pack ? 6 : op.symu ? 5 : 4;
       info[1] = op.symu ? sym_entries(g) + sym_bnd_entries(g) : box_entries(g);

@@ -1170,3 +1170,30 @@ def test_cg_breakdown_by_norms_test(mfe, ctx, oracle_mod, replay):
     assert r.breakdown and r.num_iters == 0
     assert r.history[0, 1] == 0.0 and r.history[0, 2] == 0.0
     assert list(x.to_numpy()) == [0.0, 0.0]
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (15, 16, 2), (16, 15, 31), (33, 47, 5), (7, 64, 40)])
+@pytest.mark.parametrize("field", [False, True])
+def test_cg_spmv_kernel_bits(mfe, ctx, oracle_mod, dims, field):
+    """The fast CG's SpMV (variant 1) and the same kernel on full-width values
+    (variant 11) at block and chunk edges, with unit conductivity (packed
+    values) and with a conductivity field (full-width values): the bits of the
+    oracle's row sums, in the rows a boundary entry, a neighbour's product or
+    the thread's own column contributes to."""
+    say(f"case CG SpMV {dims} field={field}")
+    ne = dims[0] * dims[1] * dims[2]
+    kappa = np.exp(np.random.default_rng(4).normal(0, 0.5, ne)) if field else None
+    kv = mfe.Vector.from_numpy(kappa, ctx) if field else None
+    _, A, _ = mfe.build_problem(*dims, ctx=ctx, kappa=kv)
+    n = A.nrows
+    assert mfe.spmv_plan(A)["kernel"] in ("box-sym-packed", "box-sym")
+    h = A.to_host(rows=False)
+    Ao = oracle_mod.CSR(np.arange(n, dtype=np.int32), h["row_offsets"], h["cols"], h["vals"])
+    xh = np.random.default_rng(sum(dims)).standard_normal(n)
+    want = oracle_mod.matvec(Ao, xh)
+    x = mfe.Vector.from_numpy(xh, ctx)
+    y = mfe.Vector(n, ctx)
+    for variant in (1, 11):
+        y.fill(7.0)
+        mfe.time_matvec(A, x, y, variant=variant, reps=1)
+        assert bits_equal(y.to_numpy(), want), variant
