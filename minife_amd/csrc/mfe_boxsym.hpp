@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
   constexpr int kWords = L.words;
   constexpr bool kHasKQ = PF != kPackNone;
   constexpr bool wpk = kHasKQ && WPK;
-  if (done && *done) return;
+  const int stop = done ? *done : 0;  // tested once the first loads are in flight
   __shared__ T xw[3][kBoxWin];
   __shared__ T up[8][kBlock];  // products of the plane before's upper slots 18 + j
                                // (j != 4), by reading row
@@ -299,16 +299,18 @@ __global__ __launch_bounds__(kBlock) void spmv_boxsym_kernel(
   if (z0 > 0 && live) load_raw(z0 - 1, 5, 9, r0);
   if (wpk && t < kSymWRec) kqs[z0 & 1][t] = WKQ[(rec0 + z0) * kSymWRec + t];
   fetch(z0);
+  SymRec<T> rprev{};
+  if (kHasKQ && z0 > 0) rprev = SymRec<T>::load(KQ + (rec0 + z0 - 1) * kSymKRec);
+  load_rec(z0);
   put_plane((z0 + 2) % 3, xa);
   put_plane(z0 % 3, xb);
+  if (stop) return;
   __syncthreads();
   if (z0 > 0 && live) {
     T u9[9];
-    load_rec(z0 - 1);
-    decode(5, 9, r0, rec, u9);
+    decode(5, 9, r0, rprev, u9);
     put_up(u9, xw[(z0 + 2) % 3][c0]);
   }
-  load_rec(z0);
   T xs[5];  // x of this row and of its upper same-plane neighbours, slots 13 .. 17
 #pragma unroll
   for (int i = 0; i < 5; ++i)

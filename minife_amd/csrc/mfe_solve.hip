@@ -895,12 +895,19 @@ void box_chunks(BoxGeom& g, int resident, int64_t cap) {
   }
 }
 
-// Resident workgroups of a packed symmetric SpMV: its plane record sits in
-// scalar registers, and with about 100 of them a SIMD holds six waves, which the
-// occupancy query does not count (FP32 at 200^3: 1,521 workgroups 67.8 us,
-// 1,690 -- within the query's seven per CU -- 83.3 us).
-static int packed_resident(const void* kernel, int cus) {
-  return std::min(resident_groups(kernel, cus), 6 * std::max(cus, 1));
+// Workgroups per CU that the z chunks of a symmetric SpMV are sized for.  The
+// chunks are also the groups of its dot's partials, so the figure belongs to the
+// format (precision, packed form, packed boundary stream) and is not asked of the
+// occupancy query, whose answer follows the compiler's register allocation and
+// would move the sums with it (and which counts no scalar registers: with the
+// plane record in about 100 of them a SIMD holds at most six waves.  FP32 at
+// 200^3 in chunks for five per CU 71.3 us, six 67.8, seven 83.3).
+static int sym_slots(bool f64, int pack, bool wpack, int cus) {
+  const bool wide = pack == kPackAll16 || pack == kPackCube16Near32 || pack == kPackCube16;
+  int per = f64 ? (wpack && wide ? 3 : 4)
+          : pack == kPackNone || pack == kPackCube16 ? 7
+          : pack == kPackAll16 || pack == kPackAll10 ? 6 : 5;
+  return per * std::max(cus, 1);
 }
 
 static bool box_applies(const mfe_csr* A) {
@@ -1842,86 +1849,6 @@ static SpmvOp<T> spmv_op(const mfe_csr* A, bool allow_sell = true, bool allow_st
   return op;
 }
 
-constexpr int kWPackRows = 1 << 23;  // rows from which the packed boundary stream is read
-
-// y = A x on stream; *tiles_out = the number of partials written (one per
-// 256 rows in the CSR and SELL formats, one per workgroup in the box layout,
-// never more than max(kVecBlocks, one per 256 rows)).
-template <typename T, bool ZERO_Y, int MODE>
-static int launch_spmv(const SpmvOp<T>& op, const T* x, T* y, const T* bvec, T* partials,
-                       const int* done, hipStream_t stream, int* tiles_out) {
-  const int n = op.n;
-  if (n == 0) {
-    if (tiles_out) *tiles_out = 0;
-    return 0;
-  }
-  const int64_t cap = std::max<int64_t>(kVecBlocks, cdiv(n, kSpmvRows));
-  if (op.symu) {
-    BoxGeom g = op.bg;
-    {
-      if (op.pack) {
-        auto run = [&](auto kern) {
-          box_chunks(g, packed_resident((const void*)kern, op.cus), cap);
-          const int groups = g.nbx * g.nby * g.nzc;
-          kern<<<groups, kBlock, 0, stream>>>(g, op.symu, op.symw, op.symtab, x, y, bvec,
-                                               partials, done, op.pw, op.pkq, op.wpw, op.wkq,
-                                               op.wpack);
-          if (tiles_out) *tiles_out = groups;
-          return (int)hipGetLastError();
-        };
-        return with_pack_form<T>(op.pack, [&](auto pf) {
-          // The packed boundary stream only where it was measured faster: FP64
-          // without ZERO_Y (the CG's kernel) on matrices that the 256 MB of
-          // last-level cache cannot hold with their vectors; elsewhere its decode
-          // costs more than the bytes it saves (packed against full: 300^3 309
-          // and 324 us, 200^3 100 and 100, 128^3 36.6 and 34.2, 64^3 12.4 and
-          // 11.0; matvec_std at 300^3 385 and 371).
-          if constexpr (!ZERO_Y && std::is_same<T, double>::value)
-            if (op.wpack && n >= kWPackRows) return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, true>);
-          return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, false>);
-        });
-      }
-    }
-    box_chunks(g, resident_groups((const void*)spmv_boxsym_kernel<T, ZERO_Y, MODE>, op.cus), cap);
-    const int groups = g.nbx * g.nby * g.nzc;
-    spmv_boxsym_kernel<T, ZERO_Y, MODE><<<groups, kBlock, 0, stream>>>(
-        g, op.symu, op.symw, op.symtab, x, y, bvec, partials, done);
-    if (tiles_out) *tiles_out = groups;
-    return (int)hipGetLastError();
-  }
-  if (op.bvals) {
-    BoxGeom g = op.bg;
-    box_chunks(g, resident_groups((const void*)spmv_box_kernel<T, ZERO_Y, MODE>, op.cus), cap);
-    const int groups = g.nbx * g.nby * g.nzc;
-    spmv_box_kernel<T, ZERO_Y, MODE><<<groups, kBlock, 0, stream>>>(g, op.bvals, x, y, bvec,
-                                                                     partials, done);
-    if (tiles_out) *tiles_out = groups;
-    return (int)hipGetLastError();
-  }
-  const int tiles = (int)cdiv(n, kSpmvRows);
-  // operands the plan did not prepare (an FP32 CSR copy that was never made):
-  // refuse rather than launch on a null array
-  if (!op.svals && (!op.vals || !op.ro || !op.cols)) return (int)hipErrorInvalidValue;
-  if (op.xl) {
-    // padding slots read entry 0, slots past the width of a slice with bases entry lane
-    const size_t lds = sizeof(T) * (size_t)std::max(op.xmaxu, kSlice);
-    spmv_sellx_kernel<T, ZERO_Y, MODE><<<tiles, kBlock, lds, stream>>>(
-        n, op.nslices, op.soff, op.slen, op.xl, op.xltail, op.xaff, op.xsbase, op.svals, op.xroff,
-        op.xrcol, op.xrpos, op.xnu, x, y, bvec, partials, done);
-  } else if (op.svals) {
-    spmv_sell_kernel<T, ZERO_Y, MODE><<<tiles, kBlock, 0, stream>>>(
-        n, op.nslices, op.soff, op.slen, op.scols, op.svals, x, y, bvec, partials, done);
-  } else if (op.stream_ok) {
-    spmv_stream_kernel<T, ZERO_Y, MODE><<<tiles, kBlock, 0, stream>>>(
-        n, op.ro, op.cols, op.vals, x, y, bvec, partials, done);
-  } else {
-    spmv_rowwise_kernel<T, ZERO_Y, MODE><<<tiles, kBlock, 0, stream>>>(
-        n, op.ro, op.cols, op.vals, x, y, bvec, partials, done);
-  }
-  if (tiles_out) *tiles_out = tiles;
-  return (int)hipGetLastError();
-}
-
 // -------------------------------------------------------------- vectors -----
 
 template <typename T>
@@ -2055,16 +1982,22 @@ __global__ __launch_bounds__(kBlock) void dot_seq_kernel(int64_t n, const double
 // ------------------------------------------------------------------- CG -----
 //
 // Per iteration k (fast mode), all on one stream:
-//   cg_p       x += alpha_{k-1} p_{k-1} (deferred, see below); p = 1*r + beta*y
+//   advance    (k > 1) breakdown() if the norms were needed; end of k-1; loop
+//              test; rtrans, beta, normr of k
+//   p          x += alpha_{k-1} p_{k-1} (deferred, see below); p = 1*r + beta*y
 //   spmv       Ap = A p, workgroup partials of p.Ap
 //   reduce     first stage of the p.Ap reduction (large n only)
 //   update     p.Ap; breakdown test; alpha = rtrans / p.Ap;
 //              r = 1*r + (-alpha)*Ap, workgroup partials of r.r (and, only
 //              when p.Ap < brkdown_tol, of ||Ap||^2 and ||p||^2)
-//   next       breakdown() if the norms were needed; end of k; loop test;
-//              rtrans, beta, normr of k+1
+// The scalars live in two records: `st` as an iteration begins (written by
+// advance) and `mid` after its alpha (written by update).  A kernel reads one
+// and its first workgroup writes the other, so every workgroup of the p update
+// can do the advance step itself (from mid and the r.r partials: the same sums
+// in the same order give all of them the same scalars) and the separate launch
+// goes away; running it twice changes nothing.
 // The per-operation timing mode runs the same sums as separate kernels
-// (reduce, alpha, norms, norms-fin, update, next).
+// (reduce, alpha, norms, norms-fin, update, next) on st alone.
 // The reference updates x right after r (cg_solve.hpp:211-212).  Here the
 // update x = 1*x + alpha*p of iteration k is applied by the next cg_p, which
 // reads p anyway (or by cg_finish after the last iteration): the same
@@ -2161,11 +2094,14 @@ __global__ void cg_init_kernel(CgState* st, int max_iter, double tol) {
 
 // Fast mode scalar kernels (one workgroup each) ------------------------------
 template <typename T>
-__global__ __launch_bounds__(kBlock) void cg_first_fast_kernel(CgState* st, const T* partials,
-                                                               int np) {
+__global__ __launch_bounds__(kBlock) void cg_first_fast_kernel(CgState* st, CgState* mid,
+                                                               const T* partials, int np) {
   __shared__ T red[4];
   const T rr = sum_partials<T>(partials, np, red);
-  if (threadIdx.x == 0) cg_begin_first(st, (double)rr);
+  if (threadIdx.x == 0) {
+    cg_begin_first(st, (double)rr);
+    *mid = *st;  // what advance reads if there is nothing to do
+  }
 }
 
 template <typename T>
@@ -2221,8 +2157,9 @@ __global__ __launch_bounds__(kBlock) void cg_next_fast_kernel(CgState* st, const
 // k restarts at 1 (history rows stay in range; the captured iterations always
 // take p = gamma r + beta p).
 template <typename T>
-__global__ __launch_bounds__(kBlock) void cg_resume_kernel(CgState* st, const T* partials, int np,
-                                                           int max_iter, double tol) {
+__global__ __launch_bounds__(kBlock) void cg_resume_kernel(CgState* st, CgState* mid,
+                                                           const T* partials, int np, int max_iter,
+                                                           double tol) {
   __shared__ T red[4];
   const T rr = sum_partials<T>(partials, np, red);
   const T rp = sum_partials<T>(partials + np, np, red);
@@ -2240,6 +2177,7 @@ __global__ __launch_bounds__(kBlock) void cg_resume_kernel(CgState* st, const T*
     st->num_iters = 0;
     st->need_norms = 0;
     st->x_pending = 0;
+    *mid = *st;
   }
 }
 
@@ -2375,45 +2313,76 @@ __device__ T pap_two_stage(const T* partials, int np, const T* red2, int ng, T* 
     const T sg = sum_partials<T>(partials + g * kStage, min(kStage, np - g * kStage), red);
     if (threadIdx.x == 0) grp[g] = sg;
   }
+  if (ngi == 1) return T(0) + grp[0];  // what the second stage gives (thread 0)
   __syncthreads();
   return sum_partials<T>(grp, ngi, red);
 }
 
 // The fast iteration's alpha step folded into the r update: every workgroup
 // forms p.Ap (pap_two_stage) and alpha = rtrans / p.Ap itself, workgroup 0
-// records them (cg_alpha_or_defer).  p.Ap < 0: breakdown, nothing updated.
+// records them in mid (cg_alpha_or_defer).  p.Ap < 0: breakdown, nothing updated.
 // p.Ap < brkdown_tol: the breakdown test's norms are needed; alpha does not
 // depend on them (cg_solve.hpp:186-201), so r is updated at once and the
 // partials of ||Ap||^2 and ||p||^2 go beside those of r.r for
-// cg_next_norms_kernel, which decides before anything else of the iteration
+// advance, which decides before anything else of the iteration
 // becomes visible (x is updated only once the iteration has ended, and r is
 // internal).  Partials: r.r at out[b], ||Ap||^2 at out[G + b], ||p||^2 at
 // out[2G + b] (G = the grid), the same per-workgroup sums as cg_update_kernel
 // and cg_norms_kernel.
-template <typename T>
+// PRE: at most kUpdPre elements per thread (small n), whose loads do not depend
+// on alpha and are in flight while p.Ap is summed; else a grid-stride loop (for
+// which loading ahead measured slower: FP32 at 200^3 136 against 131 us per
+// iteration).
+constexpr int kUpdPre = 4;
+template <typename T, bool PRE>
 __global__ __launch_bounds__(kBlock) void cg_update_alpha_kernel(
-    int64_t n, CgState* st, T* __restrict__ r, const T* __restrict__ Ap, const T* __restrict__ p,
+    int64_t n, const CgState* st, CgState* mid, T* __restrict__ r, const T* __restrict__ Ap, const T* __restrict__ p,
     const T* partials, int np, const T* red2, int ng, double* hist, T* __restrict__ out) {
-  if (st->done) return;
   __shared__ T red[4];
   __shared__ double s_pap;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  T rv[kUpdPre], av[kUpdPre];
+  if (PRE) {
+#pragma unroll
+    for (int u = 0; u < kUpdPre; ++u) {
+      const int64_t i = i0 + u * stride;
+      rv[u] = i < n ? r[i] : T(0);
+      av[u] = i < n ? Ap[i] : T(0);
+    }
+  }
+  if (st->done) return;
   const double rtrans = st->rtrans, btol = st->brkdown_tol;
   const T pap_t = pap_two_stage<T>(partials, np, red2, ng, red);  // valid in thread 0
   if (threadIdx.x == 0) {
     s_pap = (double)pap_t;
-    if (blockIdx.x == 0) cg_alpha_or_defer(st, (double)pap_t, hist);
+    if (blockIdx.x == 0) {
+      CgState c = *st;
+      cg_alpha_or_defer(&c, (double)pap_t, hist);
+      *mid = c;
+    }
   }
   __syncthreads();
   const double pAp = s_pap;
   if (pAp < btol && pAp < 0) return;
   const bool need = pAp < btol;
   const T malpha = (T)(-(rtrans / pAp));
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   T acc = T(0);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const T ri = T(1) * r[i] + malpha * Ap[i];
-    r[i] = ri;
-    acc += ri * ri;
+  if (PRE) {
+#pragma unroll
+    for (int u = 0; u < kUpdPre; ++u) {
+      const int64_t i = i0 + u * stride;
+      if (i >= n) break;
+      const T ri = T(1) * rv[u] + malpha * av[u];
+      r[i] = ri;
+      acc += ri * ri;
+    }
+  } else {
+    for (int64_t i = i0; i < n; i += stride) {
+      const T ri = T(1) * r[i] + malpha * Ap[i];
+      r[i] = ri;
+      acc += ri * ri;
+    }
   }
   acc = block_sum<T>(acc, red);
   if (threadIdx.x == 0) out[blockIdx.x] = acc;
@@ -2426,27 +2395,163 @@ __global__ __launch_bounds__(kBlock) void cg_update_alpha_kernel(
   }
 }
 
-// End of a fast iteration after cg_update_alpha_kernel: the breakdown test's
-// norms if they were needed (cg_alpha_after_norms: breakdown ends the solve
-// before the iteration counts), then cg_next with r.r.
+// The scalars an iteration begins with, for every thread of the workgroup.
+struct CgBegin {
+  double beta, gamma, alpha_prev;
+  int done, x_pending, k;
+};
+
+// The step from mid (iteration k after its update) to the start of k + 1: the
+// breakdown test's norms if they were needed (cg_alpha_after_norms: breakdown
+// ends the solve before the iteration counts), then cg_next with r.r.  The
+// partials are the G r.r values (then G of ||Ap||^2 and G of ||p||^2) that
+// cg_update_alpha_kernel left at out.  Every workgroup gets the same bits; the
+// first one records them in st.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void cg_next_norms_kernel(CgState* st, const T* out, int G,
-                                                               double* hist) {
-  if (st->done) return;
-  __shared__ T red[4];
-  __shared__ int stop;
+__device__ __forceinline__ CgBegin cg_advance(const CgState* mid, CgState* st, const T* out, int G,
+                                              double* hist, T* red) {
+  __shared__ CgBegin begin;
+  const int need = mid->need_norms;
   const T rr = sum_partials<T>(out, G, red);
-  if (st->need_norms) {
-    const T ApAp = sum_partials<T>(out + G, G, red);
-    const T pp = sum_partials<T>(out + 2 * G, G, red);
-    if (threadIdx.x == 0) {
-      cg_alpha_after_norms(st, (double)ApAp, (double)pp, hist);
-      stop = st->done;
-    }
-    __syncthreads();
-    if (stop) return;
+  T ApAp = T(0), pp = T(0);
+  if (need) {
+    ApAp = sum_partials<T>(out + G, G, red);
+    pp = sum_partials<T>(out + 2 * G, G, red);
   }
-  if (threadIdx.x == 0) cg_next(st, (double)rr);
+  if (threadIdx.x == 0) {
+    CgState s = *mid;
+    if (!s.done) {
+      if (need) cg_alpha_after_norms(&s, (double)ApAp, (double)pp, hist);
+      if (!s.done) cg_next(&s, (double)rr);
+    }
+    begin = CgBegin{s.beta, s.gamma, s.alpha_prev, s.done, s.x_pending, s.k};
+    if (blockIdx.x == 0) *st = s;
+  }
+  __syncthreads();
+  return begin;
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void cg_advance_kernel(const CgState* mid, CgState* st,
+                                                            const T* out, int G, double* hist) {
+  __shared__ T red[4];
+  (void)cg_advance<T>(mid, st, out, G, hist, red);
+}
+
+// advance and the p update (cg_p_kernel) in one launch, four elements per
+// thread; their loads do not depend on the scalars and are in flight while the
+// partials are summed.
+constexpr int kFoldPer = 4;
+template <typename T>
+__global__ __launch_bounds__(kBlock) void cg_p_next_kernel(int64_t n, const CgState* mid,
+                                                           CgState* st, const T* out, int G,
+                                                           double* hist, const T* __restrict__ r,
+                                                           T* __restrict__ p, T* __restrict__ x,
+                                                           unsigned long long* progress) {
+  __shared__ T red[4];
+  const int64_t i0 = (int64_t)blockIdx.x * (kBlock * kFoldPer) + threadIdx.x;
+  T rv[kFoldPer], pv[kFoldPer], xv[kFoldPer];
+#pragma unroll
+  for (int u = 0; u < kFoldPer; ++u) {
+    const int64_t i = i0 + u * kBlock;
+    const bool in = i < n;
+    rv[u] = in ? r[i] : T(0);
+    pv[u] = in ? p[i] : T(0);
+    xv[u] = in ? x[i] : T(0);
+  }
+  const CgBegin c = cg_advance<T>(mid, st, out, G, hist, red);
+  if (blockIdx.x == 0 && threadIdx.x == 0)  // the host reads it from pinned memory
+    __hip_atomic_store(progress, (unsigned long long)c.k | ((unsigned long long)(c.done != 0) << 32),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (c.done) return;
+  const T beta = (T)c.beta, gamma = (T)c.gamma, a = (T)c.alpha_prev;
+#pragma unroll
+  for (int u = 0; u < kFoldPer; ++u) {
+    const int64_t i = i0 + u * kBlock;
+    if (i >= n) break;
+    if (c.x_pending) x[i] = T(1) * xv[u] + a * pv[u];
+    p[i] = gamma * rv[u] + beta * pv[u];
+  }
+}
+
+constexpr int kWPackRows = 1 << 23;  // rows from which the packed boundary stream is read
+
+// y = A x on stream; *tiles_out = the number of partials written (one per
+// 256 rows in the CSR and SELL formats, one per workgroup in the box layout,
+// never more than max(kVecBlocks, one per 256 rows)).
+template <typename T, bool ZERO_Y, int MODE>
+static int launch_spmv(const SpmvOp<T>& op, const T* x, T* y, const T* bvec, T* partials,
+                       const int* done, hipStream_t stream, int* tiles_out) {
+  const int n = op.n;
+  if (n == 0) {
+    if (tiles_out) *tiles_out = 0;
+    return 0;
+  }
+  const int64_t cap = std::max<int64_t>(kVecBlocks, cdiv(n, kSpmvRows));
+  if (op.symu) {
+    BoxGeom g = op.bg;
+    {
+      if (op.pack) {
+        auto run = [&](auto kern) {
+          box_chunks(g, sym_slots(sizeof(T) == 8, op.pack, !ZERO_Y && op.wpack, op.cus), cap);
+          const int groups = g.nbx * g.nby * g.nzc;
+          kern<<<groups, kBlock, 0, stream>>>(g, op.symu, op.symw, op.symtab, x, y, bvec,
+                                               partials, done, op.pw, op.pkq, op.wpw, op.wkq,
+                                               op.wpack);
+          if (tiles_out) *tiles_out = groups;
+          return (int)hipGetLastError();
+        };
+        return with_pack_form<T>(op.pack, [&](auto pf) {
+          // The packed boundary stream only where it was measured faster: FP64
+          // without ZERO_Y (the CG's kernel) on matrices that the 256 MB of
+          // last-level cache cannot hold with their vectors; elsewhere its decode
+          // costs more than the bytes it saves (packed against full: 300^3 309
+          // and 324 us, 200^3 100 and 100, 128^3 36.6 and 34.2, 64^3 12.4 and
+          // 11.0; matvec_std at 300^3 385 and 371).
+          if constexpr (!ZERO_Y && std::is_same<T, double>::value)
+            if (op.wpack && n >= kWPackRows) return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, true>);
+          return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, false>);
+        });
+      }
+    }
+    box_chunks(g, sym_slots(sizeof(T) == 8, kPackNone, false, op.cus), cap);
+    const int groups = g.nbx * g.nby * g.nzc;
+    spmv_boxsym_kernel<T, ZERO_Y, MODE><<<groups, kBlock, 0, stream>>>(
+        g, op.symu, op.symw, op.symtab, x, y, bvec, partials, done);
+    if (tiles_out) *tiles_out = groups;
+    return (int)hipGetLastError();
+  }
+  if (op.bvals) {
+    BoxGeom g = op.bg;
+    box_chunks(g, resident_groups((const void*)spmv_box_kernel<T, ZERO_Y, MODE>, op.cus), cap);
+    const int groups = g.nbx * g.nby * g.nzc;
+    spmv_box_kernel<T, ZERO_Y, MODE><<<groups, kBlock, 0, stream>>>(g, op.bvals, x, y, bvec,
+                                                                     partials, done);
+    if (tiles_out) *tiles_out = groups;
+    return (int)hipGetLastError();
+  }
+  const int tiles = (int)cdiv(n, kSpmvRows);
+  // operands the plan did not prepare (an FP32 CSR copy that was never made):
+  // refuse rather than launch on a null array
+  if (!op.svals && (!op.vals || !op.ro || !op.cols)) return (int)hipErrorInvalidValue;
+  if (op.xl) {
+    // padding slots read entry 0, slots past the width of a slice with bases entry lane
+    const size_t lds = sizeof(T) * (size_t)std::max(op.xmaxu, kSlice);
+    spmv_sellx_kernel<T, ZERO_Y, MODE><<<tiles, kBlock, lds, stream>>>(
+        n, op.nslices, op.soff, op.slen, op.xl, op.xltail, op.xaff, op.xsbase, op.svals, op.xroff,
+        op.xrcol, op.xrpos, op.xnu, x, y, bvec, partials, done);
+  } else if (op.svals) {
+    spmv_sell_kernel<T, ZERO_Y, MODE><<<tiles, kBlock, 0, stream>>>(
+        n, op.nslices, op.soff, op.slen, op.scols, op.svals, x, y, bvec, partials, done);
+  } else if (op.stream_ok) {
+    spmv_stream_kernel<T, ZERO_Y, MODE><<<tiles, kBlock, 0, stream>>>(
+        n, op.ro, op.cols, op.vals, x, y, bvec, partials, done);
+  } else {
+    spmv_rowwise_kernel<T, ZERO_Y, MODE><<<tiles, kBlock, 0, stream>>>(
+        n, op.ro, op.cols, op.vals, x, y, bvec, partials, done);
+  }
+  if (tiles_out) *tiles_out = tiles;
+  return (int)hipGetLastError();
 }
 
 // --------------------------------------------------------- workspace -----
@@ -2524,7 +2629,6 @@ struct GraphSlot {
   hipGraphExec_t exec = nullptr;
   const void *kA = nullptr, *kvals = nullptr, *kb = nullptr, *kx = nullptr;
   uint64_t kgen = 0;
-  unsigned kflags = 0;
   void drop() {
     if (exec) hipGraphExecDestroy(exec);
     if (graph) hipGraphDestroy(graph);
@@ -2539,8 +2643,9 @@ struct CgWorkspace {
   VecSet<float> v32;
   float *f_rhs = nullptr, *f_x = nullptr;  // inner system of the mixed solve
   int64_t f_n = -1;
-  CgState* st = nullptr;
+  CgState* st = nullptr;   // as an iteration begins; [1]: mid, after its alpha
   CgState* h_st = nullptr;  // pinned
+  unsigned long long* h_progress = nullptr;  // pinned: k, and done in bit 32 (cg_p_next_kernel)
   double* hist = nullptr;
   int64_t hist_cap = 0;
   GraphSlot g64, g32;
@@ -2559,6 +2664,7 @@ static void ws_free(CgWorkspace* w) {
   hipFree(w->st);
   hipFree(w->hist);
   if (w->h_st) hipHostFree(w->h_st);
+  if (w->h_progress) hipHostFree(w->h_progress);
   delete w;
 }
 
@@ -2585,8 +2691,9 @@ static int ws_get(mfe_ctx* ctx, int max_iter, CgWorkspace** out) {
   if (!w) {
     w = new CgWorkspace();
     ctx->cg = w;
-    MFE_CHECK(ctx, hipMalloc(&w->st, sizeof(CgState)));
+    MFE_CHECK(ctx, hipMalloc(&w->st, 2 * sizeof(CgState)));
     MFE_CHECK(ctx, hipHostMalloc(&w->h_st, sizeof(CgState), hipHostMallocDefault));
+    MFE_CHECK(ctx, hipHostMalloc(&w->h_progress, sizeof(*w->h_progress), hipHostMallocCoherent));
   }
   const int64_t hneed = 4 * (int64_t)(max_iter > 0 ? max_iter : 1);
   if (w->hist_cap < hneed) {
@@ -2631,11 +2738,12 @@ static inline void mark(OpTimer* tm, int slot) {
   if (tm) tm->mark(slot);
 }
 
-// One CG iteration body (k = 1 when y_for_p == r, k >= 2 when y_for_p == p).
+// One CG iteration of replay mode or of the per-operation timing mode, all
+// scalars in st (k = 1 when y_for_p == r, k >= 2 when y_for_p == p).
 template <typename T>
 static hipError_t enqueue_iteration(const SpmvOp<T>& op, VecSet<T>& v, CgState* st,
                                     double* hist, T* x, const T* y_for_p, bool replay,
-                                    hipStream_t s, OpTimer* tm = nullptr) {
+                                    hipStream_t s, OpTimer* tm) {
   const int64_t n = v.n;
   constexpr bool kF64 = sizeof(T) == 8;
   const unsigned vg = kF64 ? upd_grid(n) : vec_grid(n);
@@ -2643,12 +2751,13 @@ static hipError_t enqueue_iteration(const SpmvOp<T>& op, VecSet<T>& v, CgState* 
   mark(tm, MFE_T_WAXPY);
   int tiles = 0;
   const int* done = &st->done;
+  const bool fused = tm && tm->fused;
   if constexpr (std::is_same<T, double>::value) {
     if (replay) {
       launch_spmv<double, true, kPlain>(op, v.p, v.Ap, nullptr, nullptr, done, s, &tiles);
-      if (!(tm && tm->fused)) mark(tm, MFE_T_MATVEC);
+      if (!fused) mark(tm, MFE_T_MATVEC);
       cg_alpha_seq_kernel<<<1, kBlock, 0, s>>>(st, n, v.Ap, v.p, hist);
-      mark(tm, tm && tm->fused ? MFE_T_MATVECDOT : MFE_T_DOT);
+      mark(tm, fused ? MFE_T_MATVECDOT : MFE_T_DOT);
       cg_update_kernel<double, false><<<vg, kBlock, 0, s>>>(n, st, v.r, v.Ap, nullptr);
       mark(tm, MFE_T_WAXPY);
       cg_next_seq_kernel<<<1, kBlock, 0, s>>>(st, n, v.r);
@@ -2657,35 +2766,192 @@ static hipError_t enqueue_iteration(const SpmvOp<T>& op, VecSet<T>& v, CgState* 
     }
   }
   launch_spmv<T, false, kDot>(op, v.p, v.Ap, nullptr, v.partials, done, s, &tiles);
-  if (!(tm && tm->fused)) mark(tm, MFE_T_MATVEC);
+  if (!fused) mark(tm, MFE_T_MATVEC);
   const int nb2 = (int)cdiv(tiles, kStage);
-  if (tm) {
-    // Timed per operation: the dot products stay kernels of their own.
-    reduce_stage_kernel<T><<<nb2, kBlock, 0, s>>>(v.partials, tiles, 1, v.red2, done);
-    cg_alpha_fast_kernel<T><<<1, kBlock, 0, s>>>(st, v.red2, nb2, hist);
-    // Fused timing: the breakdown test's norms are untimed, as breakdown()
-    // is in the reference (slot -1).
-    if (tm->fused) mark(tm, MFE_T_MATVECDOT);
-    cg_norms_kernel<T><<<vg, kBlock, 0, s>>>(n, st, v.Ap, v.p, v.partials);
-    cg_norms_fin_kernel<T><<<1, kBlock, 0, s>>>(st, v.partials, (int)vg, hist);
-    mark(tm, tm->fused ? -1 : MFE_T_DOT);
-    cg_update_kernel<T, true><<<vg, kBlock, 0, s>>>(n, st, v.r, v.Ap, v.partials);
-    mark(tm, MFE_T_WAXPY);
-    cg_next_fast_kernel<T><<<1, kBlock, 0, s>>>(st, v.partials, (int)vg);
-    mark(tm, MFE_T_DOT);
+  // Timed per operation: the dot products stay kernels of their own.
+  reduce_stage_kernel<T><<<nb2, kBlock, 0, s>>>(v.partials, tiles, 1, v.red2, done);
+  cg_alpha_fast_kernel<T><<<1, kBlock, 0, s>>>(st, v.red2, nb2, hist);
+  // Fused timing: the breakdown test's norms are untimed, as breakdown()
+  // is in the reference (slot -1).
+  if (fused) mark(tm, MFE_T_MATVECDOT);
+  cg_norms_kernel<T><<<vg, kBlock, 0, s>>>(n, st, v.Ap, v.p, v.partials);
+  cg_norms_fin_kernel<T><<<1, kBlock, 0, s>>>(st, v.partials, (int)vg, hist);
+  mark(tm, fused ? -1 : MFE_T_DOT);
+  cg_update_kernel<T, true><<<vg, kBlock, 0, s>>>(n, st, v.r, v.Ap, v.partials);
+  mark(tm, MFE_T_WAXPY);
+  cg_next_fast_kernel<T><<<1, kBlock, 0, s>>>(st, v.partials, (int)vg);
+  mark(tm, MFE_T_DOT);
+  return hipGetLastError();
+}
+
+// Rows up to which every workgroup of the p update does the advance step itself
+// (cg_p_next_kernel): each reads the r.r partials (8 KB), 4 us of a launch less
+// per iteration (100^3 42.0 -> 40.4 us, 200^3 198 -> 194).
+constexpr int64_t kFoldRows = 1 << 23;
+// Rows up to which the host launches the iterations one by one, following the
+// GPU's progress: a captured chunk costs 170 us per solve with new vectors, a
+// stop every 25 iterations and empty iterations past the end, as much as the
+// launches it saves (30^3 to 1e-10: 1.26 ms against 1.38 captured; 128^3 20.2
+// against 19.8, so from there on captured).
+constexpr int64_t kEagerRows = 1500000;
+// Iterations the host may be ahead of the one the GPU reports to have begun (8
+// measured no better, and up to this many run empty past the last one).
+constexpr int kFoldAhead = 4;
+
+// One fast CG solve's launches (see the kernels' overview): the same sums in the
+// same order as the timing mode's.
+template <typename T>
+struct FastCg {
+  const SpmvOp<T>& op;
+  VecSet<T>& v;
+  CgState *st, *mid;
+  double* hist;
+  T* x;
+  hipStream_t s;
+  unsigned long long* progress;
+  static constexpr bool kF64 = sizeof(T) == 8;
+  int64_t n() const { return v.n; }
+  unsigned ug() const { return kF64 ? upd_grid(v.n) : vec_grid(v.n); }
+  T* out() const { return v.partials + v.part_base; }  // past the SpMV's partials
+
+  // p.Ap's first stage where it has one, then the r update (and alpha)
+  hipError_t update(int tiles) const {
+    const int nb2 = (int)cdiv(tiles, kStage);
+    const bool inline_groups = nb2 <= kInlineGroups;
+    if (!inline_groups)
+      reduce_stage_kernel<T><<<nb2, kBlock, 0, s>>>(v.partials, tiles, 1, v.red2, &st->done);
+    auto run = [&](auto kern) {
+      kern<<<ug(), kBlock, 0, s>>>(n(), st, mid, v.r, v.Ap, v.p, v.partials, tiles,
+                                   inline_groups ? nullptr : v.red2, nb2, hist, out());
+    };
+    if (n() <= (int64_t)ug() * kBlock * kUpdPre) run(cg_update_alpha_kernel<T, true>);
+    else run(cg_update_alpha_kernel<T, false>);
     return hipGetLastError();
   }
-  // Same sums in the same order as above, in 3 to 4 launches instead of 6.
-  // The r update's partials sit past the SpMV's (which it may read).
-  T* out = v.partials + v.part_base;
-  const bool inline_groups = nb2 <= kInlineGroups;
-  if (!inline_groups)
-    reduce_stage_kernel<T><<<nb2, kBlock, 0, s>>>(v.partials, tiles, 1, v.red2, done);
-  cg_update_alpha_kernel<T><<<vg, kBlock, 0, s>>>(n, st, v.r, v.Ap, v.p, v.partials, tiles,
-                                                  inline_groups ? nullptr : v.red2, nb2, hist,
-                                                  out);
-  cg_next_norms_kernel<T><<<1, kBlock, 0, s>>>(st, out, (int)vg, hist);
-  return hipGetLastError();
+  // the solve's first iteration: p from y (r, or the kept p) by the scalars in st
+  hipError_t first(const T* y) const {
+    cg_p_kernel<T><<<kF64 ? stream_grid(n()) : vec_grid(n()), kBlock, 0, s>>>(n(), st, v.r, y, v.p,
+                                                                              x);
+    int tiles = 0;
+    launch_spmv<T, false, kDot>(op, v.p, v.Ap, nullptr, v.partials, &st->done, s, &tiles);
+    return update(tiles);
+  }
+  // a later one
+  hipError_t next() const {
+    if (n() <= kFoldRows) {
+      cg_p_next_kernel<T><<<(unsigned)cdiv(n(), kBlock * kFoldPer), kBlock, 0, s>>>(
+          n(), mid, st, out(), (int)ug(), hist, v.r, v.p, x, progress);
+    } else {
+      cg_advance_kernel<T><<<1, kBlock, 0, s>>>(mid, st, out(), (int)ug(), hist);
+      cg_p_kernel<T><<<kF64 ? stream_grid(n()) : vec_grid(n()), kBlock, 0, s>>>(n(), st, v.r, v.p,
+                                                                                v.p, x);
+    }
+    int tiles = 0;
+    launch_spmv<T, false, kDot>(op, v.p, v.Ap, nullptr, v.partials, &st->done, s, &tiles);
+    return update(tiles);
+  }
+  // the scalars after the last iteration
+  hipError_t settle() const {
+    cg_advance_kernel<T><<<1, kBlock, 0, s>>>(mid, st, out(), (int)ug(), hist);
+    return hipGetLastError();
+  }
+};
+
+// The captured chunk of `chunk` iterations after the first, kept in slot for the
+// same matrix, right-hand side and x.
+template <typename T, typename F>
+static int capture_chunk(mfe_ctx* ctx, const FastCg<T>& f, GraphSlot& slot, const void* key_b,
+                         const void* key_x, F&& enqueue) {
+  hipStream_t s = ctx->stream;
+  if (slot.exec && slot.kA == f.op.A && slot.kgen == f.op.gen && slot.kvals == f.op.key() &&
+      slot.kb == key_b && slot.kx == key_x)
+    return MFE_OK;
+  slot.drop();
+  MFE_CHECK(ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+  hipError_t ce = enqueue();
+  hipGraph_t g = nullptr;
+  hipError_t ee = hipStreamEndCapture(s, &g);
+  if (ce != hipSuccess) {
+    if (g) (void)hipGraphDestroy(g);
+    return hip_fail(ctx, ce, "cg capture");
+  }
+  if (ee != hipSuccess) return hip_fail(ctx, ee, "hipStreamEndCapture");
+  slot.graph = g;
+  MFE_CHECK(ctx, hipGraphInstantiate(&slot.exec, g, nullptr, nullptr, 0));
+  slot.kA = f.op.A;
+  slot.kgen = f.op.gen;
+  slot.kvals = f.op.key();
+  slot.kb = key_b;
+  slot.kx = key_x;
+  return MFE_OK;
+}
+
+// The iterations after the first, up to number `last`: launched one by one behind
+// the GPU's progress word, or in captured chunks.
+template <typename T>
+static int run_cg_rest(mfe_ctx* ctx, const FastCg<T>& f, int last, bool eager, CgWorkspace* w,
+                       GraphSlot& slot, const void* key_b, const void* key_x) {
+  hipStream_t s = ctx->stream;
+  if (f.n() <= kEagerRows) {
+    volatile unsigned long long* prog = w->h_progress;
+    unsigned long long seen = 0;
+    for (int k = 2; k <= last && !(seen >> 32); ++k) {
+      if (hipError_t e = f.next()) return hip_fail(ctx, e, "cg iteration");
+      seen = *prog;
+      for (int spin = 0; !(seen >> 32) && (int)(seen & 0xffffffffu) < k - kFoldAhead; seen = *prog)
+        if (++spin % (1 << 16) == 0) {  // not for ever: the stream may have failed
+          const hipError_t e = hipStreamQuery(s);
+          if (e == hipSuccess) break;
+          if (e != hipErrorNotReady) return hip_fail(ctx, e, "cg iteration");
+        }
+    }
+    if (hipError_t e = f.settle()) return hip_fail(ctx, e, "cg_advance_kernel");
+    return MFE_OK;
+  }
+  if (eager) {
+    for (int k = 2; k <= last; ++k) {
+      if (hipError_t e = f.next()) return hip_fail(ctx, e, "cg iteration");
+      if (k % kGraphChunk == 0) {
+        if (hipError_t e = f.settle()) return hip_fail(ctx, e, "cg_advance_kernel");
+        MFE_CHECK(ctx, hipMemcpyAsync(w->h_st, w->st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+        MFE_CHECK(ctx, hipStreamSynchronize(s));
+        if (w->h_st->done) break;
+      }
+    }
+    if (hipError_t e = f.settle()) return hip_fail(ctx, e, "cg_advance_kernel");
+    return MFE_OK;
+  }
+  const int chunks = (int)cdiv(std::max(last - 1, 0), kGraphChunk);
+  if (chunks == 0) {
+    if (hipError_t e = f.settle()) return hip_fail(ctx, e, "cg_advance_kernel");
+    return MFE_OK;
+  }
+  if (int st = capture_chunk<T>(ctx, f, slot, key_b, key_x, [&] {
+        hipError_t e = hipSuccess;
+        for (int c = 0; c < kGraphChunk && e == hipSuccess; ++c) e = f.next();
+        return e == hipSuccess ? f.settle() : e;
+      }))
+    return st;
+  for (int c = 0; c < chunks; ++c) {
+    MFE_CHECK(ctx, hipGraphLaunch(slot.exec, s));
+    if (c + 1 < chunks) {
+      MFE_CHECK(ctx, hipMemcpyAsync(w->h_st, w->st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+      MFE_CHECK(ctx, hipStreamSynchronize(s));
+      if (w->h_st->done) break;
+    }
+  }
+  return MFE_OK;
+}
+
+// The pending x update and the final state in w->h_st.
+template <typename T>
+static int finish_cg(mfe_ctx* ctx, const FastCg<T>& f, CgWorkspace* w) {
+  hipStream_t s = ctx->stream;
+  cg_finish_kernel<T><<<stream_grid(f.n()), kBlock, 0, s>>>(f.n(), w->st, f.v.p, f.x);
+  MFE_LAUNCHED(ctx, "cg_finish_kernel");
+  MFE_CHECK(ctx, hipMemcpyAsync(w->h_st, w->st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+  MFE_CHECK(ctx, hipStreamSynchronize(s));
+  return MFE_OK;
 }
 
 // Unpreconditioned CG (cg_solve.hpp:69-229) on vectors of type T from the
@@ -2693,7 +2959,7 @@ static hipError_t enqueue_iteration(const SpmvOp<T>& op, VecSet<T>& v, CgState* 
 template <typename T>
 static int run_cg(mfe_ctx* ctx, const SpmvOp<T>& op, const T* b, T* x, int max_iter,
                   double tol, bool replay, bool eager, CgWorkspace* w, VecSet<T>& v,
-                  GraphSlot& slot, const void* key_b, const void* key_x, unsigned key_flags,
+                  GraphSlot& slot, const void* key_b, const void* key_x,
                   double* times = nullptr, bool fused = false) {
   hipStream_t s = ctx->stream;
   const int64_t n = v.n;
@@ -2720,59 +2986,26 @@ static int run_cg(mfe_ctx* ctx, const SpmvOp<T>& op, const T* b, T* x, int max_i
         cg_first_seq_kernel<<<1, kBlock, 0, s>>>(w->st, n, v.r);
     } else {
       dot_partial_kernel<T><<<vg, kBlock, 0, s>>>(n, v.r, v.r, v.partials);
-      cg_first_fast_kernel<T><<<1, kBlock, 0, s>>>(w->st, v.partials, (int)vg);
+      cg_first_fast_kernel<T><<<1, kBlock, 0, s>>>(w->st, w->st + 1, v.partials, (int)vg);
     }
     mark(tm, MFE_T_DOT);
     MFE_LAUNCHED(ctx, "cg prologue");
-    // Iteration 1: p = 1*r + 0*r.
-    hipError_t he = enqueue_iteration<T>(op, v, w->st, w->hist, x, v.r, replay, s, tm);
-    if (he != hipSuccess) return hip_fail(ctx, he, "cg iteration 1");
-    if (max_iter > 1) {
-      if (eager) {
-        for (int k = 2; k <= max_iter; ++k) {
-          he = enqueue_iteration<T>(op, v, w->st, w->hist, x, v.p, replay, s, tm);
-          if (he != hipSuccess) return hip_fail(ctx, he, "cg iteration");
-          if (k % kGraphChunk == 0) {
-            MFE_CHECK(ctx, hipMemcpyAsync(w->h_st, w->st, sizeof(CgState), hipMemcpyDeviceToHost, s));
-            MFE_CHECK(ctx, hipStreamSynchronize(s));
-            if (w->h_st->done) break;
-          }
-        }
-      } else {
-        const bool reuse = slot.exec && slot.kA == op.A && slot.kgen == op.gen &&
-                           slot.kvals == op.key() && slot.kb == key_b &&
-                           slot.kx == key_x && slot.kflags == key_flags;
-        if (!reuse) {
-          slot.drop();
-          MFE_CHECK(ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-          hipError_t ce = hipSuccess;
-          for (int c = 0; c < kGraphChunk && ce == hipSuccess; ++c)
-            ce = enqueue_iteration<T>(op, v, w->st, w->hist, x, v.p, replay, s);
-          hipGraph_t g = nullptr;
-          hipError_t ee = hipStreamEndCapture(s, &g);
-          if (ce != hipSuccess) {
-            if (g) hipGraphDestroy(g);
-            return hip_fail(ctx, ce, "cg capture");
-          }
-          if (ee != hipSuccess) return hip_fail(ctx, ee, "hipStreamEndCapture");
-          slot.graph = g;
-          MFE_CHECK(ctx, hipGraphInstantiate(&slot.exec, g, nullptr, nullptr, 0));
-          slot.kA = op.A;
-          slot.kgen = op.gen;
-          slot.kvals = op.key();
-          slot.kb = key_b;
-          slot.kx = key_x;
-          slot.kflags = key_flags;
-        }
-        const int chunks = (int)cdiv(max_iter - 1, kGraphChunk);
-        for (int c = 0; c < chunks; ++c) {
-          MFE_CHECK(ctx, hipGraphLaunch(slot.exec, s));
-          MFE_CHECK(ctx, hipMemcpyAsync(w->h_st, w->st, sizeof(CgState), hipMemcpyDeviceToHost, s));
-          if (c + 1 < chunks) {
-            MFE_CHECK(ctx, hipStreamSynchronize(s));
-            if (w->h_st->done) break;
-          }
-        }
+    if (!seq && !tm) {
+      *w->h_progress = 1;  // nothing that writes it is in flight: every solve ends synchronised
+      FastCg<T> f{op, v, w->st, w->st + 1, w->hist, x, s, w->h_progress};
+      // Iteration 1: p = 1*r + 0*r.
+      if (hipError_t he = f.first(v.r)) return hip_fail(ctx, he, "cg iteration 1");
+      if (int st = run_cg_rest<T>(ctx, f, max_iter, eager, w, slot, key_b, key_x)) return st;
+      return finish_cg<T>(ctx, f, w);
+    }
+    for (int k = 1; k <= max_iter; ++k) {
+      hipError_t he =
+          enqueue_iteration<T>(op, v, w->st, w->hist, x, k == 1 ? v.r : v.p, replay, s, tm);
+      if (he != hipSuccess) return hip_fail(ctx, he, "cg iteration");
+      if (k % kGraphChunk == 0) {
+        MFE_CHECK(ctx, hipMemcpyAsync(w->h_st, w->st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+        MFE_CHECK(ctx, hipStreamSynchronize(s));
+        if (w->h_st->done) break;
       }
     }
     cg_finish_kernel<T><<<stream_grid(n), kBlock, 0, s>>>(n, w->st, v.p, x);
@@ -2796,47 +3029,15 @@ static int run_cg_resume(mfe_ctx* ctx, const SpmvOp<T>& op, T* x, int max_iter, 
   const int64_t n = v.n;
   if (n == 0) return MFE_OK;
   const unsigned vg = vec_grid(n);
+  FastCg<T> f{op, v, w->st, w->st + 1, w->hist, x, s, w->h_progress};
+  *w->h_progress = 1;
   dot_partial_kernel<T><<<vg, kBlock, 0, s>>>(n, v.r, v.r, v.partials);
   dot_partial_kernel<T><<<vg, kBlock, 0, s>>>(n, v.r, v.p, v.partials + vg);
-  cg_resume_kernel<T><<<1, kBlock, 0, s>>>(w->st, v.partials, (int)vg, max_iter, tol);
+  cg_resume_kernel<T><<<1, kBlock, 0, s>>>(w->st, w->st + 1, v.partials, (int)vg, max_iter, tol);
   MFE_LAUNCHED(ctx, "cg_resume_kernel");
-  const bool reuse = slot.exec && slot.kA == op.A && slot.kgen == op.gen &&
-                     slot.kvals == op.key() && slot.kb == key_b && slot.kx == key_x &&
-                     slot.kflags == 0;
-  if (!reuse) {
-    slot.drop();
-    MFE_CHECK(ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    hipError_t ce = hipSuccess;
-    for (int c = 0; c < kGraphChunk && ce == hipSuccess; ++c)
-      ce = enqueue_iteration<T>(op, v, w->st, w->hist, x, v.p, false, s);
-    hipGraph_t g = nullptr;
-    hipError_t ee = hipStreamEndCapture(s, &g);
-    if (ce != hipSuccess) {
-      if (g) (void)hipGraphDestroy(g);
-      return hip_fail(ctx, ce, "cg capture");
-    }
-    if (ee != hipSuccess) return hip_fail(ctx, ee, "hipStreamEndCapture");
-    slot.graph = g;
-    MFE_CHECK(ctx, hipGraphInstantiate(&slot.exec, g, nullptr, nullptr, 0));
-    slot.kA = op.A;
-    slot.kgen = op.gen;
-    slot.kvals = op.key();
-    slot.kb = key_b;
-    slot.kx = key_x;
-    slot.kflags = 0;
-  }
-  const int chunks = (int)cdiv(std::max(max_iter, 1), kGraphChunk);
-  for (int c = 0; c < chunks; ++c) {
-    MFE_CHECK(ctx, hipGraphLaunch(slot.exec, s));
-    MFE_CHECK(ctx, hipMemcpyAsync(w->h_st, w->st, sizeof(CgState), hipMemcpyDeviceToHost, s));
-    MFE_CHECK(ctx, hipStreamSynchronize(s));
-    if (w->h_st->done) break;
-  }
-  cg_finish_kernel<T><<<stream_grid(n), kBlock, 0, s>>>(n, w->st, v.p, x);
-  MFE_LAUNCHED(ctx, "cg_finish_kernel");
-  MFE_CHECK(ctx, hipMemcpyAsync(w->h_st, w->st, sizeof(CgState), hipMemcpyDeviceToHost, s));
-  MFE_CHECK(ctx, hipStreamSynchronize(s));
-  return MFE_OK;
+  if (hipError_t he = f.first(v.p)) return hip_fail(ctx, he, "cg iteration 1");
+  if (int st = run_cg_rest<T>(ctx, f, max_iter, false, w, slot, key_b, key_x)) return st;
+  return finish_cg<T>(ctx, f, w);
 }
 
 // ---- allocation-free SpMV + dot ---------------------------------------------
@@ -2942,17 +3143,10 @@ int mfe_spmv_plan(mfe_ctx* ctx, mfe_csr* A, int format, int64_t info[8]) {
     const SpmvOp<double> op = spmv_op<double>(A);
     if (op.bvals || op.symu) {  // box layout: stored entries; the CG kernel's launch
       BoxGeom g = op.bg;
-      const void* k = op.symu ? (const void*)spmv_boxsym_kernel<double, false, kDot>
-                              : (const void*)spmv_box_kernel<double, false, kDot>;
-      if (op.pack)
-        with_pack_form<double>(op.pack, [&](auto pf) {
-          k = op.wpack && A->nrows >= kWPackRows
-                  ? (const void*)spmv_boxsym_kernel<double, false, kDot, decltype(pf)::value, true>
-                  : (const void*)spmv_boxsym_kernel<double, false, kDot, decltype(pf)::value, false>;
-          return 0;
-        });
-      box_chunks(g, op.pack ? packed_resident(k, op.cus) : resident_groups(k, op.cus),
-                 std::max<int64_t>(kVecBlocks, cdiv(A->nrows, kSpmvRows)));
+      const int slots = op.symu ? sym_slots(true, op.pack, op.wpack != kPackNone, op.cus)
+                                : resident_groups((const void*)spmv_box_kernel<double, false, kDot>,
+                                                  op.cus);
+      box_chunks(g, slots, std::max<int64_t>(kVecBlocks, cdiv(A->nrows, kSpmvRows)));
       info[0] = op.pack ? 6 : op.symu ? 5 : 4;
       info[1] = op.symu ? sym_entries(g) + sym_bnd_entries(g) : box_entries(g);
       info[2] = (int64_t)g.nbx * g.nby * g.nzc;
@@ -3207,8 +3401,8 @@ int mfe_cg_solve(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_vec* x, i
   double op_times[5] = {0, 0, 0, 0, 0};
   MFE_CHECK(ctx, hipEventRecord(ctx->t_start, ctx->stream));
   if ((st = ensure_plan(ctx, A, true, false))) return st;
-  st = run_cg<double>(ctx, spmv_op<double>(A), b->d, x->d, max_iter, tol, replay, eager, w, w->v64, w->g64,
-                      b, x, flags & MFE_CG_REPLAY, times ? op_times : nullptr,
+  st = run_cg<double>(ctx, spmv_op<double>(A), b->d, x->d, max_iter, tol, replay, eager, w,
+                      w->v64, w->g64, b, x, times ? op_times : nullptr,
                       (flags & MFE_CG_FUSED) != 0);
   if (st) return st;
   MFE_CHECK(ctx, hipEventRecord(ctx->t_stop, ctx->stream));
@@ -3318,7 +3512,7 @@ int mfe_cg_solve_mixed_ex(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_
       to_f32_kernel<<<vg, kBlock, 0, s>>>(n, v.r, 1.0 / scale, w->f_rhs);
       MFE_LAUNCHED(ctx, "to_f32_kernel");
       if ((st = run_cg<float>(ctx, op32, w->f_rhs, w->f_x, max_inner, tol_k * (keep ? rn : 1.0),
-                              false, false, w, w->v32, w->g32, w->f_rhs, w->f_x, 0)))
+                              false, false, w, w->v32, w->g32, w->f_rhs, w->f_x)))
         return st;
     }
     const CgState hs = *w->h_st;

@@ -1197,3 +1197,30 @@ def test_cg_spmv_kernel_bits(mfe, ctx, oracle_mod, dims, field):
         y.fill(7.0)
         mfe.time_matvec(A, x, y, variant=variant, reps=1)
         assert bits_equal(y.to_numpy(), want), variant
+
+
+@pytest.mark.parametrize("dims,iters", [((12, 9, 7), (0, 1, 2, 3, 6, 25, 26, 60)),
+                                        ((118, 117, 119), (1, 2, 25, 26, 27, 51))])
+def test_cg_launch_forms_agree(mfe, ctx, dims, iters):
+    """The fast loop (launched one by one behind the GPU's progress, or captured;
+    the p update advancing the scalars itself) against the per-operation timing
+    mode, whose scalars and dots are kernels of their own: the same iteration
+    counts, histories and x, bit for bit, for counts around the loop's first
+    iterations and the captured chunk, and when the tolerance ends the loop."""
+    say(f"case CG launch forms {dims}")
+    mesh, A, _ = mfe.build_problem(*dims, ctx=ctx)
+    n = A.nrows
+    bh = np.random.default_rng(7).standard_normal(n)
+    bh[mesh.bc_rows_0] = 0.0
+    bh[mesh.bc_rows_1] = 0.0
+    b = mfe.Vector.from_numpy(bh, ctx)
+    x1, x2 = mfe.Vector(n, ctx), mfe.Vector(n, ctx)
+    for kw in [dict(max_iter=k, tolerance=0.0) for k in iters] + \
+            [dict(max_iter=400, tolerance=1e-3, relative=True)]:
+        x1.fill(0.5)
+        x2.fill(0.5)
+        r1 = mfe.cg_solve(A, b, x1, history=True, **kw)
+        r2 = mfe.cg_solve(A, b, x2, history=True, eager=True, **kw)
+        assert r1.num_iters == r2.num_iters and r1.normr == r2.normr, kw
+        assert bits_equal(x1.to_numpy(), x2.to_numpy()), kw
+        assert bits_equal(r1.history, r2.history), kw
