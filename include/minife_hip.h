@@ -16,7 +16,10 @@
  *     {x0,x1,y0,y1,z0,z1} in elements, as ref/utils/Box.hpp.
  *   - Ordinals are int32 and Scalar is double, as ref/src/Makefile.gnu.serial;
  *     nnz must stay below 2^31 (the reference's LocalOrdinal is int).
- *   - Handles own device memory.  Host pointers are borrowed for the call.
+ *   - Handles own device memory.  What destroyed matrices and vectors held is
+ *     kept for later ones on the same context, at most an eighth of the
+ *     device's memory over all contexts, until an allocation fails or the
+ *     context goes.  Host pointers are borrowed for the call.
  *     Calls on one ctx are ordered on its single HIP stream; a ctx is not
  *     thread-safe.  No C++ exception crosses this boundary.
  */

@@ -468,14 +468,18 @@ class simple_mesh_description:
         if not np.array_equal(self.local_box, self.global_box):
             raise NotImplementedError("one rank: local box must equal the global box")
         gx, gy, gz = int(gb[1]) + 1, int(gb[3]) + 1, int(gb[5]) + 1
-        iz, iy, ix = np.meshgrid(np.arange(gz), np.arange(gy), np.arange(gx), indexing="ij")
-        ids = (ix + gx * iy + gx * gy * iz).reshape(-1)
-        ix, iy, iz = ix.reshape(-1), iy.reshape(-1), iz.reshape(-1)
         hot, cold = (gx - 1, 0) if self.hot_face else (0, gx - 1)
-        in0 = (ix == cold) | (iy == 0) | (iz == 0) | (iy == gy - 1) | (iz == gz - 1)
-        in1 = ix == hot
-        self.bc_rows_0 = ids[in0].astype(np.int32)
-        self.bc_rows_1 = ids[in1].astype(np.int32)
+        # u = 0: the first and last z planes whole, of every other plane its
+        # first and last lines and the cold column, in ascending id
+        line = np.zeros((gy, gx), bool)
+        line[0] = line[-1] = True
+        line[:, cold] = True
+        edge = np.flatnonzero(line).astype(np.int32)
+        plane = gx * gy
+        inner = np.arange(1, gz - 1, dtype=np.int32)[:, None] * np.int32(plane) + edge
+        first = np.arange(plane, dtype=np.int32)
+        self.bc_rows_0 = np.concatenate([first, inner.reshape(-1), first + np.int32((gz - 1) * plane)])
+        self.bc_rows_1 = np.arange(hot, plane * gz, gx, dtype=np.int32)
 
     @property
     def nodes(self):

@@ -580,7 +580,7 @@ static int element_loop(mfe_ctx* ctx, const int gbox[6], const int ebox[6], mfe_
   // the Jacobian column tables, then the Gauss tables (read by every element)
   const int64_t njac = 24 * ((int64_t)Nx + Ny + Nz);
   double* djac = nullptr;
-  hipError_t e1 = hipMalloc(&djac, sizeof(double) * (size_t)njac + sizeof(HexTables));
+  hipError_t e1 = dev_alloc(ctx, &djac, sizeof(double) * (size_t)njac + sizeof(HexTables));
   if (e1 != hipSuccess) return hip_fail(ctx, e1, "hipMalloc(element tables)");
   HexTables* dtab = reinterpret_cast<HexTables*>(djac + njac);
   copy_tables_kernel<<<1, kBlock, 0, ctx->stream>>>(tab, dtab);
@@ -611,7 +611,7 @@ static int element_loop(mfe_ctx* ctx, const int gbox[6], const int ebox[6], mfe_
   if (le != hipSuccess) st = hip_fail(ctx, le, "element_gather_kernel");
   hipError_t se = hipStreamSynchronize(ctx->stream);
   if (st == MFE_OK && se != hipSuccess) st = hip_fail(ctx, se, "assembly");
-  hipFree(djac);
+  dev_free(ctx, djac);
   return st;
 }
 
@@ -649,7 +649,7 @@ int mfe_impose_dirichlet(mfe_ctx* ctx, double value, mfe_csr* A, mfe_vec* b, int
   }
   unsigned char* flags = nullptr;
   // flags[0, n): BC rows; flags[n, 2n): rows that may hold a BC column
-  hipError_t e = hipMalloc(&flags, 2 * (size_t)n);
+  hipError_t e = dev_alloc(ctx, &flags, 2 * (size_t)n);
   if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc(bc flags)");
   unsigned char* const touch = flags + n;
   // the box stencil is structurally symmetric: only the BC rows' neighbours
@@ -690,7 +690,7 @@ int mfe_impose_dirichlet(mfe_ctx* ctx, double value, mfe_csr* A, mfe_vec* b, int
   } while (0);
   hipError_t se = hipStreamSynchronize(ctx->stream);
   if (st == MFE_OK && se != hipSuccess) st = hip_fail(ctx, se, "impose_dirichlet");
-  hipFree(flags);
+  dev_free(ctx, flags);
   return st;
 }
 

@@ -183,6 +183,19 @@ int stage_buffer(mfe_ctx* ctx, void** out);
 int upload_bytes(mfe_ctx* ctx, void* dst, const void* src, size_t bytes);
 int download_bytes(mfe_ctx* ctx, void* dst, const void* src, size_t bytes);
 int hip_fail(mfe_ctx* ctx, hipError_t e, const char* what);
+// Device memory of matrices, vectors and their plans (mfe_api.hip).  dev_free
+// keeps the block for the next dev_alloc of about its size on the same context:
+// work on a context is ordered on its one stream, so a block can be handed out
+// again while kernels that used it are still queued.  Blocks kept on a device
+// are at most an eighth of its memory together (the oldest go first), all of
+// them go when an allocation fails, and a context's go with it.  Safe from
+// several threads.
+hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes);
+template <typename P>
+inline hipError_t dev_alloc(mfe_ctx* ctx, P** out, size_t bytes) {
+  return dev_alloc_bytes(ctx, reinterpret_cast<void**>(out), bytes);
+}
+void dev_free(mfe_ctx* ctx, void* p);
 // Recompute A->max_block_nnz on the device (synchronises the stream).
 int plan_spmv(mfe_ctx* ctx, mfe_csr* A);
 

@@ -823,7 +823,7 @@ static int ensure_lines(mfe_ctx* ctx, const mfe_csr* Ac) {
   if (!A->sell_ok || A->sell_lines_valid) return MFE_OK;
   const int ns = (int)A->sell_nslices;
   if (!A->sell_lines)
-    MFE_CHECK(ctx, hipMalloc(&A->sell_lines, sizeof(int) * kLineStride * (size_t)std::max(ns, 1)));
+    MFE_CHECK(ctx, dev_alloc(ctx, &A->sell_lines, sizeof(int) * kLineStride * (size_t)std::max(ns, 1)));
   if (ns > 0) {
     sell_lines_kernel<<<(unsigned)cdiv(ns, kBlock / kWave), kBlock, 0, ctx->stream>>>(
         (int)A->nrows, ns, A->sell_off, A->sell_len, A->sell_cols, A->sell_lines);

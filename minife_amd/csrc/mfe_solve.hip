@@ -606,13 +606,13 @@ __global__ __launch_bounds__(kBlock) void spmv_sellx_kernel(
 }
 
 static void sellx_release(mfe_csr* A) {
-  (void)hipFree(A->sellx_lcols);
-  (void)hipFree(A->sellx_roff);
-  (void)hipFree(A->sellx_rcol);
-  (void)hipFree(A->sellx_rpos);
-  (void)hipFree(A->sellx_nu);
-  (void)hipFree(A->sellx_aff);
-  (void)hipFree(A->sellx_sbase);
+  dev_free(A->ctx, A->sellx_lcols);
+  dev_free(A->ctx, A->sellx_roff);
+  dev_free(A->ctx, A->sellx_rcol);
+  dev_free(A->ctx, A->sellx_rpos);
+  dev_free(A->ctx, A->sellx_nu);
+  dev_free(A->ctx, A->sellx_aff);
+  dev_free(A->ctx, A->sellx_sbase);
   A->sellx_lcols = nullptr;
   A->sellx_roff = A->sellx_rcol = A->sellx_rpos = A->sellx_nu = nullptr;
   A->sellx_aff = nullptr;
@@ -625,12 +625,12 @@ static void sellx_release(mfe_csr* A) {
 void sell_release(mfe_csr* A) {
   A->plan_gen = next_plan_gen();
   sellx_release(A);
-  hipFree(A->sell_off);
-  hipFree(A->sell_len);
-  hipFree(A->sell_cols);
-  hipFree(A->sell_vals);
-  hipFree(A->sell_vals32);
-  hipFree(A->sell_lines);
+  dev_free(A->ctx, A->sell_off);
+  dev_free(A->ctx, A->sell_len);
+  dev_free(A->ctx, A->sell_cols);
+  dev_free(A->ctx, A->sell_vals);
+  dev_free(A->ctx, A->sell_vals32);
+  dev_free(A->ctx, A->sell_lines);
   A->sell_lines = nullptr;
   A->sell_lines_valid = false;
   A->sell_off = nullptr;
@@ -653,14 +653,11 @@ static void sell_disable(mfe_csr* A) {
   A->sell_max_len = maxw;
 }
 
-// hipMalloc that leaves no sticky error behind when memory is short (the
-// plan then falls back to the CSR kernels).
+// False (and a null pointer) when memory is short: the plan then falls back to
+// another format.
 template <typename P>
-static bool try_alloc(P** p, size_t bytes) {
-  if (hipMalloc(p, bytes) == hipSuccess) return true;
-  (void)hipGetLastError();
-  *p = nullptr;
-  return false;
+static bool try_alloc(mfe_ctx* ctx, P** p, size_t bytes) {
+  return dev_alloc(ctx, p, bytes) == hipSuccess;
 }
 
 // The staged-x plan of A's SELL structure (synchronises the stream).  Leaves
@@ -675,7 +672,7 @@ static int build_sellx(mfe_ctx* ctx, mfe_csr* A) {
   const int nt = (int)cdiv(n, kSpmvRows);
   const int ns = (int)A->sell_nslices;
   int2* d_counts = nullptr;
-  if (!try_alloc(&d_counts, sizeof(int2) * (size_t)nt)) return MFE_OK;
+  if (!try_alloc(ctx, &d_counts, sizeof(int2) * (size_t)nt)) return MFE_OK;
   sellx_plan_kernel<<<nt, kBlock, 0, s>>>((int)n, ns, A->row_offsets, A->cols, A->sell_off,
                                            A->sell_len, 0, d_counts, nullptr, nullptr, nullptr,
                                            nullptr, nullptr, nullptr);
@@ -683,7 +680,7 @@ static int build_sellx(mfe_ctx* ctx, mfe_csr* A) {
   hipError_t e = hipGetLastError();
   int dst = e == hipSuccess ? download_bytes(ctx, counts.data(), d_counts, sizeof(int2) * (size_t)nt)
                             : MFE_OK;
-  (void)hipFree(d_counts);
+  dev_free(ctx, d_counts);
   if (e != hipSuccess) return hip_fail(ctx, e, "sellx_plan_kernel count");
   if (dst) return dst;
   std::vector<int> roff((size_t)nt + 1), nu((size_t)nt);
@@ -700,13 +697,13 @@ static int build_sellx(mfe_ctx* ctx, mfe_csr* A) {
   roff[(size_t)nt] = (int)runs;
   if ((int64_t)maxu * (int64_t)sizeof(double) > kXLdsBytes || runs >= INT32_MAX) return MFE_OK;
   const size_t nl = (size_t)(A->sell_slots + kXTail);
-  const bool ok = try_alloc(&A->sellx_lcols, sizeof(unsigned short) * nl) &&
-                  try_alloc(&A->sellx_roff, sizeof(int) * ((size_t)nt + 1)) &&
-                  try_alloc(&A->sellx_rcol, sizeof(int) * (size_t)std::max<int64_t>(runs, 1)) &&
-                  try_alloc(&A->sellx_rpos, sizeof(int) * (size_t)std::max<int64_t>(runs, 1)) &&
-                  try_alloc(&A->sellx_nu, sizeof(int) * (size_t)nt) &&
-                  try_alloc(&A->sellx_aff, (size_t)ns) &&
-                  try_alloc(&A->sellx_sbase, sizeof(unsigned short) * kSellBaseStride * (size_t)ns);
+  const bool ok = try_alloc(ctx, &A->sellx_lcols, sizeof(unsigned short) * nl) &&
+                  try_alloc(ctx, &A->sellx_roff, sizeof(int) * ((size_t)nt + 1)) &&
+                  try_alloc(ctx, &A->sellx_rcol, sizeof(int) * (size_t)std::max<int64_t>(runs, 1)) &&
+                  try_alloc(ctx, &A->sellx_rpos, sizeof(int) * (size_t)std::max<int64_t>(runs, 1)) &&
+                  try_alloc(ctx, &A->sellx_nu, sizeof(int) * (size_t)nt) &&
+                  try_alloc(ctx, &A->sellx_aff, (size_t)ns) &&
+                  try_alloc(ctx, &A->sellx_sbase, sizeof(unsigned short) * kSellBaseStride * (size_t)ns);
   if (!ok) {
     sellx_release(A);
     A->sellx_valid = true;
@@ -761,19 +758,19 @@ __global__ void vals_to_f32_kernel(int64_t nnz, const double* __restrict__ v,
 // ---- box layout plan ---------------------------------------------------------
 
 void box_release(mfe_csr* A) {
-  hipFree(A->box_vals);
-  hipFree(A->box_vals32);
-  hipFree(A->boxsym_u);
-  hipFree(A->boxsym_w);
-  hipFree(A->boxsym_u32);
-  hipFree(A->boxsym_w32);
-  hipFree(A->boxsym_tab);
-  hipFree(A->boxpack_pw);
-  hipFree(A->boxpack_kq);
-  hipFree(A->boxpack32_pw);
-  hipFree(A->boxpack32_kq);
-  hipFree(A->boxwpack_pw);
-  hipFree(A->boxwpack_kq);
+  dev_free(A->ctx, A->box_vals);
+  dev_free(A->ctx, A->box_vals32);
+  dev_free(A->ctx, A->boxsym_u);
+  dev_free(A->ctx, A->boxsym_w);
+  dev_free(A->ctx, A->boxsym_u32);
+  dev_free(A->ctx, A->boxsym_w32);
+  dev_free(A->ctx, A->boxsym_tab);
+  dev_free(A->ctx, A->boxpack_pw);
+  dev_free(A->ctx, A->boxpack_kq);
+  dev_free(A->ctx, A->boxpack32_pw);
+  dev_free(A->ctx, A->boxpack32_kq);
+  dev_free(A->ctx, A->boxwpack_pw);
+  dev_free(A->ctx, A->boxwpack_kq);
   A->box_vals = nullptr;
   A->box_vals32 = nullptr;
   A->boxsym_u = A->boxsym_w = nullptr;
@@ -968,7 +965,7 @@ static int build_box(mfe_ctx* ctx, mfe_csr* A) {
   T** dst;
   if constexpr (std::is_same<T, double>::value) dst = &A->box_vals;
   else dst = &A->box_vals32;
-  if (!*dst && !try_alloc(dst, sizeof(T) * (size_t)box_entries(g))) return MFE_OK;
+  if (!*dst && !try_alloc(ctx, dst, sizeof(T) * (size_t)box_entries(g))) return MFE_OK;
   box_fill_kernel<T><<<(unsigned)((int64_t)g.nbx * g.nby * g.gz), kBlock, 0, ctx->stream>>>(
       g, A->row_offsets, A->vals, *dst);
   MFE_LAUNCHED(ctx, "box_fill_kernel");
@@ -1335,7 +1332,7 @@ static int build_boxsym(mfe_ctx* ctx, mfe_csr* A) {
     std::vector<int> tab;
     boxsym_tables(tab);
     if (tab.empty()) return fail(ctx, MFE_UNSUPPORTED, "symmetric layout tables");
-    if (!try_alloc(&A->boxsym_tab, sizeof(int) * tab.size())) return MFE_OK;
+    if (!try_alloc(ctx, &A->boxsym_tab, sizeof(int) * tab.size())) return MFE_OK;
     if (int st = upload_bytes(ctx, A->boxsym_tab, tab.data(), sizeof(int) * tab.size())) return st;
   }
   T **du, **dw, **dk;
@@ -1349,13 +1346,13 @@ static int build_boxsym(mfe_ctx* ctx, mfe_csr* A) {
     dk = &A->boxpack32_kq;
   }
   const int64_t groups = (int64_t)g.nbx * g.nby * g.gz;
-  if (!*du && !try_alloc(du, sizeof(T) * (size_t)sym_entries(g))) return MFE_OK;
-  if (!*dw && !try_alloc(dw, sizeof(T) * (size_t)sym_bnd_entries(g))) return MFE_OK;
+  if (!*du && !try_alloc(ctx, du, sizeof(T) * (size_t)sym_entries(g))) return MFE_OK;
+  if (!*dw && !try_alloc(ctx, dw, sizeof(T) * (size_t)sym_bnd_entries(g))) return MFE_OK;
   // without room for these the values stay at full width
-  if (!*dk) (void)try_alloc(dk, sizeof(T) * (size_t)(groups * kSymKRec));
+  if (!*dk) (void)try_alloc(ctx, dk, sizeof(T) * (size_t)(groups * kSymKRec));
   T* wkq = nullptr;
   if constexpr (f64) {
-    if (!A->boxwpack_kq) (void)try_alloc(&A->boxwpack_kq, sizeof(T) * (size_t)(groups * kSymWRec));
+    if (!A->boxwpack_kq) (void)try_alloc(ctx, &A->boxwpack_kq, sizeof(T) * (size_t)(groups * kSymWRec));
     wkq = A->boxwpack_kq;
   }
   const bool check = A->boxsym_state == 0;
@@ -1374,8 +1371,8 @@ static int build_boxsym(mfe_ctx* ctx, mfe_csr* A) {
   if (check) {
     A->boxsym_state = hw.asym ? 2 : 1;
     if (hw.asym) {  // not symmetric: the box layout with all 27 slots instead
-      hipFree(*du);
-      hipFree(*dw);
+      dev_free(ctx, *du);
+      dev_free(ctx, *dw);
       *du = nullptr;
       *dw = nullptr;
       return MFE_OK;
@@ -1449,10 +1446,10 @@ static int enqueue_pack(mfe_ctx* ctx, const T* U, int64_t groups, const unsigned
   if (form == kPackNone) return MFE_OK;
   const int nw = P::words(form);
   if (*cap < nw) {
-    hipFree(*pw);
+    dev_free(ctx, *pw);
     *pw = nullptr;
     *cap = 0;
-    if (!try_alloc(pw, sizeof(unsigned) * (size_t)(groups * nw * kBlock))) return MFE_OK;
+    if (!try_alloc(ctx, pw, sizeof(unsigned) * (size_t)(groups * nw * kBlock))) return MFE_OK;
     *cap = nw;
   }
   with_pack_form<T>(form, [&](auto pf) {
@@ -1521,7 +1518,7 @@ static int enqueue_wpack(mfe_ctx* ctx, mfe_csr* A, int64_t groups, PlanWords* wo
                          int* form_out) {
   *form_out = kPackNone;
   if (!A->boxwpack_pw &&
-      !try_alloc(&A->boxwpack_pw, sizeof(unsigned) * (size_t)(groups * sym_w_words(kPackCube16Near32))))
+      !try_alloc(ctx, &A->boxwpack_pw, sizeof(unsigned) * (size_t)(groups * sym_w_words(kPackCube16Near32))))
     return MFE_OK;
   auto fit = [&](int wd, unsigned slots) {
     int i = 0;
@@ -1620,9 +1617,9 @@ static int ensure_plan(mfe_ctx* ctx, const mfe_csr* Ac, bool need64, bool need32
     sell_release(A);
     const int64_t ns = cdiv(n, kSlice);
     int* d_width = nullptr;
-    bool ok = try_alloc(&A->sell_len, (size_t)(ns * kSlice)) &&
-              try_alloc(&A->sell_off, sizeof(int) * (size_t)(ns + 1)) &&
-              try_alloc(&d_width, sizeof(int) * (size_t)ns);
+    bool ok = try_alloc(ctx, &A->sell_len, (size_t)(ns * kSlice)) &&
+              try_alloc(ctx, &A->sell_off, sizeof(int) * (size_t)(ns + 1)) &&
+              try_alloc(ctx, &d_width, sizeof(int) * (size_t)ns);
     if (ok) {
       sell_len_kernel<<<(unsigned)cdiv(ns * kSlice, kBlock), kBlock, 0, s>>>(
           (int)n, (int)ns, A->row_offsets, A->sell_len, d_width);
@@ -1631,7 +1628,7 @@ static int ensure_plan(mfe_ctx* ctx, const mfe_csr* Ac, bool need64, bool need32
       {
         const int dst = download_bytes(ctx, width.data(), d_width, sizeof(int) * (size_t)ns);
         if (dst) {
-          (void)hipFree(d_width);
+          dev_free(ctx, d_width);
           return dst;
         }
       }
@@ -1647,7 +1644,7 @@ static int ensure_plan(mfe_ctx* ctx, const mfe_csr* Ac, bool need64, bool need32
       A->sell_nslices = ns;
       A->sell_slots = acc * kSlice;
       ok = maxw <= kSellMaxWidth && acc < INT32_MAX &&
-           try_alloc(&A->sell_cols, sizeof(int) * (size_t)(A->sell_slots + kSellTail));
+           try_alloc(ctx, &A->sell_cols, sizeof(int) * (size_t)(A->sell_slots + kSellTail));
       if (ok) {
         MFE_CHECK(ctx, hipMemsetAsync(A->sell_cols + A->sell_slots, 0, sizeof(int) * kSellTail, s));
         int ust = upload_bytes(ctx, A->sell_off, off.data(), sizeof(int) * (size_t)(ns + 1));
@@ -1658,7 +1655,7 @@ static int ensure_plan(mfe_ctx* ctx, const mfe_csr* Ac, bool need64, bool need32
         MFE_LAUNCHED(ctx, "sell_fill_kernel (columns)");
       }
     }
-    hipFree(d_width);
+    dev_free(ctx, d_width);
     A->sell_struct_valid = true;
     if (ok) {
       A->sell_ok = true;
@@ -1674,7 +1671,7 @@ static int ensure_plan(mfe_ctx* ctx, const mfe_csr* Ac, bool need64, bool need32
   const unsigned fg = (unsigned)A->sell_nslices;  // one wave per slice
   if (sell && need64 && !A->sell_vals_valid) {
     if (!A->sell_vals) {
-      if (!try_alloc(&A->sell_vals, sizeof(double) * (size_t)(A->sell_slots + kSellTail))) {
+      if (!try_alloc(ctx, &A->sell_vals, sizeof(double) * (size_t)(A->sell_slots + kSellTail))) {
         sell_disable(A);  // no room for the copy: CSR kernels
         return ensure_plan(ctx, A, need64, need32, allow_box);
       }
@@ -1688,7 +1685,7 @@ static int ensure_plan(mfe_ctx* ctx, const mfe_csr* Ac, bool need64, bool need32
   }
   if (sell && need32 && !A->sell_vals32_valid) {
     if (!A->sell_vals32) {
-      if (!try_alloc(&A->sell_vals32, sizeof(float) * (size_t)(A->sell_slots + kSellTail))) {
+      if (!try_alloc(ctx, &A->sell_vals32, sizeof(float) * (size_t)(A->sell_slots + kSellTail))) {
         sell_disable(A);
         return ensure_plan(ctx, A, need64, need32, allow_box);
       }
@@ -1702,7 +1699,7 @@ static int ensure_plan(mfe_ctx* ctx, const mfe_csr* Ac, bool need64, bool need32
   }
   if (!sell && need32 && !A->vals32_valid) {
     if (!A->vals32)
-      MFE_CHECK(ctx, hipMalloc(&A->vals32, sizeof(float) * (size_t)(A->nnz > 0 ? A->nnz : 1)));
+      MFE_CHECK(ctx, dev_alloc(ctx, &A->vals32, sizeof(float) * (size_t)(A->nnz > 0 ? A->nnz : 1)));
     if (A->nnz > 0) {
       vals_to_f32_kernel<<<(unsigned)std::min<int64_t>(cdiv(A->nnz, kBlock), 65536), kBlock, 0,
                            s>>>(A->nnz, A->vals, A->vals32);
@@ -3402,7 +3399,7 @@ int mfe_cg_solve(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_vec* x, i
   MFE_CHECK(ctx, hipEventRecord(ctx->t_start, ctx->stream));
   if ((st = ensure_plan(ctx, A, true, false))) return st;
   st = run_cg<double>(ctx, spmv_op<double>(A), b->d, x->d, max_iter, tol, replay, eager, w,
-                      w->v64, w->g64, b, x, times ? op_times : nullptr,
+                      w->v64, w->g64, b->d, x->d, times ? op_times : nullptr,
                       (flags & MFE_CG_FUSED) != 0);
   if (st) return st;
   MFE_CHECK(ctx, hipEventRecord(ctx->t_stop, ctx->stream));
