@@ -644,7 +644,22 @@ __device__ __forceinline__ void spmm_boxp_body(int wg, int nwg, BoxGeom g, int n
   double tsum[CPL], accA[CPL], accB[CPL], accC[CPL], xown[CPL];
 #pragma unroll
   for (int q = 0; q < CPL; ++q) tsum[q] = accA[q] = accB[q] = accC[q] = xown[q] = 0.0;
+  // The nine values of line sy of X plane p: three slots of each of the three
+  // rows in flight (plane p + 1 - grp, slots 9 grp + 3 (sy + 1) ..).  They are
+  // loaded one line ahead of their products.
+  double vn[3][3];
+  auto values = [&](int p, int sy) {
+#pragma unroll
+    for (int grp = 0; grp < 3; ++grp) {
+      const int zrow = p + 1 - grp;
+      const bool need = live && zrow >= z0 && zrow < z1;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        vn[grp][i] = need ? V[box_at(g, vblk, zrow, grp * 9 + (sy + 1) * 3 + i, vt)] : 0.0;
+    }
+  };
   fetch(z0 - 1);
+  values(z0 - 1, -1);
   put(0);
   __syncthreads();
   for (int p = z0 - 1; p <= z1; ++p) {
@@ -652,31 +667,33 @@ __device__ __forceinline__ void spmm_boxp_body(int wg, int nwg, BoxGeom g, int n
     if (PF && p < z1) fetch(p + 1);
     const bool pin = p >= 0 && p < g.gz;  // X plane p exists: every slot reading it is in range in z
     // the row of plane q takes its slots (sz+1)*9 .. (sz+1)*9+8 at step q + sz
-    const bool rowA = live && p + 1 >= z0 && p + 1 < z1;  // plane p+1, sz = -1
-    const bool rowB = live && p >= z0 && p < z1;          // plane p,   sz = 0
-    const bool rowC = live && p - 1 >= z0 && p - 1 < z1;  // plane p-1, sz = +1
-    if (pin) {
-      const double* wp = win[buf];
-      // one group of 9 slots at a time: its value loads, then its products
+    const bool rowC = live && p - 1 >= z0 && p - 1 < z1;  // complete after this step
+    const double* wp = win[buf];
+    // one line of the plane at a time: each cell's X piece is read from LDS once
+    // and goes into all three rows in flight.  Out of range the value and the X
+    // entry are 0: adding +0.0 leaves a sum that started at +0.0 as it is; rows
+    // that this chunk does not store are never read.
+#pragma unroll 1
+    for (int sy = -1; sy <= 1; ++sy) {
+      double v[3][3];
 #pragma unroll
-      for (int grp = 0; grp < 3; ++grp) {
-        const bool need = grp == 0 ? rowA : grp == 1 ? rowB : rowC;
-        const int zrow = grp == 0 ? p + 1 : grp == 1 ? p : p - 1;
-        double v[9];
+      for (int grp = 0; grp < 3; ++grp)
 #pragma unroll
-        for (int i = 0; i < 9; ++i) v[i] = need ? V[box_at(g, vblk, need ? zrow : 0, grp * 9 + i, vt)] : 0.0;
+        for (int i = 0; i < 3; ++i) v[grp][i] = vn[grp][i];
+      if (sy < 1) values(p, sy + 1);
+      else if (p < z1) values(p + 1, -1);
 #pragma unroll
-        for (int i = 0; i < 9; ++i) {
-          const int sy = i / 3 - 1, sx = i % 3 - 1;
-          const bool in = need && sx >= lox && sx <= hix && sy >= loy && sy <= hiy;
-          const double* xp = wp + (c0 + sy * WX + sx) * K;
+      for (int sx = -1; sx <= 1; ++sx) {
+        const double* xp = wp + (c0 + sy * WX + sx) * K;
+        double xv[CPL];
 #pragma unroll
-          for (int q = 0; q < CPL; ++q) {
-            double& a = grp == 0 ? accA[q] : grp == 1 ? accB[q] : accC[q];
-            const double next = a + v[i] * xp[col(q)];
-            a = in ? next : a;
-          }
-        }
+        for (int q = 0; q < CPL; ++q) xv[q] = xp[col(q)];
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) accA[q] += v[0][sx + 1] * xv[q];
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) accB[q] += v[1][sx + 1] * xv[q];
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) accC[q] += v[2][sx + 1] * xv[q];
       }
     }
     if (rowC) {  // the row of plane p-1 is complete
@@ -734,24 +751,22 @@ __global__ __launch_bounds__(kBlock, MINB) void spmm_boxp_kernel(
 
 // The box tiles the tuner tries: block width MX (MY = 64 / MX), XCD-contiguous
 // tile order, X prefetch, and a minimum of MINB resident workgroups per CU
-// (MINB 5: at most 96 VGPRs; the kernel needs 90).  Measured at 128^3 x 16
-// (ms per SpMM, one MI355X): 16 x 4 XCD MINB 5 0.360 (fetches 0.85 GB per
-// product, 1.15x its 0.74 GB of value and X reads), 8 x 8 prefetch 0.366;
-// 8 x 8 MINB 5 0.359 but it fetches 1.40 GB (1.89x: a 128-byte line of the
-// 16-wide value blocks serves two 8 x 8 tiles, which run on different XCDs),
-// so it is not offered; 8 x 8 XCD 0.374, 16 x 4 XCD with prefetch 0.387,
-// 8 x 8 MINB 6 (12 VGPRs spilled) 0.387.  Against the earlier form that kept three X planes in LDS (two
-// barriers per step, 38 KB): 0.427-0.430, and with columns strided over the
-// lanes (no LDS bank conflicts, SQ_LDS_BANK_CONFLICT 0 instead of 84 M) or
-// 16 x 4 blocks (30% fewer bytes fetched: whole 128-byte value lines per
-// wave) it lost its fourth resident workgroup per CU and ran 0.51-0.54 ms:
-// residency, not bytes or bank conflicts, set that kernel's time.
+// (MINB 3: at most 168 VGPRs; the kernel needs 148 and 156, the next line's nine
+// values among them).  Bound by the memory system: 1.0 GB per product at
+// 128^3 x 16 (values 0.47, X 0.27, Y 0.27), 206 us at the rate of a copy.
+// Measured there (us per SpMM, one MI355X): 8 x 8 prefetch 308, 16 x 4 XCD 326.
+// With the values loaded slot by slot, nine loads of one row ahead of 9 K
+// products, and each X piece read from LDS three times, the same tiles took 365
+// and 360 (MINB 5, five workgroups per CU); that loop line by line but without
+// the values ahead 304 and 384, with them and MINB 4 (21 VGPRs spilled) 468 for
+// 16 x 4.  8 x 8 XCD with prefetch 310, without 315; 16 x 4 with prefetch 318.
+// K = 8: 246 and 251 (before: 269 and 255).
 struct BoxVariant {
   int mx;
   bool xcd, prefetch;
   int minb;
 };
-constexpr BoxVariant kBoxVariants[] = {{16, true, false, 5}, {8, false, true, 1}};
+constexpr BoxVariant kBoxVariants[] = {{16, true, false, 3}, {8, false, true, 3}};
 constexpr int kBoxVariantCount = 2;
 
 template <int K, int V>
@@ -993,29 +1008,48 @@ static int tune_spmm(mfe_ctx* ctx, const SpmmArgs& a, int K, const double* X, do
 
 constexpr int kColStage = 1024;  // partial rows per stage-1 workgroup
 
-// out[b*K + k] = sum of in[r*K + k] over rows r in [b*chunk, (b+1)*chunk),
-// fixed order: thread (t / K) walks rows t/K, t/K + 256/K, ...; then the
-// 256/K threads of a column add up in a fixed tree.
+// Sum over rows r of [r0, r1) of in[r*K + k], k = threadIdx.x % K, fixed order:
+// thread (t / K) walks rows t/K, t/K + 256/K, ... (eight loads in flight: one at a
+// time a first stage of 1,024 rows took 10.8 us at K = 16, so 6.7); then the 256/K
+// threads of a column add up in a fixed tree.  Valid in the first K threads; sh:
+// kBlock values.
 template <int K>
-__global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const double* __restrict__ in,
-                                                             int rows, int chunk,
-                                                             double* __restrict__ out,
-                                                             const int* __restrict__ done) {
-  if (done && *done) return;
+__device__ __forceinline__ double sum_cols(const double* __restrict__ in, int r0, int r1,
+                                           double* sh) {
   constexpr int G = kBlock / K;  // threads per column
-  __shared__ double sh[kBlock];
+  constexpr int U = 8;
   const int t = (int)threadIdx.x;
   const int k = t % K, g = t / K;
-  const int r0 = (int)blockIdx.x * chunk, r1 = min(r0 + chunk, rows);
   double s = 0.0;
-  for (int r = r0 + g; r < r1; r += G) s += in[(int64_t)r * K + k];
+  int r = r0 + g;
+  for (; r + (U - 1) * G < r1; r += U * G) {
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = in[(int64_t)(r + u * G) * K + k];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s += v[u];
+  }
+  for (; r < r1; r += G) s += in[(int64_t)r * K + k];
   sh[t] = s;
   __syncthreads();
   for (int w = G / 2; w > 0; w >>= 1) {
     if (g < w) sh[t] += sh[t + w * K];
     __syncthreads();
   }
-  if (g == 0) out[(int64_t)blockIdx.x * K + k] = sh[k];
+  return sh[k];
+}
+
+// First stage: out[b*K + k] = the sum of rows [b*chunk, (b+1)*chunk).
+template <int K>
+__global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const double* __restrict__ in,
+                                                             int rows, int chunk,
+                                                             double* __restrict__ out,
+                                                             const int* __restrict__ done) {
+  if (done && *done) return;
+  __shared__ double sh[kBlock];
+  const int r0 = (int)blockIdx.x * chunk, r1 = min(r0 + chunk, rows);
+  const double s = sum_cols<K>(in, r0, r1, sh);
+  if ((int)threadIdx.x < K) out[(int64_t)blockIdx.x * K + threadIdx.x] = s;
 }
 
 // ------------------------------------------------------------ CG state -------
@@ -1091,17 +1125,23 @@ __global__ __launch_bounds__(kBlock) void multi_finish_kernel(int64_t nk, const 
     X[i] = 1.0 * X[i] + a * P[i];
 }
 
-__global__ void multi_alpha_kernel(MultiState* st, int K, const double* pAp) {
+// The second stage of the p.Ap reduction (nb rows of first-stage sums), then
+// alpha per column.
+template <int K>
+__global__ __launch_bounds__(kBlock) void multi_alpha_kernel(MultiState* st, const double* part,
+                                                             int nb) {
   if (st->done) return;
+  __shared__ double sh[kBlock];
+  const double pAp = sum_cols<K>(part, 0, nb, sh);
   const int c = (int)threadIdx.x;
   if (c < K && st->active[c]) {
-    st->pAp[c] = pAp[c];
-    if (!(pAp[c] > 0.0)) {  // non-positive curvature: stop this column
+    st->pAp[c] = pAp;
+    if (!(pAp > 0.0)) {  // non-positive curvature: stop this column
       st->breakdown[c] = 1;
       st->active[c] = 0;
       st->alpha[c] = 0.0;
     } else {
-      st->alpha[c] = st->rtrans[c] / pAp[c];
+      st->alpha[c] = st->rtrans[c] / pAp;
     }
   }
   if (c < K) {  // this iteration's X update, applied by the next P update
@@ -1146,14 +1186,20 @@ __global__ __launch_bounds__(kBlock) void multi_update_kernel(int64_t nk, const 
   }
 }
 
-__global__ void multi_next_kernel(MultiState* st, int K, const double* rr) {
+// The second stage of the r.r reduction, then the end of the iteration per column.
+template <int K>
+__global__ __launch_bounds__(kBlock) void multi_next_kernel(MultiState* st, const double* part,
+                                                            int nb) {
   if (st->done) return;
+  __shared__ double sh[kBlock];
+  const double rr = sum_cols<K>(part, 0, nb, sh);
   const int c = (int)threadIdx.x;
   const int k = st->k;
+  __syncthreads();  // every thread has read k and done
   if (c < K && st->active[c]) {
     st->oldrtrans[c] = st->rtrans[c];
-    st->rtrans[c] = rr[c];
-    st->normr[c] = sqrt(rr[c]);
+    st->rtrans[c] = rr;
+    st->normr[c] = sqrt(rr);
     st->beta[c] = st->rtrans[c] / st->oldrtrans[c];
     st->iters[c] = k;
     if (!(st->normr[c] > st->tol[c]) || k + 1 > st->max_iter) st->active[c] = 0;
@@ -1339,12 +1385,13 @@ static hipError_t enqueue_multi_iteration(MultiWorkspace* w, const mfe_csr* A, d
   int nb = 0;
   hipError_t e = launch_spmm<K>(tile, spmm_args(A, w), w->P, w->AP, w->part, done, s, &nb);
   if (e != hipSuccess) return e;
-  if ((e = reduce_cols(K, w->part, nb, w->part2, w->res, done, s)) != hipSuccess) return e;
-  multi_alpha_kernel<<<1, 64, 0, s>>>(w->st, K, w->res);
+  const int s1 = (int)std::max<int64_t>(1, cdiv(nb, kColStage));
+  reduce_cols_kernel<K><<<s1, kBlock, 0, s>>>(w->part, nb, kColStage, w->part2, done);
+  multi_alpha_kernel<K><<<1, kBlock, 0, s>>>(w->st, w->part2, s1);
   multi_update_kernel<K><<<vg, kBlock, 0, s>>>(nk, w->st, w->R, w->AP, w->part);
-  if ((e = reduce_cols(K, w->part, (int)vg, w->part2, w->res + 16, done, s)) != hipSuccess)
-    return e;
-  multi_next_kernel<<<1, 64, 0, s>>>(w->st, K, w->res + 16);
+  const int s2 = (int)std::max<int64_t>(1, cdiv(vg, kColStage));
+  reduce_cols_kernel<K><<<s2, kBlock, 0, s>>>(w->part, (int)vg, kColStage, w->part2, done);
+  multi_next_kernel<K><<<1, kBlock, 0, s>>>(w->st, w->part2, s2);
   return hipGetLastError();
 }
 
