@@ -4,8 +4,7 @@
 // Each problem owns a contiguous range of the grid's workgroups, sized by its
 // expected work (non-zeros x CG iterations, the latter ~ the box's extent).
 // The workgroups of a problem meet at a problem-local barrier (an arrival
-// counter plus a generation word, agent-scope release/acquire), so problems
-// never wait for each other.  The cooperative launch guarantees that every
+// counter, agent-scope release/acquire), so problems never wait for each other.  The cooperative launch guarantees that every
 // workgroup is resident, and every wait is bounded by a wall-clock limit: a
 // wait that exceeds it raises the batch's abort flag and all workgroups leave.
 //
@@ -47,7 +46,7 @@ struct BatchProb {
 };
 
 struct BatchState {  // per problem, zeroed before each launch
-  unsigned count, gen;
+  unsigned count, pad0;  // arrivals at the problem's barriers
   int iters, status;  // status: 0 converged or max_iter, 1 breakdown, 2 aborted
   double normr, tol, bnorm, pad;
   uint64_t t_begin, t_end;  // wall clock of the problem's first workgroup
@@ -59,41 +58,51 @@ struct BatchState {  // per problem, zeroed before each launch
 constexpr double kBatchWaitSeconds = 10.0;
 constexpr int kUnroll = 4;  // tiles per step of the vector loops
 
-// Problem-local barrier.  The workgroup's stores are complete in L2 after
-// __syncthreads (L1 writes through); thread 0 then releases them at agent
-// scope (writes the L2 back, so workgroups on other XCDs see them), arrives,
-// waits for the generation to move, and acquires (invalidates this CU's L1
-// and non-coherent L2 lines) before the workgroup reads what others wrote.
+// Problem-local barrier: an arrival counter that only grows; the barrier is
+// complete when it reaches `target` (nb more than at the last one; it may wrap).
+// The workgroup's stores are complete in L2 after __syncthreads (L1 writes
+// through); thread 0 releases them at agent scope (writes the L2 back, so
+// workgroups on other XCDs see them), arrives, waits, and acquires (invalidates
+// this CU's L1 and the XCD's non-coherent L2 lines) before the workgroup reads
+// what others wrote.  Every arrival is a read-modify-write of the same word, so
+// the one that completes it carries the releases of all earlier ones.
+// Bound by the round trips to memory: one release, one arrival, the poll.  The
+// polls are relaxed: with an acquire in each, every waiting workgroup kept
+// invalidating the L2 under the workgroups still at work (64 boxes of 16..96:
+// 290 ms, so 251; two 150^3: 233, so 183), and with a separate generation word
+// and a load of the abort flag per poll it had two more trips (30^3: 6.1 us per
+// barrier, so 3.9; the acquiring polls 11.5).  The abort flag is looked at every
+// 16th poll; a problem whose own barriers complete runs on.
 // Returns false when the batch was aborted.
-__device__ bool prob_barrier(BatchState* st, int nb, int* abort_flag, uint64_t limit_ticks) {
+__device__ bool prob_barrier(BatchState* st, unsigned target, int* abort_flag,
+                             uint64_t limit_ticks) {
   __syncthreads();
   __shared__ int s_ok;
   if (threadIdx.x == 0) {
-    __threadfence();
-    const unsigned g = __hip_atomic_load(&st->gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned arrived =
-        __hip_atomic_fetch_add(&st->count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    unsigned seen =
+        __hip_atomic_fetch_add(&st->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
     int ok = 1;
-    if (arrived == (unsigned)nb) {
-      __hip_atomic_store(&st->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_fetch_add(&st->gen, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
+    if ((int)(seen - target) < 0) {
       const uint64_t t0 = wall_clock64();
-      while (__hip_atomic_load(&st->gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == g) {
-        if (__hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-          ok = 0;
-          break;
-        }
-        if (wall_clock64() - t0 > limit_ticks) {
-          __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          ok = 0;
-          break;
+      for (unsigned polls = 1;; ++polls) {
+        seen = __hip_atomic_load(&st->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((int)(seen - target) >= 0) break;
+        if (polls % 16 == 0) {
+          if (__hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+            ok = 0;
+            break;
+          }
+          if (wall_clock64() - t0 > limit_ticks) {
+            __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ok = 0;
+            break;
+          }
         }
         __builtin_amdgcn_s_sleep(1);
       }
     }
-    if (__hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) ok = 0;
-    __threadfence();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     s_ok = ok;
   }
   __syncthreads();
@@ -292,6 +301,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8
   double* part = partials + P.part0;
   const int ntiles = (int)cdiv((int64_t)P.nslices * kWave, kBlock);
   const bool timer = i == 0 && t == 0;
+  unsigned bar = 0;  // arrivals that complete the problem's next barrier
   uint64_t tp[6] = {0, 0, 0, 0, 0, 0};
   uint64_t tc = wall_clock64();
   if (timer) st->t_begin = tc;
@@ -303,7 +313,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8
   } while (0)
 #define MFE_BARRIER()                                                  \
   do {                                                                 \
-    const bool ok_ = prob_barrier(st, nb, abort_flag, limit_ticks);    \
+    bar += (unsigned)nb;                                               \
+    const bool ok_ = prob_barrier(st, bar, abort_flag, limit_ticks);   \
     MFE_PHASE(5);                                                      \
     if (!ok_) return;                                                  \
   } while (0)
