@@ -1,10 +1,14 @@
-// Batched miniFE: many independent box problems of uneven size assembled and
-// solved by FP64 CG in ONE persistent, cooperative launch.
+// Batched miniFE: many independent box problems of uneven size assembled by two
+// launches over all of them and solved by FP64 CG in ONE persistent, cooperative
+// launch.
 //
 // Each problem owns a contiguous range of the grid's workgroups, sized by its
-// expected work (non-zeros x CG iterations, the latter ~ the box's extent).
+// expected work (non-zeros x CG iterations, the latter ~ the box's extent); the
+// ranges are laid over the XCDs one after the other, so that most problems stay
+// within one L2.
 // The workgroups of a problem meet at a problem-local barrier (an arrival
-// counter, agent-scope release/acquire), so problems never wait for each other.  The cooperative launch guarantees that every
+// counter, agent-scope release/acquire), so problems never wait for each other.
+// The cooperative launch guarantees that every
 // workgroup is resident, and every wait is bounded by a wall-clock limit: a
 // wait that exceeds it raises the batch's abort flag and all workgroups leave.
 //
@@ -14,13 +18,22 @@
 //   2. one thread per row: the row's entries summed in ascending element id,
 //      both Dirichlet passes (u = 0 on bc_rows_0, then u = 1 on bc_rows_1,
 //      row-local because the BC sets are faces of the box), stored straight
-//      into the problem's SELL-64 slices; x = 0, r = b;
-//   3. CG (cg_solve.hpp:69-229 with the fast, tree-reduced dots): p update,
-//      barrier, SpMV + p.Ap partials, barrier, x/r update + r.r partials,
-//      barrier.  Partials alternate between two buffers, so a workgroup that
+//      into the problem's SELL-64 slices and, for the CG, in an exact packed
+//      form (below); x = 0, r = b;
+//   3. CG (cg_solve.hpp:69-229 with the fast, tree-reduced dots): the last
+//      iteration's x update and p update, barrier, SpMV + p.Ap partials,
+//      barrier, r update + r.r partials, barrier.  Partials alternate between
+//      two buffers, so a workgroup that
 //      runs ahead never overwrites what a slower one is still summing.  Every
 //      workgroup sums a problem's partials in the same order, so all of them
 //      take the same scalars and leave the loop at the same iteration.
+//
+// A row or a column of a Dirichlet face (all six faces are) is the identity's, so
+// the operator couples interior nodes only, and an interior row has all its 27
+// neighbours.  The CG keeps p = 0 on the faces in the vector that rows gather
+// from and a face node's own p in its entry of A p (which equals it), so an
+// interior row sums its 27 products without a look at where it lies: the skipped
+// terms of a masked sum are the +-0.0 that leave this one unchanged.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -28,6 +41,7 @@
 
 #include "mfe_common.hpp"
 #include "mfe_hex8.hpp"
+#include "mfe_pack.hpp"
 #include "mfe_sell.hpp"
 
 namespace mfe {
@@ -43,7 +57,41 @@ struct BatchProb {
   int64_t slot0;   // base of its SELL entries
   int64_t elem0;   // base of its element scratch (44 doubles per element)
   int64_t part0;   // base of its 2*nb partials
+  int64_t tile0;   // index of its first tile's record and packed words
 };
+
+// The packed stencil values of a tile (kBlock consecutive rows), interior entries
+// of interior rows only.  Slot s of the tile holds base[s] + f q, f a field of
+// the form's width, q the largest power of two that divides all of the slot's
+// values, base their least: the assembled values of one slot differ by rounding
+// only, and both products and sums of the decoding are exact.  Widths needed:
+// 8 to 10 bits for boxes of up to about 100 elements a side, 14 to 18 for the
+// slots that are analytically zero (a cube's face neighbours, N x N x 2N's edge
+// neighbours).  Per row 36, 44 or 68 bytes instead of the 216 that a tile which
+// fits no form reads from its SELL slices.
+constexpr int kBSlots = 27;
+constexpr unsigned kBNear = (1u << 4) | (1u << 10) | (1u << 12) | (1u << 14) | (1u << 16) | (1u << 22);
+struct BatchRec {
+  double base[kBSlots];
+  uint64_t inner[kBlock / kWave];  // the wave's lanes on interior nodes
+  unsigned qhi[kBSlots];           // q's high word (the low one is 0)
+  int form;                        // BatchForm
+};
+enum BatchForm { kBFull = 0, kB10 = 1, kB10Near22 = 2, kB20 = 3 };
+// Form of bits N per slot, NN for the near ones: the fields follow each other in
+// slot order; word w of the tile's row t is at w * kBlock + t.
+template <int N, int NN>
+struct BatchPack {
+  static constexpr int width(int s) { return (kBNear >> s) & 1u ? NN : N; }
+  static constexpr int bit(int s) {
+    return s * N + __builtin_popcount(kBNear & ((1u << s) - 1u)) * (NN - N);
+  }
+  static constexpr int words = (kBSlots * N + 6 * (NN - N) + 31) / 32;
+};
+using BPack10 = BatchPack<10, 10>;      // 9 words
+using BPack10N22 = BatchPack<10, 22>;   // 11
+using BPack20 = BatchPack<20, 20>;      // 17
+constexpr int kBWords = BPack20::words;  // words kept per row of a tile
 
 struct BatchState {  // per problem, zeroed before each launch
   unsigned count, pad0;  // arrivals at the problem's barriers
@@ -74,9 +122,10 @@ constexpr int kUnroll = 4;  // tiles per step of the vector loops
 // barrier, so 3.9; the acquiring polls 11.5).  The abort flag is looked at every
 // 16th poll; a problem whose own barriers complete runs on.
 // Returns false when the batch was aborted.
-__device__ bool prob_barrier(BatchState* st, unsigned target, int* abort_flag,
+__device__ bool prob_barrier(BatchState* st, int nb, unsigned target, int* abort_flag,
                              uint64_t limit_ticks) {
   __syncthreads();
+  if (nb == 1) return true;
   __shared__ int s_ok;
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
@@ -124,10 +173,11 @@ __device__ double sum_partials_all(const double* pp, int nb, double* red) {
 
 __device__ __forceinline__ int axis_len(int i, int g) { return 1 + (i > 0) + (i < g - 1); }
 
-// Assemble row `id` of problem P (element scratch K/F), apply both Dirichlet
-// passes, store it into the SELL slices; returns b[id].
-__device__ double assemble_row(const BatchProb& P, int id, const double* K, const double* F,
-                               const int* soff, int* scols, double* svals) {
+// Assemble row `id` of problem P (element scratch K/F) into acc, apply both
+// Dirichlet passes, store it into the SELL slices; returns b[id].
+__device__ __forceinline__ double assemble_row(const BatchProb& P, int id, const double* K,
+                                               const double* F, const int* soff, int* scols,
+                                               double* svals, double (&acc)[kBSlots]) {
   const int Nx = P.Nx, Ny = P.Ny, Nz = P.Nz;
   const int gx = Nx + 1, gy = Ny + 1;
   const int64_t ne = P.ne;
@@ -135,9 +185,8 @@ __device__ double assemble_row(const BatchProb& P, int id, const double* K, cons
   const int lox = ix > 0 ? -1 : 0, hix = ix < Nx ? 1 : 0;
   const int loy = iy > 0 ? -1 : 0, hiy = iy < Ny ? 1 : 0;
   const int loz = iz > 0 ? -1 : 0, hiz = iz < Nz ? 1 : 0;
-  double acc[27];
 #pragma unroll
-  for (int s = 0; s < 27; ++s) acc[s] = 0.0;
+  for (int s = 0; s < kBSlots; ++s) acc[s] = 0.0;
   double accb = 0.0;
 #pragma unroll
   for (int dz = -1; dz <= 0; ++dz)
@@ -234,66 +283,279 @@ __device__ void pad_row(const BatchProb& P, int id, const int* soff, int* scols,
   }
 }
 
-// (A p)[row] for row < n of problem P from its SELL values, summed over the
-// row's entries in stored (ascending column) order, 0 for padding rows.  The
-// columns are not loaded: a box row's k-th stored entry is its k-th in-range
-// neighbour in (z, y, x) order, so each neighbour's x address and slot follow
-// from the row's grid position, and every value load and x gather of the row
-// is issued at once (out-of-range neighbours load slot 0 and p[row], unused).
-__device__ __forceinline__ double batch_row_sum(const BatchProb& P, int row, const int* soff,
-                                                const double* svals, const double* pv) {
-  const int slice = row / kWave, lane = row % kWave;
-  const int o = soff[slice], w = soff[slice + 1] - o;
+// The exponent of the lowest set bit of v (v != 0), as of a value 1.f * 2^e.
+__device__ __forceinline__ int low_bit_exponent(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const int ex = (int)((u >> 52) & 0x7ff);
+  const uint64_t m = (u & 0xfffffffffffffull) | (ex ? 1ull << 52 : 0ull);
+  return (ex ? ex : 1) - 1075 + __builtin_ctzll(m);
+}
+
+// The packed words of form BP of one row: field s = (v[s] - base[s]) / q, exact.
+template <typename BP>
+__device__ __forceinline__ void pack_row(const double (&v)[kBSlots], const double* base,
+                                         const double* inv_q, unsigned* w) {
+  unsigned cur = 0;
+#pragma unroll
+  for (int s = 0; s < kBSlots; ++s) {
+    const unsigned f = (unsigned)((v[s] - base[s]) * inv_q[s]);
+    const int sh = BP::bit(s) % 32, word = BP::bit(s) / 32;
+    cur |= f << sh;
+    if (sh + BP::width(s) >= 32) {
+      w[(int64_t)word * kBlock] = cur;
+      cur = sh + BP::width(s) > 32 ? f >> ((32 - sh) & 31) : 0u;
+    }
+  }
+  if ((BP::bit(kBSlots - 1) + BP::width(kBSlots - 1)) % 32)
+    w[(int64_t)(BP::words - 1) * kBlock] = cur;
+}
+
+// The record and packed words of one tile from its rows' values (all threads of
+// the workgroup; `in`: this thread's row is interior).  pw null: no packed form.
+// An interior row's entries in columns on the faces are 0.0 and are skipped by
+// the gathered p = 0 as well, so they take no part: any field does.
+__device__ __forceinline__ void pack_tile(const BatchProb& P, int id, bool in,
+                                          double (&v)[kBSlots], BatchRec* rec, unsigned* pw) {
+  __shared__ double lo[kBSlots][kBlock / kWave], hi[kBSlots][kBlock / kWave];
+  __shared__ int low[kBSlots][kBlock / kWave];
+  __shared__ double base[kBSlots], inv_q[kBSlots];
+  __shared__ int bits[kBSlots];
+  __shared__ int form_sh;
+  const int t = (int)threadIdx.x, lane = t % kWave, wave = t / kWave;
+  const uint64_t m = __ballot(in);
+  if (lane == 0) rec->inner[wave] = m;
   const int gx = P.Nx + 1, gy = P.Ny + 1;
-  const bool valid = row < P.n;
-  const int rr = valid ? row : P.n - 1;
-  const int ix = rr % gx, iy = (rr / gx) % gy, iz = rr / (gx * gy);
-  const int lox = ix > 0 ? -1 : 0, hix = ix < P.Nx ? 1 : 0;
-  const int loy = iy > 0 ? -1 : 0, hiy = iy < P.Ny ? 1 : 0;
-  const int loz = iz > 0 ? -1 : 0, hiz = iz < P.Nz ? 1 : 0;
-  const int64_t o64 = P.slot0 + (int64_t)o * kWave;
-  double v[27], xv[27];
-  bool in[27];
-  int pos = 0;
+  const int ix = id % gx, iy = (id / gx) % gy, iz = id / (gx * gy);
+  const double inf = __longlong_as_double(0x7ff0000000000000ll);
+  unsigned has = 0;  // slots whose column is interior
 #pragma unroll
-  for (int sz = -1; sz <= 1; ++sz)
+  for (int s = 0; s < kBSlots; ++s) {
+    const int jx = ix + s % 3 - 1, jy = iy + (s / 3) % 3 - 1, jz = iz + s / 9 - 1;
+    const bool h = in && jx > 0 && jx < P.Nx && jy > 0 && jy < P.Ny && jz > 0 && jz < P.Nz;
+    has |= (h ? 1u : 0u) << s;
+    double a = h ? v[s] : inf, b = h ? v[s] : -inf;
+    int e = h && v[s] != 0.0 ? low_bit_exponent(v[s]) : 4096;
 #pragma unroll
-    for (int sy = -1; sy <= 1; ++sy)
+    for (int d = 1; d < kWave; d <<= 1) {
+      a = fmin(a, __shfl_xor(a, d));
+      b = fmax(b, __shfl_xor(b, d));
+      e = min(e, __shfl_xor(e, d));
+    }
+    if (lane == 0) {
+      lo[s][wave] = a;
+      hi[s][wave] = b;
+      low[s][wave] = e;
+    }
+  }
+  __syncthreads();
+  if (t < kBSlots) {
+    double a = lo[t][0], b = hi[t][0];
+    int e = low[t][0];
 #pragma unroll
-      for (int sx = -1; sx <= 1; ++sx) {
-        const int q = (sz + 1) * 9 + (sy + 1) * 3 + (sx + 1);
-        in[q] = valid && sx >= lox && sx <= hix && sy >= loy && sy <= hiy && sz >= loz &&
-                sz <= hiz;
-        v[q] = svals[sell_pos(o64, in[q] ? pos : 0, w, lane)];
-        xv[q] = pv[in[q] ? rr + sx + gx * (sy + gy * sz) : rr];
-        pos += in[q] ? 1 : 0;
-      }
+    for (int w = 1; w < kBlock / kWave; ++w) {
+      a = fmin(a, lo[t][w]);
+      b = fmax(b, hi[t][w]);
+      e = min(e, low[t][w]);
+    }
+    int need = 0;
+    if (a > b) {  // the slot is in no interior row's range
+      a = 0.0;
+      e = 0;
+    } else if (e == 4096) {  // every value is 0.0
+      e = 0;
+    } else if (!(e > -1000 && e < 900)) {  // 2^e and 2^-e are not both normal
+      need = 64;
+      e = 0;
+    } else {
+      const double r = (b - a) * ldexp(1.0, -e);  // too large a range only rounds to one
+      need = r <= 1023.0 ? 10 : r <= 1048575.0 ? 20 : r <= 4194303.0 ? 22 : 64;
+    }
+    const double q = ldexp(1.0, e);
+    base[t] = a;
+    inv_q[t] = ldexp(1.0, -e);
+    bits[t] = need;
+    rec->base[t] = a;
+    rec->qhi[t] = (unsigned)__double2hiint(q);
+  }
+  __syncthreads();
+  if (t == 0) {
+    int all = 0, cube = 0, near = 0;
+    for (int s = 0; s < kBSlots; ++s) {
+      all = max(all, bits[s]);
+      if ((kBNear >> s) & 1u) near = max(near, bits[s]);
+      else cube = max(cube, bits[s]);
+    }
+    const int f = !pw ? kBFull
+                      : all <= 10 ? kB10 : cube <= 10 && near <= 22 ? kB10Near22
+                                               : all <= 20 ? kB20 : kBFull;
+    form_sh = f;
+    rec->form = f;
+  }
+  __syncthreads();
+  const int form = form_sh;
+  if (form == kBFull) return;
+#pragma unroll
+  for (int s = 0; s < kBSlots; ++s)
+    if (!((has >> s) & 1u)) v[s] = base[s];
+  if (form == kB10) pack_row<BPack10>(v, base, inv_q, pw + t);
+  else if (form == kB10Near22) pack_row<BPack10N22>(v, base, inv_q, pw + t);
+  else pack_row<BPack20>(v, base, inv_q, pw + t);
+}
+
+// The 27 entries of p around row `row` of a problem whose planes hold `plane`
+// nodes; an unsigned byte offset from a pointer that is the same for every lane
+// (rows < 2^29: the matrix alone takes 324 bytes a row).
+__device__ __forceinline__ void gather27(const double* pv, int row, int gx, int plane,
+                                         double (&xv)[kBSlots]) {
+  const unsigned off = 8u * (unsigned)row;
+#pragma unroll
+  for (int s = 0; s < kBSlots; ++s) {
+    const double* q = pv + ((s % 3 - 1) + gx * ((s / 3) % 3 - 1) + (int64_t)plane * (s / 9 - 1));
+    xv[s] = *reinterpret_cast<const double*>(reinterpret_cast<const char*>(q) + off);
+  }
+}
+
+// (A p)[row] of an interior row, its 27 entries in ascending column order, from
+// the packed words w of the row's tile.
+template <typename BP>
+__device__ __forceinline__ double packed_row_sum(const unsigned* __restrict__ w,
+                                                 const BatchRec* __restrict__ rec,
+                                                 const double* pv, int row, int gx, int plane,
+                                                 double* own) {
+  unsigned f[BP::words];
+#pragma unroll
+  for (int i = 0; i < BP::words; ++i) f[i] = w[i * kBlock];
+  double xv[kBSlots];
+  gather27(pv, row, gx, plane, xv);
   double sum = 0.0;
 #pragma unroll
-  for (int q = 0; q < 27; ++q)
-    if (in[q]) sum += v[q] * xv[q];
+  for (int s = 0; s < kBSlots; ++s) {
+    const unsigned u = pack_field(f + BP::bit(s) / 32, BP::width(s), BP::bit(s) % 32);
+    const double v = (double)u * __hiloint2double((int)rec->qhi[s], 0) + rec->base[s];
+    sum += v * xv[s];
+  }
+  *own = xv[kBSlots / 2];
   return sum;
 }
 
-// WAVES: the minimum waves per SIMD the register allocation must allow (the
-// element math alone wants ~200 VGPRs, i.e. 2 waves; more waves hide more of
-// the CG's memory latency at the price of some spilling in the element phase).
-template <int WAVES>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8))) void batch_kernel(
+// The same from the row's SELL values (27 of them: its slice is as wide).
+__device__ __forceinline__ double full_row_sum(const BatchProb& P, const int* __restrict__ soff,
+                                               const double* __restrict__ svals,
+                                               const double* pv, int row, int gx, int plane,
+                                               double* own) {
+  const int slice = row / kWave, lane = row % kWave;
+  const int o = soff[slice], w = soff[slice + 1] - o;
+  const int64_t o64 = P.slot0 + (int64_t)o * kWave;
+  double v[kBSlots], xv[kBSlots];
+#pragma unroll
+  for (int s = 0; s < kBSlots; ++s) v[s] = svals[sell_pos(o64, s, w, lane)];
+  gather27(pv, row, gx, plane, xv);
+  double sum = 0.0;
+#pragma unroll
+  for (int s = 0; s < kBSlots; ++s) sum += v[s] * xv[s];
+  *own = xv[kBSlots / 2];
+  return sum;
+}
+
+// Element matrices and source vectors of every problem (Hex8 element math, k = 1).
+__global__ __launch_bounds__(kBlock) void batch_elements_kernel(
     const BatchProb* __restrict__ probs, const int* __restrict__ blk2prob, HexTables tab,
-    const int* __restrict__ soff_all, int* scols, double* svals, double* KF, double* b,
-    double* x, double* r, double* p, double* Ap, double* partials, BatchState* states,
-    int* abort_flag, int max_iter, double rel_tol, uint64_t limit_ticks) {
-  __shared__ double red[4];
-  const int pi = blk2prob[blockIdx.x];
+    double* KF, BatchState* states) {
+  const int wg = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
+  const int pi = blk2prob[wg];
   const BatchProb P = probs[pi];
-  BatchState* st = states + pi;
-  const int i = (int)blockIdx.x - P.b0, nb = P.nb, t = (int)threadIdx.x;
+  const int i = wg - P.b0, t = (int)threadIdx.x;
   const int64_t ne = P.ne;
   double* K = KF + P.elem0;
   double* F = K + 36 * ne;
+  const uint64_t tc = wall_clock64();
+  const double hx = 1.0 / P.Nx, hy = 1.0 / P.Ny, hz = 1.0 / P.Nz;
+  for (int64_t e = (int64_t)i * kBlock + t; e < ne; e += (int64_t)P.nb * kBlock) {
+    const int ex = (int)(e % P.Nx);
+    const int ey = (int)((e / P.Nx) % P.Ny);
+    const int ez = (int)(e / ((int64_t)P.Nx * P.Ny));
+    const double x0 = 1.0 * ex / P.Nx;
+    const double y0 = 1.0 * ey / P.Ny;
+    const double z0 = (1.0 * ez) / P.Nz;
+    const double x1 = x0 + hx, y1 = y0 + hy, z1 = z0 + hz;
+    const double c[24] = {x0, y0, z0, x1, y0, z0, x1, y1, z0, x0, y1, z0,
+                          x0, y0, z1, x1, y0, z1, x1, y1, z1, x0, y1, z1};
+    double Ke[36], Fe[8];
+    hex8_element<false>(c, tab, 1.0, Ke, Fe);
+#pragma unroll
+    for (int q = 0; q < 36; ++q) K[(int64_t)q * ne + e] = Ke[q];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) F[(int64_t)q * ne + e] = Fe[q];
+  }
+  if (i == 0 && t == 0) {
+    BatchState* st = states + pi;
+    st->t_begin = tc;
+    st->t_phase[0] = wall_clock64() - tc;
+  }
+}
+
+// Rows of every problem: gather, Dirichlet, SELL store, packed form; x = 0,
+// r = b, p = 0 (the faces keep it), and the partials of b.b.
+__global__ __launch_bounds__(kBlock) void batch_rows_kernel(
+    const BatchProb* __restrict__ probs, const int* __restrict__ blk2prob,
+    const int* __restrict__ soff_all, const double* __restrict__ KF, int* scols, double* svals,
+    BatchRec* recs, unsigned* words, double* b, double* x, double* r, double* p,
+    double* partials, BatchState* states) {
+  __shared__ double red[4];
+  const int wg = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
+  const int pi = blk2prob[wg];
+  const BatchProb P = probs[pi];
+  const int i = wg - P.b0, nb = P.nb, t = (int)threadIdx.x;
+  const double* K = KF + P.elem0;
+  const double* F = K + 36 * (int64_t)P.ne;
   const int* soff = soff_all + P.soff0;
-  double* bp = b + P.row0;
+  const int gx = P.Nx + 1, gy = P.Ny + 1;
+  const int ntiles = (int)cdiv((int64_t)P.nslices * kWave, kBlock);
+  const uint64_t tc = wall_clock64();
+  double acc = 0.0;
+  for (int tile = i; tile < ntiles; tile += nb) {
+    const int row = tile * kBlock + t;
+    double v[kBSlots];
+    bool in = false;
+    if (row < P.n) {
+      const double bv = assemble_row(P, row, K, F, soff, scols, svals, v);
+      const int ix = row % gx, iy = (row / gx) % gy, iz = row / (gx * gy);
+      in = ix > 0 && ix < P.Nx && iy > 0 && iy < P.Ny && iz > 0 && iz < P.Nz;
+      b[P.row0 + row] = bv;
+      x[P.row0 + row] = 0.0;
+      r[P.row0 + row] = bv;
+      p[P.row0 + row] = 0.0;
+      acc += bv * bv;
+    } else if (row < P.nslices * kWave) {
+      pad_row(P, row, soff, scols, svals);
+    }
+    pack_tile(P, row, in, v, recs + P.tile0 + tile,
+              words ? words + (P.tile0 + tile) * (int64_t)(kBWords * kBlock) : nullptr);
+  }
+  const double v0 = block_sum<double>(acc, red);
+  if (t == 0) partials[P.part0 + i] = v0;
+  if (i == 0 && t == 0) states[pi].t_phase[1] = wall_clock64() - tc;
+}
+
+// The CG of every problem.  WAVES: the minimum waves per SIMD the register
+// allocation must allow.
+template <int WAVES>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8))) void batch_kernel(
+    const BatchProb* __restrict__ probs, const int* __restrict__ blk2prob,
+    const int* __restrict__ soff_all, const double* __restrict__ svals,
+    const BatchRec* __restrict__ recs, const unsigned* __restrict__ words, double* x, double* r,
+    double* p, double* Ap, double* partials, BatchState* states, int* abort_flag, int max_iter,
+    double rel_tol, uint64_t limit_ticks) {
+  __shared__ double red[4];
+  const int wg = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
+  const int pi = blk2prob[wg];
+  const BatchProb P = probs[pi];
+  BatchState* st = states + pi;
+  const int i = wg - P.b0, nb = P.nb, t = (int)threadIdx.x;
+  const int lane = t % kWave, wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int* soff = soff_all + P.soff0;
+  const BatchRec* prec = recs + P.tile0;
+  const int gx = P.Nx + 1, plane = gx * (P.Ny + 1);
   double* xp = x + P.row0;
   double* rp = r + P.row0;
   double* pp = p + P.row0;
@@ -304,90 +566,51 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8
   unsigned bar = 0;  // arrivals that complete the problem's next barrier
   uint64_t tp[6] = {0, 0, 0, 0, 0, 0};
   uint64_t tc = wall_clock64();
-  if (timer) st->t_begin = tc;
 #define MFE_PHASE(k)                  \
   do {                                \
     const uint64_t now_ = wall_clock64(); \
     tp[k] += now_ - tc;               \
     tc = now_;                        \
   } while (0)
-#define MFE_BARRIER()                                                  \
-  do {                                                                 \
-    bar += (unsigned)nb;                                               \
-    const bool ok_ = prob_barrier(st, bar, abort_flag, limit_ticks);   \
-    MFE_PHASE(5);                                                      \
-    if (!ok_) return;                                                  \
+#define MFE_BARRIER()                                                    \
+  do {                                                                   \
+    bar += (unsigned)nb;                                                 \
+    const bool ok_ = prob_barrier(st, nb, bar, abort_flag, limit_ticks); \
+    MFE_PHASE(5);                                                        \
+    if (!ok_) return;                                                    \
   } while (0)
+  // a row's own p: in p on interior nodes, in A p on the faces
+  auto own_p = [&](int tile) {
+    return (prec[tile].inner[wave] >> lane) & 1u ? pp : App;
+  };
 
-  // 1. element matrices and source vectors (Hex8 element math, k = 1)
-  {
-    const double hx = 1.0 / P.Nx, hy = 1.0 / P.Ny, hz = 1.0 / P.Nz;
-    for (int64_t e = (int64_t)i * kBlock + t; e < ne; e += (int64_t)nb * kBlock) {
-      const int ex = (int)(e % P.Nx);
-      const int ey = (int)((e / P.Nx) % P.Ny);
-      const int ez = (int)(e / ((int64_t)P.Nx * P.Ny));
-      const double x0 = 1.0 * ex / P.Nx;
-      const double y0 = 1.0 * ey / P.Ny;
-      const double z0 = (1.0 * ez) / P.Nz;
-      const double x1 = x0 + hx, y1 = y0 + hy, z1 = z0 + hz;
-      const double c[24] = {x0, y0, z0, x1, y0, z0, x1, y1, z0, x0, y1, z0,
-                            x0, y0, z1, x1, y0, z1, x1, y1, z1, x0, y1, z1};
-      double Ke[36], Fe[8];
-      hex8_element<WAVES >= 3>(c, tab, 1.0, Ke, Fe);
-#pragma unroll
-      for (int q = 0; q < 36; ++q) K[(int64_t)q * ne + e] = Ke[q];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) F[(int64_t)q * ne + e] = Fe[q];
-    }
-  }
-  MFE_PHASE(0);
-  MFE_BARRIER();
-
-  // 2. rows: gather, Dirichlet, SELL store; x = 0, r = b
-  double acc = 0.0;
-  for (int tile = i; tile < ntiles; tile += nb) {
-    const int row = tile * kBlock + t;
-    if (row < P.n) {
-      const double bv = assemble_row(P, row, K, F, soff, scols, svals);
-      bp[row] = bv;
-      xp[row] = 0.0;
-      rp[row] = bv;
-      acc += bv * bv;
-    } else if (row < P.nslices * kWave) {
-      pad_row(P, row, soff, scols, svals);
-    }
-  }
-  {
-    const double v0 = block_sum<double>(acc, red);
-    if (t == 0) part[i] = v0;
-  }
-  MFE_PHASE(1);
-  MFE_BARRIER();
   double rtrans = sum_partials_all(part, nb, red);
   int buf = 1;
   const double bnorm = sqrt(rtrans);
   const double tol = rel_tol * bnorm;
-  double normr = bnorm, oldrtrans = 0.0;
+  double normr = bnorm, oldrtrans = 0.0, alpha = 0.0, acc = 0.0;
   int status = 0, k = 1;
-
-  // 3. CG
   for (; k <= max_iter && normr > tol; ++k) {
     const double beta = k == 1 ? 0.0 : rtrans / oldrtrans;
-    // four of the workgroup's tiles per step, loads before stores
+    // x takes the last iteration's alpha p on the way to the next p, so that p is
+    // read once; four of the workgroup's tiles per step, loads before stores
     for (int tile = i; tile < ntiles; tile += kUnroll * nb) {
-      double rv[kUnroll], pv[kUnroll];
+      double rv[kUnroll], pv[kUnroll], xv[kUnroll];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        const int row = (tile + u * nb) * kBlock + t;
-        const bool ok = tile + u * nb < ntiles && row < P.n;
+        const int tl = tile + u * nb, row = tl * kBlock + t;
+        const bool ok = tl < ntiles && row < P.n;
         rv[u] = ok ? rp[row] : 0.0;
-        pv[u] = ok && k > 1 ? pp[row] : 0.0;
+        pv[u] = ok && k > 1 ? own_p(tl)[row] : 0.0;
+        xv[u] = ok && k > 1 ? xp[row] : 0.0;
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        const int row = (tile + u * nb) * kBlock + t;
-        if (tile + u * nb < ntiles && row < P.n)
-          pp[row] = k == 1 ? 1.0 * rv[u] + 0.0 * rv[u] : 1.0 * rv[u] + beta * pv[u];
+        const int tl = tile + u * nb, row = tl * kBlock + t;
+        if (tl < ntiles && row < P.n) {
+          if (k > 1) xp[row] = 1.0 * xv[u] + alpha * pv[u];
+          own_p(tl)[row] = k == 1 ? 1.0 * rv[u] + 0.0 * rv[u] : 1.0 * rv[u] + beta * pv[u];
+        }
       }
     }
     MFE_PHASE(2);
@@ -395,12 +618,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8
     acc = 0.0;
     for (int tile = i; tile < ntiles; tile += nb) {
       const int row = tile * kBlock + t;
-      if (row / kWave < P.nslices) {
-        const double sum = batch_row_sum(P, row, soff, svals, pp);
-        if (row < P.n) {
-          App[row] = sum;
-          acc += sum * pp[row];
-        }
+      const BatchRec* rec = prec + tile;
+      const int form = rec->form;
+      if ((rec->inner[wave] >> lane) & 1u) {
+        const unsigned* w = words + (P.tile0 + tile) * (int64_t)(kBWords * kBlock) + t;
+        double sum, own;
+        if (form == kB10) sum = packed_row_sum<BPack10>(w, rec, pp, row, gx, plane, &own);
+        else if (form == kB10Near22)
+          sum = packed_row_sum<BPack10N22>(w, rec, pp, row, gx, plane, &own);
+        else if (form == kB20) sum = packed_row_sum<BPack20>(w, rec, pp, row, gx, plane, &own);
+        else sum = full_row_sum(P, soff, svals, pp, row, gx, plane, &own);
+        App[row] = sum;
+        acc += sum * own;
+      } else if (row < P.n) {
+        const double own = App[row];
+        acc += own * own;
       }
     }
     {
@@ -415,16 +647,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8
       status = 1;
       break;
     }
-    const double alpha = rtrans / pAp;
+    alpha = rtrans / pAp;
     acc = 0.0;
     for (int tile = i; tile < ntiles; tile += kUnroll * nb) {
-      double xv[kUnroll], pv[kUnroll], rv[kUnroll], av[kUnroll];
+      double rv[kUnroll], av[kUnroll];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         const int row = (tile + u * nb) * kBlock + t;
         const bool ok = tile + u * nb < ntiles && row < P.n;
-        xv[u] = ok ? xp[row] : 0.0;
-        pv[u] = ok ? pp[row] : 0.0;
         rv[u] = ok ? rp[row] : 0.0;
         av[u] = ok ? App[row] : 0.0;
       }
@@ -432,7 +662,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8
       for (int u = 0; u < kUnroll; ++u) {
         const int row = (tile + u * nb) * kBlock + t;
         if (tile + u * nb < ntiles && row < P.n) {
-          xp[row] = 1.0 * xv[u] + alpha * pv[u];
           const double r1 = 1.0 * rv[u] + (-alpha) * av[u];
           rp[row] = r1;
           acc += r1 * r1;
@@ -450,10 +679,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8
     buf ^= 1;
     normr = sqrt(rtrans);
   }
+  if (status == 0 && k > 1) {  // the last iteration's x
+    for (int tile = i; tile < ntiles; tile += nb) {
+      const int row = tile * kBlock + t;
+      if (row < P.n) xp[row] = 1.0 * xp[row] + alpha * own_p(tile)[row];
+    }
+    MFE_PHASE(4);
+  }
 #undef MFE_BARRIER
 #undef MFE_PHASE
   if (timer) {
-    for (int q = 0; q < 6; ++q) st->t_phase[q] = tp[q];
+    for (int q = 2; q < 6; ++q) st->t_phase[q] = tp[q];
     st->t_end = wall_clock64();
     st->iters = k - 1;
     st->status = status;
@@ -484,6 +720,8 @@ struct mfe_batch {
   int* d_scols = nullptr;
   double* d_svals = nullptr;
   double* d_KF = nullptr;
+  BatchRec* d_recs = nullptr;
+  unsigned* d_words = nullptr;  // null: every tile reads its SELL slices
   double *d_b = nullptr, *d_x = nullptr, *d_r = nullptr, *d_p = nullptr, *d_Ap = nullptr;
   double* d_part = nullptr;
   BatchState* d_states = nullptr;
@@ -496,6 +734,8 @@ struct mfe_batch {
     (void)hipFree(d_scols);
     (void)hipFree(d_svals);
     (void)hipFree(d_KF);
+    (void)hipFree(d_recs);
+    (void)hipFree(d_words);
     (void)hipFree(d_b);
     (void)hipFree(d_x);
     (void)hipFree(d_r);
@@ -585,7 +825,7 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
   // Problem layout and slice widths (closed form: a row's length is the
   // product of its per-axis neighbour counts).
   std::vector<double> work((size_t)nprob);
-  int64_t row0 = 0, soff0 = 0, slot0 = 0, elem0 = 0;
+  int64_t row0 = 0, soff0 = 0, slot0 = 0, elem0 = 0, tile0 = 0;
   for (int q = 0; q < nprob; ++q) {
     BatchProb P{};
     P.Nx = dims[3 * q];
@@ -599,6 +839,7 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
     P.soff0 = soff0;
     P.slot0 = slot0;
     P.elem0 = elem0;
+    P.tile0 = tile0;
     int acc = 0;
     for (int s = 0; s < P.nslices; ++s) {
       B->soff.push_back(acc);
@@ -616,6 +857,7 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
     soff0 += P.nslices + 1;
     slot0 += (int64_t)acc * kWave + kSellTail;  // each problem keeps its own over-read tail
     elem0 += 44 * (int64_t)P.ne;
+    tile0 += cdiv((int64_t)P.nslices * kWave, kBlock);
     // CG iterations grow with the largest side (the smallest mesh width)
     const double nnz = (3.0 * gx - 2) * (3.0 * gy - 2) * (3.0 * gz - 2);
     work[(size_t)q] = nnz * (double)std::max(P.Nx, std::max(P.Ny, P.Nz));
@@ -639,6 +881,7 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
   BALLOC(B->d_scols, sizeof(int) * (size_t)B->slots);
   BALLOC(B->d_svals, sizeof(double) * (size_t)B->slots);
   BALLOC(B->d_KF, sizeof(double) * (size_t)elem0);
+  BALLOC(B->d_recs, sizeof(BatchRec) * (size_t)tile0);
   BALLOC(B->d_b, sizeof(double) * (size_t)B->rows);
   BALLOC(B->d_x, sizeof(double) * (size_t)B->rows);
   BALLOC(B->d_r, sizeof(double) * (size_t)B->rows);
@@ -648,6 +891,13 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
   BALLOC(B->d_states, sizeof(BatchState) * (size_t)nprob);
   BALLOC(B->d_abort, sizeof(int));
 #undef BALLOC
+  // the packed words last: a batch that fits without them still runs
+  const char* pack = std::getenv("MINIFE_BATCH_PACK");
+  if (!(pack && std::atoi(pack) == 0) &&
+      hipMalloc(&B->d_words, sizeof(unsigned) * kBWords * kBlock * (size_t)tile0) != hipSuccess) {
+    (void)hipGetLastError();
+    B->d_words = nullptr;
+  }
   // zero everything once: the per-problem tails stay value 0, column 0
   auto fill = [&]() -> int {
     MFE_CHECK(ctx, hipMemsetAsync(B->d_scols, 0, sizeof(int) * (size_t)B->slots, s));
@@ -721,19 +971,28 @@ int mfe_batch_solve(mfe_ctx* ctx, mfe_batch* B, int max_iter, double rel_tol, in
     for (int q = 0; q < B->nprob; ++q) {
       const BatchProb& P = B->probs[(size_t)q];
       const double stored = (double)B->soff[(size_t)(P.soff0 + P.nslices)] * kWave;
-      work[(size_t)q] = (double)B->last_iters[(size_t)q] * (12.0 * stored + 88.0 * P.n) +
-                        400.0 * P.ne;
+      const double spmv = B->d_words ? 64.0 * P.n : 8.0 * stored + 24.0 * P.n;
+      work[(size_t)q] = (double)B->last_iters[(size_t)q] * (spmv + 64.0 * P.n);
     }
     batch_assign(B, work, B->capacity);
     if (int st2 = batch_upload_assignment(ctx, B)) return st2;
   }
   HexTables tab;
   host_tables(tab);
-  void* args[] = {&B->d_probs, &B->d_blk2prob, &tab,        &B->d_soff,   &B->d_scols,
-                  &B->d_svals, &B->d_KF,       &B->d_b,     &B->d_x,      &B->d_r,
-                  &B->d_p,     &B->d_Ap,       &B->d_part,  &B->d_states, &B->d_abort,
-                  &max_iter,   &rel_tol,       &limit};
+  void* args[] = {&B->d_probs, &B->d_blk2prob, &B->d_soff,   &B->d_svals, &B->d_recs,
+                  &B->d_words, &B->d_x,        &B->d_r,      &B->d_p,     &B->d_Ap,
+                  &B->d_part,  &B->d_states,   &B->d_abort,  &max_iter,   &rel_tol,
+                  &limit};
   MFE_CHECK(ctx, hipEventRecord(ctx->t_start, s));
+  const unsigned grid = (unsigned)B->grid;
+  batch_elements_kernel<<<grid, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, tab, B->d_KF,
+                                                B->d_states);
+  MFE_CHECK(ctx, hipGetLastError());
+  batch_rows_kernel<<<grid, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, B->d_soff, B->d_KF,
+                                            B->d_scols, B->d_svals, B->d_recs, B->d_words,
+                                            B->d_b, B->d_x, B->d_r, B->d_p, B->d_part,
+                                            B->d_states);
+  MFE_CHECK(ctx, hipGetLastError());
   MFE_CHECK(ctx, hipLaunchCooperativeKernel(B->kernel, dim3((unsigned)B->grid),
                                             dim3(kBlock), args, 0, s));
   MFE_CHECK(ctx, hipEventRecord(ctx->t_stop, s));

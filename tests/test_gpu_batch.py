@@ -129,3 +129,25 @@ def test_batch_64_boxes(mfe, oracle_mod):
     for p in sorted(picks):
         err = check_against_single_solve(oracle_mod, B, p, tuple(int(v) for v in dims[p]))
         say(f"  problem {p} at 1e-13: |x - x_oracle|/|x_oracle| = {err:.2e}")
+
+
+# No interior node, one, a tile's edge (256 rows), slots of 10 bits, cubes (the
+# near-zero slots up to 22), analytically zero edge neighbours and 2a^2 = b^2 + c^2
+# (20 bits).
+@pytest.mark.parametrize("dims", [(1, 1, 40), (2, 2, 2), (7, 7, 3), (24, 20, 31), (33, 33, 33),
+                                  (48, 48, 96), (75, 15, 105)])
+def test_batch_packed_values_are_exact(mfe, monkeypatch, dims):
+    """The CG on packed stencil values gives the bits of the CG on the values
+    themselves (the partial sums of both are grouped alike)."""
+    say(f"batch packed {dims}")
+    boxes = [dims, (5, 4, 3)]
+    out, xs = [], []
+    for pack in ("1", "0"):
+        monkeypatch.setenv("MINIFE_BATCH_PACK", pack)
+        B = mfe.Batch(boxes)
+        out.append(B.solve(max_iter=60, rel_tol=1e-12))
+        xs.append([B.download(p, matrix=False)["x"] for p in range(2)])
+    assert out[0]["iters"].tolist() == out[1]["iters"].tolist()
+    assert out[0]["iters"][0] > 0
+    for a, b in zip(*xs):
+        assert bits_equal(a, b)
