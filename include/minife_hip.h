@@ -315,29 +315,27 @@ int mfe_time_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y
  * reference solves one box per run).  Problem p is the unit cube meshed with
  * dims[3p..3p+2] = (nx, ny, nz) hex8 elements, unit conductivity, the
  * reference's source and Dirichlet faces.  mfe_batch_solve assembles every
- * problem and solves it with FP64 CG to ||r|| <= rel_tol * ||b|| in ONE
- * cooperative persistent launch; each assembled operator is bit-identical to
- * the reference's (generate_matrix_structure + assemble_FE_data + both
- * impose_dirichlet passes, driver.hpp:181-218).  Needs cooperative launch and
- * at least one resident workgroup per problem (else MFE_UNSUPPORTED). */
+ * problem and solves it with FP64 CG to ||r|| <= rel_tol * ||b||, all problems
+ * that are not done in the same launches; each assembled operator is
+ * bit-identical to the reference's (generate_matrix_structure +
+ * assemble_FE_data + both impose_dirichlet passes, driver.hpp:181-218).  At
+ * most two problems per compute unit (else MFE_UNSUPPORTED). */
 int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out);
 void mfe_batch_destroy(mfe_batch* batch);
 /* p = -1: {problems, workgroups, total rows, stored SELL entries, total
  * non-zeros, 0}; p >= 0: {rows, non-zeros, elements, workgroups, first
  * workgroup, stored SELL entries} of problem p. */
 int mfe_batch_info(const mfe_batch* batch, int p, int64_t info[6]);
-/* iters[nprob], rel_residual[nprob] (recursive ||r||/||b||) and the launch's
+/* iters[nprob], rel_residual[nprob] (recursive ||r||/||b||) and the solve's
  * GPU time in seconds (all nullable).  MFE_BREAKDOWN if a problem hit
- * non-positive p.Ap; MFE_HIP_ERROR if a problem barrier waited past its
- * 10 s limit (the launch is then abandoned by every workgroup). */
+ * non-positive p.Ap. */
 int mfe_batch_solve(mfe_ctx* ctx, mfe_batch* batch, int max_iter, double rel_tol, int* iters,
                     double* rel_residual, double* seconds);
 /* seconds[nprob]: each problem's time in the last solve (its first
- * workgroup's wall clock from entry to exit); phases[6*nprob] (nullable):
- * that workgroup's seconds in element math, row assembly, p updates, SpMVs,
- * x/r updates and barrier waits.  Every solve after the first re-divides the
- * workgroups in proportion to the traffic the previous solve's iteration
- * counts moved (the batch tunes its own balance). */
+ * workgroup's wall clock from the first launch to its end); phases[6*nprob]
+ * (nullable): that workgroup's seconds in element math, row assembly, x and p
+ * updates, SpMVs and r updates, and the rest, in which it waits for the other
+ * workgroups' end. */
 int mfe_batch_timing(const mfe_batch* batch, double* seconds, double* phases);
 /* Problem p's assembled operator as CSR (row_offsets[n+1], cols[nnz],
  * vals[nnz]), its right-hand side b[n] and solution x[n]; any may be NULL. */

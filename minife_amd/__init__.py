@@ -738,7 +738,7 @@ def cg_solve_multi(A: CSRMatrix, B: Vector, X: Vector, nrhs: int, max_iter: int 
 
 class Batch:
     """Many independent box problems (dims: (nprob, 3) elements per side),
-    assembled and solved by FP64 CG in one cooperative persistent launch."""
+    assembled and solved by FP64 CG together, every launch over all that are not done."""
 
     def __init__(self, dims, ctx: Context | None = None):
         self.ctx = ctx or default_context()

@@ -1,16 +1,14 @@
-// Batched miniFE: many independent box problems of uneven size assembled by two
-// launches over all of them and solved by FP64 CG in ONE persistent, cooperative
-// launch.
+// Batched miniFE: many independent box problems of uneven size, assembled and
+// solved by FP64 CG together: every launch works on all problems that are not
+// done.
 //
-// Each problem owns a contiguous range of the grid's workgroups, sized by its
-// expected work (non-zeros x CG iterations, the latter ~ the box's extent); the
-// ranges are laid over the XCDs one after the other, so that most problems stay
-// within one L2.
-// The workgroups of a problem meet at a problem-local barrier (an arrival
-// counter, agent-scope release/acquire), so problems never wait for each other.
-// The cooperative launch guarantees that every
-// workgroup is resident, and every wait is bounded by a wall-clock limit: a
-// wait that exceeds it raises the batch's abort flag and all workgroups leave.
+// A problem's rows fall into tiles of kBlock rows; a workgroup owns a few
+// consecutive tiles of one problem, the same ones in every launch.  The problems
+// are laid out with the ones expected to iterate longest first (the largest
+// side), so that the launches can end before the first problem of the tail that
+// is done.  (Laying a launch over the XCDs in contiguous ranges, so that a problem
+// stays within one L2, took 112.5 instead of 110.5 ms at 64 boxes: problems that
+// are done leave their XCD idle.)
 //
 // Per problem (same arithmetic as the single-box path, so the assembled
 // operator is bit-identical to the reference's):
@@ -20,14 +18,19 @@
 //      row-local because the BC sets are faces of the box), stored straight
 //      into the problem's SELL-64 slices and, for the CG, in an exact packed
 //      form (below); x = 0, r = b;
-//   3. CG (cg_solve.hpp:69-229 with the fast, tree-reduced dots): the last
-//      iteration's x update and p update, barrier, SpMV + p.Ap partials,
-//      barrier, r update + r.r partials, barrier.  Partials alternate between
-//      two buffers, so a workgroup that
-//      runs ahead never overwrites what a slower one is still summing.  Every
-//      workgroup sums a problem's partials in the same order, so all of them
-//      take the same scalars and leave the loop at the same iteration.
+//   3. CG (cg_solve.hpp:69-229 with the fast, tree-reduced dots), three launches
+//      per iteration: the last iteration's x update and the p update, SpMV with
+//      p.Ap partials, r update with r.r partials.  Every workgroup sums its
+//      problem's partials in the same order, so all of them take the same
+//      scalars; the problem's first one writes the state.  The host launches a
+//      few iterations ahead of the GPU, which reports the iteration it is in and
+//      the problems that are done in pinned words.
 //
+// Against one cooperative launch whose workgroups each ran their problem's whole
+// CG, meeting at problem-local barriers (3.9 us each, and the phases
+// of a problem as slow as its slowest workgroup): 64 boxes of 16..96 171 ms, so 110;
+// two 150^3 110, so 72; 12 of 20..64 13.1, so 7.2; one 30^3 1.26, so 0.87.
+
 // A row or a column of a Dirichlet face (all six faces are) is the identity's, so
 // the operator couples interior nodes only, and an interior row has all its 27
 // neighbours.  The CG keeps p = 0 on the faces in the vector that rows gather
@@ -52,11 +55,12 @@ struct BatchProb {
   int ne;          // elements
   int nslices;     // ceil(n / 64)
   int b0, nb;      // first workgroup, workgroup count
+  int tpb, ntiles; // tiles per workgroup and in all
   int64_t row0;    // base of the problem's rows in the vectors
   int64_t soff0;   // base of its nslices+1 slice offsets
   int64_t slot0;   // base of its SELL entries
   int64_t elem0;   // base of its element scratch (44 doubles per element)
-  int64_t part0;   // base of its 2*nb partials
+  int64_t part0;   // base of its 2*nb partials: nb of r.r, nb of p.Ap
   int64_t tile0;   // index of its first tile's record and packed words
 };
 
@@ -93,70 +97,23 @@ using BPack10N22 = BatchPack<10, 22>;   // 11
 using BPack20 = BatchPack<20, 20>;      // 17
 constexpr int kBWords = BPack20::words;  // words kept per row of a tile
 
-struct BatchState {  // per problem, zeroed before each launch
-  unsigned count, pad0;  // arrivals at the problem's barriers
-  int iters, status;  // status: 0 converged or max_iter, 1 breakdown, 2 aborted
-  double normr, tol, bnorm, pad;
+struct BatchState {  // per problem, zeroed before each solve
+  unsigned done_at;    // iteration at which the problem ended; 0: it has not
+  int iters, status;   // status: 0 converged or max_iter, 1 breakdown
+  int pad;
+  double normr, tol, bnorm;
+  double alpha;        // of the last complete iteration
+  double rtrans[2];    // r.r at the start of iteration k at [k & 1]
   uint64_t t_begin, t_end;  // wall clock of the problem's first workgroup
   // that workgroup's clock ticks per phase: element math, row assembly,
-  // p update, SpMV, x/r update, barrier waits
-  uint64_t t_phase[6];
+  // x and p update, SpMV, r update
+  uint64_t t_phase[5];
 };
 
-constexpr double kBatchWaitSeconds = 10.0;
 constexpr int kUnroll = 4;  // tiles per step of the vector loops
-
-// Problem-local barrier: an arrival counter that only grows; the barrier is
-// complete when it reaches `target` (nb more than at the last one; it may wrap).
-// The workgroup's stores are complete in L2 after __syncthreads (L1 writes
-// through); thread 0 releases them at agent scope (writes the L2 back, so
-// workgroups on other XCDs see them), arrives, waits, and acquires (invalidates
-// this CU's L1 and the XCD's non-coherent L2 lines) before the workgroup reads
-// what others wrote.  Every arrival is a read-modify-write of the same word, so
-// the one that completes it carries the releases of all earlier ones.
-// Bound by the round trips to memory: one release, one arrival, the poll.  The
-// polls are relaxed: with an acquire in each, every waiting workgroup kept
-// invalidating the L2 under the workgroups still at work (64 boxes of 16..96:
-// 290 ms, so 251; two 150^3: 233, so 183), and with a separate generation word
-// and a load of the abort flag per poll it had two more trips (30^3: 6.1 us per
-// barrier, so 3.9; the acquiring polls 11.5).  The abort flag is looked at every
-// 16th poll; a problem whose own barriers complete runs on.
-// Returns false when the batch was aborted.
-__device__ bool prob_barrier(BatchState* st, int nb, unsigned target, int* abort_flag,
-                             uint64_t limit_ticks) {
-  __syncthreads();
-  if (nb == 1) return true;
-  __shared__ int s_ok;
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    unsigned seen =
-        __hip_atomic_fetch_add(&st->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-    int ok = 1;
-    if ((int)(seen - target) < 0) {
-      const uint64_t t0 = wall_clock64();
-      for (unsigned polls = 1;; ++polls) {
-        seen = __hip_atomic_load(&st->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if ((int)(seen - target) >= 0) break;
-        if (polls % 16 == 0) {
-          if (__hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-            ok = 0;
-            break;
-          }
-          if (wall_clock64() - t0 > limit_ticks) {
-            __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ok = 0;
-            break;
-          }
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    s_ok = ok;
-  }
-  __syncthreads();
-  return s_ok != 0;
-}
+constexpr int kMaxPart = 1024;  // a problem's workgroups (every one sums all partials)
+constexpr int kBatchProblemsPerCu = 2;  // more are refused
+constexpr unsigned kAhead = 6;  // iterations the host launches ahead of the GPU's
 
 // Sum of a problem's nb partials in a fixed order (the same in every workgroup).
 __device__ double sum_partials_all(const double* pp, int nb, double* red) {
@@ -457,14 +414,30 @@ __device__ __forceinline__ double full_row_sum(const BatchProb& P, const int* __
   return sum;
 }
 
+// What a workgroup works on.
+struct BatchWg {
+  int pi, i;   // problem, index within it
+  int t0, t1;  // tiles
+};
+__device__ __forceinline__ BatchWg batch_wg(const BatchProb* __restrict__ probs,
+                                            const int* __restrict__ blk2prob) {
+  const int wg = (int)blockIdx.x;
+  BatchWg w;
+  w.pi = blk2prob[wg];
+  const BatchProb& P = probs[w.pi];
+  w.i = wg - P.b0;
+  w.t0 = w.i * P.tpb;
+  w.t1 = min(w.t0 + P.tpb, P.ntiles);
+  return w;
+}
+
 // Element matrices and source vectors of every problem (Hex8 element math, k = 1).
 __global__ __launch_bounds__(kBlock) void batch_elements_kernel(
     const BatchProb* __restrict__ probs, const int* __restrict__ blk2prob, HexTables tab,
     double* KF, BatchState* states) {
-  const int wg = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
-  const int pi = blk2prob[wg];
-  const BatchProb P = probs[pi];
-  const int i = wg - P.b0, t = (int)threadIdx.x;
+  const BatchWg wg = batch_wg(probs, blk2prob);
+  const BatchProb P = probs[wg.pi];
+  const int i = wg.i, t = (int)threadIdx.x;
   const int64_t ne = P.ne;
   double* K = KF + P.elem0;
   double* F = K + 36 * ne;
@@ -488,7 +461,7 @@ __global__ __launch_bounds__(kBlock) void batch_elements_kernel(
     for (int q = 0; q < 8; ++q) F[(int64_t)q * ne + e] = Fe[q];
   }
   if (i == 0 && t == 0) {
-    BatchState* st = states + pi;
+    BatchState* st = states + wg.pi;
     st->t_begin = tc;
     st->t_phase[0] = wall_clock64() - tc;
   }
@@ -502,18 +475,16 @@ __global__ __launch_bounds__(kBlock) void batch_rows_kernel(
     BatchRec* recs, unsigned* words, double* b, double* x, double* r, double* p,
     double* partials, BatchState* states) {
   __shared__ double red[4];
-  const int wg = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
-  const int pi = blk2prob[wg];
-  const BatchProb P = probs[pi];
-  const int i = wg - P.b0, nb = P.nb, t = (int)threadIdx.x;
+  const BatchWg wg = batch_wg(probs, blk2prob);
+  const BatchProb P = probs[wg.pi];
+  const int t = (int)threadIdx.x;
   const double* K = KF + P.elem0;
   const double* F = K + 36 * (int64_t)P.ne;
   const int* soff = soff_all + P.soff0;
   const int gx = P.Nx + 1, gy = P.Ny + 1;
-  const int ntiles = (int)cdiv((int64_t)P.nslices * kWave, kBlock);
   const uint64_t tc = wall_clock64();
   double acc = 0.0;
-  for (int tile = i; tile < ntiles; tile += nb) {
+  for (int tile = wg.t0; tile < wg.t1; ++tile) {
     const int row = tile * kBlock + t;
     double v[kBSlots];
     bool in = false;
@@ -533,169 +504,197 @@ __global__ __launch_bounds__(kBlock) void batch_rows_kernel(
               words ? words + (P.tile0 + tile) * (int64_t)(kBWords * kBlock) : nullptr);
   }
   const double v0 = block_sum<double>(acc, red);
-  if (t == 0) partials[P.part0 + i] = v0;
-  if (i == 0 && t == 0) states[pi].t_phase[1] = wall_clock64() - tc;
+  if (t == 0) partials[P.part0 + wg.i] = v0;
+  if (wg.i == 0 && t == 0) states[wg.pi].t_phase[1] = wall_clock64() - tc;
 }
 
-// The CG of every problem.  WAVES: the minimum waves per SIMD the register
-// allocation must allow.
-template <int WAVES>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, 8))) void batch_kernel(
+// A row's own p: in p on interior nodes, in A p on the faces.
+__device__ __forceinline__ double* own_p(const BatchRec* __restrict__ rec, int wave, int lane,
+                                         double* pp, double* App) {
+  return (rec->inner[wave] >> lane) & 1u ? pp : App;
+}
+
+// The problem's first workgroup at its end in iteration k.
+__device__ __forceinline__ void batch_end(BatchState* st, int* host, int pi, unsigned k,
+                                          double normr, int status) {
+  st->done_at = k;
+  st->iters = (int)(k - 1);
+  st->normr = normr;
+  st->status = status;
+  st->t_end = wall_clock64();
+  __hip_atomic_store(host + 1 + pi, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Start of iteration k: the convergence test, x += alpha p of the iteration
+// before, and p = r + beta p unless the problem is done.  x rides along because
+// p is read here anyway (40 bytes per row; with x in the r update 24 + 48
+// instead of 40 + 24 for the two).  The loads of the first tiles are issued
+// before the sum of the partials.
+__global__ __launch_bounds__(kBlock) void batch_p_kernel(
     const BatchProb* __restrict__ probs, const int* __restrict__ blk2prob,
-    const int* __restrict__ soff_all, const double* __restrict__ svals,
-    const BatchRec* __restrict__ recs, const unsigned* __restrict__ words, double* x, double* r,
-    double* p, double* Ap, double* partials, BatchState* states, int* abort_flag, int max_iter,
-    double rel_tol, uint64_t limit_ticks) {
+    const BatchRec* __restrict__ recs, double* __restrict__ x, const double* __restrict__ r,
+    double* p, double* Ap, const double* __restrict__ partials, BatchState* states, int* host,
+    unsigned k, int max_iter, double rel_tol) {
   __shared__ double red[4];
-  const int wg = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
-  const int pi = blk2prob[wg];
-  const BatchProb P = probs[pi];
-  BatchState* st = states + pi;
-  const int i = wg - P.b0, nb = P.nb, t = (int)threadIdx.x;
+  const int t = (int)threadIdx.x;
+  if (blockIdx.x == 0 && t == 0)
+    __hip_atomic_store(host, (int)k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  const uint64_t tc = wall_clock64();
+  const BatchWg wg = batch_wg(probs, blk2prob);
+  const BatchProb& P = probs[wg.pi];
+  BatchState* st = states + wg.pi;
+  // (the first workgroup may be writing done_at = k)
+  const unsigned done_at = st->done_at;
+  if (done_at && done_at < k) return;
   const int lane = t % kWave, wave = __builtin_amdgcn_readfirstlane(t / kWave);
-  const int* soff = soff_all + P.soff0;
   const BatchRec* prec = recs + P.tile0;
-  const int gx = P.Nx + 1, plane = gx * (P.Ny + 1);
+  const int n = P.n;
   double* xp = x + P.row0;
-  double* rp = r + P.row0;
+  const double* rp = r + P.row0;
   double* pp = p + P.row0;
   double* App = Ap + P.row0;
-  double* part = partials + P.part0;
-  const int ntiles = (int)cdiv((int64_t)P.nslices * kWave, kBlock);
-  const bool timer = i == 0 && t == 0;
-  unsigned bar = 0;  // arrivals that complete the problem's next barrier
-  uint64_t tp[6] = {0, 0, 0, 0, 0, 0};
-  uint64_t tc = wall_clock64();
-#define MFE_PHASE(k)                  \
-  do {                                \
-    const uint64_t now_ = wall_clock64(); \
-    tp[k] += now_ - tc;               \
-    tc = now_;                        \
-  } while (0)
-#define MFE_BARRIER()                                                    \
-  do {                                                                   \
-    bar += (unsigned)nb;                                                 \
-    const bool ok_ = prob_barrier(st, nb, bar, abort_flag, limit_ticks); \
-    MFE_PHASE(5);                                                        \
-    if (!ok_) return;                                                    \
-  } while (0)
-  // a row's own p: in p on interior nodes, in A p on the faces
-  auto own_p = [&](int tile) {
-    return (prec[tile].inner[wave] >> lane) & 1u ? pp : App;
+  double rv[kUnroll], pv[kUnroll], xv[kUnroll];
+  auto load = [&](int tile) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int row = (tile + u) * kBlock + t;
+      const bool ok = tile + u < wg.t1 && row < n;
+      rv[u] = ok ? rp[row] : 0.0;
+      pv[u] = ok && k > 1 ? own_p(prec + tile + u, wave, lane, pp, App)[row] : 0.0;
+      xv[u] = ok && k > 1 ? xp[row] : 0.0;
+    }
   };
+  load(wg.t0);
+  const double rtrans = sum_partials_all(partials + P.part0, P.nb, red);
+  const double normr = sqrt(rtrans);
+  const double tol = k == 1 ? rel_tol * normr : st->tol;
+  const double alpha = k == 1 ? 0.0 : st->alpha;
+  const double beta = k == 1 ? 0.0 : rtrans / st->rtrans[(k - 1) & 1];
+  const bool stop = k > (unsigned)max_iter || !(normr > tol);
+  for (int tile = wg.t0; tile < wg.t1;) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int row = (tile + u) * kBlock + t;
+      if (tile + u < wg.t1 && row < n) {
+        if (k > 1) xp[row] = 1.0 * xv[u] + alpha * pv[u];
+        if (!stop)
+          own_p(prec + tile + u, wave, lane, pp, App)[row] =
+              k == 1 ? 1.0 * rv[u] + 0.0 * rv[u] : 1.0 * rv[u] + beta * pv[u];
+      }
+    }
+    tile += kUnroll;
+    if (tile < wg.t1) load(tile);
+  }
+  if (wg.i == 0 && t == 0) {
+    st->rtrans[k & 1] = rtrans;
+    if (k == 1) {
+      st->tol = tol;
+      st->bnorm = normr;
+    }
+    if (stop) batch_end(st, host, wg.pi, k, normr, 0);
+    st->t_phase[2] += wall_clock64() - tc;
+  }
+}
 
-  double rtrans = sum_partials_all(part, nb, red);
-  int buf = 1;
-  const double bnorm = sqrt(rtrans);
-  const double tol = rel_tol * bnorm;
-  double normr = bnorm, oldrtrans = 0.0, alpha = 0.0, acc = 0.0;
-  int status = 0, k = 1;
-  for (; k <= max_iter && normr > tol; ++k) {
-    const double beta = k == 1 ? 0.0 : rtrans / oldrtrans;
-    // x takes the last iteration's alpha p on the way to the next p, so that p is
-    // read once; four of the workgroup's tiles per step, loads before stores
-    for (int tile = i; tile < ntiles; tile += kUnroll * nb) {
-      double rv[kUnroll], pv[kUnroll], xv[kUnroll];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int tl = tile + u * nb, row = tl * kBlock + t;
-        const bool ok = tl < ntiles && row < P.n;
-        rv[u] = ok ? rp[row] : 0.0;
-        pv[u] = ok && k > 1 ? own_p(tl)[row] : 0.0;
-        xv[u] = ok && k > 1 ? xp[row] : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int tl = tile + u * nb, row = tl * kBlock + t;
-        if (tl < ntiles && row < P.n) {
-          if (k > 1) xp[row] = 1.0 * xv[u] + alpha * pv[u];
-          own_p(tl)[row] = k == 1 ? 1.0 * rv[u] + 0.0 * rv[u] : 1.0 * rv[u] + beta * pv[u];
-        }
-      }
+// A p and the partials of p.Ap.  About 63 bytes per row; 64 boxes of 16..96 average
+// 2.7 TB/s, two 150^3 3.1: bound by the 27 entries of p per row going through
+// the L1s.  128 registers (four waves per SIMD; with three 122 ms for the whole
+// solve instead of 112, with five the 150^3 boxes lose 2%).  With p staged in
+// LDS, three windows for four tiles at a time, 115 to 124 ms.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void batch_spmv_kernel(
+    const BatchProb* __restrict__ probs, const int* __restrict__ blk2prob,
+    const int* __restrict__ soff_all, const double* __restrict__ svals,
+    const BatchRec* __restrict__ recs, const unsigned* __restrict__ words,
+    const double* __restrict__ p, double* Ap, double* __restrict__ partials,
+    BatchState* states) {
+  __shared__ double red[4];
+  const uint64_t tc = wall_clock64();
+  const BatchWg wg = batch_wg(probs, blk2prob);
+  const BatchProb& P = probs[wg.pi];
+  BatchState* st = states + wg.pi;
+  if (st->done_at) return;
+  const int t = (int)threadIdx.x;
+  const int lane = t % kWave, wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int* soff = soff_all + P.soff0;
+  const int n = P.n, gx = P.Nx + 1, plane = gx * (P.Ny + 1);
+  const double* pp = p + P.row0;
+  double* App = Ap + P.row0;
+  double acc = 0.0;
+  for (int tile = wg.t0; tile < wg.t1; ++tile) {
+    const int row = tile * kBlock + t;
+    const BatchRec* rec = recs + P.tile0 + tile;
+    const int form = rec->form;
+    if ((rec->inner[wave] >> lane) & 1u) {
+      const unsigned* w = words + (P.tile0 + tile) * (int64_t)(kBWords * kBlock) + t;
+      double sum, own;
+      if (form == kB10) sum = packed_row_sum<BPack10>(w, rec, pp, row, gx, plane, &own);
+      else if (form == kB10Near22)
+        sum = packed_row_sum<BPack10N22>(w, rec, pp, row, gx, plane, &own);
+      else if (form == kB20) sum = packed_row_sum<BPack20>(w, rec, pp, row, gx, plane, &own);
+      else sum = full_row_sum(P, soff, svals, pp, row, gx, plane, &own);
+      App[row] = sum;
+      acc += sum * own;
+    } else if (row < n) {
+      const double own = App[row];
+      acc += own * own;
     }
-    MFE_PHASE(2);
-    MFE_BARRIER();
-    acc = 0.0;
-    for (int tile = i; tile < ntiles; tile += nb) {
-      const int row = tile * kBlock + t;
-      const BatchRec* rec = prec + tile;
-      const int form = rec->form;
-      if ((rec->inner[wave] >> lane) & 1u) {
-        const unsigned* w = words + (P.tile0 + tile) * (int64_t)(kBWords * kBlock) + t;
-        double sum, own;
-        if (form == kB10) sum = packed_row_sum<BPack10>(w, rec, pp, row, gx, plane, &own);
-        else if (form == kB10Near22)
-          sum = packed_row_sum<BPack10N22>(w, rec, pp, row, gx, plane, &own);
-        else if (form == kB20) sum = packed_row_sum<BPack20>(w, rec, pp, row, gx, plane, &own);
-        else sum = full_row_sum(P, soff, svals, pp, row, gx, plane, &own);
-        App[row] = sum;
-        acc += sum * own;
-      } else if (row < P.n) {
-        const double own = App[row];
-        acc += own * own;
-      }
-    }
-    {
-      const double v0 = block_sum<double>(acc, red);
-      if (t == 0) part[buf * nb + i] = v0;
-    }
-    MFE_PHASE(3);
-    MFE_BARRIER();
-    const double pAp = sum_partials_all(part + buf * nb, nb, red);
-    buf ^= 1;
-    if (!(pAp > 0.0)) {  // non-positive curvature: the operator is not SPD here
-      status = 1;
-      break;
-    }
-    alpha = rtrans / pAp;
-    acc = 0.0;
-    for (int tile = i; tile < ntiles; tile += kUnroll * nb) {
-      double rv[kUnroll], av[kUnroll];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int row = (tile + u * nb) * kBlock + t;
-        const bool ok = tile + u * nb < ntiles && row < P.n;
-        rv[u] = ok ? rp[row] : 0.0;
-        av[u] = ok ? App[row] : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int row = (tile + u * nb) * kBlock + t;
-        if (tile + u * nb < ntiles && row < P.n) {
-          const double r1 = 1.0 * rv[u] + (-alpha) * av[u];
-          rp[row] = r1;
-          acc += r1 * r1;
-        }
-      }
-    }
-    {
-      const double v0 = block_sum<double>(acc, red);
-      if (t == 0) part[buf * nb + i] = v0;
-    }
-    MFE_PHASE(4);
-    MFE_BARRIER();
-    oldrtrans = rtrans;
-    rtrans = sum_partials_all(part + buf * nb, nb, red);
-    buf ^= 1;
-    normr = sqrt(rtrans);
   }
-  if (status == 0 && k > 1) {  // the last iteration's x
-    for (int tile = i; tile < ntiles; tile += nb) {
-      const int row = tile * kBlock + t;
-      if (row < P.n) xp[row] = 1.0 * xp[row] + alpha * own_p(tile)[row];
+  const double v0 = block_sum<double>(acc, red);
+  if (t == 0) partials[P.part0 + P.nb + wg.i] = v0;
+  if (wg.i == 0 && t == 0) st->t_phase[3] += wall_clock64() - tc;
+}
+
+// alpha = r.r / p.Ap, r -= alpha Ap, and the partials of r.r.
+__global__ __launch_bounds__(kBlock) void batch_r_kernel(
+    const BatchProb* __restrict__ probs, const int* __restrict__ blk2prob,
+    double* __restrict__ r, const double* __restrict__ Ap, double* partials, BatchState* states,
+    int* host, unsigned k) {
+  __shared__ double red[4];
+  const uint64_t tc = wall_clock64();
+  const BatchWg wg = batch_wg(probs, blk2prob);
+  const BatchProb& P = probs[wg.pi];
+  BatchState* st = states + wg.pi;
+  if (st->done_at) return;  // (also what a breakdown of this iteration may have written)
+  const int t = (int)threadIdx.x, n = P.n;
+  double* rp = r + P.row0;
+  const double* App = Ap + P.row0;
+  double rv[kUnroll], av[kUnroll];
+  auto load = [&](int tile) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int row = (tile + u) * kBlock + t;
+      const bool ok = tile + u < wg.t1 && row < n;
+      rv[u] = ok ? rp[row] : 0.0;
+      av[u] = ok ? App[row] : 0.0;
     }
-    MFE_PHASE(4);
+  };
+  load(wg.t0);
+  const double pAp = sum_partials_all(partials + P.part0 + P.nb, P.nb, red);
+  const double rtrans = st->rtrans[k & 1];
+  if (!(pAp > 0.0)) {  // non-positive curvature: the operator is not SPD here
+    if (wg.i == 0 && t == 0) batch_end(st, host, wg.pi, k, sqrt(rtrans), 1);
+    return;
   }
-#undef MFE_BARRIER
-#undef MFE_PHASE
-  if (timer) {
-    for (int q = 2; q < 6; ++q) st->t_phase[q] = tp[q];
-    st->t_end = wall_clock64();
-    st->iters = k - 1;
-    st->status = status;
-    st->normr = normr;
-    st->tol = tol;
-    st->bnorm = bnorm;
+  const double alpha = rtrans / pAp;
+  double acc = 0.0;
+  for (int tile = wg.t0; tile < wg.t1;) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int row = (tile + u) * kBlock + t;
+      if (tile + u < wg.t1 && row < n) {
+        const double r1 = 1.0 * rv[u] + (-alpha) * av[u];
+        rp[row] = r1;
+        acc += r1 * r1;
+      }
+    }
+    tile += kUnroll;
+    if (tile < wg.t1) load(tile);
+  }
+  const double v0 = block_sum<double>(acc, red);
+  if (t == 0) partials[P.part0 + wg.i] = v0;
+  if (wg.i == 0 && t == 0) {
+    st->alpha = alpha;
+    st->t_phase[4] += wall_clock64() - tc;
   }
 }
 
@@ -705,15 +704,14 @@ using namespace mfe;
 
 struct mfe_batch {
   mfe_ctx* ctx = nullptr;
-  int nprob = 0, grid = 0, capacity = 0;
-  const void* kernel = nullptr;  // the batch_kernel instance (occupancy) in use
+  int nprob = 0, grid = 0;
   double tick_seconds = 1e-8;  // wall clock period
   std::vector<double> last_seconds;  // per problem, previous solve
   std::vector<double> last_phases;   // per problem x 6 phases, previous solve
   std::vector<BatchProb> probs;
   std::vector<int> soff;      // all problems' slice offsets
   std::vector<int> blk2prob;  // problem of each workgroup
-  std::vector<int> last_iters;  // iterations of the previous solve (rebalancing)
+  std::vector<int> order;     // the problems as they are laid out
   BatchProb* d_probs = nullptr;
   int* d_blk2prob = nullptr;
   int* d_soff = nullptr;
@@ -725,7 +723,7 @@ struct mfe_batch {
   double *d_b = nullptr, *d_x = nullptr, *d_r = nullptr, *d_p = nullptr, *d_Ap = nullptr;
   double* d_part = nullptr;
   BatchState* d_states = nullptr;
-  int* d_abort = nullptr;
+  int* h_words = nullptr;  // pinned: the iteration the GPU is in, then a flag per problem
   int64_t rows = 0, slots = 0;
   void release() {
     (void)hipFree(d_probs);
@@ -743,48 +741,43 @@ struct mfe_batch {
     (void)hipFree(d_Ap);
     (void)hipFree(d_part);
     (void)hipFree(d_states);
-    (void)hipFree(d_abort);
+    if (h_words) (void)hipHostFree(h_words);
   }
 };
 
 static int host_axis_len(int i, int g) { return 1 + (i > 0) + (i < g - 1); }
 
-// Workgroups per problem: one each, then the rest one at a time to the
-// problem with the most work per workgroup (capped at its tile count).
-static void batch_assign(mfe_batch* B, const std::vector<double>& work, int grid) {
-  const int nprob = B->nprob;
-  std::vector<int> nb((size_t)nprob, 1);
-  int left = grid - nprob;
-  while (left > 0) {
-    int best = -1;
-    double bw = -1;
-    for (int q = 0; q < nprob; ++q) {
-      const int tiles = (int)cdiv((int64_t)B->probs[(size_t)q].nslices * kWave, kBlock);
-      if (nb[(size_t)q] >= tiles) continue;
-      const double w = work[(size_t)q] / nb[(size_t)q];
-      if (w > bw) {
-        bw = w;
-        best = q;
-      }
-    }
-    if (best < 0) break;
-    ++nb[(size_t)best];
-    --left;
-  }
-  B->blk2prob.clear();
+// The problems' workgroups: the problems in descending order of their largest
+// side.  Up to 4 tiles per workgroup where that still leaves 16 workgroups per CU
+// (one step of the vector loops, and fewer partials for each to sum: 64 boxes of
+// 16..96 take 112 ms, with 2 tiles 127, with 8 113), more where a problem would
+// have more than kMaxPart.
+static void batch_layout(mfe_batch* B, int cus) {
+  int64_t tiles = 0;
+  for (const BatchProb& P : B->probs) tiles += P.ntiles;
+  const int least = (int)std::max<int64_t>(1, std::min<int64_t>(kUnroll, tiles / (16 * cus)));
+  auto side = [&](int q) {
+    const BatchProb& P = B->probs[(size_t)q];
+    return std::max(P.Nx, std::max(P.Ny, P.Nz));
+  };
+  B->order.resize((size_t)B->nprob);
+  for (int q = 0; q < B->nprob; ++q) B->order[(size_t)q] = q;
+  std::stable_sort(B->order.begin(), B->order.end(),
+                   [&](int a, int b) { return side(a) > side(b); });
   int64_t part0 = 0;
-  for (int q = 0; q < nprob; ++q) {
+  for (int q : B->order) {
     BatchProb& P = B->probs[(size_t)q];
+    P.tpb = std::max(least, (int)cdiv(P.ntiles, kMaxPart));
     P.b0 = (int)B->blk2prob.size();
-    P.nb = nb[(size_t)q];
+    P.nb = (int)cdiv(P.ntiles, P.tpb);
     P.part0 = part0;
     part0 += 2 * (int64_t)P.nb;
-    for (int k = 0; k < P.nb; ++k) B->blk2prob.push_back(q);
+    B->blk2prob.insert(B->blk2prob.end(), (size_t)P.nb, q);
   }
   B->grid = (int)B->blk2prob.size();
 }
 
-static int batch_upload_assignment(mfe_ctx* ctx, mfe_batch* B) {
+static int batch_upload_layout(mfe_ctx* ctx, mfe_batch* B) {
   hipStream_t s = ctx->stream;
   MFE_CHECK(ctx, hipMemcpyAsync(B->d_probs, B->probs.data(), sizeof(BatchProb) * B->probs.size(),
                                 hipMemcpyHostToDevice, s));
@@ -803,28 +796,13 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
     if (dims[q] < 1 || dims[q] > 1024)
       return fail(ctx, MFE_BAD_ARG, "batch_create: box sides must be in [1, 1024] elements");
   MFE_CHECK(ctx, hipSetDevice(ctx->device));
-  int waves = 2;
-  if (const char* e = std::getenv("MINIFE_BATCH_WAVES")) waves = std::atoi(e);
-  if (waves < 2 || waves > 4) waves = 2;
-  const void* kern = waves == 4 ? (const void*)batch_kernel<4>
-                                : waves == 3 ? (const void*)batch_kernel<3> : (const void*)batch_kernel<2>;
-  int per_cu = 0;
-  MFE_CHECK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kBlock, 0));
-  int coop = 0;
-  MFE_CHECK(ctx, hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
-  const int grid = per_cu * ctx->cu_count;
-  if (!coop || grid < nprob)
-    return fail(ctx, MFE_UNSUPPORTED, "batch_create: needs a cooperative launch with at least one "
-                                      "resident workgroup per problem");
+  if (nprob > kBatchProblemsPerCu * ctx->cu_count)
+    return fail(ctx, MFE_UNSUPPORTED, "batch_create: more than two problems per compute unit");
   mfe_batch* B = new mfe_batch();
   B->ctx = ctx;
   B->nprob = nprob;
-  B->grid = grid;
-  B->capacity = grid;
-  B->kernel = kern;
   // Problem layout and slice widths (closed form: a row's length is the
   // product of its per-axis neighbour counts).
-  std::vector<double> work((size_t)nprob);
   int64_t row0 = 0, soff0 = 0, slot0 = 0, elem0 = 0, tile0 = 0;
   for (int q = 0; q < nprob; ++q) {
     BatchProb P{};
@@ -857,15 +835,13 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
     soff0 += P.nslices + 1;
     slot0 += (int64_t)acc * kWave + kSellTail;  // each problem keeps its own over-read tail
     elem0 += 44 * (int64_t)P.ne;
-    tile0 += cdiv((int64_t)P.nslices * kWave, kBlock);
-    // CG iterations grow with the largest side (the smallest mesh width)
-    const double nnz = (3.0 * gx - 2) * (3.0 * gy - 2) * (3.0 * gz - 2);
-    work[(size_t)q] = nnz * (double)std::max(P.Nx, std::max(P.Ny, P.Nz));
+    P.ntiles = (int)cdiv((int64_t)P.nslices * kWave, kBlock);
+    tile0 += P.ntiles;
     B->probs.push_back(P);
   }
   B->rows = row0;
   B->slots = slot0;
-  batch_assign(B, work, grid);
+  batch_layout(B, ctx->cu_count);
   hipStream_t s = ctx->stream;
   auto fail_oom = [&](hipError_t e) {
     B->release();
@@ -876,7 +852,7 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
 #define BALLOC(ptr, bytes) \
   if ((e = hipMalloc(&(ptr), (bytes))) != hipSuccess) return fail_oom(e)
   BALLOC(B->d_probs, sizeof(BatchProb) * (size_t)nprob);
-  BALLOC(B->d_blk2prob, sizeof(int) * (size_t)B->capacity);  // any later re-division fits
+  BALLOC(B->d_blk2prob, sizeof(int) * B->blk2prob.size());
   BALLOC(B->d_soff, sizeof(int) * B->soff.size());
   BALLOC(B->d_scols, sizeof(int) * (size_t)B->slots);
   BALLOC(B->d_svals, sizeof(double) * (size_t)B->slots);
@@ -887,10 +863,12 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
   BALLOC(B->d_r, sizeof(double) * (size_t)B->rows);
   BALLOC(B->d_p, sizeof(double) * (size_t)B->rows);
   BALLOC(B->d_Ap, sizeof(double) * (size_t)B->rows);
-  BALLOC(B->d_part, sizeof(double) * 2 * (size_t)B->capacity);
+  BALLOC(B->d_part, sizeof(double) * 2 * B->blk2prob.size());
   BALLOC(B->d_states, sizeof(BatchState) * (size_t)nprob);
-  BALLOC(B->d_abort, sizeof(int));
 #undef BALLOC
+  if ((e = hipHostMalloc(&B->h_words, sizeof(int) * (1 + (size_t)nprob),
+                         hipHostMallocCoherent)) != hipSuccess)
+    return fail_oom(e);
   // the packed words last: a batch that fits without them still runs
   const char* pack = std::getenv("MINIFE_BATCH_PACK");
   if (!(pack && std::atoi(pack) == 0) &&
@@ -902,7 +880,7 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
   auto fill = [&]() -> int {
     MFE_CHECK(ctx, hipMemsetAsync(B->d_scols, 0, sizeof(int) * (size_t)B->slots, s));
     MFE_CHECK(ctx, hipMemsetAsync(B->d_svals, 0, sizeof(double) * (size_t)B->slots, s));
-    if (int st2 = batch_upload_assignment(ctx, B)) return st2;
+    if (int st2 = batch_upload_layout(ctx, B)) return st2;
     MFE_CHECK(ctx, hipMemcpyAsync(B->d_soff, B->soff.data(), sizeof(int) * B->soff.size(),
                                   hipMemcpyHostToDevice, s));
     MFE_CHECK(ctx, hipStreamSynchronize(s));
@@ -958,31 +936,13 @@ int mfe_batch_solve(mfe_ctx* ctx, mfe_batch* B, int max_iter, double rel_tol, in
   MFE_CHECK(ctx, hipSetDevice(ctx->device));
   hipStream_t s = ctx->stream;
   MFE_CHECK(ctx, hipMemsetAsync(B->d_states, 0, sizeof(BatchState) * (size_t)B->nprob, s));
-  MFE_CHECK(ctx, hipMemsetAsync(B->d_abort, 0, sizeof(int), s));
+  std::fill(B->h_words, B->h_words + 1 + B->nprob, 0);  // nothing is in flight
   int rate_khz = 0;
   MFE_CHECK(ctx, hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, ctx->device));
   if (rate_khz <= 0) rate_khz = 100000;
   B->tick_seconds = 1.0 / (1e3 * (double)rate_khz);
-  uint64_t limit = (uint64_t)(kBatchWaitSeconds * 1e3 * (double)rate_khz);
-  // Autotuned balance: after a solve, give each problem workgroups in
-  // proportion to the traffic its measured iterations moved.
-  if ((int)B->last_iters.size() == B->nprob) {
-    std::vector<double> work((size_t)B->nprob);
-    for (int q = 0; q < B->nprob; ++q) {
-      const BatchProb& P = B->probs[(size_t)q];
-      const double stored = (double)B->soff[(size_t)(P.soff0 + P.nslices)] * kWave;
-      const double spmv = B->d_words ? 64.0 * P.n : 8.0 * stored + 24.0 * P.n;
-      work[(size_t)q] = (double)B->last_iters[(size_t)q] * (spmv + 64.0 * P.n);
-    }
-    batch_assign(B, work, B->capacity);
-    if (int st2 = batch_upload_assignment(ctx, B)) return st2;
-  }
   HexTables tab;
   host_tables(tab);
-  void* args[] = {&B->d_probs, &B->d_blk2prob, &B->d_soff,   &B->d_svals, &B->d_recs,
-                  &B->d_words, &B->d_x,        &B->d_r,      &B->d_p,     &B->d_Ap,
-                  &B->d_part,  &B->d_states,   &B->d_abort,  &max_iter,   &rel_tol,
-                  &limit};
   MFE_CHECK(ctx, hipEventRecord(ctx->t_start, s));
   const unsigned grid = (unsigned)B->grid;
   batch_elements_kernel<<<grid, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, tab, B->d_KF,
@@ -993,31 +953,52 @@ int mfe_batch_solve(mfe_ctx* ctx, mfe_batch* B, int max_iter, double rel_tol, in
                                             B->d_b, B->d_x, B->d_r, B->d_p, B->d_part,
                                             B->d_states);
   MFE_CHECK(ctx, hipGetLastError());
-  MFE_CHECK(ctx, hipLaunchCooperativeKernel(B->kernel, dim3((unsigned)B->grid),
-                                            dim3(kBlock), args, 0, s));
+  volatile int* host = B->h_words;
+  int active = B->nprob;  // problems order[0 .. active) are launched
+  for (unsigned k = 1; k <= (unsigned)max_iter + 1; ++k) {
+    while (active > 0 && host[1 + B->order[(size_t)active - 1]]) --active;
+    if (active == 0) break;
+    const BatchProb& last = B->probs[(size_t)B->order[(size_t)active - 1]];
+    const unsigned g = (unsigned)(last.b0 + last.nb);
+    batch_p_kernel<<<g, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, B->d_recs, B->d_x, B->d_r,
+                                        B->d_p, B->d_Ap, B->d_part, B->d_states, B->h_words, k,
+                                        max_iter, rel_tol);
+    if (k <= (unsigned)max_iter) {
+      batch_spmv_kernel<<<g, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, B->d_soff, B->d_svals,
+                                             B->d_recs, B->d_words, B->d_p, B->d_Ap, B->d_part,
+                                             B->d_states);
+      batch_r_kernel<<<g, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, B->d_r, B->d_Ap, B->d_part,
+                                          B->d_states, B->h_words, k);
+    }
+    MFE_CHECK(ctx, hipGetLastError());
+    for (unsigned spin = 1; (unsigned)host[0] + kAhead < k; ++spin)
+      if (spin % (1 << 16) == 0) {  // not for ever: the stream may have failed
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipSuccess) break;
+        if (e != hipErrorNotReady) return hip_fail(ctx, e, "batch_solve: iteration");
+      }
+  }
   MFE_CHECK(ctx, hipEventRecord(ctx->t_stop, s));
   MFE_CHECK(ctx, hipEventSynchronize(ctx->t_stop));
   float ms = 0;
   MFE_CHECK(ctx, hipEventElapsedTime(&ms, ctx->t_start, ctx->t_stop));
   if (seconds) *seconds = 1e-3 * ms;
-  int aborted = 0;
   std::vector<BatchState> hs((size_t)B->nprob);
-  MFE_CHECK(ctx, hipMemcpy(&aborted, B->d_abort, sizeof(int), hipMemcpyDeviceToHost));
   MFE_CHECK(ctx, hipMemcpy(hs.data(), B->d_states, sizeof(BatchState) * hs.size(),
                            hipMemcpyDeviceToHost));
-  if (aborted)
-    return fail(ctx, MFE_HIP_ERROR, "batch_solve: a problem barrier waited past its limit; "
-                                    "the launch was abandoned");
   int status = MFE_OK;
-  B->last_iters.assign((size_t)B->nprob, 0);
   B->last_seconds.assign((size_t)B->nprob, 0.0);
   B->last_phases.assign((size_t)B->nprob * 6, 0.0);
   for (int q = 0; q < B->nprob; ++q) {
-    B->last_iters[(size_t)q] = hs[(size_t)q].iters;
     B->last_seconds[(size_t)q] =
         (double)(hs[(size_t)q].t_end - hs[(size_t)q].t_begin) * B->tick_seconds;
-    for (int ph = 0; ph < 6; ++ph)
-      B->last_phases[(size_t)q * 6 + ph] = (double)hs[(size_t)q].t_phase[ph] * B->tick_seconds;
+    double rest = B->last_seconds[(size_t)q];  // between its workgroups of two launches
+    for (int ph = 0; ph < 5; ++ph) {
+      const double sec = (double)hs[(size_t)q].t_phase[ph] * B->tick_seconds;
+      B->last_phases[(size_t)q * 6 + ph] = sec;
+      rest -= sec;
+    }
+    B->last_phases[(size_t)q * 6 + 5] = std::max(rest, 0.0);
     if (iters) iters[q] = hs[(size_t)q].iters;
     if (rel_residual)
       rel_residual[q] = hs[(size_t)q].bnorm > 0 ? hs[(size_t)q].normr / hs[(size_t)q].bnorm
