@@ -110,6 +110,7 @@ struct BatchState {  // per problem, zeroed before each solve
   uint64_t t_phase[5];
 };
 
+constexpr int kPPad = 2;    // entries of p before and after the problems' (packed_pair_sum)
 constexpr int kUnroll = 4;  // tiles per step of the vector loops
 constexpr int kMaxPart = 1024;  // a problem's workgroups (every one sums all partials)
 constexpr int kBatchProblemsPerCu = 2;  // more are refused
@@ -395,7 +396,54 @@ __device__ __forceinline__ double packed_row_sum(const unsigned* __restrict__ w,
   return sum;
 }
 
-// The same from the row's SELL values (27 of them: its slice is as wide).
+struct __attribute__((aligned(8))) PairD {
+  double a, b;
+};
+
+// (A p) of rows `row` and row + 1, each over its 27 entries in ascending column
+// order, from the packed words w of row `row` in its tile (row even there).  The
+// rows of a line share their neighbours: four entries of p, two loads, serve both.
+// A row that is not interior gets a sum that is not used; its neighbour's loads
+// reach at most one entry past the problem's rows.
+template <typename BP>
+__device__ __forceinline__ void packed_pair_sum(const unsigned* __restrict__ w,
+                                                const BatchRec* __restrict__ rec,
+                                                const double* pv, int row, int gx, int plane,
+                                                double (&sum)[2], double (&own)[2]) {
+  unsigned f0[BP::words], f1[BP::words];
+#pragma unroll
+  for (int i = 0; i < BP::words; ++i) {
+    const uint2 v = *reinterpret_cast<const uint2*>(w + i * kBlock);
+    f0[i] = v.x;
+    f1[i] = v.y;
+  }
+  const unsigned off = 8u * (unsigned)row;
+  double x[9][4];
+#pragma unroll
+  for (int l = 0; l < 9; ++l) {
+    const double* q = pv + (gx * (l % 3 - 1) + (int64_t)plane * (l / 3 - 1));
+    const PairD lo = *reinterpret_cast<const PairD*>(reinterpret_cast<const char*>(q - 1) + off);
+    const PairD hi = *reinterpret_cast<const PairD*>(reinterpret_cast<const char*>(q + 1) + off);
+    x[l][0] = lo.a;
+    x[l][1] = lo.b;
+    x[l][2] = hi.a;
+    x[l][3] = hi.b;
+  }
+  sum[0] = sum[1] = 0.0;
+#pragma unroll
+  for (int s = 0; s < kBSlots; ++s) {
+    const double q = __hiloint2double((int)rec->qhi[s], 0), base = rec->base[s];
+    const int at = BP::bit(s) / 32, sh = BP::bit(s) % 32;
+    const double v0 = (double)pack_field(f0 + at, BP::width(s), sh) * q + base;
+    const double v1 = (double)pack_field(f1 + at, BP::width(s), sh) * q + base;
+    sum[0] += v0 * x[s / 3][s % 3];
+    sum[1] += v1 * x[s / 3][s % 3 + 1];
+  }
+  own[0] = x[4][1];
+  own[1] = x[4][2];
+}
+
+// One row from its SELL values (27 of them: its slice is as wide).
 __device__ __forceinline__ double full_row_sum(const BatchProb& P, const int* __restrict__ soff,
                                                const double* __restrict__ svals,
                                                const double* pv, int row, int gx, int plane,
@@ -596,11 +644,16 @@ __global__ __launch_bounds__(kBlock) void batch_p_kernel(
   }
 }
 
-// A p and the partials of p.Ap.  About 63 bytes per row; 64 boxes of 16..96 average
-// 2.7 TB/s, two 150^3 3.1: bound by the 27 entries of p per row going through
-// the L1s.  128 registers (four waves per SIMD; with three 122 ms for the whole
-// solve instead of 112, with five the 150^3 boxes lose 2%).  With p staged in
-// LDS, three windows for four tiles at a time, 115 to 124 ms.
+// A p and the partials of p.Ap.  About 46 bytes per row come from and go to
+// memory (44 of them floor); bound by the 27 entries of p per row that go through
+// the L1s, and the waits for them: row by row two 150^3 run at 2.3 TB/s, 33 vector
+// memory instructions per 64 rows.  PAIR: two rows per thread, whose lines share
+// their entries (27 per 128 rows): their whole solve 72.2 ms, so 64.4; 64 boxes of
+// 16..96 110.6, so 106.6.  For launches of few tiles (one per workgroup) it
+// leaves half the waves idle: 12 of 20..64 7.5 ms, row by row 7.2.
+// 128 registers (four waves per SIMD): three 108 ms, five 121 (64 boxes).  With p
+// staged in LDS, three windows for four tiles at a time, row by row: 115 to 124.
+template <bool PAIR>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void batch_spmv_kernel(
     const BatchProb* __restrict__ probs, const int* __restrict__ blk2prob,
     const int* __restrict__ soff_all, const double* __restrict__ svals,
@@ -620,23 +673,63 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
   const double* pp = p + P.row0;
   double* App = Ap + P.row0;
   double acc = 0.0;
-  for (int tile = wg.t0; tile < wg.t1; ++tile) {
-    const int row = tile * kBlock + t;
-    const BatchRec* rec = recs + P.tile0 + tile;
-    const int form = rec->form;
-    if ((rec->inner[wave] >> lane) & 1u) {
-      const unsigned* w = words + (P.tile0 + tile) * (int64_t)(kBWords * kBlock) + t;
-      double sum, own;
-      if (form == kB10) sum = packed_row_sum<BPack10>(w, rec, pp, row, gx, plane, &own);
-      else if (form == kB10Near22)
-        sum = packed_row_sum<BPack10N22>(w, rec, pp, row, gx, plane, &own);
-      else if (form == kB20) sum = packed_row_sum<BPack20>(w, rec, pp, row, gx, plane, &own);
-      else sum = full_row_sum(P, soff, svals, pp, row, gx, plane, &own);
-      App[row] = sum;
-      acc += sum * own;
-    } else if (row < n) {
-      const double own = App[row];
-      acc += own * own;
+  if constexpr (PAIR) {
+    // two waves per tile, two rows per thread
+    for (int tile = wg.t0 + wave / 2; tile < wg.t1; tile += kBlock / kWave / 2) {
+      const int half = wave % 2, row = tile * kBlock + half * 2 * kWave + 2 * lane;
+      const BatchRec* rec = recs + P.tile0 + tile;
+      const int form = rec->form;
+      const uint64_t m0 = rec->inner[2 * half], m1 = rec->inner[2 * half + 1];
+      const unsigned in = (unsigned)((lane < kWave / 2 ? m0 : m1) >> (2 * lane % kWave)) & 3u;
+      double sum[2], own[2];
+      if (in) {
+        const unsigned* w = words + (P.tile0 + tile) * (int64_t)(kBWords * kBlock) +
+                            (half * 2 * kWave + 2 * lane);
+        if (form == kB10) packed_pair_sum<BPack10>(w, rec, pp, row, gx, plane, sum, own);
+        else if (form == kB10Near22)
+          packed_pair_sum<BPack10N22>(w, rec, pp, row, gx, plane, sum, own);
+        else if (form == kB20) packed_pair_sum<BPack20>(w, rec, pp, row, gx, plane, sum, own);
+        else {
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            if ((in >> h) & 1u) sum[h] = full_row_sum(P, soff, svals, pp, row + h, gx, plane, &own[h]);
+        }
+      }
+      if (in == 3u) {
+        *reinterpret_cast<PairD*>(App + row) = PairD{sum[0], sum[1]};
+        acc += sum[0] * own[0];
+        acc += sum[1] * own[1];
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if ((in >> h) & 1u) {
+            App[row + h] = sum[h];
+            acc += sum[h] * own[h];
+          } else if (row + h < n) {
+            const double pv = App[row + h];
+            acc += pv * pv;
+          }
+      }
+    }
+  } else {
+    for (int tile = wg.t0; tile < wg.t1; ++tile) {
+      const int row = tile * kBlock + t;
+      const BatchRec* rec = recs + P.tile0 + tile;
+      const int form = rec->form;
+      if ((rec->inner[wave] >> lane) & 1u) {
+        const unsigned* w = words + (P.tile0 + tile) * (int64_t)(kBWords * kBlock) + t;
+        double sum, own;
+        if (form == kB10) sum = packed_row_sum<BPack10>(w, rec, pp, row, gx, plane, &own);
+        else if (form == kB10Near22)
+          sum = packed_row_sum<BPack10N22>(w, rec, pp, row, gx, plane, &own);
+        else if (form == kB20) sum = packed_row_sum<BPack20>(w, rec, pp, row, gx, plane, &own);
+        else sum = full_row_sum(P, soff, svals, pp, row, gx, plane, &own);
+        App[row] = sum;
+        acc += sum * own;
+      } else if (row < n) {
+        const double own = App[row];
+        acc += own * own;
+      }
     }
   }
   const double v0 = block_sum<double>(acc, red);
@@ -705,6 +798,7 @@ using namespace mfe;
 struct mfe_batch {
   mfe_ctx* ctx = nullptr;
   int nprob = 0, grid = 0;
+  bool pairs = false;  // the SpMV takes two rows per thread
   double tick_seconds = 1e-8;  // wall clock period
   std::vector<double> last_seconds;  // per problem, previous solve
   std::vector<double> last_phases;   // per problem x 6 phases, previous solve
@@ -737,7 +831,7 @@ struct mfe_batch {
     (void)hipFree(d_b);
     (void)hipFree(d_x);
     (void)hipFree(d_r);
-    (void)hipFree(d_p);
+    (void)hipFree(d_p ? d_p - kPPad : nullptr);
     (void)hipFree(d_Ap);
     (void)hipFree(d_part);
     (void)hipFree(d_states);
@@ -756,6 +850,7 @@ static void batch_layout(mfe_batch* B, int cus) {
   int64_t tiles = 0;
   for (const BatchProb& P : B->probs) tiles += P.ntiles;
   const int least = (int)std::max<int64_t>(1, std::min<int64_t>(kUnroll, tiles / (16 * cus)));
+  B->pairs = least >= 2;
   auto side = [&](int q) {
     const BatchProb& P = B->probs[(size_t)q];
     return std::max(P.Nx, std::max(P.Ny, P.Nz));
@@ -861,7 +956,8 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
   BALLOC(B->d_b, sizeof(double) * (size_t)B->rows);
   BALLOC(B->d_x, sizeof(double) * (size_t)B->rows);
   BALLOC(B->d_r, sizeof(double) * (size_t)B->rows);
-  BALLOC(B->d_p, sizeof(double) * (size_t)B->rows);
+  BALLOC(B->d_p, sizeof(double) * ((size_t)B->rows + 2 * kPPad));
+  B->d_p += kPPad;
   BALLOC(B->d_Ap, sizeof(double) * (size_t)B->rows);
   BALLOC(B->d_part, sizeof(double) * 2 * B->blk2prob.size());
   BALLOC(B->d_states, sizeof(BatchState) * (size_t)nprob);
@@ -964,9 +1060,9 @@ int mfe_batch_solve(mfe_ctx* ctx, mfe_batch* B, int max_iter, double rel_tol, in
                                         B->d_p, B->d_Ap, B->d_part, B->d_states, B->h_words, k,
                                         max_iter, rel_tol);
     if (k <= (unsigned)max_iter) {
-      batch_spmv_kernel<<<g, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, B->d_soff, B->d_svals,
-                                             B->d_recs, B->d_words, B->d_p, B->d_Ap, B->d_part,
-                                             B->d_states);
+      auto spmv = B->pairs ? batch_spmv_kernel<true> : batch_spmv_kernel<false>;
+      spmv<<<g, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, B->d_soff, B->d_svals, B->d_recs,
+                                B->d_words, B->d_p, B->d_Ap, B->d_part, B->d_states);
       batch_r_kernel<<<g, kBlock, 0, s>>>(B->d_probs, B->d_blk2prob, B->d_r, B->d_Ap, B->d_part,
                                           B->d_states, B->h_words, k);
     }

@@ -140,13 +140,23 @@ def test_batch_packed_values_are_exact(mfe, monkeypatch, dims):
     """The CG on packed stencil values gives the bits of the CG on the values
     themselves (the partial sums of both are grouped alike)."""
     say(f"batch packed {dims}")
-    boxes = [dims, (5, 4, 3)]
+    same_bits_without_packing(mfe, monkeypatch, [dims, (5, 4, 3)])
+
+
+def test_batch_packed_values_are_exact_two_rows_per_thread(mfe, monkeypatch):
+    """The same where the launches are large enough for two rows per thread."""
+    boxes = [(128, 128, 128), (48, 48, 96), (75, 15, 105), (2, 2, 2), (1, 1, 40), (31, 30, 17)]
+    say(f"batch packed {boxes}")
+    same_bits_without_packing(mfe, monkeypatch, boxes)
+
+
+def same_bits_without_packing(mfe, monkeypatch, boxes):
     out, xs = [], []
     for pack in ("1", "0"):
         monkeypatch.setenv("MINIFE_BATCH_PACK", pack)
         B = mfe.Batch(boxes)
         out.append(B.solve(max_iter=60, rel_tol=1e-12))
-        xs.append([B.download(p, matrix=False)["x"] for p in range(2)])
+        xs.append([B.download(p, matrix=False)["x"] for p in range(len(boxes))])
     assert out[0]["iters"].tolist() == out[1]["iters"].tolist()
     assert out[0]["iters"][0] > 0
     for a, b in zip(*xs):
