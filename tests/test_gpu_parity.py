@@ -797,6 +797,33 @@ def test_dirichlet_on_uploaded_matrices(mfe, ctx, oracle_mod, maxlen):
         assert bits_equal(b.to_numpy(), bo)
 
 
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 3, 1), (63, 1, 2), (7, 9, 11)])
+@pytest.mark.parametrize("share", [0.0, 0.02, 0.3, 1.0])
+def test_dirichlet_on_boxes_with_any_rows(mfe, ctx, oracle_mod, dims, share):
+    """impose_dirichlet on a box matrix visits the rows next to the BC rows, two
+    at a time by each wave: none, few, many and all rows of boxes whose 64-row
+    groups end inside and at the last row, bit for bit as the oracle."""
+    say(f"case dirichlet box {dims} share={share}")
+    mesh = mfe.simple_mesh_description([0, dims[0], 0, dims[1], 0, dims[2]])
+    A = mfe.CSRMatrix(ctx)
+    assert mfe.generate_matrix_structure(mesh, A) == 0
+    rng = np.random.default_rng(sum(dims))
+    bh = rng.standard_normal(A.nrows)
+    b = mfe.Vector.from_numpy(np.zeros(A.nrows), ctx)
+    mfe.assemble_FE_data(mesh, A, b)
+    b = mfe.Vector.from_numpy(bh, ctx)
+    h = A.to_host(rows=False)
+    Ao = oracle_mod.CSR(np.arange(A.nrows, dtype=np.int32), h["row_offsets"], h["cols"],
+                        h["vals"].copy())
+    bo = bh.copy()
+    for value in (0.0, 1.0):
+        rows = np.flatnonzero(rng.random(A.nrows) < share).astype(np.int32)
+        mfe.impose_dirichlet(value, A, b, 0, 0, 0, rows)
+        oracle_mod.impose_dirichlet(value, Ao, bo, rows)
+        assert bits_equal(A.to_host(rows=False, row_offsets=False, cols=False)["vals"], Ao.vals)
+        assert bits_equal(b.to_numpy(), bo)
+
+
 def test_dirichlet_bc_rows_beyond_one_staging_chunk(mfe, ctx, oracle_mod):
     """impose_dirichlet reads the BC row list through a pinned buffer of
     262,144 rows at a time, waiting for the kernels before each refill:
