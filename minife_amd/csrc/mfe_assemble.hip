@@ -79,12 +79,17 @@ __host__ __device__ constexpr int tri4(int a, int b) {  // packed 4 x 4 upper tr
 // phase A slot of K entry (m, n), m <= n, m a lower corner
 __host__ __device__ constexpr int fuse_a(int m, int n) { return n < 4 ? tri4(m, n) : 10 + m * 4 + (n - 4); }
 
+// Bound by the FP64 operations of the elements (about 3,000 vector instructions
+// per 64 elements, 57% of the issue slots) and the waits of two waves per SIMD:
+// element loop at 300^3 5.73 ms with the Gauss tables read through the scalar
+// cache and every Jacobian entry used, 5.12 with constant tables, 4.96 without
+// the entries that are zero.  (Three workgroups per CU, 168 registers and 224
+// bytes of scratch: 7.27.)
 template <bool ZERO_START>
 // (launch bounds: two workgroups per CU, which the 60 KB of LDS allow, so at
 // most 256 registers per lane)
 __global__ __launch_bounds__(kBlock, 2) void element_gather_kernel(
-    int Nx, int Ny, int Nz, int tiles_x, int nzc, int zc, const HexTables* __restrict__ tab,
-    const double* __restrict__ jac, const double* __restrict__ kappa, double Q,
+    int Nx, int Ny, int Nz, int tiles_x, int nzc, int zc, const double* __restrict__ jac, const double* __restrict__ kappa, double Q,
     const int* __restrict__ ro, double* __restrict__ vals, double* __restrict__ b) {
   static_assert(kFuseSide * kFuseSide == kBlock, "one element per thread");
   __shared__ double sh[kFuseA][kBlock];
@@ -139,8 +144,8 @@ __global__ __launch_bounds__(kBlock, 2) void element_gather_kernel(
     double K[36], F[8];
     if (layer && elive) {
       const int64_t e = ex + (int64_t)Nx * (ey + (int64_t)Ny * ez);
-      hex8_element_jac<true>(jac + (int64_t)ex * 24, jac + (int64_t)(Nx + ey) * 24,
-                             jac + (int64_t)(Nx + Ny + ez) * 24, *tab, kappa ? kappa[e] : 1.0, K,
+      hex8_element_jac(jac + (int64_t)ex * 24, jac + (int64_t)(Nx + ey) * 24,
+                             jac + (int64_t)(Nx + Ny + ez) * 24, kappa ? kappa[e] : 1.0, K,
                              F, Q);
     }
     __syncthreads();  // the previous step's reads are done
@@ -617,11 +622,11 @@ static int element_loop(mfe_ctx* ctx, const int gbox[6], const int ebox[6], mfe_
   const unsigned grid = (unsigned)((int64_t)m.nbx * m.nby * m.nzc);
   if (zero)
     element_gather_kernel<true><<<grid, kBlock, 0, ctx->stream>>>(
-        Nx, Ny, Nz, m.nbx, m.nzc, m.zc, dtab, djac, kappa ? kappa->d : nullptr, source,
+        Nx, Ny, Nz, m.nbx, m.nzc, m.zc, djac, kappa ? kappa->d : nullptr, source,
         A->row_offsets, A->vals, b->d);
   else
     element_gather_kernel<false><<<grid, kBlock, 0, ctx->stream>>>(
-        Nx, Ny, Nz, m.nbx, m.nzc, m.zc, dtab, djac, kappa ? kappa->d : nullptr, source,
+        Nx, Ny, Nz, m.nbx, m.nzc, m.zc, djac, kappa ? kappa->d : nullptr, source,
         A->row_offsets, A->vals, b->d);
   hipError_t le = hipGetLastError();
   csr_values_changed(A);

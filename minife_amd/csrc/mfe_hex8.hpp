@@ -16,7 +16,7 @@ struct HexTables {
   double gw[2];    // Gauss weights
 };
 
-inline void host_gauss_pts(double pts[2], double wts[2]) {
+__host__ __device__ constexpr void host_gauss_pts(double pts[2], double wts[2]) {
   const double x2 = 0.577350269;  // truncated 1/sqrt(3), gauss_pts.hpp:41
   pts[0] = -x2;
   wts[0] = 1.0;
@@ -24,8 +24,8 @@ inline void host_gauss_pts(double pts[2], double wts[2]) {
   wts[1] = 1.0;
 }
 
-inline void host_tables(HexTables& t) {
-  double gp[2], gw[2];
+__host__ __device__ constexpr void host_tables(HexTables& t) {
+  double gp[2] = {}, gw[2] = {};
   host_gauss_pts(gp, gw);
   t.gw[0] = gw[0];
   t.gw[1] = gw[1];
@@ -55,6 +55,12 @@ inline void host_tables(HexTables& t) {
         s[6] = 0.125 * up1 * vp1 * wp1;
         s[7] = 0.125 * u * vp1 * wp1;
       }
+}
+
+__host__ __device__ constexpr HexTables host_tables() {
+  HexTables t{};
+  host_tables(t);
+  return t;
 }
 
 // Exodus hex8 corner layout (Hex8_box_utils.hpp:41-57).
@@ -141,30 +147,85 @@ __host__ __device__ inline void jac_column(const HexTables& tab, int q, int axis
   out[2] = s2;
 }
 
-// hex8_element for an element whose Jacobian columns come from tables:
+// hex8_element for a box element, whose Jacobian columns come from tables:
 // jx[3q + a] = J[a][0] at Gauss point q for the element's x index (likewise
 // jy, jz), as jac_column makes them.  Same bits as hex8_element on the
-// element's coordinates.  LEAN keeps two Gauss points in flight (only the
-// innermost loop is unrolled); same arithmetic.
-template <bool LEAN = false>
+// element's coordinates, with fewer operations:
+//   - The Gauss tables are compile-time constants here (made by the same
+//     expressions), and the weights of 1.0 drop out.
+//   - J[0][1] and J[0][2] are +0.0: in jac_column's sums for the y and z axes,
+//     corners 0 and 1, 2 and 3, 4 and 5, 6 and 7 have the same coordinate and
+//     opposite d/dx, so each pair cancels.  What they multiply drops out (a
+//     term of +-0.0 in a sum that another term keeps from being zero): det J
+//     = J[0][0] term0, and the gradients' x components are products of one factor.
+//   - A gradient's magnitude along an axis is shared by the two corners that
+//     differ along it: it is multiplied once and the sign goes to the product;
+//     so are the products of the x components.
+// Two Gauss points at a time (the scheduling barriers): the registers hold K, F
+// and two points' gradients.
 __device__ __forceinline__ void hex8_element_jac(const double* jx, const double* jy,
-                                                 const double* jz, const HexTables& tab, double k,
-                                                 double K[36], double F[8], double Q = 1.0) {
+                                                 const double* jz, double k, double K[36],
+                                                 double F[8], double Q = 1.0) {
+  constexpr HexTables T = host_tables();
+  static_assert(T.gw[0] == 1.0 && T.gw[1] == 1.0, "weights that drop out");
 #pragma unroll
   for (int i = 0; i < 36; ++i) K[i] = 0;
 #pragma unroll
   for (int i = 0; i < 8; ++i) F[i] = 0;
-  int q = 0;
-#pragma unroll(LEAN ? 1 : 2)
-  for (int ig = 0; ig < 2; ++ig)
-#pragma unroll(LEAN ? 1 : 2)
-    for (int jg = 0; jg < 2; ++jg)
 #pragma unroll
-      for (int kg = 0; kg < 2; ++kg, ++q)
-        hex8_gauss_point<true>(jx[3 * q], jy[3 * q], jz[3 * q], jx[3 * q + 1], jy[3 * q + 1],
-                               jz[3 * q + 1], jx[3 * q + 2], jy[3 * q + 2], jz[3 * q + 2],
-                               tab.gv + 24 * q, tab.psi + 8 * q, k, tab.gw[ig], tab.gw[jg],
-                               tab.gw[kg], K, F, Q);
+  for (int q = 0; q < 8; ++q) {
+    const double J00 = jx[3 * q], J10 = jx[3 * q + 1], J20 = jx[3 * q + 2];
+    const double J11 = jy[3 * q + 1], J21 = jy[3 * q + 2];
+    const double J12 = jz[3 * q + 1], J22 = jz[3 * q + 2];
+    const double term0 = J22 * J11 - J21 * J12;
+    const double detJ = J00 * term0;
+    const double inv_detJ = 1.0 / detJ;
+    const double ixx = term0 * inv_detJ;
+    const double inv[2][3] = {
+        {-(J22 * J10 - J20 * J12) * inv_detJ, (J22 * J00) * inv_detJ, -(J12 * J00) * inv_detJ},
+        {(J21 * J10 - J20 * J11) * inv_detJ, -(J21 * J00) * inv_detJ, (J11 * J00) * inv_detJ}};
+    const double kdw = k * detJ;
+    // the corners (1, y, z), (x, 1, z), (x, y, 1) of index lo + 2 hi
+    double dx[4], dxdx[4][4];  // d/dx of corner (1, y, z) and their products
+#pragma unroll
+    for (int c = 0; c < 4; ++c) dx[c] = T.gv[24 * q + 3 * corner_of(1, c & 1, c >> 1)] * ixx;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int e = c; e < 4; ++e) dxdx[c][e] = dx[c] * dx[e];
+    double d[2][8];  // d/dy and d/dz
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      double m[3][4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int lo = c & 1, hi = c >> 1;
+        m[0][c] = T.gv[24 * q + 3 * corner_of(1, lo, hi)] * inv[a][0];
+        m[1][c] = T.gv[24 * q + 3 * corner_of(lo, 1, hi) + 1] * inv[a][1];
+        m[2][c] = T.gv[24 * q + 3 * corner_of(lo, hi, 1) + 2] * inv[a][2];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int x = corner_x(i), y = corner_y(i), z = corner_z(i);
+        const double p0 = m[0][y + 2 * z], p1 = m[1][x + 2 * z], p2 = m[2][x + 2 * y];
+        d[a][i] = (x ? p0 : -p0) + (y ? p1 : -p1) + (z ? p2 : -p2);
+      }
+    }
+    int off = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int n = i; n < 8; ++n) {
+        const int ci = corner_y(i) + 2 * corner_z(i), cn = corner_y(n) + 2 * corner_z(n);
+        const double xx = dxdx[ci < cn ? ci : cn][ci < cn ? cn : ci];
+        K[off++] += kdw * ((corner_x(i) == corner_x(n) ? xx : -xx) + (d[0][i] * d[0][n]) +
+                           (d[1][i] * d[1][n]));
+      }
+    const double term = Q * detJ;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) F[i] += T.psi[8 * q + i] * term;
+    if (q % 2) __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 // Hex8::diffusionMatrix_symm (Hex8.hpp:259-361) and Hex8::sourceVector

@@ -797,6 +797,19 @@ def test_dirichlet_on_uploaded_matrices(mfe, ctx, oracle_mod, maxlen):
         assert bits_equal(b.to_numpy(), bo)
 
 
+@pytest.mark.parametrize("dims", [(1000, 1, 2), (2, 777, 1), (1, 2, 901), (15, 16, 31), (16, 15, 1)])
+def test_element_loop_uses_only_zero_terms_less(mfe, ctx, oracle_mod, dims):
+    """The element matrices leave out the Jacobian entries that a box makes zero
+    and share the magnitudes of mirrored gradients: rows and right-hand side
+    equal the oracle's bit for bit where the coordinates round most (long
+    boxes) and at the edges of the 15-element tiles."""
+    say(f"case element loop {dims}")
+    mesh, A, b, _ = build_stages(mfe, ctx, dims)
+    P = oracle_mod.build_problem(*dims)
+    assert bits_equal(A.to_host(rows=False, row_offsets=False, cols=False)["vals"], P["A"].vals)
+    assert bits_equal(b.to_numpy(), P["b"])
+
+
 @pytest.mark.parametrize("dims", [(1, 1, 1), (2, 3, 1), (63, 1, 2), (7, 9, 11)])
 @pytest.mark.parametrize("share", [0.0, 0.02, 0.3, 1.0])
 def test_dirichlet_on_boxes_with_any_rows(mfe, ctx, oracle_mod, dims, share):
