@@ -106,23 +106,26 @@ def boxsym_bytes(dims, plan: dict, value_bytes: int = 8) -> int:
     return full + value_bytes * (14 * n + 282 * nb * gz + 9 * gx * gy * (plan["z_chunks"] - 1))
 
 
+PACKED_BOUNDARY_ROWS = 1 << 23  # rows from which the CG's kernel reads it packed
+
+
 def boxpack_bytes(dims, plan: dict, value_bytes: int = 8) -> int:
     """HBM bytes of one SpMV on the symmetric box layout with packed upper
     values: as boxsym_bytes, but a row's packed slots cost its 32-bit words
-    of fields instead of value_bytes each, plus a base and a power of two
-    (value_bytes each) per (block, plane, slot) and a codes flag per (block,
-    plane); where the FP64 boundary stream is packed too (the CG's kernel
-    reads it so), its words and 13 (base, power of two) pairs and a flag per
-    (block, plane) instead of its 282 values."""
+    of fields instead of value_bytes each, plus a record of 30 values per
+    (block, plane): 14 bases, 14 powers of two and the codes flag as words, the
+    rest padding; where the CG's kernel reads the FP64 boundary stream packed too
+    (from 2^23 rows on), its words and 13 (base, power of two) pairs and a
+    flag per (block, plane) instead of its 282 values."""
     import minife_amd as mfe
     gx, gy, gz = dims
     n = gx * gy * gz
     nb = plan["blocks_x"] * plan["blocks_y"]
     words, fulls = mfe.pack_row_layout(plan["pack"] if value_bytes == 8 else plan["pack_fp32"])
-    wform = plan.get("wpack") if value_bytes == 8 else None  # FP64 only
+    wform = plan.get("wpack") if value_bytes == 8 and n >= PACKED_BOUNDARY_ROWS else None
     wbytes = (4 * mfe.pack_bnd_words(wform) + value_bytes * 27 - value_bytes * 282) if wform else 0
     return (boxsym_bytes(dims, plan, value_bytes) - value_bytes * (14 - fulls) * n
-            + 4 * words * n + value_bytes * (2 * 14 + 1) * nb * gz + wbytes * nb * gz)
+            + 4 * words * n + value_bytes * (2 * 14 + 2) * nb * gz + wbytes * nb * gz)
 
 
 def plan_bytes(n: int, nnz: int, plan: dict, value_bytes: int = 8, dims=None) -> int:
@@ -238,9 +241,10 @@ def cpu_baseline(A_dev, b_dev, n, nnz, iters: int, omp_iters: int):
 
 def bench_batched(mfe, ctx):
     """64 boxes, sides uniform on [16, 96] (seed 0): assembly + FP64 CG to
-    1e-10 in one persistent launch.  Equivalent bytes per problem and
+    1e-10 together.  Equivalent bytes per problem and
     iteration: 12 B per stored SELL entry + 88 B per row (p update, x gather,
-    Ap, x/r update), plus nothing for assembly (not counted)."""
+    Ap, x/r update), plus nothing for assembly (not counted); the packed values
+    move fewer."""
     from minife_amd.workloads import batch_boxes
     B = mfe.Batch(batch_boxes(0), ctx)
     B.solve(max_iter=5000, rel_tol=1e-10)  # warm (code objects, first touch)
@@ -256,7 +260,7 @@ def bench_batched(mfe, ctx):
                "seconds": float(out["problem_seconds"][slow]),
                "phase_seconds": {k: round(float(v), 5)
                                  for k, v in zip(B.PHASES, out["phase_seconds"][slow])}}
-    res = {"workload": "64 boxes, sides U[16,96] seed 0, assemble + FP64 CG to 1e-10, one launch",
+    res = {"workload": "64 boxes, sides U[16,96] seed 0, assemble + FP64 CG to 1e-10 together",
            "seconds": out["seconds"], "problems": B.nprob, "workgroups": tot["workgroups"],
            "rows": tot["rows"], "nnz": tot["nnz"], "iters_total": int(out["iters"].sum()),
            "iters_max": int(out["iters"].max()),
@@ -585,7 +589,7 @@ def main():
             log(f"cpu baseline {cpu['value']:.3f} it/s ({cpu['sample']})")
 
     form = {v: k for k, v in mfe.PACK_FORMS.items()}.get(plan.get("pack"), 0)
-    wpk = "true" if plan.get("wpack") else "false"
+    wpk = "true" if plan.get("wpack") and n >= PACKED_BOUNDARY_ROWS else "false"
     traffic = measured_traffic(N, CG_KERNEL_PROFILE_NAMES.get(plan["kernel"], "").format(
         form=form, wpk=wpk))
     # Assembly (the element loop, perform_element_loop): bounded by the FP64

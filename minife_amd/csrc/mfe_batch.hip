@@ -644,12 +644,13 @@ __global__ __launch_bounds__(kBlock) void batch_p_kernel(
   }
 }
 
-// A p and the partials of p.Ap.  About 46 bytes per row come from and go to
-// memory (44 of them floor); bound by the 27 entries of p per row that go through
-// the L1s, and the waits for them: row by row two 150^3 run at 2.3 TB/s, 33 vector
-// memory instructions per 64 rows.  PAIR: two rows per thread, whose lines share
-// their entries (27 per 128 rows): their whole solve 72.2 ms, so 64.4; 64 boxes of
-// 16..96 110.6, so 106.6.  For launches of few tiles (one per workgroup) it
+// A p and the partials of p.Ap.  Two 150^3, row by row: 76 bytes per row read (46 of
+// packed values and records, p by several XCDs; a cube's form) and 8 written, 4.1
+// TB/s, 33 vector memory instructions per 64 rows, waves waiting half their time.
+// PAIR: two rows per thread, whose lines share their entries (27 per 128 rows):
+// their whole solve 72.2 ms, so 64.4; 64 boxes of 16..96 110.6, so 106.6.
+// Workgroups of neighbouring tiles on one XCD (groups of 4 to 64) change nothing.
+// For launches of few tiles (one per workgroup) PAIR
 // leaves half the waves idle: 12 of 20..64 7.5 ms, row by row 7.2.
 // 128 registers (four waves per SIMD): three 108 ms, five 121 (64 boxes).  With p
 // staged in LDS, three windows for four tiles at a time, row by row: 115 to 124.
