@@ -72,7 +72,7 @@ __global__ void copy_tables_kernel(HexTables tab, HexTables* __restrict__ out) {
 // upper block (10) and the upper source terms (4).
 constexpr int kFuseSide = 16;                    // elements per tile side
 constexpr int kFuseStep = kFuseSide - 1;         // tile pitch in elements
-constexpr int kFuseA = 30, kFuseB = 14;          // LDS entries per element per phase
+constexpr int kFuseA = 30;                       // LDS entries per element (the first phase's)
 __host__ __device__ constexpr int tri4(int a, int b) {  // packed 4 x 4 upper triangle, a <= b
   return a * 4 - a * (a - 1) / 2 + (b - a);
 }

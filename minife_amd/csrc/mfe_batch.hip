@@ -129,8 +129,6 @@ __device__ double sum_partials_all(const double* pp, int nb, double* red) {
   return r;
 }
 
-__device__ __forceinline__ int axis_len(int i, int g) { return 1 + (i > 0) + (i < g - 1); }
-
 // Assemble row `id` of problem P (element scratch K/F) into acc, apply both
 // Dirichlet passes, store it into the SELL slices; returns b[id].
 __device__ __forceinline__ double assemble_row(const BatchProb& P, int id, const double* K,
@@ -502,7 +500,7 @@ __global__ __launch_bounds__(kBlock) void batch_elements_kernel(
     const double c[24] = {x0, y0, z0, x1, y0, z0, x1, y1, z0, x0, y1, z0,
                           x0, y0, z1, x1, y0, z1, x1, y1, z1, x0, y1, z1};
     double Ke[36], Fe[8];
-    hex8_element<false>(c, tab, 1.0, Ke, Fe);
+    hex8_element(c, tab, 1.0, Ke, Fe);
 #pragma unroll
     for (int q = 0; q < 36; ++q) K[(int64_t)q * ne + e] = Ke[q];
 #pragma unroll

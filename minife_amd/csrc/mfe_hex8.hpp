@@ -75,10 +75,9 @@ __host__ __device__ constexpr int packed(int a, int b) {
   return a <= b ? a * 8 - a * (a - 1) / 2 + (b - a) : b * 8 - b * (b - 1) / 2 + (a - b);
 }
 
-// One Gauss point of Hex8::diffusionMatrix_symm (Hex8.hpp:259-361) and, with
-// SRC, of Hex8::sourceVector (Hex8.hpp:363-410), given that point's Jacobian
+// One Gauss point of Hex8::diffusionMatrix_symm (Hex8.hpp:259-361) and of
+// Hex8::sourceVector (Hex8.hpp:363-410), given that point's Jacobian
 // J[a][b] (gradients_and_invJ_and_detJ, Hex8.hpp:177-257, after the J sums).
-template <bool SRC>
 __device__ __forceinline__ void hex8_gauss_point(double J00, double J01, double J02, double J10,
                                                  double J11, double J12, double J20, double J21,
                                                  double J22, const double* g, const double* psi,
@@ -117,12 +116,10 @@ __device__ __forceinline__ void hex8_gauss_point(double J00, double J01, double 
     for (int n = m + 1; n < 8; ++n)
       K[off++] += kdw * ((dx[m] * dx[n]) + (dy[m] * dy[n]) + (dz[m] * dz[n]));
   }
-  if (SRC) {
-    // sourceVector: term = Q*detJ*wi*wj*wk, reference Q = 1.0 (Hex8.hpp:379,402).
-    const double term = Q * detJ * wi * wj * wk;
+  // sourceVector: term = Q*detJ*wi*wj*wk, reference Q = 1.0 (Hex8.hpp:379,402).
+  const double term = Q * detJ * wi * wj * wk;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) F[i] += psi[i] * term;
-  }
+  for (int i = 0; i < 8; ++i) F[i] += psi[i] * term;
 }
 
 // Column b of the Jacobian at Gauss point q, J[a][b] = sum_i grad_i[a] *
@@ -231,9 +228,6 @@ __device__ __forceinline__ void hex8_element_jac(const double* jx, const double*
 // Hex8::diffusionMatrix_symm (Hex8.hpp:259-361) and Hex8::sourceVector
 // (Hex8.hpp:363-410) for one element; J, detJ are evaluated once per Gauss
 // point and shared (the reference evaluates the same expressions twice).
-// LEAN keeps one Gauss point in flight (the loops are not unrolled), which
-// holds the register footprint near the 44 accumulators; same arithmetic.
-template <bool LEAN = false>
 __device__ __forceinline__ void hex8_element(const double c[24], const HexTables& tab, double k,
                                              double K[36], double F[8], double Q = 1.0) {
 #pragma unroll
@@ -241,11 +235,11 @@ __device__ __forceinline__ void hex8_element(const double c[24], const HexTables
 #pragma unroll
   for (int i = 0; i < 8; ++i) F[i] = 0;
   int q = 0;
-#pragma unroll(LEAN ? 1 : 2)
+#pragma unroll
   for (int ig = 0; ig < 2; ++ig) {
-#pragma unroll(LEAN ? 1 : 2)
+#pragma unroll
     for (int jg = 0; jg < 2; ++jg) {
-#pragma unroll(LEAN ? 1 : 2)
+#pragma unroll
       for (int kg = 0; kg < 2; ++kg, ++q) {
         const double* g = tab.gv + 24 * q;
         double J00 = 0, J01 = 0, J02 = 0, J10 = 0, J11 = 0, J12 = 0, J20 = 0, J21 = 0, J22 = 0;
@@ -257,37 +251,10 @@ __device__ __forceinline__ void hex8_element(const double c[24], const HexTables
           J10 += g1 * x; J11 += g1 * y; J12 += g1 * z;
           J20 += g2 * x; J21 += g2 * y; J22 += g2 * z;
         }
-        hex8_gauss_point<!LEAN>(J00, J01, J02, J10, J11, J12, J20, J21, J22, g, tab.psi + 8 * q, k,
-                                tab.gw[ig], tab.gw[jg], tab.gw[kg], K, F, Q);
+        hex8_gauss_point(J00, J01, J02, J10, J11, J12, J20, J21, J22, g, tab.psi + 8 * q, k,
+                         tab.gw[ig], tab.gw[jg], tab.gw[kg], K, F, Q);
       }
     }
-  }
-  if (LEAN) {  // the source vector in a pass of its own: detJ from the same expressions
-    q = 0;
-#pragma unroll 1
-    for (int ig = 0; ig < 2; ++ig)
-#pragma unroll 1
-      for (int jg = 0; jg < 2; ++jg)
-#pragma unroll 1
-        for (int kg = 0; kg < 2; ++kg, ++q) {
-          const double* g = tab.gv + 24 * q;
-          double J00 = 0, J01 = 0, J02 = 0, J10 = 0, J11 = 0, J12 = 0, J20 = 0, J21 = 0, J22 = 0;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const double g0 = g[3 * i], g1 = g[3 * i + 1], g2 = g[3 * i + 2];
-            const double x = c[3 * i], y = c[3 * i + 1], z = c[3 * i + 2];
-            J00 += g0 * x; J01 += g0 * y; J02 += g0 * z;
-            J10 += g1 * x; J11 += g1 * y; J12 += g1 * z;
-            J20 += g2 * x; J21 += g2 * y; J22 += g2 * z;
-          }
-          const double term0 = J22 * J11 - J21 * J12;
-          const double term1 = J22 * J01 - J21 * J02;
-          const double term2 = J12 * J01 - J11 * J02;
-          const double detJ = J00 * term0 - J10 * term1 + J20 * term2;
-          const double term = Q * detJ * tab.gw[ig] * tab.gw[jg] * tab.gw[kg];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) F[i] += tab.psi[8 * q + i] * term;
-        }
   }
 }
 
