@@ -19,6 +19,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <tuple>
 #include <type_traits>
 
 #include "mfe_box.hpp"
@@ -1725,7 +1726,7 @@ int box_prepare(mfe_ctx* ctx, const mfe_csr* Ac) {
 template <typename T>
 struct SpmvOp {
   const mfe_csr* A = nullptr;
-  uint64_t gen = 0;  // A->plan_gen when made: captured graphs are keyed on it
+  uint64_t gen = 0;  // A->plan_gen when made
   int n = 0;
   const int* ro = nullptr;
   const int* cols = nullptr;
@@ -1754,9 +1755,13 @@ struct SpmvOp {
   const unsigned* wpw = nullptr;
   const T* wkq = nullptr;
   BoxGeom bg{};
-  const void* key() const {
-    return pack ? (const void*)pw : symu ? (const void*)symu : bvals ? (const void*)bvals
-         : svals ? (const void*)svals : (const void*)vals;
+  // All that a launch chooses its kernel by or hands to it: a captured graph may be
+  // replayed for an operand that ties equal.  (Values that change in place stay
+  // covered; a rebuilt plan may take another packed form in the same memory.)
+  auto tie() const {
+    return std::tie(A, gen, n, ro, cols, vals, stream_ok, nslices, soff, slen, scols, svals, xl,
+                    xltail, xaff, xsbase, xroff, xrcol, xrpos, xnu, xmaxu, cus, bvals, symu, symw,
+                    symtab, pack, pw, pkq, wpack, wpw, wkq, bg.gx, bg.gy, bg.gz, bg.nbx, bg.nby);
   }
 };
 
@@ -2621,17 +2626,17 @@ struct VecSet {
   }
 };
 
+template <typename T>
 struct GraphSlot {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  const void *kA = nullptr, *kvals = nullptr, *kb = nullptr, *kx = nullptr;
-  uint64_t kgen = 0;
+  SpmvOp<T> op;           // what the captured SpMVs read
+  const T* x = nullptr;   // what the captured p updates write (besides the workspace)
   void drop() {
     if (exec) hipGraphExecDestroy(exec);
     if (graph) hipGraphDestroy(graph);
     exec = nullptr;
     graph = nullptr;
-    kA = kvals = kb = kx = nullptr;
   }
 };
 
@@ -2645,7 +2650,8 @@ struct CgWorkspace {
   unsigned long long* h_progress = nullptr;  // pinned: k, and done in bit 32 (cg_p_next_kernel)
   double* hist = nullptr;
   int64_t hist_cap = 0;
-  GraphSlot g64, g32;
+  GraphSlot<double> g64;
+  GraphSlot<float> g32;
   OpTimer timer;
 };
 
@@ -2666,7 +2672,7 @@ static void ws_free(CgWorkspace* w) {
 }
 
 template <typename T>
-static int vecset_prepare(mfe_ctx* ctx, VecSet<T>& v, int64_t n, GraphSlot& g) {
+static int vecset_prepare(mfe_ctx* ctx, VecSet<T>& v, int64_t n, GraphSlot<T>& g) {
   if (v.n == n) return MFE_OK;
   g.drop();
   v.release();
@@ -2854,15 +2860,12 @@ struct FastCg {
   }
 };
 
-// The captured chunk of `chunk` iterations after the first, kept in slot for the
-// same matrix, right-hand side and x.
+// The captured chunk of iterations after the first, kept in slot for the same
+// operand and x.
 template <typename T, typename F>
-static int capture_chunk(mfe_ctx* ctx, const FastCg<T>& f, GraphSlot& slot, const void* key_b,
-                         const void* key_x, F&& enqueue) {
+static int capture_chunk(mfe_ctx* ctx, const FastCg<T>& f, GraphSlot<T>& slot, F&& enqueue) {
   hipStream_t s = ctx->stream;
-  if (slot.exec && slot.kA == f.op.A && slot.kgen == f.op.gen && slot.kvals == f.op.key() &&
-      slot.kb == key_b && slot.kx == key_x)
-    return MFE_OK;
+  if (slot.exec && slot.op.tie() == f.op.tie() && slot.x == f.x) return MFE_OK;
   slot.drop();
   MFE_CHECK(ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   hipError_t ce = enqueue();
@@ -2875,11 +2878,8 @@ static int capture_chunk(mfe_ctx* ctx, const FastCg<T>& f, GraphSlot& slot, cons
   if (ee != hipSuccess) return hip_fail(ctx, ee, "hipStreamEndCapture");
   slot.graph = g;
   MFE_CHECK(ctx, hipGraphInstantiate(&slot.exec, g, nullptr, nullptr, 0));
-  slot.kA = f.op.A;
-  slot.kgen = f.op.gen;
-  slot.kvals = f.op.key();
-  slot.kb = key_b;
-  slot.kx = key_x;
+  slot.op = f.op;
+  slot.x = f.x;
   return MFE_OK;
 }
 
@@ -2887,7 +2887,7 @@ static int capture_chunk(mfe_ctx* ctx, const FastCg<T>& f, GraphSlot& slot, cons
 // the GPU's progress word, or in captured chunks.
 template <typename T>
 static int run_cg_rest(mfe_ctx* ctx, const FastCg<T>& f, int last, bool eager, CgWorkspace* w,
-                       GraphSlot& slot, const void* key_b, const void* key_x) {
+                       GraphSlot<T>& slot) {
   hipStream_t s = ctx->stream;
   if (f.n() <= kEagerRows) {
     volatile unsigned long long* prog = w->h_progress;
@@ -2923,7 +2923,7 @@ static int run_cg_rest(mfe_ctx* ctx, const FastCg<T>& f, int last, bool eager, C
     if (hipError_t e = f.settle()) return hip_fail(ctx, e, "cg_advance_kernel");
     return MFE_OK;
   }
-  if (int st = capture_chunk<T>(ctx, f, slot, key_b, key_x, [&] {
+  if (int st = capture_chunk<T>(ctx, f, slot, [&] {
         hipError_t e = hipSuccess;
         for (int c = 0; c < kGraphChunk && e == hipSuccess; ++c) e = f.next();
         return e == hipSuccess ? f.settle() : e;
@@ -2956,8 +2956,7 @@ static int finish_cg(mfe_ctx* ctx, const FastCg<T>& f, CgWorkspace* w) {
 template <typename T>
 static int run_cg(mfe_ctx* ctx, const SpmvOp<T>& op, const T* b, T* x, int max_iter,
                   double tol, bool replay, bool eager, CgWorkspace* w, VecSet<T>& v,
-                  GraphSlot& slot, const void* key_b, const void* key_x,
-                  double* times = nullptr, bool fused = false) {
+                  GraphSlot<T>& slot, double* times = nullptr, bool fused = false) {
   hipStream_t s = ctx->stream;
   const int64_t n = v.n;
   OpTimer* tm = (eager && times) ? &w->timer : nullptr;
@@ -2992,7 +2991,7 @@ static int run_cg(mfe_ctx* ctx, const SpmvOp<T>& op, const T* b, T* x, int max_i
       FastCg<T> f{op, v, w->st, w->st + 1, w->hist, x, s, w->h_progress};
       // Iteration 1: p = 1*r + 0*r.
       if (hipError_t he = f.first(v.r)) return hip_fail(ctx, he, "cg iteration 1");
-      if (int st = run_cg_rest<T>(ctx, f, max_iter, eager, w, slot, key_b, key_x)) return st;
+      if (int st = run_cg_rest<T>(ctx, f, max_iter, eager, w, slot)) return st;
       return finish_cg<T>(ctx, f, w);
     }
     for (int k = 1; k <= max_iter; ++k) {
@@ -3020,8 +3019,7 @@ static int run_cg(mfe_ctx* ctx, const SpmvOp<T>& op, const T* b, T* x, int max_i
 // ||r|| <= tol.  Uses the same captured chunk as run_cg's k >= 2 iterations.
 template <typename T>
 static int run_cg_resume(mfe_ctx* ctx, const SpmvOp<T>& op, T* x, int max_iter, double tol,
-                         CgWorkspace* w, VecSet<T>& v, GraphSlot& slot, const void* key_b,
-                         const void* key_x) {
+                         CgWorkspace* w, VecSet<T>& v, GraphSlot<T>& slot) {
   hipStream_t s = ctx->stream;
   const int64_t n = v.n;
   if (n == 0) return MFE_OK;
@@ -3033,7 +3031,7 @@ static int run_cg_resume(mfe_ctx* ctx, const SpmvOp<T>& op, T* x, int max_iter, 
   cg_resume_kernel<T><<<1, kBlock, 0, s>>>(w->st, w->st + 1, v.partials, (int)vg, max_iter, tol);
   MFE_LAUNCHED(ctx, "cg_resume_kernel");
   if (hipError_t he = f.first(v.p)) return hip_fail(ctx, he, "cg iteration 1");
-  if (int st = run_cg_rest<T>(ctx, f, max_iter, false, w, slot, key_b, key_x)) return st;
+  if (int st = run_cg_rest<T>(ctx, f, max_iter, false, w, slot)) return st;
   return finish_cg<T>(ctx, f, w);
 }
 
@@ -3399,7 +3397,7 @@ int mfe_cg_solve(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_vec* x, i
   MFE_CHECK(ctx, hipEventRecord(ctx->t_start, ctx->stream));
   if ((st = ensure_plan(ctx, A, true, false))) return st;
   st = run_cg<double>(ctx, spmv_op<double>(A), b->d, x->d, max_iter, tol, replay, eager, w,
-                      w->v64, w->g64, b->d, x->d, times ? op_times : nullptr,
+                      w->v64, w->g64, times ? op_times : nullptr,
                       (flags & MFE_CG_FUSED) != 0);
   if (st) return st;
   MFE_CHECK(ctx, hipEventRecord(ctx->t_stop, ctx->stream));
@@ -3502,14 +3500,13 @@ int mfe_cg_solve_mixed_ex(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_
     if (keep && outer > 0) {
       to_f32_kernel<<<vg, kBlock, 0, s>>>(n, v.r, 1.0, w->v32.r);
       MFE_LAUNCHED(ctx, "to_f32_kernel");
-      if ((st = run_cg_resume<float>(ctx, op32, w->f_x, max_inner, tol_k * rn, w, w->v32, w->g32,
-                                     w->f_rhs, w->f_x)))
+      if ((st = run_cg_resume<float>(ctx, op32, w->f_x, max_inner, tol_k * rn, w, w->v32, w->g32)))
         return st;
     } else {
       to_f32_kernel<<<vg, kBlock, 0, s>>>(n, v.r, 1.0 / scale, w->f_rhs);
       MFE_LAUNCHED(ctx, "to_f32_kernel");
       if ((st = run_cg<float>(ctx, op32, w->f_rhs, w->f_x, max_inner, tol_k * (keep ? rn : 1.0),
-                              false, false, w, w->v32, w->g32, w->f_rhs, w->f_x)))
+                              false, false, w, w->v32, w->g32)))
         return st;
     }
     const CgState hs = *w->h_st;
