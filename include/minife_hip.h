@@ -19,7 +19,9 @@
  *   - Handles own device memory.  What destroyed matrices and vectors held is
  *     kept for later ones on the same context, at most an eighth of the
  *     device's memory over all contexts, until an allocation fails or the
- *     context goes.  Host pointers are borrowed for the call.
+ *     context goes; the memory of one that was used on another context than
+ *     its own goes back to the driver when it is destroyed.  Host pointers are
+ *     borrowed for the call.
  *     Calls on one ctx are ordered on its single HIP stream; a ctx is not
  *     thread-safe.  No C++ exception crosses this boundary.
  */

@@ -88,7 +88,7 @@ hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes) {
   return hipSuccess;
 }
 
-void dev_free(mfe_ctx* ctx, void* p) {
+void dev_free(mfe_ctx* ctx, void* p, bool shared) {
   if (!p) return;
   DevPool* P = pool_of(ctx);
   if (!P) {
@@ -97,12 +97,12 @@ void dev_free(mfe_ctx* ctx, void* p) {
   }
   std::lock_guard<std::mutex> lock(P->mu);
   auto it = P->live.find(p);
-  if (it == P->live.end()) {
+  const size_t bytes = it == P->live.end() ? 0 : it->second;
+  if (it != P->live.end()) P->live.erase(it);
+  if (shared || bytes == 0) {
     (void)hipFree(p);
     return;
   }
-  const size_t bytes = it->second;
-  P->live.erase(it);
   if (!P->cap) {
     size_t free_b = 0, total = 0;
     if (hipMemGetInfo(&free_b, &total) == hipSuccess) P->cap = total / 8;
@@ -305,7 +305,7 @@ int mfe_timer_stop(mfe_ctx* ctx, double* ms) {
 static void csr_release(mfe_csr* A) {
   for (void* p : {(void*)A->rows, (void*)A->row_offsets, (void*)A->cols, (void*)A->vals,
                   (void*)A->vals32})
-    dev_free(A->ctx, p);
+    csr_free(A, p);
   A->rows = A->row_offsets = A->cols = nullptr;
   A->vals = nullptr;
   A->vals32 = nullptr;
@@ -348,6 +348,7 @@ int mfe_csr_shape(const mfe_csr* A, int64_t* nrows, int64_t* nnz) {
 namespace mfe {
 // (Re)allocate A's arrays for nrows/nnz; contents undefined.
 int csr_alloc(mfe_ctx* ctx, mfe_csr* A, int64_t nrows, int64_t nnz) {
+  uses(ctx, A);
   MFE_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   csr_release(A);
   if (nrows < 0 || nnz < 0 || nnz > INT32_MAX || nrows >= INT32_MAX)
@@ -414,6 +415,7 @@ int mfe_csr_upload(mfe_ctx* ctx, mfe_csr* A, int64_t nrows, int64_t nnz, const i
 int mfe_csr_download(mfe_ctx* ctx, const mfe_csr* A, int* rows, int* row_offsets, int* cols,
                      double* vals) {
   if (!ctx || !A) return MFE_BAD_ARG;
+  uses(ctx, A);
   MFE_CHECK(ctx, hipSetDevice(ctx->device));
   hipStream_t s = ctx->stream;
   if (rows && A->nrows)
@@ -467,7 +469,7 @@ void mfe_vec_destroy(mfe_vec* v) {
   if (!v) return;
   hipSetDevice(v->ctx->device);
   hipStreamSynchronize(v->ctx->stream);
-  if (v->owns) dev_free(v->ctx, v->d);
+  if (v->owns) dev_free(v->ctx, v->d, v->shared);
   mfe_ctx* ctx = v->ctx;
   delete v;
   ctx_release(ctx);
@@ -493,6 +495,7 @@ int64_t mfe_vec_size(const mfe_vec* v) { return v ? v->n : -1; }
 
 int mfe_vec_upload(mfe_ctx* ctx, mfe_vec* v, const double* host, int64_t n) {
   if (!ctx || !v || (n > 0 && !host) || n != v->n) return MFE_BAD_ARG;
+  uses(ctx, v);
   if (n) MFE_CHECK(ctx, hipMemcpyAsync(v->d, host, sizeof(double) * n, hipMemcpyHostToDevice,
                                        ctx->stream));
   MFE_CHECK(ctx, hipStreamSynchronize(ctx->stream));
@@ -501,6 +504,7 @@ int mfe_vec_upload(mfe_ctx* ctx, mfe_vec* v, const double* host, int64_t n) {
 
 int mfe_vec_download(mfe_ctx* ctx, const mfe_vec* v, double* host, int64_t n) {
   if (!ctx || !v || (n > 0 && !host) || n != v->n) return MFE_BAD_ARG;
+  uses(ctx, v);
   if (n) MFE_CHECK(ctx, hipMemcpyAsync(host, v->d, sizeof(double) * n, hipMemcpyDeviceToHost,
                                        ctx->stream));
   MFE_CHECK(ctx, hipStreamSynchronize(ctx->stream));
@@ -520,6 +524,7 @@ extern "C" {
 
 int mfe_vec_fill(mfe_ctx* ctx, mfe_vec* v, double value) {
   if (!ctx || !v) return MFE_BAD_ARG;
+  uses(ctx, v);
   if (v->n == 0) return MFE_OK;
   fill_kernel<<<(unsigned)cdiv(v->n, kBlock), kBlock, 0, ctx->stream>>>(v->n, value, v->d);
   MFE_LAUNCHED(ctx, "fill_kernel");
@@ -564,6 +569,7 @@ int mfe_verify_solution(mfe_ctx* ctx, const int g[6], const mfe_vec* xv, double 
 int mfe_verify_solution_ex(mfe_ctx* ctx, const int g[6], const mfe_vec* xv, double tolerance,
                            int whole, int hot_face, double* max_err) {
   if (!ctx || !g || !xv) return MFE_BAD_ARG;
+  uses(ctx, xv);
   const int gx = g[1] + 1, gy = g[3] + 1, gz = g[5] + 1;
   if (g[0] != 0 || g[2] != 0 || g[4] != 0 || (int64_t)gx * gy * gz != xv->n)
     return fail(ctx, MFE_BAD_ARG, "verify_solution: box does not match x");

@@ -568,6 +568,8 @@ int mfe_perform_element_loop(mfe_ctx* ctx, const int gbox[6], const int ebox[6],
 static int element_loop(mfe_ctx* ctx, const int gbox[6], const int ebox[6], mfe_csr* A,
                         mfe_vec* b, const mfe_vec* kappa, double source) {
   if (!ctx || !A || !b || !box_ok(gbox) || !ebox) return MFE_BAD_ARG;
+  uses(ctx, A, b);
+  if (kappa) uses(ctx, kappa);
   if (!same_box(gbox, ebox))
     return fail(ctx, MFE_UNSUPPORTED, "one rank: the element box must be the global box");
   MFE_CHECK(ctx, hipSetDevice(ctx->device));
@@ -660,6 +662,7 @@ int mfe_impose_dirichlet(mfe_ctx* ctx, double value, mfe_csr* A, mfe_vec* b, int
   (void)gny;
   (void)gnz;
   if (!ctx || !A || !b || nbc < 0 || (nbc > 0 && !bc_rows)) return MFE_BAD_ARG;
+  uses(ctx, A, b);
   if (b->n != A->nrows) return fail(ctx, MFE_BAD_ARG, "b length != rows");
   MFE_CHECK(ctx, hipSetDevice(ctx->device));
   const int64_t n = A->nrows;
@@ -721,6 +724,7 @@ int mfe_impose_dirichlet(mfe_ctx* ctx, double value, mfe_csr* A, mfe_vec* b, int
 extern "C" int mfe_element_gradient(mfe_ctx* ctx, const int gbox[6], const mfe_vec* lambda,
                                     const mfe_vec* utilde, mfe_vec* grad) {
   if (!ctx || !box_ok(gbox) || !lambda || !utilde || !grad) return MFE_BAD_ARG;
+  uses(ctx, lambda, utilde, grad);
   const int Nx = gbox[1], Ny = gbox[3], Nz = gbox[5];
   const int64_t n = (int64_t)(Nx + 1) * (Ny + 1) * (Nz + 1);
   const int64_t ne = (int64_t)Nx * Ny * Nz;

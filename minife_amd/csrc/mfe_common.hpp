@@ -62,6 +62,7 @@ struct mfe_ctx {
 
 struct mfe_csr {
   mfe_ctx* ctx = nullptr;
+  mutable std::atomic<bool> shared{false};  // see uses()
   int64_t nrows = 0, nnz = 0;
   int* rows = nullptr;
   int* row_offsets = nullptr;
@@ -159,6 +160,7 @@ struct mfe_csr {
 
 struct mfe_vec {
   mfe_ctx* ctx = nullptr;
+  mutable std::atomic<bool> shared{false};  // see uses()
   int64_t n = 0;
   double* d = nullptr;
   bool owns = true;  // false for mfe_vec_wrap views
@@ -186,16 +188,32 @@ int hip_fail(mfe_ctx* ctx, hipError_t e, const char* what);
 // Device memory of matrices, vectors and their plans (mfe_api.hip).  dev_free
 // keeps the block for the next dev_alloc of about its size on the same context:
 // work on a context is ordered on its one stream, so a block can be handed out
-// again while kernels that used it are still queued.  Blocks kept on a device
-// are at most an eighth of its memory together (the oldest go first), all of
-// them go when an allocation fails, and a context's go with it.  Safe from
-// several threads.
+// again while kernels that used it are still queued.  What another context's
+// stream may have used (shared, see uses()) goes to hipFree, which waits for the
+// device.  Blocks kept on a device are at most an eighth of its memory together
+// (the oldest go first), all of them go when an allocation fails, and a context's
+// go with it.  Safe from several threads.
 hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes);
 template <typename P>
 inline hipError_t dev_alloc(mfe_ctx* ctx, P** out, size_t bytes) {
   return dev_alloc_bytes(ctx, reinterpret_cast<void**>(out), bytes);
 }
-void dev_free(mfe_ctx* ctx, void* p);
+void dev_free(mfe_ctx* ctx, void* p, bool shared = false);
+// A block of A's own.
+inline void csr_free(const mfe_csr* A, void* p) { dev_free(A->ctx, p, A->shared); }
+// Every entry point says which handles it is about to use on ctx: one that was
+// made on another context is marked for good, and its memory is not kept.
+inline void uses(const mfe_ctx* ctx, const mfe_csr* A) {
+  if (A->ctx != ctx) A->shared = true;
+}
+inline void uses(const mfe_ctx* ctx, const mfe_vec* v) {
+  if (v->ctx != ctx) v->shared = true;
+}
+template <typename H, typename... Hs>
+inline void uses(const mfe_ctx* ctx, const H* h, const Hs*... hs) {
+  uses(ctx, h);
+  uses(ctx, hs...);
+}
 // Recompute A->max_block_nnz on the device (synchronises the stream).
 int plan_spmv(mfe_ctx* ctx, mfe_csr* A);
 

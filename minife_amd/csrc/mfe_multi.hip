@@ -1452,6 +1452,7 @@ extern "C" {
 
 int mfe_spmm_tune(mfe_ctx* ctx, const mfe_csr* A, int nrhs, int* tile, double* ms, int* ntiles) {
   if (!ctx || !A || !k_ok(nrhs)) return MFE_BAD_ARG;
+  uses(ctx, A);
   MFE_CHECK(ctx, hipSetDevice(ctx->device));
   MultiWorkspace* w = nullptr;
   int st;
@@ -1468,6 +1469,7 @@ int mfe_spmm_tune(mfe_ctx* ctx, const mfe_csr* A, int nrhs, int* tile, double* m
 
 int mfe_spmm_select(mfe_ctx* ctx, const mfe_csr* A, int nrhs, int tile) {
   if (!ctx || !A || !k_ok(nrhs)) return MFE_BAD_ARG;
+  uses(ctx, A);
   if (tile < 0 || tile >= tile_count(nrhs)) return fail(ctx, MFE_BAD_ARG, "spmm_select: no such tile");
   MFE_CHECK(ctx, hipSetDevice(ctx->device));
   MultiWorkspace* w = nullptr;
@@ -1504,6 +1506,7 @@ int mfe_spmm_tile_info(int nrhs, int tile, int* cols_per_lane, int* unroll, int*
 
 int mfe_spmm(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* X, mfe_vec* Y, int nrhs, int tile) {
   if (!ctx || !A || !X || !Y || !k_ok(nrhs)) return MFE_BAD_ARG;
+  uses(ctx, A, X, Y);
   const int64_t nk = A->nrows * nrhs;
   if (X->n != nk || Y->n != nk) return fail(ctx, MFE_BAD_ARG, "spmm: X and Y need nrows*nrhs values");
   if (tile >= tile_count(nrhs)) return fail(ctx, MFE_BAD_ARG, "spmm: no such tile");
@@ -1544,6 +1547,7 @@ int mfe_cg_solve_multi(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* B, mfe_vec
                        int max_iter, double rel_tol, int* iters, double* rel_residual,
                        double* seconds) {
   if (!ctx || !A || !B || !X || !k_ok(nrhs) || max_iter < 0) return MFE_BAD_ARG;
+  uses(ctx, A, B, X);
   if (!A->has_local_indices)
     return fail(ctx, MFE_NOT_LOCAL,
                 "cg_solve_multi: A.has_local_indices is false; call make_local_matrix(A) first");

@@ -607,13 +607,13 @@ __global__ __launch_bounds__(kBlock) void spmv_sellx_kernel(
 }
 
 static void sellx_release(mfe_csr* A) {
-  dev_free(A->ctx, A->sellx_lcols);
-  dev_free(A->ctx, A->sellx_roff);
-  dev_free(A->ctx, A->sellx_rcol);
-  dev_free(A->ctx, A->sellx_rpos);
-  dev_free(A->ctx, A->sellx_nu);
-  dev_free(A->ctx, A->sellx_aff);
-  dev_free(A->ctx, A->sellx_sbase);
+  csr_free(A, A->sellx_lcols);
+  csr_free(A, A->sellx_roff);
+  csr_free(A, A->sellx_rcol);
+  csr_free(A, A->sellx_rpos);
+  csr_free(A, A->sellx_nu);
+  csr_free(A, A->sellx_aff);
+  csr_free(A, A->sellx_sbase);
   A->sellx_lcols = nullptr;
   A->sellx_roff = A->sellx_rcol = A->sellx_rpos = A->sellx_nu = nullptr;
   A->sellx_aff = nullptr;
@@ -626,12 +626,12 @@ static void sellx_release(mfe_csr* A) {
 void sell_release(mfe_csr* A) {
   A->plan_gen = next_plan_gen();
   sellx_release(A);
-  dev_free(A->ctx, A->sell_off);
-  dev_free(A->ctx, A->sell_len);
-  dev_free(A->ctx, A->sell_cols);
-  dev_free(A->ctx, A->sell_vals);
-  dev_free(A->ctx, A->sell_vals32);
-  dev_free(A->ctx, A->sell_lines);
+  csr_free(A, A->sell_off);
+  csr_free(A, A->sell_len);
+  csr_free(A, A->sell_cols);
+  csr_free(A, A->sell_vals);
+  csr_free(A, A->sell_vals32);
+  csr_free(A, A->sell_lines);
   A->sell_lines = nullptr;
   A->sell_lines_valid = false;
   A->sell_off = nullptr;
@@ -759,19 +759,19 @@ __global__ void vals_to_f32_kernel(int64_t nnz, const double* __restrict__ v,
 // ---- box layout plan ---------------------------------------------------------
 
 void box_release(mfe_csr* A) {
-  dev_free(A->ctx, A->box_vals);
-  dev_free(A->ctx, A->box_vals32);
-  dev_free(A->ctx, A->boxsym_u);
-  dev_free(A->ctx, A->boxsym_w);
-  dev_free(A->ctx, A->boxsym_u32);
-  dev_free(A->ctx, A->boxsym_w32);
-  dev_free(A->ctx, A->boxsym_tab);
-  dev_free(A->ctx, A->boxpack_pw);
-  dev_free(A->ctx, A->boxpack_kq);
-  dev_free(A->ctx, A->boxpack32_pw);
-  dev_free(A->ctx, A->boxpack32_kq);
-  dev_free(A->ctx, A->boxwpack_pw);
-  dev_free(A->ctx, A->boxwpack_kq);
+  csr_free(A, A->box_vals);
+  csr_free(A, A->box_vals32);
+  csr_free(A, A->boxsym_u);
+  csr_free(A, A->boxsym_w);
+  csr_free(A, A->boxsym_u32);
+  csr_free(A, A->boxsym_w32);
+  csr_free(A, A->boxsym_tab);
+  csr_free(A, A->boxpack_pw);
+  csr_free(A, A->boxpack_kq);
+  csr_free(A, A->boxpack32_pw);
+  csr_free(A, A->boxpack32_kq);
+  csr_free(A, A->boxwpack_pw);
+  csr_free(A, A->boxwpack_kq);
   A->box_vals = nullptr;
   A->box_vals32 = nullptr;
   A->boxsym_u = A->boxsym_w = nullptr;
@@ -1372,8 +1372,8 @@ static int build_boxsym(mfe_ctx* ctx, mfe_csr* A) {
   if (check) {
     A->boxsym_state = hw.asym ? 2 : 1;
     if (hw.asym) {  // not symmetric: the box layout with all 27 slots instead
-      dev_free(ctx, *du);
-      dev_free(ctx, *dw);
+      csr_free(A, *du);
+      csr_free(A, *dw);
       *du = nullptr;
       *dw = nullptr;
       return MFE_OK;
@@ -1417,8 +1417,9 @@ static int with_pack_form(int form, F&& f) {
 // left kPackNone when they do not fit in memory.  Enqueues the packing; the
 // caller checks words->pack_bad.
 template <typename T>
-static int enqueue_pack(mfe_ctx* ctx, const T* U, int64_t groups, const unsigned* fits, T* kq,
-                        unsigned** pw, int* cap, PlanWords* words, int* form_out) {
+static int enqueue_pack(mfe_ctx* ctx, const mfe_csr* A, const T* U, int64_t groups,
+                        const unsigned* fits, T* kq, unsigned** pw, int* cap, PlanWords* words,
+                        int* form_out) {
   using P = SymPack;
   constexpr bool f64 = std::is_same<T, double>::value;
   *form_out = kPackNone;
@@ -1447,7 +1448,7 @@ static int enqueue_pack(mfe_ctx* ctx, const T* U, int64_t groups, const unsigned
   if (form == kPackNone) return MFE_OK;
   const int nw = P::words(form);
   if (*cap < nw) {
-    dev_free(ctx, *pw);
+    csr_free(A, *pw);
     *pw = nullptr;
     *cap = 0;
     if (!try_alloc(ctx, pw, sizeof(unsigned) * (size_t)(groups * nw * kBlock))) return MFE_OK;
@@ -1558,11 +1559,11 @@ static int build_boxpack(mfe_ctx* ctx, mfe_csr* A) {
   plan_words_kernel<<<1, kWave, 0, ctx->stream>>>(words);
   int form = kPackNone, wform = kPackNone, st = MFE_OK;
   if constexpr (f64) {
-    st = enqueue_pack<double>(ctx, A->boxsym_u, groups, A->boxpack_fits, A->boxpack_kq,
+    st = enqueue_pack<double>(ctx, A, A->boxsym_u, groups, A->boxpack_fits, A->boxpack_kq,
                               &A->boxpack_pw, &A->boxpack_cap, words, &form);
     if (!st && form != kPackNone) st = enqueue_wpack(ctx, A, groups, words, &wform);
   } else {
-    st = enqueue_pack<float>(ctx, A->boxsym_u32, groups, A->boxpack32_fits, A->boxpack32_kq,
+    st = enqueue_pack<float>(ctx, A, A->boxsym_u32, groups, A->boxpack32_fits, A->boxpack32_kq,
                              &A->boxpack32_pw, &A->boxpack32_cap, words, &form);
   }
   if (st) return st;
@@ -3101,6 +3102,7 @@ void mfe_cg_workspace_free(mfe_ctx* ctx) {
 
 static int check_vec(mfe_ctx* ctx, const mfe_vec* v, int64_t n, const char* what) {
   if (!v || v->n != n) return fail(ctx, MFE_BAD_ARG, std::string(what) + ": length mismatch");
+  uses(ctx, v);
   return MFE_OK;
 }
 
@@ -3125,6 +3127,7 @@ static int read_scalar(mfe_ctx* ctx, const double* d, double* out) {
 int mfe_spmv_plan(mfe_ctx* ctx, mfe_csr* A, int format, int64_t info[8]) {
   if (!ctx || !A || (format != MFE_SPMV_AUTO && format != MFE_SPMV_CSR && format != MFE_SPMV_SELL))
     return MFE_BAD_ARG;
+  uses(ctx, A);
   MFE_CHECK(ctx, hipSetDevice(ctx->device));
   if (format != A->spmv_format) {
     MFE_CHECK(ctx, hipStreamSynchronize(ctx->stream));
@@ -3180,6 +3183,7 @@ int mfe_spmv_plan(mfe_ctx* ctx, mfe_csr* A, int format, int64_t info[8]) {
 
 int mfe_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y) {
   if (!ctx || !A) return MFE_BAD_ARG;
+  uses(ctx, A);
   int st;
   if ((st = check_vec(ctx, x, A->nrows, "matvec x")) || (st = check_vec(ctx, y, A->nrows, "matvec y")))
     return st;
@@ -3193,6 +3197,7 @@ int mfe_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y) {
 int mfe_matvec_and_dot(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y,
                        double* result) {
   if (!ctx || !A || !result) return MFE_BAD_ARG;
+  uses(ctx, A);
   int st;
   if ((st = check_vec(ctx, x, A->nrows, "matvec x")) || (st = check_vec(ctx, y, A->nrows, "matvec y")))
     return st;
@@ -3215,6 +3220,7 @@ int mfe_matvec_and_dot(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec
 int mfe_matvec_and_dot_noalloc(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y,
                                double* result_device) {
   if (!ctx || !A || !result_device) return MFE_BAD_ARG;
+  uses(ctx, A);
   int st;
   if ((st = check_vec(ctx, x, A->nrows, "matvec x")) || (st = check_vec(ctx, y, A->nrows, "matvec y")))
     return st;
@@ -3245,6 +3251,7 @@ int mfe_matvec_and_dot_noalloc(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x,
 
 int mfe_matvec_fp32(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y) {
   if (!ctx || !A) return MFE_BAD_ARG;
+  uses(ctx, A);
   int st;
   if ((st = check_vec(ctx, x, A->nrows, "matvec x")) || (st = check_vec(ctx, y, A->nrows, "matvec y")))
     return st;
@@ -3266,6 +3273,7 @@ int mfe_matvec_fp32(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y
 int mfe_time_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y, int variant,
                     int reps, double* avg_ms) {
   if (!ctx || !A || !avg_ms || reps <= 0 || variant < 0 || variant > 12) return MFE_BAD_ARG;
+  uses(ctx, A);
   int st;
   if ((st = check_vec(ctx, x, A->nrows, "matvec x")) || (st = check_vec(ctx, y, A->nrows, "matvec y")))
     return st;
@@ -3338,6 +3346,7 @@ int mfe_time_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y
 
 int mfe_dot(mfe_ctx* ctx, const mfe_vec* x, const mfe_vec* y, double* result) {
   if (!ctx || !x || !y || !result) return MFE_BAD_ARG;
+  uses(ctx, x, y);
   if (y->n < x->n) return fail(ctx, MFE_BAD_ARG, "dot: y shorter than x");
   const int64_t n = x->n;
   const unsigned g = vec_grid(n);
@@ -3352,6 +3361,7 @@ int mfe_dot(mfe_ctx* ctx, const mfe_vec* x, const mfe_vec* y, double* result) {
 
 int mfe_dot_replay(mfe_ctx* ctx, const mfe_vec* x, const mfe_vec* y, double* result) {
   if (!ctx || !x || !y || !result) return MFE_BAD_ARG;
+  uses(ctx, x, y);
   if (y->n < x->n) return fail(ctx, MFE_BAD_ARG, "dot: y shorter than x");
   dot_seq_kernel<<<1, kBlock, 0, ctx->stream>>>(x->n, x->d, y->d, ctx->d_scalars);
   MFE_LAUNCHED(ctx, "dot_seq_kernel");
@@ -3361,6 +3371,7 @@ int mfe_dot_replay(mfe_ctx* ctx, const mfe_vec* x, const mfe_vec* y, double* res
 int mfe_waxpby(mfe_ctx* ctx, double alpha, const mfe_vec* x, double beta, const mfe_vec* y,
                mfe_vec* w) {
   if (!ctx || !x || !y || !w) return MFE_BAD_ARG;
+  uses(ctx, x, y, w);
   if (y->n < x->n || w->n < x->n) return fail(ctx, MFE_BAD_ARG, "waxpby: y and w must be at least as long as x");
   if (x->n == 0) return MFE_OK;
   waxpby_kernel<double><<<vec_grid(x->n), kBlock, 0, ctx->stream>>>(x->n, alpha, x->d, beta, y->d,
@@ -3373,6 +3384,7 @@ int mfe_cg_solve(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_vec* x, i
                  double tolerance, unsigned flags, int* num_iters, double* normr,
                  double* times, double* history) {
   if (!ctx || !A || !num_iters || !normr) return MFE_BAD_ARG;
+  uses(ctx, A);
   if (!A->has_local_indices)
     return fail(ctx, MFE_NOT_LOCAL,
                 "cg_solve: A.has_local_indices is false; call make_local_matrix(A) first");
@@ -3425,6 +3437,7 @@ int mfe_cg_solve_mixed_ex(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_
                           double* rel_residual, double* times) {
   if (!ctx || !A || !outer_iters || !inner_iters || !rel_residual || max_outer < 0 || max_inner < 0)
     return MFE_BAD_ARG;
+  uses(ctx, A);
   const bool keep = (flags & MFE_MIXED_KEEP_DIRECTION) != 0;
   if (!A->has_local_indices)
     return fail(ctx, MFE_NOT_LOCAL,
