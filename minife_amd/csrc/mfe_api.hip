@@ -38,12 +38,18 @@ struct DevPool {
   std::map<uint64_t, Block> idle;              // kept blocks by age
   size_t idle_bytes = 0, cap = 0;
   uint64_t clock = 0;
-  // Gives a kept block back to the driver (mu held).
-  std::map<uint64_t, Block>::iterator drop(std::map<uint64_t, Block>::iterator it) {
-    (void)hipStreamSynchronize(it->second.ctx->stream);
-    (void)hipFree(it->second.p);
+  // Takes a kept block out (mu held); the caller gives it to release().
+  std::map<uint64_t, Block>::iterator take(std::map<uint64_t, Block>::iterator it,
+                                           std::vector<void*>& out) {
+    out.push_back(it->second.p);
     idle_bytes -= it->second.bytes;
     return idle.erase(it);
+  }
+  // Gives blocks back to the driver, without the mutex: hipFree waits for the
+  // device, other contexts' work included, and their threads go on meanwhile.  No
+  // stream is waited for by name: another thread may be capturing it.
+  static void release(const std::vector<void*>& blocks) {
+    for (void* p : blocks) (void)hipFree(p);
   }
 };
 constexpr int kPoolDevices = 64;
@@ -59,7 +65,7 @@ hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes) {
   if (!P) return hipMalloc(out, bytes);
   const size_t unit = bytes < (size_t(1) << 20) ? 512 : size_t(2) << 20;
   const size_t want = (bytes + unit - 1) / unit * unit;
-  std::lock_guard<std::mutex> lock(P->mu);
+  std::unique_lock<std::mutex> lock(P->mu);
   auto best = P->idle.end();  // the smallest kept block of at most 1/8 more
   for (auto it = P->idle.begin(); it != P->idle.end(); ++it)
     if (it->second.ctx == ctx && it->second.bytes >= want &&
@@ -73,17 +79,23 @@ hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes) {
     P->idle.erase(best);
     return hipSuccess;
   }
+  lock.unlock();
   hipError_t e = hipMalloc(out, want);
-  if (e != hipSuccess && !P->idle.empty()) {
+  if (e != hipSuccess) {
     (void)hipGetLastError();
-    for (auto it = P->idle.begin(); it != P->idle.end();) it = P->drop(it);
-    e = hipMalloc(out, want);
+    std::vector<void*> all;
+    lock.lock();
+    for (auto it = P->idle.begin(); it != P->idle.end();) it = P->take(it, all);
+    lock.unlock();
+    DevPool::release(all);
+    if (!all.empty()) e = hipMalloc(out, want);
   }
   if (e != hipSuccess) {
     (void)hipGetLastError();  // nothing sticky: the caller decides
     *out = nullptr;
     return e;
   }
+  lock.lock();
   P->live[*out] = want;
   return hipSuccess;
 }
@@ -95,31 +107,39 @@ void dev_free(mfe_ctx* ctx, void* p, bool shared) {
     (void)hipFree(p);
     return;
   }
-  std::lock_guard<std::mutex> lock(P->mu);
-  auto it = P->live.find(p);
-  const size_t bytes = it == P->live.end() ? 0 : it->second;
-  if (it != P->live.end()) P->live.erase(it);
-  if (shared || bytes == 0) {
-    (void)hipFree(p);
-    return;
+  std::vector<void*> gone;
+  {
+    std::lock_guard<std::mutex> lock(P->mu);
+    auto it = P->live.find(p);
+    const size_t bytes = it == P->live.end() ? 0 : it->second;
+    if (it != P->live.end()) P->live.erase(it);
+    if (shared || bytes == 0) {
+      gone.push_back(p);
+    } else {
+      if (!P->cap) {
+        size_t free_b = 0, total = 0;
+        if (hipMemGetInfo(&free_b, &total) == hipSuccess) P->cap = total / 8;
+      }
+      P->idle[P->clock++] = DevPool::Block{p, bytes, ctx};
+      P->idle_bytes += bytes;
+      for (auto old = P->idle.begin(); P->idle_bytes > P->cap && old != P->idle.end();)
+        old = P->take(old, gone);
+    }
   }
-  if (!P->cap) {
-    size_t free_b = 0, total = 0;
-    if (hipMemGetInfo(&free_b, &total) == hipSuccess) P->cap = total / 8;
-  }
-  P->idle[P->clock++] = DevPool::Block{p, bytes, ctx};
-  P->idle_bytes += bytes;
-  for (auto old = P->idle.begin(); P->idle_bytes > P->cap && old != P->idle.end();)
-    old = P->drop(old);
+  DevPool::release(gone);
 }
 
 // The blocks kept for ctx go (its stream has drained).
 static void dev_drop(mfe_ctx* ctx) {
   DevPool* P = pool_of(ctx);
   if (!P) return;
-  std::lock_guard<std::mutex> lock(P->mu);
-  for (auto it = P->idle.begin(); it != P->idle.end();)
-    it = it->second.ctx == ctx ? P->drop(it) : std::next(it);
+  std::vector<void*> gone;
+  {
+    std::lock_guard<std::mutex> lock(P->mu);
+    for (auto it = P->idle.begin(); it != P->idle.end();)
+      it = it->second.ctx == ctx ? P->take(it, gone) : std::next(it);
+  }
+  DevPool::release(gone);
 }
 
 // Largest non-zero count of any kSpmvRows-row tile: ro[min(r0+R,n)] - ro[r0].

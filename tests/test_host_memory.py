@@ -175,3 +175,29 @@ for name, (make, call) in calls.items():
             gone = stub.stub_frees() - before
             assert (gone > 0) == foreign, (name, type(h).__name__, foreign, gone)
 """)
+
+
+@pytest.mark.parametrize("why", ["cap", "failure"])
+def test_giving_kept_memory_back_leaves_other_streams_alone(stub_lib, why):
+    """Memory that one context kept goes when another context's thread frees more
+    than the device keeps, or runs out of memory -- without a wait for the first
+    one's stream, which its own thread may be capturing."""
+    run(stub_lib, f"why = {why!r}" + """
+stub.stub_capacity(256 * MB)      # 32 MB may be kept
+c1, c2 = m.Context(0), m.Context(0)
+kept = [vec(8, c2) for _ in range(3)]
+for v in kept: v.close()
+assert stub.stub_frees() == 0
+stub.stub_thread_stream(0)
+stub.stub_begin_capture(1)        # c2's stream
+if why == "cap":
+    vs = [vec(8, c1) for _ in range(2)]
+    for v in vs: v.close()
+    assert stub.stub_frees() == 1
+else:
+    v = vec(240, c1)
+    assert stub.stub_frees() == 3
+    v.close()
+stub.stub_end_capture(1)
+assert stub.stub_capture_breaks() == 0 and stub.stub_foreign_waits() == 0
+""")
