@@ -18,8 +18,8 @@
  *     nnz must stay below 2^31 (the reference's LocalOrdinal is int).
  *   - Handles own device memory.  What destroyed matrices and vectors held is
  *     kept for later ones on the same context, at most an eighth of the
- *     device's memory over all contexts, until an allocation fails or the
- *     context goes; the memory of one that was used on another context than
+ *     device's memory over all contexts, until an allocation of the library
+ *     fails, mfe_trim_memory is called or the context goes; the memory of one that was used on another context than
  *     its own goes back to the driver when it is destroyed.  Host pointers are
  *     borrowed for the call.
  *     Calls on one ctx are ordered on its single HIP stream; a ctx is not
@@ -74,6 +74,10 @@ int mfe_ctx_create(int device, mfe_ctx** out);
 void mfe_ctx_destroy(mfe_ctx* ctx);
 const char* mfe_last_error(const mfe_ctx* ctx);
 int mfe_ctx_synchronize(mfe_ctx* ctx);
+/* Gives the memory kept for later matrices and vectors on ctx's device (of all
+ * contexts) back to the driver, where other allocators of the process find it;
+ * bytes (nullable) receives how much that was. */
+int mfe_trim_memory(mfe_ctx* ctx, int64_t* bytes);
 /* Device name, compute-unit count and HBM bytes of ctx's device. */
 int mfe_device_info(mfe_ctx* ctx, char* name, int name_len, int* cu_count,
                     int64_t* hbm_bytes);

@@ -70,7 +70,7 @@ T_WAXPY, T_DOT, T_MATVEC, T_MATVECDOT, T_TOTAL = range(5)
 
 # Every extern "C" symbol declared in include/minife_hip.h.
 EXPORTS = [
-    "mfe_ctx_create", "mfe_ctx_destroy", "mfe_last_error", "mfe_ctx_synchronize",
+    "mfe_ctx_create", "mfe_ctx_destroy", "mfe_last_error", "mfe_ctx_synchronize", "mfe_trim_memory",
     "mfe_device_info", "mfe_timer_start", "mfe_timer_stop",
     "mfe_csr_create", "mfe_csr_destroy", "mfe_csr_shape", "mfe_csr_upload", "mfe_csr_download",
     "mfe_vec_create", "mfe_vec_destroy", "mfe_vec_size", "mfe_vec_upload", "mfe_vec_download",
@@ -171,6 +171,7 @@ def lib() -> ctypes.CDLL:
         "mfe_ctx_destroy": ([_vp], None),
         "mfe_last_error": ([_vp], ctypes.c_char_p),
         "mfe_ctx_synchronize": ([_vp], ctypes.c_int),
+        "mfe_trim_memory": ([_vp, ctypes.POINTER(_i64)], ctypes.c_int),
         "mfe_device_info": ([_vp, ctypes.c_char_p, ctypes.c_int, ctypes.POINTER(ctypes.c_int),
                              ctypes.POINTER(_i64)], ctypes.c_int),
         "mfe_timer_start": ([_vp], ctypes.c_int),
@@ -270,6 +271,13 @@ class Context:
 
     def synchronize(self):
         self.check(lib().mfe_ctx_synchronize(self.h), "synchronize")
+
+    def trim_memory(self) -> int:
+        """Gives the device memory kept for later matrices and vectors back to the
+        driver (torch's allocator then finds it); returns the bytes."""
+        n = _i64(0)
+        self.check(lib().mfe_trim_memory(self.h, ctypes.byref(n)), "trim_memory")
+        return n.value
 
     def device_info(self) -> dict:
         buf = ctypes.create_string_buffer(256)

@@ -59,10 +59,37 @@ DevPool* pool_of(const mfe_ctx* ctx) {
 }
 }  // namespace
 
+// Gives every block kept on ctx's device back to the driver; their bytes.
+static size_t dev_trim(mfe_ctx* ctx) {
+  DevPool* P = pool_of(ctx);
+  if (!P) return 0;
+  std::vector<void*> all;
+  size_t bytes = 0;
+  {
+    std::lock_guard<std::mutex> lock(P->mu);
+    bytes = P->idle_bytes;
+    for (auto it = P->idle.begin(); it != P->idle.end();) it = P->take(it, all);
+  }
+  DevPool::release(all);
+  return bytes;
+}
+
+hipError_t dev_malloc_bytes(mfe_ctx* ctx, void** out, size_t bytes) {
+  hipError_t e = hipMalloc(out, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  if (dev_trim(ctx) > 0) e = hipMalloc(out, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // nothing sticky: the caller decides
+    *out = nullptr;
+  }
+  return e;
+}
+
 hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes) {
   *out = nullptr;
   DevPool* P = pool_of(ctx);
-  if (!P) return hipMalloc(out, bytes);
+  if (!P) return dev_malloc_bytes(ctx, out, bytes);
   const size_t unit = bytes < (size_t(1) << 20) ? 512 : size_t(2) << 20;
   const size_t want = (bytes + unit - 1) / unit * unit;
   std::unique_lock<std::mutex> lock(P->mu);
@@ -80,21 +107,8 @@ hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes) {
     return hipSuccess;
   }
   lock.unlock();
-  hipError_t e = hipMalloc(out, want);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    std::vector<void*> all;
-    lock.lock();
-    for (auto it = P->idle.begin(); it != P->idle.end();) it = P->take(it, all);
-    lock.unlock();
-    DevPool::release(all);
-    if (!all.empty()) e = hipMalloc(out, want);
-  }
-  if (e != hipSuccess) {
-    (void)hipGetLastError();  // nothing sticky: the caller decides
-    *out = nullptr;
-    return e;
-  }
+  const hipError_t e = dev_malloc_bytes(ctx, out, want);
+  if (e != hipSuccess) return e;
   lock.lock();
   P->live[*out] = want;
   return hipSuccess;
@@ -244,7 +258,7 @@ int mfe_ctx_create(int device, mfe_ctx** out) {
     return bail(MFE_HIP_ERROR);
   if (hipEventCreate(&c->t_start) != hipSuccess || hipEventCreate(&c->t_stop) != hipSuccess)
     return bail(MFE_HIP_ERROR);
-  if (hipMalloc(&c->d_scalars, 64 * sizeof(double)) != hipSuccess) return bail(MFE_OOM);
+  if (dev_malloc(c, &c->d_scalars, 64 * sizeof(double)) != hipSuccess) return bail(MFE_OOM);
   if (hipHostMalloc(&c->h_scalars, 64 * sizeof(double), hipHostMallocDefault) != hipSuccess)
     return bail(MFE_OOM);
   hipDeviceProp_t prop;
@@ -289,6 +303,14 @@ const char* mfe_last_error(const mfe_ctx* ctx) { return ctx ? ctx->err.c_str() :
 int mfe_ctx_synchronize(mfe_ctx* ctx) {
   if (!ctx) return MFE_BAD_ARG;
   MFE_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+  return MFE_OK;
+}
+
+int mfe_trim_memory(mfe_ctx* ctx, int64_t* bytes) {
+  if (!ctx) return MFE_BAD_ARG;
+  MFE_CHECK(ctx, hipSetDevice(ctx->device));
+  const size_t freed = dev_trim(ctx);
+  if (bytes) *bytes = (int64_t)freed;
   return MFE_OK;
 }
 

@@ -944,7 +944,7 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
   };
   hipError_t e;
 #define BALLOC(ptr, bytes) \
-  if ((e = hipMalloc(&(ptr), (bytes))) != hipSuccess) return fail_oom(e)
+  if ((e = dev_malloc(ctx, &(ptr), (bytes))) != hipSuccess) return fail_oom(e)
   BALLOC(B->d_probs, sizeof(BatchProb) * (size_t)nprob);
   BALLOC(B->d_blk2prob, sizeof(int) * B->blk2prob.size());
   BALLOC(B->d_soff, sizeof(int) * B->soff.size());
@@ -967,10 +967,8 @@ int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out) 
   // the packed words last: a batch that fits without them still runs
   const char* pack = std::getenv("MINIFE_BATCH_PACK");
   if (!(pack && std::atoi(pack) == 0) &&
-      hipMalloc(&B->d_words, sizeof(unsigned) * kBWords * kBlock * (size_t)tile0) != hipSuccess) {
-    (void)hipGetLastError();
+      dev_malloc(ctx, &B->d_words, sizeof(unsigned) * kBWords * kBlock * (size_t)tile0) != hipSuccess)
     B->d_words = nullptr;
-  }
   // zero everything once: the per-problem tails stay value 0, column 0
   auto fill = [&]() -> int {
     MFE_CHECK(ctx, hipMemsetAsync(B->d_scols, 0, sizeof(int) * (size_t)B->slots, s));

@@ -191,14 +191,22 @@ int hip_fail(mfe_ctx* ctx, hipError_t e, const char* what);
 // again while kernels that used it are still queued.  What another context's
 // stream may have used (shared, see uses()) goes to hipFree, which waits for the
 // device.  Blocks kept on a device are at most an eighth of its memory together
-// (the oldest go first), all of them go when an allocation fails, and a context's
-// go with it.  Safe from several threads.
+// (the oldest go first), all of them go when an allocation of the library fails
+// or mfe_trim_memory asks for it, and a context's go with it.  Safe from several
+// threads.
 hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes);
 template <typename P>
 inline hipError_t dev_alloc(mfe_ctx* ctx, P** out, size_t bytes) {
   return dev_alloc_bytes(ctx, reinterpret_cast<void**>(out), bytes);
 }
 void dev_free(mfe_ctx* ctx, void* p, bool shared = false);
+// hipMalloc of memory that is not kept (workspaces; hipFree frees it) and, when
+// that fails, once more after the kept blocks have gone back.
+hipError_t dev_malloc_bytes(mfe_ctx* ctx, void** out, size_t bytes);
+template <typename P>
+inline hipError_t dev_malloc(mfe_ctx* ctx, P** out, size_t bytes) {
+  return dev_malloc_bytes(ctx, reinterpret_cast<void**>(out), bytes);
+}
 // A block of A's own.
 inline void csr_free(const mfe_csr* A, void* p) { dev_free(A->ctx, p, A->shared); }
 // Every entry point says which handles it is about to use on ctx: one that was

@@ -374,7 +374,7 @@ static int build_stage_plan(mfe_ctx* ctx, const mfe_csr* A, int R, SpmmPlan& p) 
   if (n == 0 || n > INT_MAX - R) return MFE_OK;
   const int nt = (int)cdiv(n, R);
   hipStream_t s = ctx->stream;
-  MFE_CHECK(ctx, hipMalloc(&p.uoff, sizeof(int) * ((size_t)nt + 1)));
+  MFE_CHECK(ctx, dev_malloc(ctx, &p.uoff, sizeof(int) * ((size_t)nt + 1)));
   stage_plan_kernel<<<nt, kBlock, 0, s>>>((int)n, R, A->row_offsets, A->cols, 0, nullptr, p.uoff,
                                           nullptr, nullptr);
   MFE_LAUNCHED(ctx, "stage_plan_kernel count");
@@ -401,8 +401,8 @@ static int build_stage_plan(mfe_ctx* ctx, const mfe_csr* A, int R, SpmmPlan& p) 
   if (total > INT_MAX) return MFE_OK;
   MFE_CHECK(ctx, hipMemcpyAsync(p.uoff, h.data(), sizeof(int) * ((size_t)nt + 1),
                                 hipMemcpyHostToDevice, s));
-  MFE_CHECK(ctx, hipMalloc(&p.ucols, sizeof(int) * (size_t)std::max<int64_t>(total, 1)));
-  MFE_CHECK(ctx, hipMalloc(&p.lcols, sizeof(unsigned short) * (size_t)std::max<int64_t>(A->nnz, 1)));
+  MFE_CHECK(ctx, dev_malloc(ctx, &p.ucols, sizeof(int) * (size_t)std::max<int64_t>(total, 1)));
+  MFE_CHECK(ctx, dev_malloc(ctx, &p.lcols, sizeof(unsigned short) * (size_t)std::max<int64_t>(A->nnz, 1)));
   stage_plan_kernel<<<nt, kBlock, 0, s>>>((int)n, R, A->row_offsets, A->cols, 1, p.uoff, nullptr,
                                           p.ucols, p.lcols);
   MFE_LAUNCHED(ctx, "stage_plan_kernel fill");
@@ -1336,16 +1336,16 @@ static int multi_prepare(mfe_ctx* ctx, int64_t n, int K, MultiWorkspace** out) {
   if (w->nk != nk || w->K != K) {
     w->release();
     const size_t bytes = sizeof(double) * (size_t)std::max<int64_t>(nk, 1);
-    MFE_CHECK(ctx, hipMalloc(&w->R, bytes));
-    MFE_CHECK(ctx, hipMalloc(&w->P, bytes));
-    MFE_CHECK(ctx, hipMalloc(&w->AP, bytes));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->R, bytes));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->P, bytes));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->AP, bytes));
     // partial rows: the SpMM's workgroups (at most n with one row each) or
     // the vector kernels' grid
     w->part_rows = std::max<int64_t>(n, kVecBlocks) + 1;
-    MFE_CHECK(ctx, hipMalloc(&w->part, sizeof(double) * (size_t)(w->part_rows * K)));
-    MFE_CHECK(ctx, hipMalloc(&w->part2, sizeof(double) * (size_t)((cdiv(w->part_rows, kColStage) + 1) * K)));
-    MFE_CHECK(ctx, hipMalloc(&w->res, sizeof(double) * 64));
-    MFE_CHECK(ctx, hipMalloc(&w->st, sizeof(MultiState)));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->part, sizeof(double) * (size_t)(w->part_rows * K)));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->part2, sizeof(double) * (size_t)((cdiv(w->part_rows, kColStage) + 1) * K)));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->res, sizeof(double) * 64));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->st, sizeof(MultiState)));
     MFE_CHECK(ctx, hipHostMalloc(&w->h_st, sizeof(MultiState), hipHostMallocDefault));
     w->nk = nk;
     w->K = K;

@@ -2679,13 +2679,13 @@ static int vecset_prepare(mfe_ctx* ctx, VecSet<T>& v, int64_t n, GraphSlot<T>& g
   v.release();
   const int64_t tiles = cdiv(n, kSpmvRows);
   const size_t bytes = sizeof(T) * (size_t)(n > 0 ? n : 1);
-  MFE_CHECK(ctx, hipMalloc(&v.r, bytes));
-  MFE_CHECK(ctx, hipMalloc(&v.p, bytes));
-  MFE_CHECK(ctx, hipMalloc(&v.Ap, bytes));
+  MFE_CHECK(ctx, dev_malloc(ctx, &v.r, bytes));
+  MFE_CHECK(ctx, dev_malloc(ctx, &v.p, bytes));
+  MFE_CHECK(ctx, dev_malloc(ctx, &v.Ap, bytes));
   v.part_base = tiles > kVecBlocks ? tiles : kVecBlocks;
-  MFE_CHECK(ctx, hipMalloc(&v.partials, sizeof(T) * 4 * (size_t)v.part_base));
+  MFE_CHECK(ctx, dev_malloc(ctx, &v.partials, sizeof(T) * 4 * (size_t)v.part_base));
   const int64_t n2 = cdiv(tiles, kStage) > 0 ? cdiv(tiles, kStage) : 1;
-  MFE_CHECK(ctx, hipMalloc(&v.red2, sizeof(T) * (size_t)n2));
+  MFE_CHECK(ctx, dev_malloc(ctx, &v.red2, sizeof(T) * (size_t)n2));
   v.n = n;
   return MFE_OK;
 }
@@ -2695,7 +2695,7 @@ static int ws_get(mfe_ctx* ctx, int max_iter, CgWorkspace** out) {
   if (!w) {
     w = new CgWorkspace();
     ctx->cg = w;
-    MFE_CHECK(ctx, hipMalloc(&w->st, 2 * sizeof(CgState)));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->st, 2 * sizeof(CgState)));
     MFE_CHECK(ctx, hipHostMalloc(&w->h_st, sizeof(CgState), hipHostMallocDefault));
     MFE_CHECK(ctx, hipHostMalloc(&w->h_progress, sizeof(*w->h_progress), hipHostMallocCoherent));
   }
@@ -2706,7 +2706,7 @@ static int ws_get(mfe_ctx* ctx, int max_iter, CgWorkspace** out) {
     hipFree(w->hist);
     w->hist = nullptr;
     w->hist_cap = 0;
-    MFE_CHECK(ctx, hipMalloc(&w->hist, sizeof(double) * (size_t)hneed));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->hist, sizeof(double) * (size_t)hneed));
     w->hist_cap = hneed;
   }
   *out = w;
@@ -3111,7 +3111,7 @@ static int ensure_partials(mfe_ctx* ctx, int64_t count) {
   hipFree(ctx->d_partials);
   ctx->d_partials = nullptr;
   ctx->partials_cap = 0;
-  MFE_CHECK(ctx, hipMalloc(&ctx->d_partials, sizeof(double) * (size_t)count));
+  MFE_CHECK(ctx, dev_malloc(ctx, &ctx->d_partials, sizeof(double) * (size_t)count));
   ctx->partials_cap = (size_t)count;
   return MFE_OK;
 }
@@ -3459,8 +3459,8 @@ int mfe_cg_solve_mixed_ex(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_
     hipFree(w->f_x);
     w->f_rhs = w->f_x = nullptr;
     w->g32.drop();
-    MFE_CHECK(ctx, hipMalloc(&w->f_rhs, sizeof(float) * (size_t)(n > 0 ? n : 1)));
-    MFE_CHECK(ctx, hipMalloc(&w->f_x, sizeof(float) * (size_t)(n > 0 ? n : 1)));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->f_rhs, sizeof(float) * (size_t)(n > 0 ? n : 1)));
+    MFE_CHECK(ctx, dev_malloc(ctx, &w->f_x, sizeof(float) * (size_t)(n > 0 ? n : 1)));
     w->f_n = n;
   }
   MFE_CHECK(ctx, hipEventRecord(ctx->t_start, s));

@@ -156,7 +156,7 @@ calls = {
 }
 # take no vector or matrix, or do not touch its memory
 exempt = {x for x in m.EXPORTS if x.startswith(("mfe_ctx_", "mfe_timer_", "mfe_batch_"))} | {
-    "mfe_last_error", "mfe_device_info", "mfe_csr_create", "mfe_csr_destroy", "mfe_csr_shape",
+    "mfe_last_error", "mfe_device_info", "mfe_trim_memory", "mfe_csr_create", "mfe_csr_destroy", "mfe_csr_shape",
     "mfe_vec_create", "mfe_vec_destroy", "mfe_vec_size", "mfe_vec_wrap", "mfe_make_local_matrix",
     "mfe_soln", "mfe_spmm_tile_info"}
 assert set(calls) | exempt == set(m.EXPORTS), set(calls) ^ (set(m.EXPORTS) - exempt)
@@ -200,4 +200,53 @@ else:
     v.close()
 stub.stub_end_capture(1)
 assert stub.stub_capture_breaks() == 0 and stub.stub_foreign_waits() == 0
+""")
+
+
+WORKSPACES = {
+    "cg_solve": "m.cg_solve(A, b, x, max_iter=2)",
+    "cg_solve_mixed": "m.cg_solve_mixed(A, b, x, max_outer=1, max_inner=2)",
+    "matvec_fp32": "m.matvec_fp32(A, b, x)",
+    "matvec_and_dot": "m.matvec_and_dot(A, b, x)",
+    "dot": "m.dot(b, x)",
+    "spmm": "m.spmm(A, X, X2, 16)",
+    "cg_solve_multi": "m.cg_solve_multi(A, X, X2, 16, max_iter=2)",
+    "batch": "m.Batch([(40, 40, 40), (30, 30, 30)], ctx)",
+}
+
+
+@pytest.mark.parametrize("what", sorted(WORKSPACES))
+def test_workspaces_get_the_kept_memory(stub_lib, what):
+    """Calls whose own allocations fit the device only once the memory kept for
+    matrices and vectors has gone back."""
+    run(stub_lib, f"what, call = {what!r}, {WORKSPACES[what]!r}" + """
+ctx = m.Context(0)
+_, A, b = m.build_problem(40, ctx=ctx)
+x = m.Vector(A.nrows, ctx)
+X, X2 = m.Vector(16 * A.nrows, ctx), m.Vector(16 * A.nrows, ctx)
+m.matvec(A, b, x)                     # A's plan
+m.spmm(A, X, X2, 16, tile=0)
+other = m.Context(0)                  # leaves its memory: half of it is another context's
+stub.stub_capacity(1 << 40)
+for c in (ctx, other):
+    kept = [m.Vector(8 * MB // 8, c) for _ in range(40)]
+    for v in kept: v.close()
+frees = stub.stub_frees()
+stub.stub_capacity(stub.stub_used())  # nothing is left but what is kept
+eval(call)
+assert stub.stub_frees() > frees
+""")
+
+
+def test_trim_memory(stub_lib):
+    """The kept memory of every context goes back when asked for, and only that."""
+    run(stub_lib, """
+c1, c2 = m.Context(0), m.Context(0)
+a = vec(4, c1)
+vec(6, c1).close()
+vec(8, c2).close()
+used = stub.stub_used()
+assert c1.trim_memory() == 14 * MB and stub.stub_used() == used - 14 * MB
+assert c1.trim_memory() == 0 and stub.stub_used() == used - 14 * MB
+a.fill(1.0)
 """)
