@@ -2691,14 +2691,13 @@ static int vecset_prepare(mfe_ctx* ctx, VecSet<T>& v, int64_t n, GraphSlot<T>& g
 }
 
 static int ws_get(mfe_ctx* ctx, int max_iter, CgWorkspace** out) {
+  if (!ctx->cg) ctx->cg = new CgWorkspace();
   CgWorkspace* w = ctx->cg;
-  if (!w) {
-    w = new CgWorkspace();
-    ctx->cg = w;
-    MFE_CHECK(ctx, dev_malloc(ctx, &w->st, 2 * sizeof(CgState)));
-    MFE_CHECK(ctx, hipHostMalloc(&w->h_st, sizeof(CgState), hipHostMallocDefault));
+  // each by itself: an earlier call may have failed at any of them
+  if (!w->st) MFE_CHECK(ctx, dev_malloc(ctx, &w->st, 2 * sizeof(CgState)));
+  if (!w->h_st) MFE_CHECK(ctx, hipHostMalloc(&w->h_st, sizeof(CgState), hipHostMallocDefault));
+  if (!w->h_progress)
     MFE_CHECK(ctx, hipHostMalloc(&w->h_progress, sizeof(*w->h_progress), hipHostMallocCoherent));
-  }
   const int64_t hneed = 4 * (int64_t)(max_iter > 0 ? max_iter : 1);
   if (w->hist_cap < hneed) {
     w->g64.drop();

@@ -250,3 +250,22 @@ assert c1.trim_memory() == 14 * MB and stub.stub_used() == used - 14 * MB
 assert c1.trim_memory() == 0 and stub.stub_used() == used - 14 * MB
 a.fill(1.0)
 """)
+
+
+@pytest.mark.parametrize("nth", [1, 2])
+def test_solve_after_a_failed_workspace(stub_lib, nth):
+    """A solve whose pinned words could not be allocated reports it, and the next
+    one allocates them."""
+    run(stub_lib, f"nth = {nth}" + """
+ctx = m.Context(0)
+_, A, b = m.build_problem(6, ctx=ctx)
+x = m.Vector(A.nrows, ctx)
+m.matvec(A, b, x)
+stub.stub_host_fail(nth)
+try:
+    m.cg_solve(A, b, x, max_iter=2)
+    assert False
+except m.MfeError as e:
+    assert e.status == m.MFE_OOM
+m.cg_solve(A, b, x, max_iter=2)
+""")
