@@ -3457,6 +3457,7 @@ int mfe_cg_solve_mixed_ex(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_
     hipFree(w->f_rhs);
     hipFree(w->f_x);
     w->f_rhs = w->f_x = nullptr;
+    w->f_n = -1;
     w->g32.drop();
     MFE_CHECK(ctx, dev_malloc(ctx, &w->f_rhs, sizeof(float) * (size_t)(n > 0 ? n : 1)));
     MFE_CHECK(ctx, dev_malloc(ctx, &w->f_x, sizeof(float) * (size_t)(n > 0 ? n : 1)));

@@ -269,3 +269,27 @@ except m.MfeError as e:
     assert e.status == m.MFE_OOM
 m.cg_solve(A, b, x, max_iter=2)
 """)
+
+
+def test_mixed_solve_after_a_failed_workspace(stub_lib):
+    """The mixed solve's inner vectors could not grow for a larger system: that
+    solve reports it, and the next one of the first size allocates its own."""
+    run(stub_lib, """
+ctx = m.Context(0)
+def problem(n):
+    _, A, b = m.build_problem(n, ctx=ctx)
+    return A, b, m.Vector(A.nrows, ctx)
+small, large = problem(6), problem(40)
+m.cg_solve_mixed(*small, max_outer=1, max_inner=2, outer_tol=-1.0)
+m.cg_solve(*large, max_iter=2)
+m.matvec_fp32(*large)            # all that the large system needs but the inner vectors
+ctx.trim_memory()
+stub.stub_capacity(stub.stub_used() + 4096)
+try:
+    m.cg_solve_mixed(*large, max_outer=1, max_inner=2)
+    assert False
+except m.MfeError as e:
+    assert e.status == m.MFE_OOM
+stub.stub_capacity(1 << 30)
+m.cg_solve_mixed(*small, max_outer=1, max_inner=2, outer_tol=-1.0)
+""")
