@@ -3,6 +3,8 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <set>
+#include <tuple>
 #include <unordered_map>
 
 #include "mfe_common.hpp"
@@ -36,12 +38,20 @@ struct DevPool {
   std::mutex mu;
   std::unordered_map<void*, size_t> live;      // blocks handed out
   std::map<uint64_t, Block> idle;              // kept blocks by age
+  std::set<std::tuple<mfe_ctx*, size_t, uint64_t>> fit;  // the same by context, bytes, age
   size_t idle_bytes = 0, cap = 0;
   uint64_t clock = 0;
+  // Keeps a block (mu held).
+  void keep(mfe_ctx* ctx, void* p, size_t bytes) {
+    fit.emplace(ctx, bytes, clock);
+    idle[clock++] = Block{p, bytes, ctx};
+    idle_bytes += bytes;
+  }
   // Takes a kept block out (mu held); the caller gives it to release().
   std::map<uint64_t, Block>::iterator take(std::map<uint64_t, Block>::iterator it,
                                            std::vector<void*>& out) {
     out.push_back(it->second.p);
+    fit.erase({it->second.ctx, it->second.bytes, it->first});
     idle_bytes -= it->second.bytes;
     return idle.erase(it);
   }
@@ -93,17 +103,15 @@ hipError_t dev_alloc_bytes(mfe_ctx* ctx, void** out, size_t bytes) {
   const size_t unit = bytes < (size_t(1) << 20) ? 512 : size_t(2) << 20;
   const size_t want = (bytes + unit - 1) / unit * unit;
   std::unique_lock<std::mutex> lock(P->mu);
-  auto best = P->idle.end();  // the smallest kept block of at most 1/8 more
-  for (auto it = P->idle.begin(); it != P->idle.end(); ++it)
-    if (it->second.ctx == ctx && it->second.bytes >= want &&
-        it->second.bytes - want <= want / 8 &&
-        (best == P->idle.end() || it->second.bytes < best->second.bytes))
-      best = it;
-  if (best != P->idle.end()) {
-    *out = best->second.p;
-    P->live[*out] = best->second.bytes;
-    P->idle_bytes -= best->second.bytes;
-    P->idle.erase(best);
+  // the smallest kept block of at most 1/8 more, the oldest of those
+  const auto best = P->fit.lower_bound({ctx, want, 0});
+  if (best != P->fit.end() && std::get<0>(*best) == ctx &&
+      std::get<1>(*best) - want <= want / 8) {
+    std::vector<void*> block;
+    const size_t got = std::get<1>(*best);
+    P->take(P->idle.find(std::get<2>(*best)), block);
+    *out = block[0];
+    P->live[*out] = got;
     return hipSuccess;
   }
   lock.unlock();
@@ -134,8 +142,7 @@ void dev_free(mfe_ctx* ctx, void* p, bool shared) {
         size_t free_b = 0, total = 0;
         if (hipMemGetInfo(&free_b, &total) == hipSuccess) P->cap = total / 8;
       }
-      P->idle[P->clock++] = DevPool::Block{p, bytes, ctx};
-      P->idle_bytes += bytes;
+      P->keep(ctx, p, bytes);
       for (auto old = P->idle.begin(); P->idle_bytes > P->cap && old != P->idle.end();)
         old = P->take(old, gone);
     }

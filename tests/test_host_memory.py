@@ -293,3 +293,39 @@ except m.MfeError as e:
 stub.stub_capacity(1 << 30)
 m.cg_solve_mixed(*small, max_outer=1, max_inner=2, outer_tol=-1.0)
 """)
+
+
+def test_allocating_among_many_kept_blocks(stub_lib):
+    """A thousand allocations that find no block of their size take about as long
+    beside 50,000 kept blocks as beside none (a look at every block takes more than
+    a hundred times as long)."""
+    run(stub_lib, """
+ctx = m.Context(0)
+h = ctypes.c_void_p()
+def seconds():
+    best = 1e9
+    for _ in range(3):
+        t = time.perf_counter()
+        vs = []
+        for _ in range(1000):
+            L.mfe_vec_create(ctx.h, 512, ctypes.byref(h))
+            vs.append(h.value)
+        best = min(best, time.perf_counter() - t)
+        for v in vs: L.mfe_vec_destroy(ctypes.c_void_p(v))
+        ctx.trim_memory()
+    return best
+stub.stub_capacity(1 << 40)
+few = seconds()
+vs = []
+for _ in range(50000):
+    L.mfe_vec_create(ctx.h, 8, ctypes.byref(h))
+    vs.append(h.value)
+for v in vs: L.mfe_vec_destroy(ctypes.c_void_p(v))
+# (not seconds(): it gives the kept blocks back)
+t = time.perf_counter()
+for _ in range(1000):
+    L.mfe_vec_create(ctx.h, 512, ctypes.byref(h))
+many = time.perf_counter() - t
+print(many, few)
+assert many < 5 * few, (many, few)
+""")
