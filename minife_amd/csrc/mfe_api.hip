@@ -1,5 +1,6 @@
 // Context, handle, timer and verification entry points of libminife_hip.so.
 #include <cmath>
+#include <condition_variable>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -36,6 +37,8 @@ struct DevPool {
     mfe_ctx* ctx;
   };
   std::mutex mu;
+  std::condition_variable left;                // leaving became 0
+  size_t leaving = 0;                          // blocks on their way to hipFree
   std::unordered_map<void*, size_t> live;      // blocks handed out
   std::map<uint64_t, Block> idle;              // kept blocks by age
   std::set<std::tuple<mfe_ctx*, size_t, uint64_t>> fit;  // the same by context, bytes, age
@@ -47,7 +50,7 @@ struct DevPool {
     idle[clock++] = Block{p, bytes, ctx};
     idle_bytes += bytes;
   }
-  // Takes a kept block out (mu held); the caller gives it to release().
+  // Takes a kept block out (mu held).
   std::map<uint64_t, Block>::iterator take(std::map<uint64_t, Block>::iterator it,
                                            std::vector<void*>& out) {
     out.push_back(it->second.p);
@@ -55,11 +58,15 @@ struct DevPool {
     idle_bytes -= it->second.bytes;
     return idle.erase(it);
   }
-  // Gives blocks back to the driver, without the mutex: hipFree waits for the
-  // device, other contexts' work included, and their threads go on meanwhile.  No
-  // stream is waited for by name: another thread may be capturing it.
-  static void release(const std::vector<void*>& blocks) {
+  // Gives blocks back to the driver, without the mutex (the caller counted them as
+  // leaving while it held it): hipFree waits for the device, other contexts' work
+  // included, and their threads go on meanwhile.  No stream is waited for by name:
+  // another thread may be capturing it.
+  void release(const std::vector<void*>& blocks) {
     for (void* p : blocks) (void)hipFree(p);
+    std::lock_guard<std::mutex> lock(mu);
+    leaving -= blocks.size();
+    if (leaving == 0) left.notify_all();
   }
 };
 constexpr int kPoolDevices = 64;
@@ -69,7 +76,8 @@ DevPool* pool_of(const mfe_ctx* ctx) {
 }
 }  // namespace
 
-// Gives every block kept on ctx's device back to the driver; their bytes.
+// Gives every block kept on ctx's device back to the driver; their bytes.  On
+// return what other threads were giving back is free too.
 static size_t dev_trim(mfe_ctx* ctx) {
   DevPool* P = pool_of(ctx);
   if (!P) return 0;
@@ -79,8 +87,11 @@ static size_t dev_trim(mfe_ctx* ctx) {
     std::lock_guard<std::mutex> lock(P->mu);
     bytes = P->idle_bytes;
     for (auto it = P->idle.begin(); it != P->idle.end();) it = P->take(it, all);
+    P->leaving += all.size();
   }
-  DevPool::release(all);
+  P->release(all);
+  std::unique_lock<std::mutex> lock(P->mu);
+  P->left.wait(lock, [&] { return P->leaving == 0; });
   return bytes;
 }
 
@@ -88,7 +99,8 @@ hipError_t dev_malloc_bytes(mfe_ctx* ctx, void** out, size_t bytes) {
   hipError_t e = hipMalloc(out, bytes);
   if (e == hipSuccess) return e;
   (void)hipGetLastError();
-  if (dev_trim(ctx) > 0) e = hipMalloc(out, bytes);
+  (void)dev_trim(ctx);
+  e = hipMalloc(out, bytes);  // (also where another thread gave the memory back)
   if (e != hipSuccess) {
     (void)hipGetLastError();  // nothing sticky: the caller decides
     *out = nullptr;
@@ -146,8 +158,9 @@ void dev_free(mfe_ctx* ctx, void* p, bool shared) {
       for (auto old = P->idle.begin(); P->idle_bytes > P->cap && old != P->idle.end();)
         old = P->take(old, gone);
     }
+    P->leaving += gone.size();
   }
-  DevPool::release(gone);
+  P->release(gone);
 }
 
 // The blocks kept for ctx go (its stream has drained).
@@ -159,8 +172,9 @@ static void dev_drop(mfe_ctx* ctx) {
     std::lock_guard<std::mutex> lock(P->mu);
     for (auto it = P->idle.begin(); it != P->idle.end();)
       it = it->second.ctx == ctx ? P->take(it, gone) : std::next(it);
+    P->leaving += gone.size();
   }
-  DevPool::release(gone);
+  P->release(gone);
 }
 
 // Largest non-zero count of any kSpmvRows-row tile: ro[min(r0+R,n)] - ro[r0].

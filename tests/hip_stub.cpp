@@ -4,10 +4,12 @@
 // whether something has been launched on it that nobody has waited for.
 #include <hip/hip_runtime_api.h>
 
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 struct ihipStream_t {
@@ -25,6 +27,7 @@ uint64_t tick = 0;
 std::map<char*, Alloc> live;
 std::vector<ihipStream_t*> streams;
 size_t used = 0, capacity = size_t(1) << 30;
+int free_delay_ms = 0;
 long mallocs = 0, frees = 0, hazards = 0, foreign_waits = 0, capture_breaks = 0, host_fail = 0;
 thread_local ihipStream_t* mine = nullptr;  // the stream of the context this thread works for
 
@@ -58,6 +61,7 @@ extern "C" {
 
 // ---- for the tests -------------------------------------------------------------
 void stub_capacity(size_t bytes) { capacity = bytes; }
+void stub_free_delay(int ms) { free_delay_ms = ms; }
 size_t stub_used() { return used; }
 long stub_mallocs() { return mallocs; }
 long stub_frees() { return frees; }
@@ -108,6 +112,7 @@ hipError_t hipMalloc(void** out, size_t bytes) {
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {  // waits for the whole device
+  if (p && free_delay_ms > 0) std::this_thread::sleep_for(std::chrono::milliseconds(free_delay_ms));
   std::lock_guard<std::recursive_mutex> lock(mu);
   if (!p) return hipSuccess;
   auto it = live.find(static_cast<char*>(p));

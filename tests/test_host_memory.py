@@ -329,3 +329,20 @@ many = time.perf_counter() - t
 print(many, few)
 assert many < 5 * few, (many, few)
 """)
+
+
+def test_allocation_waits_for_memory_that_is_being_given_back(stub_lib):
+    """An allocation that the device has no room for while another thread is still
+    giving kept memory back succeeds once that is done."""
+    run(stub_lib, """
+stub.stub_capacity(512 * MB)
+c1, c2 = m.Context(0), m.Context(0)
+vec(60, c2).close()
+stub.stub_capacity(stub.stub_used() + MB)
+stub.stub_free_delay(500)
+t = threading.Thread(target=c2.trim_memory)
+t.start()
+time.sleep(0.1)
+v = vec(40, c1)
+t.join()
+""")
