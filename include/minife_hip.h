@@ -312,7 +312,8 @@ int mfe_cg_solve_mixed_ex(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* b, mfe_
  * layout applies, 9 and 10 are 1 and 2 on the box layout with all 27 slots
  * stored where the symmetric one applies, 11 and 12 are 1 and 2 on the
  * symmetric layout's full-width values where their packed form is read (for
- * comparison). */
+ * comparison), 13 is 1 on the packed boundary stream, where there is one,
+ * whatever the number of rows (1 reads it from 2^23 rows on). */
 int mfe_time_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y, int variant,
                     int reps, double* avg_ms);
 

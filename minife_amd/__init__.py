@@ -671,7 +671,7 @@ def time_matvec(A: CSRMatrix, x: Vector, y: Vector, variant: int = 1, reps: int 
     on the context's stream); variant 1 is the kernel inside the fast cg_solve,
     variant 2 the FP32 kernel inside cg_solve_mixed, 3 and 4 the same two on
     the CSR kernels whatever A's plan, 6 variant 1 on plain SELL-64 where the
-    plan stages x."""
+    plan stages x, 13 variant 1 on the packed boundary stream whatever the size."""
     ms = ctypes.c_double(0)
     A.ctx.check(lib().mfe_time_matvec(A.ctx.h, A.h, x.h, y.h, int(variant), int(reps),
                                       ctypes.byref(ms)), "time_matvec")

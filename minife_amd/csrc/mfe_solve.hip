@@ -1722,6 +1722,8 @@ int box_prepare(mfe_ctx* ctx, const mfe_csr* Ac) {
   return build_box<double>(ctx, A);
 }
 
+constexpr int64_t kWPackRows = 1 << 23;  // rows from which the packed boundary stream is read
+
 // What one SpMV launch reads: the SELL copy when the plan has one for T,
 // else the CSR arrays (FP64 values, or the CSR FP32 copy).
 template <typename T>
@@ -1752,7 +1754,8 @@ struct SpmvOp {
   int pack = kPackNone;           // the symmetric layout's packed form (a PackForm), if used
   const unsigned* pw = nullptr;   // its words
   const T* pkq = nullptr;         // its (base, power of two) per (block, plane, slot)
-  int wpack = kPackNone;          // the boundary stream's packed form, if used (with pack)
+  int wpack = kPackNone;          // the boundary stream's packed form, if there is one (with pack)
+  int64_t wrows = kWPackRows;     // rows from which it is read
   const unsigned* wpw = nullptr;
   const T* wkq = nullptr;
   BoxGeom bg{};
@@ -1762,7 +1765,7 @@ struct SpmvOp {
   auto tie() const {
     return std::tie(A, gen, n, ro, cols, vals, stream_ok, nslices, soff, slen, scols, svals, xl,
                     xltail, xaff, xsbase, xroff, xrcol, xrpos, xnu, xmaxu, cus, bvals, symu, symw,
-                    symtab, pack, pw, pkq, wpack, wpw, wkq, bg.gx, bg.gy, bg.gz, bg.nbx, bg.nby);
+                    symtab, pack, pw, pkq, wpack, wrows, wpw, wkq, bg.gx, bg.gy, bg.gz, bg.nbx, bg.nby);
   }
 };
 
@@ -2477,8 +2480,6 @@ __global__ __launch_bounds__(kBlock) void cg_p_next_kernel(int64_t n, const CgSt
   }
 }
 
-constexpr int kWPackRows = 1 << 23;  // rows from which the packed boundary stream is read
-
 // y = A x on stream; *tiles_out = the number of partials written (one per
 // 256 rows in the CSR and SELL formats, one per workgroup in the box layout,
 // never more than max(kVecBlocks, one per 256 rows)).
@@ -2512,7 +2513,7 @@ static int launch_spmv(const SpmvOp<T>& op, const T* x, T* y, const T* bvec, T* 
           // and 324 us, 200^3 100 and 100, 128^3 36.6 and 34.2, 64^3 12.4 and
           // 11.0; matvec_std at 300^3 385 and 371).
           if constexpr (!ZERO_Y && std::is_same<T, double>::value)
-            if (op.wpack && n >= kWPackRows) return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, true>);
+            if (op.wpack && n >= op.wrows) return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, true>);
           return run(spmv_boxsym_kernel<T, ZERO_Y, MODE, decltype(pf)::value, false>);
         });
       }
@@ -3271,7 +3272,7 @@ int mfe_matvec_fp32(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y
 
 int mfe_time_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y, int variant,
                     int reps, double* avg_ms) {
-  if (!ctx || !A || !avg_ms || reps <= 0 || variant < 0 || variant > 12) return MFE_BAD_ARG;
+  if (!ctx || !A || !avg_ms || reps <= 0 || variant < 0 || variant > 13) return MFE_BAD_ARG;
   uses(ctx, A);
   int st;
   if ((st = check_vec(ctx, x, A->nrows, "matvec x")) || (st = check_vec(ctx, y, A->nrows, "matvec y")))
@@ -3303,8 +3304,10 @@ int mfe_time_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y
     if (!f32 && !A->box_vals_valid && (st = build_box<double>(ctx, Am))) return st;
     if (f32 && !A->box_vals32_valid && (st = build_box<float>(ctx, Am))) return st;
   }
-  // variant 6: variant 1 on the SELL kernel without the staged x
+  // variant 6: variant 1 on the SELL kernel without the staged x; variant 13:
+  // variant 1 on the packed boundary stream however few rows there are
   SpmvOp<double> op64 = spmv_op<double>(A, !csr_only, variant != 6, !no_box, !no_sym, !no_pack);
+  if (variant == 13) op64.wrows = 0;
   SpmvOp<float> op32 = spmv_op<float>(A, !csr_only, true, !no_box, !no_sym, !no_pack);
   CgWorkspace* w = nullptr;
   if (f32) {
