@@ -340,9 +340,10 @@ int mfe_batch_solve(mfe_ctx* ctx, mfe_batch* batch, int max_iter, double rel_tol
                     double* rel_residual, double* seconds);
 /* seconds[nprob]: each problem's time in the last solve (its first
  * workgroup's wall clock from the first launch to its end); phases[6*nprob]
- * (nullable): that workgroup's seconds in element math, row assembly, x and p
- * updates, SpMVs and r updates, and the rest, in which it waits for the other
- * workgroups' end. */
+ * (nullable): the seconds of that workgroup in its own kernels -- elements
+ * (element math), rows (row assembly), xp_update (x and p updates), spmv,
+ * r_update -- and outside_first_workgroup, the rest: the time in which the
+ * problem's other workgroups and the other problems run, and between launches. */
 int mfe_batch_timing(const mfe_batch* batch, double* seconds, double* phases);
 /* Problem p's assembled operator as CSR (row_offsets[n+1], cols[nnz],
  * vals[nnz]), its right-hand side b[n] and solution x[n]; any may be NULL. */

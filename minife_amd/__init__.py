@@ -782,7 +782,8 @@ class Batch:
         return dict(iters=iters, rel_residual=rel, seconds=sec.value, status=st,
                     problem_seconds=per, phase_seconds=ph)
 
-    PHASES = ("elements", "rows", "p_update", "spmv", "xr_update", "barrier_wait")
+    # phase_seconds' columns: the problem's first workgroup in its own kernels, then the rest
+    PHASES = ("elements", "rows", "xp_update", "spmv", "r_update", "outside_first_workgroup")
 
     def download(self, p: int, matrix: bool = True) -> dict:
         inf = self.info(p)
