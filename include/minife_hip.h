@@ -326,7 +326,10 @@ int mfe_time_matvec(mfe_ctx* ctx, const mfe_csr* A, const mfe_vec* x, mfe_vec* y
  * that are not done in the same launches; each assembled operator is
  * bit-identical to the reference's (generate_matrix_structure +
  * assemble_FE_data + both impose_dirichlet passes, driver.hpp:181-218).  At
- * most two problems per compute unit (else MFE_UNSUPPORTED). */
+ * most two problems per compute unit (else MFE_UNSUPPORTED).
+ * The CG reads the stencil values in an exact packed form where they fit one; with
+ * MINIFE_BATCH_PACK=0 in the environment when the batch is created it reads them at
+ * full width, with the same results (for comparison). */
 int mfe_batch_create(mfe_ctx* ctx, int nprob, const int* dims, mfe_batch** out);
 void mfe_batch_destroy(mfe_batch* batch);
 /* p = -1: {problems, workgroups, total rows, stored SELL entries, total

@@ -21,3 +21,13 @@ def test_batch_phases_are_the_ones_the_header_describes():
     at = [re.search(rf"\b{name}\b", doc) for name in minife_amd.Batch.PHASES]
     assert len(at) == 6 and all(at), list(zip(minife_amd.Batch.PHASES, at))
     assert [a.start() for a in at] == sorted(a.start() for a in at)
+
+
+def test_environment_variables_are_documented():
+    """Every environment variable that the library reads is described in its header."""
+    with open(os.path.join(ROOT, "include", "minife_hip.h")) as f:
+        text = f.read()
+    for name in sorted(os.listdir(CSRC)):
+        with open(os.path.join(CSRC, name)) as f:
+            for var in re.findall(r'getenv\("(\w+)"\)', f.read()):
+                assert var in text, (name, var)
