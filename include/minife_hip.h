@@ -52,7 +52,7 @@ typedef struct mfe_batch mfe_batch;
 /* cg_solve flags */
 #define MFE_CG_REPLAY       0x1u /* sequential dots: reference's exact trajectory */
 #define MFE_CG_TOL_RELATIVE 0x2u /* stop on ||r|| <= tol*||b|| instead of ||r|| <= tol */
-#define MFE_CG_EAGER        0x4u /* launch kernels one by one instead of HIP graphs */
+#define MFE_CG_EAGER        0x4u /* launch kernels one by one, whatever the size, no HIP graphs */
 /* With MFE_CG_EAGER: time as the reference's MINIFE_FUSED build does
  * (cg_solve.hpp:172-175,206-209): each iteration's SpMV and p.Ap sum in
  * MFE_T_MATVECDOT instead of MATVEC + DOT, the breakdown test's norms untimed.
@@ -247,8 +247,8 @@ int mfe_waxpby(mfe_ctx* ctx, double alpha, const mfe_vec* x, double beta, const 
  * MFE_BREAKDOWN (num_iters = last completed k).  times (nullable) receives
  * seconds in the MFE_T_* slots: TOTAL always; WAXPY, DOT and MATVEC (and
  * MATVECDOT with MFE_CG_FUSED) only with MFE_CG_EAGER (GPU time between kernel
- * groups; a HIP graph launch cannot be split, so graph mode leaves them 0).  history (nullable) receives 4 doubles per
- * iteration k (entry k-1): {rtrans, p_ap_dot, alpha, beta}.
+ * groups; otherwise they stay 0: the fused kernels and graph launches cannot be
+ * split).  history (nullable) receives 4 doubles per iteration k (entry k-1): {rtrans, p_ap_dot, alpha, beta}.
  * flags: MFE_CG_REPLAY reproduces the reference's sequential dot products and
  * hence its scalar trajectory bit for bit; the default fast mode uses tree
  * reductions (deterministic, not bit-identical to the serial sum). */

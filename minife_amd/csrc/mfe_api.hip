@@ -27,7 +27,9 @@ int hip_fail(mfe_ctx* ctx, hipError_t e, const char* what) {
 // A new matrix of 300^3 takes 14 GB with its plan.  Allocating and freeing that
 // for every matrix of a parameter study costs more than assembling it: memory
 // given back to the driver is cleared before it is handed out again (assembly
-// and first product at 300^3: 371 ms, of which 18 in kernels).
+// and first product at 300^3: 371 ms, of which 18 in kernels at the time; with
+// kept memory and 11 ms of kernels 11.4).  A process's first matrix is not helped
+// by it: 14.6 ms, in memory that the driver had ready.
 
 namespace {
 struct DevPool {

@@ -83,7 +83,8 @@ __host__ __device__ constexpr int fuse_a(int m, int n) { return n < 4 ? tri4(m, 
 // per 64 elements, 57% of the issue slots) and the waits of two waves per SIMD:
 // element loop at 300^3 5.73 ms with the Gauss tables read through the scalar
 // cache and every Jacobian entry used, 5.12 with constant tables, 4.96 without
-// the entries that are zero.  (Three workgroups per CU, 168 registers and 224
+// the entries that are zero (into memory that was written before; the first time
+// 6.2-6.6 ms, so 5.6-5.8).  (Three workgroups per CU, 168 registers and 224
 // bytes of scratch: 7.27.)
 template <bool ZERO_START>
 // (launch bounds: two workgroups per CU, which the 60 KB of LDS allow, so at

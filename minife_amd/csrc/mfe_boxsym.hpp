@@ -7,20 +7,19 @@
 // Each row stores only its 14 upper slots s = 13..26 (the diagonal, the
 // same-plane neighbours after it, the next plane's nine), 256 rows per
 // (block, plane, slot) as in the box layout.  Lower slot s of row r is
-// upper slot 26 - s of the neighbour r + off(s), which the workgroup holds in
-// LDS: the previous plane's nine upper-plane slots and the current plane's
-// four same-plane upper slots, for the block's 16 x 16 nodes plus the ring
-// around it.  The block's own entries go to LDS as the rows are loaded; a
-// lower value whose neighbour lies outside the block comes from a second
-// stream of kSymNB values per (block, plane) -- the row's own CSR entry --
-// which is written into the ring cell the row reads.  About 15 values per
-// row instead of 27; every row's products are still added in ascending slot
-// order over its in-range slots, so y has the bits of matvec_std.
+// upper slot 26 - s of the neighbour r + off(s).  A neighbour in the block forms
+// the product with its own x entry and leaves it in LDS for row r; a lower
+// value whose neighbour lies outside the block comes from a second stream of
+// kSymNB values per (block, plane) -- the row's own CSR entry -- and the thread
+// that loads it leaves its product with the ring's x entry in the same place.
+// About 15 values per row instead of 27; every row's products are still added in
+// ascending slot order over its in-range slots, so y has the bits of matvec_std.
 //
-// The LDS arrays are indexed by the reading row: up[j][t] holds the value row
-// t reads for its lower slot whose neighbour's mirrored slot is j (written by
-// that neighbour, or from the boundary stream), so every read is stride-1
-// and the arrays hold 256 entries per slot (34 KB in all for FP64: four
+// The LDS arrays are indexed by the reading row: up[j][t] and sm[i][t] hold the
+// product row t adds for the lower slot whose mirrored slot is 18 + j of the plane
+// before (its own column's stays in a register) or 14 + i of the same plane, so
+// every read is stride-1 and the arrays hold 256 entries per slot (32 KB with the
+// three planes of x for FP64, a little more with the packed boundary stream: four
 // workgroups per CU).
 #pragma once
 

@@ -139,8 +139,9 @@ struct mfe_csr {
   // The packed form of the symmetric layout's upper values (mfe_boxsym.hpp),
   // per precision: boxpack_form (a PackForm; kPackNone: the SpMV reads the
   // full values), the packed words (boxpack_cap words per row allocated), and
-  // per (block, plane, slot) the base and the power of two of the offsets,
-  // side by side (boxpack_kq[2 * group], boxpack_kq[2 * group + 1]).
+  // a record of kSymKRec values per (block, plane) (SymRec: the slots' bases,
+  // then their powers of two and the codes flag as 32-bit words; until the
+  // packing each slot's greatest multiple and power of two, side by side).
   bool boxpack_valid = false, boxpack32_valid = false;
   // Per field width (mfe_pack.hpp's kPackWidths), the upper slots (and the FP64
   // boundary stream's lower slots) whose every group fits it, found while the

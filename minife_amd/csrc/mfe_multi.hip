@@ -569,8 +569,9 @@ __global__ __launch_bounds__(kBlock) void spmm_sell_kernel(
 // p), of plane p (slots 9-17) and of plane p-1 (slots 18-26, after which that
 // row is complete and stored).  Each row still adds its in-range products in
 // ascending slot order from 0.0: per column, the bits of the single-vector
-// SpMV.  The values are loaded one group of 9 slots at a time (every lane of a
-// node loads them; one fetch per wave and address).  Partials: the dot of
+// SpMV.  A step goes line by line: three slots of each of the three rows, whose
+// nine values are loaded one line ahead (every lane of a node loads them; one fetch
+// per wave and address).  Partials: the dot of
 // each completed row with X of its own node (held from the step that had that
 // plane in LDS), per thread over its planes in order, then over the rows of
 // the workgroup.  XCD: workgroup i runs on XCD i % 8, and each XCD takes a
@@ -638,8 +639,6 @@ __device__ __forceinline__ void spmm_boxp_body(int wg, int nwg, BoxGeom g, int n
       if (e < MW * K) win[buf][e] = xr[k];
     }
   };
-  const int lox = ix > 0 ? -1 : 0, hix = ix < g.gx - 1 ? 1 : 0;
-  const int loy = iy > 0 ? -1 : 0, hiy = iy < g.gy - 1 ? 1 : 0;
   const int c0 = (ty + 1) * WX + (tx + 1);
   double tsum[CPL], accA[CPL], accB[CPL], accC[CPL], xown[CPL];
 #pragma unroll

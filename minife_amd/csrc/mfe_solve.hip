@@ -7,10 +7,11 @@
 // That is exactly matvec_std's arithmetic (SparseMatrix_functions.hpp:566-572)
 // with HBM traffic of one pass over vals/cols.  No MFMA: the operator is sparse.
 //
-// CG: one HIP stream, device-resident scalars, fused kernels, and chunks of
-// iterations captured in a HIP graph and replayed; every kernel first checks a
-// device "done" flag so the reference's data-dependent loop test
-// (cg_solve.hpp:152) stops the work without host round trips.  The kernels are
+// CG: one HIP stream, device-resident scalars and fused kernels, launched one by
+// one behind the GPU's progress word (small systems) or in chunks of iterations
+// captured in a HIP graph and replayed; every kernel checks a device "done" flag so
+// the reference's data-dependent loop test (cg_solve.hpp:152) stops the work
+// without host round trips.  The kernels are
 // templated on the vector type: double for cg_solve, float for the inner solve
 // of the mixed-precision refinement.
 #include <algorithm>
@@ -898,8 +899,12 @@ void box_chunks(BoxGeom& g, int resident, int64_t cap) {
 // format (precision, packed form, packed boundary stream) and is not asked of the
 // occupancy query, whose answer follows the compiler's register allocation and
 // would move the sums with it (and which counts no scalar registers: with the
-// plane record in about 100 of them a SIMD holds at most six waves.  FP32 at
-// 200^3 in chunks for five per CU 71.3 us, six 67.8, seven 83.3).
+// plane record in about 100 of them a SIMD holds at most six waves).  They are the
+// chunks that the sums had before the products were handed over, not the fastest
+// ones: FP32 all12 at 200^3 takes 71.3 us in chunks for five per CU, 67.8 for six,
+// 83.3 for seven, but with other groups a mixed solve to 1e-11 there ended 1.0e-9
+// (two of its own runs: 4e-10) from the x it had given.  The figure of the packed
+// boundary stream also holds below kWPackRows, where the boundary is read in full.
 static int sym_slots(bool f64, int pack, bool wpack, int cus) {
   const bool wide = pack == kPackAll16 || pack == kPackCube16Near32 || pack == kPackCube16;
   int per = f64 ? (wpack && wide ? 3 : 4)
@@ -947,8 +952,6 @@ __global__ __launch_bounds__(kBlock) void box_fill_kernel(BoxGeom g, const int* 
       }
 }
 
-// The box layout of A's values as T (synchronises nothing; on the stream).
-// Returns MFE_OK with the layout absent when it does not fit in memory.
 // Sets A->box_geom for A's current box, freeing the layouts (and forgetting
 // the symmetry check) when it changes.  Every builder below relies on it.
 static void box_set_geometry(mfe_csr* A) {
@@ -960,6 +963,8 @@ static void box_set_geometry(mfe_csr* A) {
   }
 }
 
+// The box layout of A's values as T (synchronises nothing; on the stream).
+// Returns MFE_OK with the layout absent when it does not fit in memory.
 template <typename T>
 static int build_box(mfe_ctx* ctx, mfe_csr* A) {
   const BoxGeom g = A->box_geom;
@@ -1722,7 +1727,8 @@ int box_prepare(mfe_ctx* ctx, const mfe_csr* Ac) {
   return build_box<double>(ctx, A);
 }
 
-constexpr int64_t kWPackRows = 1 << 23;  // rows from which the packed boundary stream is read
+// Rows from which the packed boundary stream is read (measured at launch_spmv).
+constexpr int64_t kWPackRows = 1 << 23;
 
 // What one SpMV launch reads: the SELL copy when the plan has one for T,
 // else the CSR arrays (FP64 values, or the CSR FP32 copy).
