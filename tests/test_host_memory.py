@@ -302,30 +302,20 @@ def test_allocating_among_many_kept_blocks(stub_lib):
     run(stub_lib, """
 ctx = m.Context(0)
 h = ctypes.c_void_p()
+def create(doubles):
+    L.mfe_vec_create(ctx.h, doubles, ctypes.byref(h))
+    return ctypes.c_void_p(h.value)
 def seconds():
     best = 1e9
-    for _ in range(3):
+    for _ in range(5):
         t = time.perf_counter()
-        vs = []
-        for _ in range(1000):
-            L.mfe_vec_create(ctx.h, 512, ctypes.byref(h))
-            vs.append(h.value)
+        for _ in range(1000): create(512)   # (never destroyed: nothing to find)
         best = min(best, time.perf_counter() - t)
-        for v in vs: L.mfe_vec_destroy(ctypes.c_void_p(v))
-        ctx.trim_memory()
     return best
 stub.stub_capacity(1 << 40)
 few = seconds()
-vs = []
-for _ in range(50000):
-    L.mfe_vec_create(ctx.h, 8, ctypes.byref(h))
-    vs.append(h.value)
-for v in vs: L.mfe_vec_destroy(ctypes.c_void_p(v))
-# (not seconds(): it gives the kept blocks back)
-t = time.perf_counter()
-for _ in range(1000):
-    L.mfe_vec_create(ctx.h, 512, ctypes.byref(h))
-many = time.perf_counter() - t
+for v in [create(8) for _ in range(50000)]: L.mfe_vec_destroy(v)
+many = seconds()
 print(many, few)
 assert many < 5 * few, (many, few)
 """)
